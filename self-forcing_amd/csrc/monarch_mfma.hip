@@ -364,20 +364,40 @@ struct S2Lds {
     static constexpr int kPitch = 2 * D, kTile = 32 * kPitch;
     static constexpr int kWave = 2 * kTile + 512;
     static __host__ __device__ constexpr size_t bytes() { return 4 * (size_t)kWave; }
+    // a team of waves on one column: two chunks of each matrix, and two cl buffers per wave
+    static __host__ __device__ constexpr size_t team_bytes(int waves) { return 4 * (size_t)kTile + waves * 512; }
 };
 
 __device__ __forceinline__ void s2_load_lds4(const char* base, uint32_t off, uint32_t lds_addr) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds_addr), "v"(off), "s"(base) : "memory", "m0");
 }
+// waits until at most N of the wave's vector memory operations are outstanding
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
 
-// The four waves of a workgroup share nothing: each streams the rows of its own (a, j) through its own part of LDS
-// (global_load_lds_dwordx4, 1 KB contiguous per instruction, requested as soon as the buffer's last reader is done) and
-// synchronises with its own loads only (vector memory operations complete in order, so waiting until only the loads
-// issued after a tile's are outstanding means that tile has landed).
-template <class E, int D>
-__global__ __launch_bounds__(256) void monarch_step2_kernel(MonarchArgs p) {
+// The step is bound by reading the Kbar / Y rows once (604 MB at the 480p chunk shape), so a column's rows are loaded by one
+// workgroup whatever the number of its query rows; a wave holds 32 of them (O^T and the query operand are 96 registers):
+//   TEAM = 1 (b1 <= 32): a wave per column (a, j), four to a workgroup that share nothing: each streams its column's rows
+//       through its own part of LDS (global_load_lds_dwordx4, 1 KB contiguous per instruction) and waits for its own loads
+//       only (vector memory operations complete in order, so when only the loads issued after a tile's are outstanding,
+//       that tile has landed).
+//   TEAM = 2..4 (b1 <= 128 per grid slice): a workgroup of TEAM waves per column; each loads its share of a chunk, two
+//       buffers per matrix, one barrier before the logits and one before the output products.  (A pass over the rows for
+//       every 32 query rows, as before, took 518 us at the 720p grid, b1 = 45, and 96 us at three frames tied, b1 = 90;
+//       this form 299 and 70.  Two query tiles in one wave need 290 registers and spill.)
+// split (TEAM = 1): 1, 2 or 4 waves of a workgroup share a column's rows, 32-row chunks dealt in turn, and merge (maximum,
+// sum, output) through LDS at the end: with few (a, j) columns the chip is otherwise idle and a wave's chain of dependent
+// chunks (about 2.5 us each) is the whole time.
+template <class E, int D, int TEAM>
+__global__ __launch_bounds__(TEAM == 1 ? 256 : 64 * TEAM) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void monarch_step2_kernel(MonarchArgs p) {
     using L = S2Lds<D>;
     constexpr int DS = D / 16, DT = D / 32, CPR = D / 8;
+    constexpr int NG = CPR / 2;                            // 1 KB pieces of a chunk
+    constexpr int MYG = (NG + TEAM - 1) / TEAM;            // pieces a wave loads (a team of three loads the last ones twice)
+    constexpr bool SOLO = TEAM == 1;
     extern __shared__ __attribute__((aligned(256))) char lds_s2[];
 
     const int tid = threadIdx.x;
@@ -387,15 +407,18 @@ __global__ __launch_bounds__(256) void monarch_step2_kernel(MonarchArgs p) {
     const int hf = lane >> 5;
 
     const int b2 = p.b2;
-    const int njg = (b2 + 3) / 4;
+    const int split = SOLO ? p.s2_split : 1;
+    const int per_wg = SOLO ? 4 / split : 1;               // columns of a workgroup
+    const int sp = SOLO ? wave & (split - 1) : 0;
+    const int njg = (b2 + per_wg - 1) / per_wg;
     const int a = blockIdx.x / njg;
-    const int jraw = (blockIdx.x % njg) * 4 + wave;
+    const int jraw = (blockIdx.x % njg) * per_wg + (SOLO ? wave / split : 0);
     const bool j_ok = jraw < b2;
     const int j = j_ok ? jraw : b2 - 1;
     const int ul = blockIdx.y;
     const int unit = p.unit0 + ul;
     const int b = unit / p.H, h = unit % p.H;
-    const int i0 = blockIdx.z * 32;
+    const int i0 = SOLO ? 0 : blockIdx.z * 128 + wave * 32;
 
     const int f_lim = p.causal ? min(p.nf, (a / p.causal + 1) * p.causal) : p.nf;
     const int r_lim = f_lim * p.b1;
@@ -407,8 +430,10 @@ __global__ __launch_bounds__(256) void monarch_step2_kernel(MonarchArgs p) {
     const char* clp = (const char*)(p.cl + (int64_t)ul * p.cl_unit + (int64_t)(a * b2 + j) * p.cl_aj);
     const uint32_t cl_ld = p.cl_row * 4;                  // bytes between the cl values of consecutive rows
 
-    char* const wl = lds_s2 + wave * L::kWave;
+    char* const wl = lds_s2 + (SOLO ? wave * L::kWave : 0);
+    char* const cll = SOLO ? wl + 2 * L::kTile : lds_s2 + 4 * L::kTile + wave * 512;      // this wave's two cl buffers
     const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)wl;
+    const uint32_t cl0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)cll;
 
     // logits operand (B): this lane's query row Q[a, i0 + m, j, :] (zero past b1)
     u32x4 qb[DS];
@@ -443,39 +468,46 @@ __global__ __launch_bounds__(256) void monarch_step2_kernel(MonarchArgs p) {
 
     const float sc2 = p.scale * kLog2e;
     const f32x16 kZero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    f32x16 oacc[DT];               // O^T[d = 32 dt + 8 g + 4 hf + e, i = m]
+    f32x16 oacc[DT];               // O^T[d = 32 dt + 8 g + 4 hf + e, i = i0 + m]
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) oacc[dt] = kZero;
     float mrun = -INFINITY, lrun = 0.f;
 
-    auto issue_k = [&](int n) {
+    auto issue = [&](const char* mat, int n, uint32_t dst) {
 #pragma unroll
-        for (int g = 0; g < CPR / 2; ++g) {
+        for (int g0 = 0; g0 < MYG; ++g0) {
+            const int g = SOLO ? g0 : min(wave * MYG + g0, NG - 1);
             const int P = g * 64 + lane;
             const int r = P / CPR, c = (P % CPR) ^ s1_swz<CPR>(r);
             const uint32_t off = (uint32_t)min(32 * n + r, r_lim - 1) * (2 * D) + (uint32_t)c * 16;
-            s1_load_lds16(kb, off, lds0 + (uint32_t)g * 1024);
-        }
-        s2_load_lds4(clp, (uint32_t)(32 * n + m) * cl_ld, lds0 + 2 * L::kTile + (uint32_t)(n & 1) * 256);   // lanes >= 32 repeat
-    };
-    auto issue_y = [&](int n) {
-#pragma unroll
-        for (int g = 0; g < CPR / 2; ++g) {
-            const int P = g * 64 + lane;
-            const int r = P / CPR, c = (P % CPR) ^ s1_swz<CPR>(r);
-            const uint32_t off = (uint32_t)min(32 * n + r, r_lim - 1) * (2 * D) + (uint32_t)c * 16;
-            s1_load_lds16(yb, off, lds0 + L::kTile + (uint32_t)g * 1024);
+            s1_load_lds16(mat, off, dst + (uint32_t)g * 1024);
         }
     };
-    issue_k(0);
-    issue_y(0);
-    for (int n = 0; n < nch; ++n) {
+    // buffers of the chunk at position `it` of this wave's sequence: a team alternates between two pairs
+    auto buf = [&](int it) { return SOLO ? 0u : (uint32_t)(it & 1) * 2 * L::kTile; };
+    auto issue_k = [&](int n, int it) {
+        issue(kb, n, lds0 + buf(it));
+        s2_load_lds4(clp, (uint32_t)(32 * n + m) * cl_ld, cl0 + (uint32_t)(it & 1) * 256);   // lanes >= 32 repeat
+    };
+    auto issue_y = [&](int n, int it) { issue(yb, n, lds0 + buf(it) + L::kTile); };
+    if (sp < nch) {
+        issue_k(sp, 0);
+        issue_y(sp, 0);
+    }
+    for (int n = sp, it = 0; n < nch; n += split, ++it) {
+        const bool more = n + split < nch;
         // Kbar and cl of chunk n have landed when only the Y loads issued after them are outstanding
-        if (D == 128) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-        const char* kt = wl;
-        const char* yt = wl + L::kTile;
-        const char* clt = wl + 2 * L::kTile + (n & 1) * 256;
+        wait_vm<MYG>();
+        if (!SOLO) {
+            lds_barrier();         // every wave's share is there, and every wave is done with the chunk before
+            if (more) {
+                issue_k(n + 1, it + 1);
+                issue_y(n + 1, it + 1);
+            }
+        }
+        const char* kt = wl + buf(it);
+        const char* yt = kt + L::kTile;
+        const char* clt = cll + (it & 1) * 256;
 
         f32x16 s;
 #pragma unroll
@@ -486,8 +518,10 @@ __global__ __launch_bounds__(256) void monarch_step2_kernel(MonarchArgs p) {
         f32x4 cc[4];
 #pragma unroll
         for (int g = 0; g < 4; ++g) cc[g] = *(const f32x4*)(clt + (8 * g + 4 * hf) * 4);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // the Kbar tile has been read: the next chunk's may land on it
-        if (n + 1 < nch) issue_k(n + 1);
+        if (SOLO) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // the Kbar tile has been read: the next chunk's may land on it
+            if (more) issue_k(n + split, it + 1);
+        }
 
         float mx = -INFINITY;
 #pragma unroll
@@ -517,13 +551,10 @@ __global__ __launch_bounds__(256) void monarch_step2_kernel(MonarchArgs p) {
             pb[st].z = pack2<E>(s[8 * st + 4], s[8 * st + 5]);
             pb[st].w = pack2<E>(s[8 * st + 6], s[8 * st + 7]);
         }
-        // Y of chunk n has landed when only the Kbar / cl loads of chunk n + 1 are outstanding
-        if (n + 1 < nch) {
-            if (D == 128) asm volatile("s_waitcnt vmcnt(9)" ::: "memory");
-            else asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
-        } else {
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        }
+        // Y of chunk n has landed when only the loads issued after it are outstanding
+        if (more) wait_vm<SOLO ? MYG + 1 : 2 * MYG + 1>();
+        else wait_vm<0>();
+        if (!SOLO) lds_barrier();
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
 #pragma unroll
@@ -536,33 +567,78 @@ __global__ __launch_bounds__(256) void monarch_step2_kernel(MonarchArgs p) {
                 oacc[dt] = E::mfma32(ay, pb[st], oacc[dt]);
             }
         }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // the Y tile has been read
-        if (n + 1 < nch) issue_y(n + 1);
+        if (SOLO) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // the Y tile has been read
+            if (more) issue_y(n + split, it + 1);
+        }
     }
 
-    // epilogue: O[i, d] = O^T / l, turned through the wave's LDS (the operand buffers are dead: every load has landed)
-    const float ltot = xhalf_sum(lrun);
-    const float inv = 1.f / ltot;
-    if (p.stats != nullptr && hf == 0 && j_ok && i0 + m < p.b1)
-        p.stats[((int64_t)unit * (p.na * b2) + a * b2 + j) * p.stats_ld + i0 + m] = mrun + log2f(ltot);
+    // epilogue: O[i, d] = O^T / l, turned through LDS (the operand buffers are dead: every load has landed)
+    uint16_t* const og = (uint16_t*)p.out + (int64_t)b * p.os[0] + (int64_t)h * p.os[2];
+    float* const stats = p.stats ? p.stats + ((int64_t)unit * (p.na * b2) + a * b2 + j) * p.stats_ld : nullptr;
+    float ltot = xhalf_sum(lrun);
+    if (split == 1) {
+        if (!SOLO) lds_barrier();
+        char* const ol = SOLO ? wl : lds_s2 + wave * L::kTile;
+        const float inv = 1.f / ltot;
+        if (stats && hf == 0 && j_ok && i0 + m < p.b1) stats[i0 + m] = mrun + log2f(ltot);
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
+        for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            u32x2 w;
-            w.x = pack2<E>(oacc[dt][4 * g + 0] * inv, oacc[dt][4 * g + 1] * inv);
-            w.y = pack2<E>(oacc[dt][4 * g + 2] * inv, oacc[dt][4 * g + 3] * inv);
-            *(u32x2*)(wl + m * L::kPitch + (32 * dt + 8 * g + 4 * hf) * 2) = w;
-        }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    {
-        uint16_t* og = (uint16_t*)p.out + (int64_t)b * p.os[0] + (int64_t)h * p.os[2];
+            for (int g = 0; g < 4; ++g) {
+                u32x2 w;
+                w.x = pack2<E>(oacc[dt][4 * g + 0] * inv, oacc[dt][4 * g + 1] * inv);
+                w.y = pack2<E>(oacc[dt][4 * g + 2] * inv, oacc[dt][4 * g + 3] * inv);
+                *(u32x2*)(ol + m * L::kPitch + (32 * dt + 8 * g + 4 * hf) * 2) = w;
+            }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         for (int c = lane; c < 32 * CPR; c += 64) {
-            int r = c / CPR, ch = c % CPR;
-            int i = i0 + r;
+            const int r = c / CPR, ch = c % CPR;
+            const int i = i0 + r;
             if (i < p.b1 && j_ok) {
-                u32x4 w = *(const u32x4*)(wl + r * L::kPitch + ch * 16);
+                const u32x4 w = *(const u32x4*)(ol + r * L::kPitch + ch * 16);
                 *(u32x4*)(og + (p.qmap.row(a, i) + j) * p.os[1] + ch * 8) = w;
+            }
+        }
+        return;
+    }
+    if constexpr (SOLO) {
+        // merge of the `split` waves of a column: statistics through the (dead) cl buffers, outputs through the waves' tile
+        // buffers as fp32 rows of 4 D bytes, 16-byte pieces XOR-ed with the row
+        char* const col = lds_s2 + (wave - sp) * L::kWave;                // the column's first wave
+        if (hf == 0) {
+            *(float*)(cll + m * 4) = mrun;
+            *(float*)(cll + 128 + m * 4) = ltot;
+        }
+        lds_barrier();
+        float M = -INFINITY, sum = 0.f;
+        for (int w = 0; w < split; ++w) M = fmaxf(M, *(const float*)(col + w * L::kWave + 2 * L::kTile + m * 4));
+        for (int w = 0; w < split; ++w) {
+            const char* c = col + w * L::kWave + 2 * L::kTile + m * 4;
+            sum += *(const float*)(c + 128) * exp2f(*(const float*)c - M);           // a wave without chunks: 0 * exp2(-inf)
+        }
+        const float fac = exp2f(mrun - M) / sum;
+        if (stats && sp == 0 && hf == 0 && j_ok && m < p.b1) stats[m] = M + log2f(sum);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const f32x4 w = {oacc[dt][4 * g + 0] * fac, oacc[dt][4 * g + 1] * fac, oacc[dt][4 * g + 2] * fac, oacc[dt][4 * g + 3] * fac};
+                *(f32x4*)(wl + m * (4 * D) + (((8 * dt + 2 * g + hf) ^ m) & (D / 4 - 1)) * 16) = w;
+            }
+        lds_barrier();
+        const int rows = 32 / split;                                      // this wave's share of the rows
+        for (int c = lane; c < rows * CPR; c += 64) {
+            const int r = sp * rows + c / CPR, ch = c % CPR;
+            f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;
+            for (int w = 0; w < split; ++w) {
+                const char* row = col + w * L::kWave + r * (4 * D);
+                lo += *(const f32x4*)(row + (((2 * ch) ^ r) & (D / 4 - 1)) * 16);
+                hi += *(const f32x4*)(row + (((2 * ch + 1) ^ r) & (D / 4 - 1)) * 16);
+            }
+            if (r < p.b1 && j_ok) {
+                const u32x4 w = {pack2<E>(lo.x, lo.y), pack2<E>(lo.z, lo.w), pack2<E>(hi.x, hi.y), pack2<E>(hi.z, hi.w)};
+                *(u32x4*)(og + (p.qmap.row(a, r) + j) * p.os[1] + ch * 8) = w;
             }
         }
     }
@@ -828,6 +904,42 @@ static int enqueue_step1(const MonarchArgs& a, int nunits, hipStream_t stream, c
     return SFM_OK;
 }
 
+// Enqueues step 2: a wave per column (a, j) of up to 32 query rows, a team of waves for more.
+template <class E, int D>
+static int enqueue_step2(const MonarchArgs& a, int nunits, hipStream_t stream) {
+    const int team = a.b1 > 96 ? 4 : (a.b1 + 31) / 32;
+    const void* fn = team == 4 ? (const void*)monarch_step2_kernel<E, D, 4> : team == 3 ? (const void*)monarch_step2_kernel<E, D, 3>
+                   : team == 2 ? (const void*)monarch_step2_kernel<E, D, 2> : (const void*)monarch_step2_kernel<E, D, 1>;
+    const size_t lds = team > 1 ? S2Lds<D>::team_bytes(team) : S2Lds<D>::bytes();
+    MonarchArgs a2 = a;
+    a2.s2_split = 1;
+    if (team == 1) {
+        // Up to two columns per compute unit leave most SIMDs idle and four waves share each: 21 cached frames of 480p against
+        // one head 60.5 -> 41.9 us for the whole call, 2 heads 75.7 -> 65.4, 8 heads and one query frame (416 columns) 117 ->
+        // 108; at 624 columns (4 heads) sharing by two or four loses 2 %.  The rule looks at all units of the call, not at
+        // those of this pass, so that the results do not depend on how a call is cut into passes.
+        const int64_t columns = (int64_t)a.B * a.H * a.na * a.b2;
+        const int nch = (a.nf * a.b1 + 31) / 32;
+        if (columns <= 2 * (int64_t)cu_count()) a2.s2_split = nch >= 8 ? 4 : nch >= 4 ? 2 : 1;
+    }
+    const int per_wg = team > 1 ? 1 : 4 / a2.s2_split;
+    if (lds > 64 * 1024) {
+        hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) {
+            set_error("hipFuncSetAttribute failed: %s", hipGetErrorString(e));
+            return SFM_ERR_HIP;
+        }
+    }
+    const dim3 grid(a.na * ((a.b2 + per_wg - 1) / per_wg), nunits, team > 1 ? (a.b1 + 127) / 128 : 1);
+    void* args[] = {&a2};
+    hipError_t e = hipLaunchKernel(fn, grid, dim3(team > 1 ? 64 * team : 256), args, lds, stream);
+    if (e != hipSuccess) {
+        set_error("hip launch failed: %s", hipGetErrorString(e));
+        return SFM_ERR_HIP;
+    }
+    return SFM_OK;
+}
+
 template <class E, int D>
 static int launch_t(const MonarchArgs& a, int nunits, hipStream_t stream, const StepEvents* ev) {
     if (ev) (void)hipEventRecord(ev->ev[0], stream);
@@ -835,17 +947,7 @@ static int launch_t(const MonarchArgs& a, int nunits, hipStream_t stream, const 
     a0.rb = nullptr;
     if (int rc = enqueue_step1<E, D>(a0, nunits, stream)) return rc;
     if (ev) (void)hipEventRecord(ev->ev[1], stream);
-    const int njg = (a.b2 + 3) / 4;
-    dim3 g2(a.na * njg, nunits, (a.b1 + 31) / 32);
-    {
-        hipError_t e = hipFuncSetAttribute((const void*)monarch_step2_kernel<E, D>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)S2Lds<D>::bytes());
-        if (e != hipSuccess) {
-            set_error("hipFuncSetAttribute failed: %s", hipGetErrorString(e));
-            return SFM_ERR_HIP;
-        }
-    }
-    hipLaunchKernelGGL((monarch_step2_kernel<E, D>), g2, dim3(256), S2Lds<D>::bytes(), stream, a);
+    if (int rc = enqueue_step2<E, D>(a, nunits, stream)) return rc;
     if (ev) (void)hipEventRecord(ev->ev[2], stream);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) {
@@ -887,19 +989,12 @@ static int launch_rep_t(const MonarchArgs& a, int nunits, hipStream_t stream) {
 // pass's step 2 writes the output (the earlier ones write it too: it is overwritten).
 template <class E, int D>
 static int launch_iter_t(const MonarchArgs& a, int nunits, int num_iters, hipStream_t stream) {
-    const int njg = (a.b2 + 3) / 4;
     const int nq = (a.b1 + 31) / 32;
-    const dim3 g2(a.na * njg, nunits, nq);
     const int nt = (a.b2 + 31) / 32;
     const void* fn1 = nt == 4 ? (const void*)monarch_step1_kernel<E, D, 4, false, true>
                     : nt == 3 ? (const void*)monarch_step1_kernel<E, D, 3, false, true>
                     : nt == 2 ? (const void*)monarch_step1_kernel<E, D, 2, false, true>
                               : (const void*)monarch_step1_kernel<E, D, 1, false, true>;
-    hipError_t e = hipFuncSetAttribute((const void*)monarch_step2_kernel<E, D>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S2Lds<D>::bytes());
-    if (e != hipSuccess) {
-        set_error("hipFuncSetAttribute failed: %s", hipGetErrorString(e));
-        return SFM_ERR_HIP;
-    }
     for (int it = 0; it < num_iters; ++it) {
         const bool last = it + 1 == num_iters;
         MonarchArgs a1 = a;
@@ -908,14 +1003,14 @@ static int launch_iter_t(const MonarchArgs& a, int nunits, int num_iters, hipStr
         if (int rc = enqueue_step1<E, D>(a1, nunits, stream, fn1)) return rc;
         MonarchArgs a2 = a;
         if (last) a2.stats = nullptr;
-        hipLaunchKernelGGL((monarch_step2_kernel<E, D>), g2, dim3(256), S2Lds<D>::bytes(), stream, a2);
+        if (int rc = enqueue_step2<E, D>(a2, nunits, stream)) return rc;
         if (!last) {
             const int rc = nq == 1 ? launch_rep_t<E, D, 1>(a, nunits, stream) : nq == 2 ? launch_rep_t<E, D, 2>(a, nunits, stream)
                          : nq == 3 ? launch_rep_t<E, D, 3>(a, nunits, stream) : launch_rep_t<E, D, 4>(a, nunits, stream);
             if (rc) return rc;
         }
     }
-    e = hipGetLastError();
+    const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         set_error("hip launch failed: %s", hipGetErrorString(e));
         return SFM_ERR_HIP;

@@ -171,6 +171,7 @@ struct MonarchArgs {
     int n_achunks;
     int s1_wgs;      // step-1 workgroups, 0 = one per CU (tuning override)
     int s1_groups;   // wave groups per step-1 workgroup
+    int s2_split;    // step-2 waves that share the rows of one (a, j) column: 1, 2 or 4
     int s1_total;    // step-1 work items: (unit, k, a-chunk, f) tiles
 };
 
