@@ -62,7 +62,9 @@ struct S1Lds {
 // IT: a pass of the iterated refinement (wan/modules/monarch_attn.py:1716-1722): the logits are scaled per (a, f, k, j)
 //     column and, after the first pass, the query operand of tile (f, k) is the column's representative p.rep[a, j, (f, k)]
 //     instead of Q[a, k, j]; the operand is then fetched for every tile.
-template <class E, int D, int NT, bool WR = false, bool IT = false>
+// KO: Kbar and cl only.  Every refinement pass but the last needs nothing of V: a pass of the refinement at three frames
+//     tied (a = 1, f = 7, b1 = 90, b2 = 52, 12 heads) writes 100 MB instead of 200 and takes 93 us instead of 136.
+template <class E, int D, int NT, bool WR = false, bool IT = false, bool KO = false>
 __global__ __launch_bounds__(NT > 2 ? 512 : 640) __attribute__((amdgpu_waves_per_eu(NT > 2 ? 2 : 3, NT > 2 ? 2 : 3)))
 void monarch_step1_kernel(MonarchArgs p) {
     using L = S1Lds<D, NT>;
@@ -138,7 +140,7 @@ void monarch_step1_kernel(MonarchArgs p) {
             const int r = P / CPR, c = (P % CPR) ^ s1_swz<CPR>(r);
             const uint32_t off = (krow0 + (uint32_t)min(r, b2 - 1)) * ks1 * 2 + (uint32_t)c * 16;
             s1_load_lds16(kg, off, dst + (uint32_t)g * 1024);
-            s1_load_lds16(vg, off, dst + L::kTile + (uint32_t)g * 1024);
+            if (!KO) s1_load_lds16(vg, off, dst + L::kTile + (uint32_t)g * 1024);
         }
     };
     // K rows 32 t + m as the logits' A operand
@@ -178,9 +180,8 @@ void monarch_step1_kernel(MonarchArgs p) {
     for (int r = 0; r < rounds; ++r) {
         const bool fresh = r < mine;     // in its last round a group may have no tile left: it repeats its previous one
         // Vector memory operations complete in order: this wave's part of tile r has landed when only the Kbar / Y
-        // stores of the round before (the last 8 * D / 64 operations it issued) are outstanding.
-        if (D == 128) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+        // stores of the round before (the last 8 * D / 64 operations it issued, half as many without Y) are outstanding.
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((KO ? 4 : 8) * D / 64) : "memory");
         lds_barrier();                   // tile r is in LDS; every wave has finished reading the tile before it
         if (fresh) cur = nxt;
         const char* kt = lds + (r & 1) * 2 * L::kTile;
@@ -296,7 +297,7 @@ void monarch_step1_kernel(MonarchArgs p) {
         // holds, for each of the four row groups rb, the piece 4 (dt0 + bit 3) + 2 bit 4 + hf of column
         // (c & 7) + 8 rb, so that one store instruction writes 128 contiguous bytes of each of 8 rows.
 #pragma unroll
-        for (int which = 0; which < 2; ++which) {
+        for (int which = 0; which < (KO ? 1 : 2); ++which) {
             const char* tbase = which == 0 ? kt : vt;
             char* og = (char*)(which == 0 ? p.kbar : p.y) + (size_t)srow * (D * 2);
 #pragma unroll
@@ -645,6 +646,166 @@ void monarch_step2_kernel(MonarchArgs p) {
 }
 
 // ------------------------------------------------------------------------------------------------
+// The left factor's row statistics alone, for the refinement passes whose output is not wanted:
+//   stats[i] = log2 sum_r exp2(s log2e <Q_i, Kbar_r> - cl_r)
+// Step 2 without Y and the output: bound by reading the Kbar rows once.  The wave arrangements are step 2's; a lone wave
+// holds two chunks in its LDS, a team four, of which three are in flight.  At three frames tied (b1 = 90, 21 cached frames
+// of 480p, 12 heads) it takes 43 us against 74 us for step 2.
+// ------------------------------------------------------------------------------------------------
+template <int D, int TEAM>
+struct StLds {
+    static constexpr int kPitch = 2 * D, kTile = 32 * kPitch;
+    static constexpr int kBufs = TEAM == 1 ? 2 : 4;
+    static constexpr int kWave = kBufs * (kTile + 256);       // TEAM = 1: a wave's tiles, then its cl values
+    static __host__ __device__ constexpr size_t bytes() { return TEAM == 1 ? 4 * (size_t)kWave : kBufs * (kTile + TEAM * 256); }
+};
+
+template <class E, int D, int TEAM>
+__global__ __launch_bounds__(TEAM == 1 ? 256 : 64 * TEAM)
+void monarch_left_stats_kernel(MonarchArgs p) {
+    using L = StLds<D, TEAM>;
+    constexpr int DS = D / 16, CPR = D / 8;
+    constexpr int NG = CPR / 2;                            // 1 KB pieces of a chunk
+    constexpr int MYG = (NG + TEAM - 1) / TEAM;            // pieces a wave loads (a team of three loads the last ones twice)
+    constexpr int NB = L::kBufs;
+    constexpr bool SOLO = TEAM == 1;
+    extern __shared__ __attribute__((aligned(256))) char lds_s2[];
+
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63;
+    const int m = lane & 31;
+    const int hf = lane >> 5;
+
+    const int b2 = p.b2;
+    const int split = SOLO ? p.s2_split : 1;
+    const int per_wg = SOLO ? 4 / split : 1;               // columns of a workgroup
+    const int sp = SOLO ? wave & (split - 1) : 0;
+    const int njg = (b2 + per_wg - 1) / per_wg;
+    const int a = blockIdx.x / njg;
+    const int jraw = (blockIdx.x % njg) * per_wg + (SOLO ? wave / split : 0);
+    const bool j_ok = jraw < b2;
+    const int j = j_ok ? jraw : b2 - 1;
+    const int ul = blockIdx.y;
+    const int unit = p.unit0 + ul;
+    const int b = unit / p.H, h = unit % p.H;
+    const int i0 = SOLO ? 0 : wave * 32;
+    const int r_lim = p.nf * p.b1;
+    const int nch = (r_lim + 31) / 32;
+
+    const int64_t blk = (int64_t)ul * p.ws_unit + (int64_t)(a * b2 + j) * p.ws_aj;
+    const char* kb = (const char*)p.kbar + blk * (2 * D);
+    const char* clp = (const char*)(p.cl + (int64_t)ul * p.cl_unit + (int64_t)(a * b2 + j) * p.cl_aj);
+    const uint32_t cl_ld = p.cl_row * 4;
+
+    char* const wl = lds_s2 + (SOLO ? wave * L::kWave : 0);
+    char* const cll = SOLO ? wl + NB * L::kTile : lds_s2 + NB * (L::kTile + wave * 256);
+    const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)wl;
+    const uint32_t cl0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)cll;
+
+    u32x4 qb[DS];                                          // logits operand (B): this lane's query row (zero past b1)
+    {
+        const uint16_t* qg = (const uint16_t*)p.q + (int64_t)b * p.qs[0] + (int64_t)h * p.qs[2];
+        const uint16_t* qrow = qg + (p.qmap.row(a, min(i0 + m, p.b1 - 1)) + j) * p.qs[1] + 8 * hf;
+#pragma unroll
+        for (int ds = 0; ds < DS; ++ds) qb[ds] = *(const u32x4*)(qrow + 16 * ds);
+#pragma unroll
+        for (int ds = 0; ds < DS; ++ds) asm volatile("" : "+v"(qb[ds]));       // waited for here, before the first chunk's loads
+        if (i0 + m >= p.b1) {
+#pragma unroll
+            for (int ds = 0; ds < DS; ++ds) qb[ds] = u32x4{0u, 0u, 0u, 0u};
+        }
+    }
+    const uint32_t a_off = (uint32_t)m * L::kPitch + (uint32_t)((hf ^ s1_swz<CPR>(m)) << 4);   // Kbar row m as the logits' A operand
+    const float sc2 = p.scale * kLog2e;
+    const f32x16 kZero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float mrun = -INFINITY, lrun = 0.f;
+
+    auto issue = [&](int n, int it) {
+        const uint32_t dst = lds0 + (uint32_t)(it % NB) * L::kTile;
+#pragma unroll
+        for (int g0 = 0; g0 < MYG; ++g0) {
+            const int g = SOLO ? g0 : min(wave * MYG + g0, NG - 1);
+            const int P = g * 64 + lane;
+            const int r = P / CPR, c = (P % CPR) ^ s1_swz<CPR>(r);
+            const uint32_t off = (uint32_t)min(32 * n + r, r_lim - 1) * (2 * D) + (uint32_t)c * 16;
+            s1_load_lds16(kb, off, dst + (uint32_t)g * 1024);
+        }
+        s2_load_lds4(clp, (uint32_t)(32 * n + m) * cl_ld, cl0 + (uint32_t)(it % NB) * 256);   // lanes >= 32 repeat
+    };
+#pragma unroll
+    for (int it = 0; it < NB - 1; ++it)
+        if (sp + it * split < nch) issue(sp + it * split, it);
+    for (int n = sp, it = 0; n < nch; n += split, ++it) {
+        // vector memory operations complete in order: chunk n has landed when only the chunks requested after it are
+        // outstanding.  The buffer of the chunk before is free once its reads have been waited for.
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (SOLO) {
+            if (n + split < nch) {
+                issue(n + split, it + 1);
+                wait_vm<MYG + 1>();
+            } else {
+                wait_vm<0>();
+            }
+        } else {
+            if (n + 2 < nch) wait_vm<2 * (MYG + 1)>();
+            else if (n + 1 < nch) wait_vm<MYG + 1>();
+            else wait_vm<0>();
+            lds_barrier();         // every wave's share is there, and every wave is done with the chunk before
+            if (n + 3 < nch) issue(n + 3, it + 3);
+        }
+        const char* kt = wl + (it % NB) * L::kTile;
+        const char* clt = cll + (it % NB) * 256;
+        f32x16 s;
+#pragma unroll
+        for (int ds = 0; ds < DS; ++ds) {
+            const u32x4 ak = *(const u32x4*)(kt + (a_off ^ (uint32_t)(ds << 5)));
+            s = E::mfma32(ak, qb[ds], ds ? s : kZero);
+        }
+        f32x4 cc[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) cc[g] = *(const f32x4*)(clt + (8 * g + 4 * hf) * 4);
+        float mx = -INFINITY;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const int r = 32 * n + 8 * (v >> 2) + 4 * hf + (v & 3);
+            const float z = r < r_lim ? s[v] * sc2 - cc[v >> 2][v & 3] : -INFINITY;
+            s[v] = z;
+            mx = fmaxf(mx, z);
+        }
+        mx = xhalf_max(mx);
+        const float mnew = fmaxf(mrun, mx);        // finite: chunk n has at least one valid row
+        float psum = 0.f;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) psum += exp2f(s[v] - mnew);
+        lrun = lrun * exp2f(mrun - mnew) + psum;
+        mrun = mnew;
+    }
+
+    float* const stats = p.stats + ((int64_t)unit * (p.na * b2) + a * b2 + j) * p.stats_ld;
+    float ltot = xhalf_sum(lrun);
+    if constexpr (SOLO) {
+        if (split > 1) {           // merge of the waves of a column through the (dead) cl buffers, in step 2's order
+            if (hf == 0) {
+                *(float*)(cll + m * 4) = mrun;
+                *(float*)(cll + 128 + m * 4) = ltot;
+            }
+            lds_barrier();
+            const char* col = cll - sp * L::kWave;
+            float M = -INFINITY, sum = 0.f;
+            for (int w = 0; w < split; ++w) M = fmaxf(M, *(const float*)(col + w * L::kWave + m * 4));
+            for (int w = 0; w < split; ++w) {
+                const char* c = col + w * L::kWave + m * 4;
+                sum += *(const float*)(c + 128) * exp2f(*(const float*)c - M);           // a wave without chunks: 0 * exp2(-inf)
+            }
+            mrun = M;
+            ltot = sum;
+        }
+    }
+    if (sp == 0 && hf == 0 && j_ok && i0 + m < p.b1) stats[i0 + m] = mrun + log2f(ltot);
+}
+
+// ------------------------------------------------------------------------------------------------
 // iterated refinement: the next pass's query representatives (wan/modules/monarch_attn.py:1741-1744)
 //   rep[a, j, r, :] = sum_i L[i, r] Q[a, i, j, :],   wgt[a, j, r] = sum_i L[i, r],   r = (f, k)
 // with L[i, r] = exp2(s log2e <Q_i, Kbar_r> - cl_r - stats_i), stats = the left factor's row statistics that step 2 wrote.
@@ -904,13 +1065,17 @@ static int enqueue_step1(const MonarchArgs& a, int nunits, hipStream_t stream, c
     return SFM_OK;
 }
 
-// Enqueues step 2: a wave per column (a, j) of up to 32 query rows, a team of waves for more.
+// Enqueues step 2: a wave per column (a, j) of up to 32 query rows, a team of waves for more.  `stats_only` (b1 <= 128):
+// the row statistics without the output.
 template <class E, int D>
-static int enqueue_step2(const MonarchArgs& a, int nunits, hipStream_t stream) {
+static int enqueue_step2(const MonarchArgs& a, int nunits, hipStream_t stream, bool stats_only = false) {
     const int team = a.b1 > 96 ? 4 : (a.b1 + 31) / 32;
-    const void* fn = team == 4 ? (const void*)monarch_step2_kernel<E, D, 4> : team == 3 ? (const void*)monarch_step2_kernel<E, D, 3>
+    const void* fn = stats_only ? (team == 4 ? (const void*)monarch_left_stats_kernel<E, D, 4> : team == 3 ? (const void*)monarch_left_stats_kernel<E, D, 3>
+                                   : team == 2 ? (const void*)monarch_left_stats_kernel<E, D, 2> : (const void*)monarch_left_stats_kernel<E, D, 1>)
+                   : team == 4 ? (const void*)monarch_step2_kernel<E, D, 4> : team == 3 ? (const void*)monarch_step2_kernel<E, D, 3>
                    : team == 2 ? (const void*)monarch_step2_kernel<E, D, 2> : (const void*)monarch_step2_kernel<E, D, 1>;
-    const size_t lds = team > 1 ? S2Lds<D>::team_bytes(team) : S2Lds<D>::bytes();
+    const size_t lds = stats_only ? (team == 4 ? StLds<D, 4>::bytes() : team == 3 ? StLds<D, 3>::bytes() : team == 2 ? StLds<D, 2>::bytes() : StLds<D, 1>::bytes())
+                       : team > 1 ? S2Lds<D>::team_bytes(team) : S2Lds<D>::bytes();
     MonarchArgs a2 = a;
     a2.s2_split = 1;
     if (team == 1) {
@@ -985,12 +1150,17 @@ static int launch_rep_t(const MonarchArgs& a, int nunits, hipStream_t stream) {
     return SFM_OK;
 }
 
-// num_iters passes of [step 1 with the pass's query operands | step 2 | representatives for the next pass]; the last
-// pass's step 2 writes the output (the earlier ones write it too: it is overwritten).
+// num_iters - 1 passes of [step 1 with the pass's query operands, Kbar only | row statistics of the left factor |
+// representatives for the next pass], then a whole forward with the last representatives.  (With whole forwards in every
+// pass a three-pass call at three frames tied took 696 us, now 572.)
 template <class E, int D>
 static int launch_iter_t(const MonarchArgs& a, int nunits, int num_iters, hipStream_t stream) {
     const int nq = (a.b1 + 31) / 32;
     const int nt = (a.b2 + 31) / 32;
+    const void* fnk = nt == 4 ? (const void*)monarch_step1_kernel<E, D, 4, false, true, true>
+                    : nt == 3 ? (const void*)monarch_step1_kernel<E, D, 3, false, true, true>
+                    : nt == 2 ? (const void*)monarch_step1_kernel<E, D, 2, false, true, true>
+                              : (const void*)monarch_step1_kernel<E, D, 1, false, true, true>;
     const void* fn1 = nt == 4 ? (const void*)monarch_step1_kernel<E, D, 4, false, true>
                     : nt == 3 ? (const void*)monarch_step1_kernel<E, D, 3, false, true>
                     : nt == 2 ? (const void*)monarch_step1_kernel<E, D, 2, false, true>
@@ -1000,10 +1170,10 @@ static int launch_iter_t(const MonarchArgs& a, int nunits, int num_iters, hipStr
         MonarchArgs a1 = a;
         a1.rb = nullptr;
         a1.iter_mode = it == 0 ? 1 : 2;
-        if (int rc = enqueue_step1<E, D>(a1, nunits, stream, fn1)) return rc;
+        if (int rc = enqueue_step1<E, D>(a1, nunits, stream, last ? fn1 : fnk)) return rc;
         MonarchArgs a2 = a;
         if (last) a2.stats = nullptr;
-        if (int rc = enqueue_step2<E, D>(a2, nunits, stream)) return rc;
+        if (int rc = enqueue_step2<E, D>(a2, nunits, stream, !last)) return rc;
         if (!last) {
             const int rc = nq == 1 ? launch_rep_t<E, D, 1>(a, nunits, stream) : nq == 2 ? launch_rep_t<E, D, 2>(a, nunits, stream)
                          : nq == 3 ? launch_rep_t<E, D, 3>(a, nunits, stream) : launch_rep_t<E, D, 4>(a, nunits, stream);

@@ -129,6 +129,18 @@ def test_mfma_refinement_against_the_oracle_and_the_fp32_kernels(dtype, h, w, D,
     assert_close_16bit(fast, slow.float(), dtype)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("b1,fk", [(1, 2), (1, 33), (31, 1), (32, 4), (33, 1), (16, 9), (64, 2), (65, 1), (96, 1), (97, 2), (128, 1)])
+def test_refinement_around_query_tiles_and_row_chunks(b1, fk, D):
+    """The passes before the last form Kbar and the row statistics only: block rows on both sides of every query tile, one
+    to nine chunks of 32 rows, and columns few enough for waves to share."""
+    q = randn((1, b1 * 5, 1, D), 400 + b1, torch.bfloat16)
+    k, v = (randn((1, fk * b1 * 5, 1, D), 401 + b1 + i, torch.bfloat16) for i in range(2))
+    ref = monarch.monarch_attn(q, k, v, 1, 1, 1, b1, 5, num_iters=3, dtype=torch.float32)
+    out = mattn.monarch_attn(q.to(DEV), k.to(DEV), v.to(DEV), 1, 1, 1, b1, 5, num_iters=3)
+    assert_close_16bit(out, ref, torch.bfloat16)
+
+
 def test_mfma_refinement_golden_vectors_in_bf16():
     """The reference's own refinement outputs (float64 golden vectors), inputs rounded to bf16: D = 64 case of the
     fixture, num_iters 2, 3 and 8, on the MFMA kernels."""
