@@ -813,21 +813,25 @@ void monarch_left_stats_kernel(MonarchArgs p) {
 // LDS; the logits come out as S[i, r] (A = query rows, B = Kbar rows), so that a lane holds a column r, and
 // rep^T[d, r] = sum_i Q^T[d, i] L[i, r] takes Q^T from transposing reads of the column's query rows, which sit in the
 // wave's LDS for the whole kernel.  NQ = 32-row tiles of the query rows i (b1 <= 32 NQ <= 128: three frames tied per
-// block give b1 = 90); with one tile the logits' A operand stays in registers, with more it is read from the LDS rows.
-// A workgroup is 4 waves (NQ <= 2) or 3 (more LDS per wave).
+// block give b1 = 90).  With one tile a wave owns a column and its query rows, and the logits' A operand stays in
+// registers; 4 waves to a workgroup.  With more tiles the rows of one column fill the LDS of a wave or two, so a
+// workgroup of 8 waves (7 at four tiles) owns one column: one copy of its query rows, chunks of Kbar rows dealt in turn
+// (a chunk's representatives need no other chunk's).  A wave per column with its own copy held one workgroup of three
+// waves on a compute unit, each with a serial chain of 20 chunks, at b1 = 90, 630 rows: 74 us, now 60.
 // ------------------------------------------------------------------------------------------------
 template <int D, int NQ>
 struct RepLds {
     static constexpr int kPitch = 2 * D, kTile = 32 * kPitch;
     static constexpr int kBuf = kTile + 256;               // [Kbar chunk | cl values]
-    static constexpr int kQ = 2 * kBuf;                    // offset of the query rows
-    static constexpr int kWave = 2 * kBuf + NQ * kTile;
-    static constexpr int kWaves = NQ <= 2 ? 4 : 3;
-    static __host__ __device__ constexpr size_t bytes() { return (size_t)kWaves * kWave; }
+    static constexpr bool kShared = NQ > 1;                // a workgroup's waves share one column
+    static constexpr int kWaves = NQ == 1 ? 4 : NQ < 4 ? 8 : 7;
+    static constexpr int kWave = 2 * kBuf + (kShared ? 0 : kTile);      // bytes per wave, its query rows behind its buffers
+    static constexpr int kQ = kShared ? kWaves * kWave : 2 * kBuf;      // offset of the query rows (from the workgroup's / the wave's LDS)
+    static __host__ __device__ constexpr size_t bytes() { return (size_t)kWaves * kWave + (kShared ? NQ * kTile : 0); }
 };
 
 template <class E, int D, int NQ>
-__global__ __launch_bounds__(256) void monarch_rep_kernel(MonarchArgs p) {
+__global__ __launch_bounds__(64 * (RepLds<D, NQ>::kWaves)) void monarch_rep_kernel(MonarchArgs p) {
     using L = RepLds<D, NQ>;
     constexpr int DS = D / 16, DT = D / 32, CPR = D / 8;
     extern __shared__ __attribute__((aligned(256))) char lds_s2[];
@@ -839,11 +843,13 @@ __global__ __launch_bounds__(256) void monarch_rep_kernel(MonarchArgs p) {
     const int hf = lane >> 5;
 
     const int b2 = p.b2;
-    const int njg = (b2 + L::kWaves - 1) / L::kWaves;
+    const int per_wg = L::kShared ? 1 : L::kWaves;         // columns of a workgroup
+    const int njg = (b2 + per_wg - 1) / per_wg;
     const int a = blockIdx.x / njg;
-    const int jraw = (blockIdx.x % njg) * L::kWaves + wave;
-    if (jraw >= b2) return;                               // the waves of a workgroup share nothing
-    const int j = jraw;
+    const int j = (blockIdx.x % njg) * per_wg + (L::kShared ? 0 : wave);
+    if (j >= b2) return;                                  // never in a shared workgroup, which has barriers
+    constexpr int step = L::kShared ? L::kWaves : 1;       // this wave's chunks: n0, n0 + step, ...
+    const int n0 = L::kShared ? wave : 0;
     const int ul = blockIdx.y;
     const int unit = p.unit0 + ul;
     const int b = unit / p.H, h = unit % p.H;
@@ -859,16 +865,16 @@ __global__ __launch_bounds__(256) void monarch_rep_kernel(MonarchArgs p) {
 
     char* const wl = lds_s2 + wave * L::kWave;
     const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)wl;
-    char* const qt = wl + L::kQ;                          // the column's query rows, laid out like chunks of scratch rows
+    char* const qt = (L::kShared ? lds_s2 : wl) + L::kQ;  // the column's query rows, laid out like chunks of scratch rows
+    const uint32_t qt0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)qt;
 
     const uint16_t* qg = (const uint16_t*)p.q + (int64_t)b * p.qs[0] + (int64_t)h * p.qs[2];
     // query rows into LDS (rows past b1 repeat the last one; their weights are zero)
-#pragma unroll
-    for (int g = 0; g < NQ * (CPR / 2); ++g) {
+    for (int g = n0; g < NQ * (CPR / 2); g += step) {
         const int P = g * 64 + lane;
         const int r = P / CPR, c = (P % CPR) ^ s1_swz<CPR>(r);
         const uint32_t off = (uint32_t)((p.qmap.row(a, min(r, p.b1 - 1)) + j) * p.qs[1] * 2) + (uint32_t)c * 16;
-        s1_load_lds16((const char*)qg, off, lds0 + L::kQ + (uint32_t)g * 1024);
+        s1_load_lds16((const char*)qg, off, qt0 + (uint32_t)g * 1024);
     }
     // one tile: the logits operand (A) is this lane's query row Q[a, m, j, :] (zero past b1), kept in registers
     u32x4 qa[DS];
@@ -930,17 +936,21 @@ __global__ __launch_bounds__(256) void monarch_rep_kernel(MonarchArgs p) {
     const float sc2 = p.scale * kLog2e;
     const f32x16 kZero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 
-    issue(0, 0);
-    for (int n = 0; n < nch; ++n) {
+    if (L::kShared) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        lds_barrier();             // every wave's share of the query rows is there
+    }
+    if (n0 < nch) issue(n0, 0);
+    for (int n = n0, buf = 0; n < nch; n += step, buf ^= 1) {
         // everything older than the chunk requested last (the stores of the chunk before included) is waited for
-        if (n + 1 < nch) {
-            issue(n + 1, (n + 1) & 1);
+        if (n + step < nch) {
+            issue(n + step, buf ^ 1);
             if (D == 128) asm volatile("s_waitcnt vmcnt(9)" ::: "memory");
             else asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
         } else {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
-        const char* kt = wl + (n & 1) * L::kBuf;
+        const char* kt = wl + buf * L::kBuf;
         const float cc = *(const float*)(kt + L::kTile + m * 4);
         const bool rok = 32 * n + m < r_lim;
         float wsum = 0.f;
@@ -1145,14 +1155,14 @@ static int launch_rep_t(const MonarchArgs& a, int nunits, hipStream_t stream) {
         set_error("hipFuncSetAttribute failed: %s", hipGetErrorString(e));
         return SFM_ERR_HIP;
     }
-    const int njg = (a.b2 + L::kWaves - 1) / L::kWaves;
+    const int njg = L::kShared ? a.b2 : (a.b2 + L::kWaves - 1) / L::kWaves;
     hipLaunchKernelGGL((monarch_rep_kernel<E, D, NQ>), dim3(a.na * njg, nunits), dim3(64 * L::kWaves), L::bytes(), stream, a);
     return SFM_OK;
 }
 
 // num_iters - 1 passes of [step 1 with the pass's query operands, Kbar only | row statistics of the left factor |
 // representatives for the next pass], then a whole forward with the last representatives.  (With whole forwards in every
-// pass a three-pass call at three frames tied took 696 us, now 572.)
+// pass a three-pass call at three frames tied took 696 us.)
 template <class E, int D>
 static int launch_iter_t(const MonarchArgs& a, int nunits, int num_iters, hipStream_t stream) {
     const int nq = (a.b1 + 31) / 32;
