@@ -409,7 +409,7 @@ template <> constexpr int left_dtype<F16>() { return SFM_F16; }
 struct Parts {
     bool left;     // 4-7: statistics and gradients of the left factor without the [i x r] matrices in memory
     bool fwd;      // 1-3: the forward's MFMA step 1 recomputes Kbar, Y, c and R straight into the scratch ([t][aj] rows)
-    bool dqa;      // 8 and the scatter of dq: dQ of the left factor in its own kernel, which also adds the right factor's part
+    bool dqa;      // 8: the left factor's kernel forms its dQ too (with `dqk` in the caller's rows, to which the right factor's is added)
     bool right;    // 9, the right factor's softmax backward, 11-13 and the scatter of dk / dv in one kernel per tile t
     bool dqk;      // 10 in a kernel that reads K where the caller has it (with `right`: no gathered copy of K is needed)
 };
@@ -448,17 +448,16 @@ Layout make_layout(const MonarchArgs& p, int n, size_t e, const Parts& f) {
     l.dS1 = take(true, n * p.b1 * AJ * NL * e);
     l.Kbar = take(true, n * AJ * RR * D * e);
     l.Y = take(true, n * AJ * RR * D * e);
-    const size_t nz = f.left ? (size_t)(p.b1 + 31) / 32 : 1;      // the fused left factor writes one partial slab per 32 query rows
-    l.dKbar = take(true, nz * n * AJ * RR * D * e);
-    l.dY = take(true, nz * n * AJ * RR * D * e);
+    l.dKbar = take(true, n * AJ * RR * D * e);
+    l.dY = take(true, n * AJ * RR * D * e);
     l.c = take(true, n * AJ * RR * 4);
-    l.dc = take(true, nz * n * AJ * RR * 4);
+    l.dc = take(true, n * AJ * RR * 4);
     l.S2f = take(!f.left, n * AJ * p.b1 * RR * 4);
     l.dLmf = take(!f.left, n * AJ * p.b1 * RR * 4);
     l.L = take(!f.left, n * AJ * p.b1 * RR * e);
-    l.dS2 = take(true, n * AJ * p.b1 * ((RR + 7) / 8 * 8) * e);                         // rows padded to 8 for the fused kernels
-    l.dQa = take(!f.dqa, n * MQ * D * 4);
-    l.dQk = take(true, n * MQ * D * 4);
+    l.dS2 = take(!f.dqa, n * AJ * p.b1 * ((RR + 7) / 8 * 8) * e);                         // rows padded to 8 for the fused kernels
+    l.dQa = take(!f.dqa || !f.dqk, n * MQ * D * 4);
+    l.dQk = take(!f.dqa || !f.dqk, n * MQ * D * 4);
     l.dKk = take(!f.right, n * MK * D * 4);
     l.dVk = take(!f.right, n * MK * D * 4);
     l.total = o;
@@ -517,6 +516,7 @@ int run(const MonarchBwdArgs& g, int n, void* workspace, hipStream_t stream) {
 
     const int64_t nseg = (int64_t)n * b1 * AJ * nf;
     const bool fused_left = parts.left, fused_fwd = parts.fwd, fused_dqa = parts.dqa, fused_right = parts.right;
+    const bool dq_direct = parts.dqa && parts.dqk;       // both parts of dq go to the caller's rows
     const int ds2_ld = fused_left ? (RR + 7) / 8 * 8 : RR;
     const int rb_ld = fused_fwd ? 64 : b2;
     if (fused_right && ((uintptr_t)g.dk | (uintptr_t)g.dv | (uintptr_t)p.v) % 16) {
@@ -588,8 +588,9 @@ int run(const MonarchBwdArgs& g, int n, void* workspace, hipStream_t stream) {
         if (!cx.status)
             cx.status = launch_monarch_bwd_left(left_dtype<E>(), D, n, b1, b2, AJ, nf, p.causal, s, p.q, p.qs, g.dout, saved ? g.fout : nullptr,
                                                 g.dos, p.qmap, H, p.unit0, ws + lay.Kbar, ws + lay.Y, (const float*)(ws + lay.c),
-                                                fused_fwd ? 1 : 0, ws + lay.dKbar, ws + lay.dY, (float*)(ws + lay.dc), ws + lay.dS2, ds2_ld,
-                                                saved ? g.fstats : nullptr, (b1 + 31) / 32 * 32, stream);
+                                                fused_fwd ? 1 : 0, ws + lay.dKbar, ws + lay.dY, (float*)(ws + lay.dc),
+                                                fused_dqa ? nullptr : ws + lay.dS2, ds2_ld,
+                                                !fused_dqa ? nullptr : dq_direct ? g.dq : (float*)(ws + lay.dQa), dq_direct ? g.dqs : nullptr, saved ? g.fstats : nullptr, (b1 + 31) / 32 * 32, stream);
     } else {
         // 4, 5. per unit and (a, j): S2 = q_i . Kbar_r, dLm = dO_i . Y_r; the [RR x D] matrix of column aj is every AJ-th row
         for (int u = 0; u < n && !cx.status; ++u) {
@@ -647,7 +648,7 @@ int run(const MonarchBwdArgs& g, int n, void* workspace, hipStream_t stream) {
     if (parts.dqk) {
         if (!cx.status)
             cx.status = launch_monarch_bwd_dqk(left_dtype<E>(), D, nuk, b1, b2, AJ, nf, s, p.k, p.ks, p.kmap, ws + lay.dS1,
-                                               (float*)(ws + lay.dQk), H, p.unit0, stream);
+                                               dq_direct ? g.dq : (float*)(ws + lay.dQk), dq_direct ? g.dqs : nullptr, p.qmap, H, p.unit0, stream);
     } else {
         gemm(cx, false, false, AJ, D, NL, s, 0.f, dS1_uk, Kk_uk, dQk_uk, tE, tF, nuk);
     }
@@ -662,10 +663,7 @@ int run(const MonarchBwdArgs& g, int n, void* workspace, hipStream_t stream) {
     // scatter the gradients back to the callers' layouts
     {
         const int64_t tq = (int64_t)n * MQ * (D / 4);
-        if (fused_dqa)
-            cx.status = launch_monarch_bwd_dqa(left_dtype<E>(), D, n, b1, b2, AJ, nf, s, ws + lay.Kbar, ws + lay.dS2, ds2_ld,
-                                               (const float*)(ws + lay.dQk), g.dq, g.dqs, p.qmap, H, p.unit0, stream);
-        else
+        if (!dq_direct)
             hipLaunchKernelGGL(scatter_dq, dim3((unsigned)((tq + 255) / 256)), dim3(256), 0, stream, (const float*)(ws + lay.dQa),
                                (const float*)(ws + lay.dQk), g.dq, g.dqs[0], g.dqs[1], g.dqs[2], p.qmap, na, H, D, p.unit0, tq);
         const int64_t tk = (int64_t)n * b1 * (g.kv_f1 - g.kv_f0) * b2 * (D / 4);

@@ -224,16 +224,13 @@ int launch_monarch_bwd_gemm(const MonarchBwdArgs& g, int dtype, int nunits, void
 // step 1 of the MFMA forward alone, with the scratch strides of `a` and, if a.rb is set, the right factor written out
 int launch_monarch_step1(const MonarchArgs& a, int dtype, int nunits, hipStream_t stream);
 // fused left-factor part of the backward (monarch_bwd_left.hip): q, dout (and out, with stats) are the callers' tensors,
-// 16-byte aligned rows; everything else in the GEMM path's scratch layouts
+// 16-byte aligned rows; everything else in the GEMM path's scratch layouts.  dS2 (for a library product) and its dQ = s dS2
+// Kbar are each optional; dQ goes to the caller's rows (dqs) or, with dqs NULL, to a float matrix [u][aj][i][D]
 bool monarch_bwd_left_supported(int dtype, int D, int b1);
 int launch_monarch_bwd_left(int dtype, int D, int n, int b1, int b2, int AJ, int nf, int causal, float scale, const void* q,
                             const int64_t* qs, const void* dout, const void* out, const int64_t* os, const TokMap& qmap, int H,
                             int unit0, const void* kbar, const void* y, const float* c, int c_rows, void* dkbar, void* dy, float* dc,
-                            void* ds2, int ds2_ld, const float* stats, int stats_ld, hipStream_t stream);
-// dq rows (caller's layout) = s dS2 Kbar per (unit, a, j) + the right factor's dQk; same limits as the left kernel
-int launch_monarch_bwd_dqa(int dtype, int D, int n, int b1, int b2, int AJ, int nf, float scale, const void* kbar, const void* ds2,
-                           int ds2_ld, const float* dqk, float* dq, const int64_t* dqs, const TokMap& map, int H, int unit0,
-                           hipStream_t stream);
+                            void* ds2, int ds2_ld, float* dq, const int64_t* dqs, const float* stats, int stats_ld, hipStream_t stream);
 // fused right-factor part of the backward (monarch_bwd_right.hip): per tile t = (unit, k, f) the dS1 block (scratch, for
 // dQ = s dS1 K) and the finished dK / dV rows of kv block-frames [f0, f1) in the caller's tensors; q, k and v are the caller's tensors too
 bool monarch_bwd_right_supported(int dtype, int D, int b2, int AJ);
@@ -242,10 +239,12 @@ int launch_monarch_bwd_right(int dtype, int D, int64_t ntiles, int b1, int b2, i
                              const int64_t* qs, const TokMap& qmap, void* ds1, void* dk, void* dv, const int64_t* dks, int64_t row0,
                              const TokMap& kmap, int H, int unit0, int f0, int f1, hipStream_t stream);
 
-// dQ of the right factor (monarch_bwd_right.hip): dqk[(u, k)][aj][:] = s sum_{f, l} dS1 K, float; k is the caller's tensor
+// dQ of the right factor (monarch_bwd_right.hip): dqk[(u, k)][aj][:] = s sum_{f, l} dS1 K, float, or, with dqs given, added
+// to the caller's rows; k is the caller's tensor
 bool monarch_bwd_dqk_supported(int dtype, int D, int b2, int AJ);
 int launch_monarch_bwd_dqk(int dtype, int D, int64_t nuk, int b1, int b2, int AJ, int nf, float scale, const void* k, const int64_t* ks,
-                           const TokMap& kmap, const void* ds1, float* dqk, int H, int unit0, hipStream_t stream);
+                           const TokMap& kmap, const void* ds1, float* dqk, const int64_t* dqs, const TokMap& qmap, int H, int unit0,
+                           hipStream_t stream);
 
 // backward of the dense attention (dense_attn_bwd.hip); scratch is 2*B*H*q_tokens floats
 bool dense_bwd_supported(int dtype, int D);

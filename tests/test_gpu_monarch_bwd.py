@@ -180,6 +180,29 @@ def test_16bit_gradients_across_the_fused_kernels_limits(h, w, Fq, Fk, D, causal
     _close(vd.grad, vr.grad, dtype)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("b1,Fk,part", [(1, 3, 0), (31, 2, 0), (32, 1, 0), (33, 2, 0), (64, 1, 0), (65, 2, 0), (96, 1, 0), (97, 2, 0), (128, 1, 0),
+                                        (32, 2, "SW_BWD_DQA_GEMM"), (70, 2, "SW_BWD_DQA_GEMM"), (70, 2, "SW_BWD_DQK_GEMM")])
+def test_gradients_around_the_left_factors_query_tiles(b1, Fk, part, D, switches):
+    """Block rows on both sides of every 32-row query tile (one wave, teams of two to four), with the left factor's dQ formed
+    in its kernel or by a library product from dS2, with the saved row statistics and recomputing them."""
+    switches(getattr(sfa.lib, part) if part else 0)
+    w, H, dtype = 4, 2, torch.bfloat16
+    q0, do = (randn((1, b1 * w, H, D), 500 + b1 + i, dtype) for i in range(2))
+    k0, v0 = (randn((1, Fk * b1 * w, H, D), 502 + b1 + i, dtype) for i in range(2))
+    qr, kr, vr = _leaf(q0.double()), _leaf(k0.double()), _leaf(v0.double())
+    monarch.monarch_attn(qr, kr, vr, 1, 1, 1, b1, w).backward(do.double())
+    qd, kd, vd, dod = q0.to(DEV), k0.to(DEV), v0.to(DEV), do.to(DEV)
+    tiling = (1, 1, 1, b1, w)
+    out, stats = mattn._monarch_fwd_stats(qd, kd, vd, tiling, D ** -0.5, 0, 0)
+    assert stats is not None
+    for kept in ({}, {"out": out, "stats": stats}):
+        dq, dk, dv = mattn._monarch_bwd(qd, kd, vd, dod, tiling, D ** -0.5, 0, 0, **kept)
+        _close(dq, qr.grad, dtype)
+        _close(dk, kr.grad, dtype)
+        _close(dv, vr.grad, dtype)
+
+
 @pytest.mark.parametrize("causal", [False, True])
 def test_backward_with_and_without_the_forwards_saved_tensors(causal):
     """sfm_monarch_bwd recomputes the left factor's row statistics; sfm_monarch_bwd_saved takes them (and the output)
