@@ -188,6 +188,16 @@ int sfm_full_attention_with_kv_cache(const sfm_dense_desc* desc, const void* q, 
                                      const void* new_k, const void* new_v, const int64_t new_stride[3],
                                      int64_t start_idx, int64_t end_idx, void* out, float* lse, void* stream);
 
+/* The same with a workspace, which lets few queries be split over the keys: sfm_dense_workspace_bytes says how much (0: the
+ * call would not be split).  With less, or NULL, the call runs unsplit. */
+int sfm_dense_workspace_bytes(const sfm_dense_desc* desc, size_t* bytes);
+int sfm_dense_fwd_ws(const sfm_dense_desc* desc, const void* q, const void* k, const void* v, void* out,
+                     float* lse, void* workspace, size_t workspace_bytes, void* stream);
+int sfm_full_attention_with_kv_cache_ws(const sfm_dense_desc* desc, const void* q, void* k_cache, void* v_cache,
+                                        const void* new_k, const void* new_v, const int64_t new_stride[3],
+                                        int64_t start_idx, int64_t end_idx, void* out, float* lse, void* workspace,
+                                        size_t workspace_bytes, void* stream);
+
 /* Backward of sfm_dense_fwd / sfm_full_attention_with_kv_cache.  Replaces _attn_bwd_preprocess, _attn_bwd and
  * _attention.backward (attn_patch.py:121-166, 169-302, 354-413): bf16 / fp16, head_dim 64 or 128.
  *   fwd                 the forward descriptor; o_stride describes both `out` and `dout`

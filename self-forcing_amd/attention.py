@@ -30,9 +30,18 @@ def _dense_fwd(q, k, v, sm_scale, want_lse):
     lse = torch.empty((q.shape[0], q.shape[2], q.shape[1]), dtype=torch.float32, device=q.device) if want_lse else None
     d = _dense_desc(q, k, v, out, sm_scale)
     with torch.cuda.device(q.device):
-        _l.check(_l.load().sfm_dense_fwd(C.byref(d), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-                                         lse.data_ptr() if want_lse else None, _stream(q)))
+        ws, nbytes = _dense_workspace(d, q.device)
+        _l.check(_l.load().sfm_dense_fwd_ws(C.byref(d), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+                                            lse.data_ptr() if want_lse else None, ws.data_ptr() if nbytes else None, nbytes, _stream(q)))
     return out, lse
+
+
+def _dense_workspace(d, device):
+    """(partials of a call that is split over the keys, bytes): most calls need none.  Allocated for the call, so that it
+    follows the allocator's rules for streams and graph capture as the output does."""
+    n = C.c_size_t(0)
+    _l.check(_l.load().sfm_dense_workspace_bytes(C.byref(d), C.byref(n)))
+    return (torch.empty(n.value, dtype=torch.uint8, device=device) if n.value else None), n.value
 
 
 def _dense_bwd(q, k, v, out, lse, dout, sm_scale, kv0=0, kv1=None):
@@ -162,7 +171,9 @@ def _dense_cache_fwd(q, k_cache, v_cache, new_k, new_v, start_idx, end_idx, sm_s
     lse = torch.empty((q.shape[0], q.shape[2], q.shape[1]), dtype=torch.float32, device=q.device) if want_lse else None
     d = _dense_desc(q, k_cache, v_cache, out, sm_scale)
     with torch.cuda.device(q.device):
-        _l.check(_l.load().sfm_full_attention_with_kv_cache(
+        ws, nbytes = _dense_workspace(d, q.device)
+        _l.check(_l.load().sfm_full_attention_with_kv_cache_ws(
             C.byref(d), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), new_k.data_ptr(), new_v.data_ptr(),
-            _l.strides3(new_k), start_idx, end_idx, out.data_ptr(), lse.data_ptr() if want_lse else None, _stream(q)))
+            _l.strides3(new_k), start_idx, end_idx, out.data_ptr(), lse.data_ptr() if want_lse else None,
+            ws.data_ptr() if nbytes else None, nbytes, _stream(q)))
     return out, lse

@@ -14,6 +14,10 @@
 // barrier per tile.  A wave's matrix and vector work are interleaved in its instruction stream: the logits of
 // tile n + 1 are contracted while the exponentials of tile n are taken, and the maximum of tile n + 1 is reduced
 // while tile n's P V products run.
+//
+// Few queries (fewer workgroups than half of what the chip holds) are split over the keys: a workgroup takes its query
+// block against one range of key tiles and leaves an fp32 partial (unnormalised O, row maximum, row sum), which
+// dense_merge_kernel combines; see dense_split for the rule.
 
 #include "sfm_common.hpp"
 
@@ -56,7 +60,7 @@ template <class E, int D, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void dense_fwd_kernel(sfm_dense_desc p, const uint16_t* __restrict__ q,
                                                         const uint16_t* __restrict__ kp,
                                                         const uint16_t* __restrict__ vp, uint16_t* __restrict__ out,
-                                                        float* __restrict__ lse) {
+                                                        float* __restrict__ lse, int nsplit, float* __restrict__ part) {
     using L = DnLds<D, NW>;
     constexpr int DS = D / 16, DT = D / 32;
     constexpr int NTH = 64 * NW;
@@ -66,18 +70,24 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, hf = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // the query blocks of one (batch, head) go to one XCD: its K / V rows are fetched from memory once, not once per XCD
-    const int nq = p.q_tokens, nk = p.kv_tokens;
+    const int nq = p.q_tokens;
     const int nqb = (nq + 32 * NW - 1) / (32 * NW);
-    const int total = nqb * p.B * p.H;
+    const int total = nqb * nsplit * p.B * p.H;
     const int item = xcd_item(total);
     if (item >= total) return;
-    const int unit = item / nqb;
+    const int us = item / nqb;                     // (unit, range of key tiles)
+    const int unit = us / nsplit, sp = us - unit * nsplit;
     const int b = unit / p.H, h = unit % p.H;
-    const int q0 = (item - unit * nqb) * (32 * NW) + wave * 32;
+    const int q0 = (item - us * nqb) * (32 * NW) + wave * 32;
+    // this workgroup's keys: tiles [tile0, tile0 + ntile) of 64, nk keys in all
+    const int alltiles = (p.kv_tokens + 63) / 64;
+    const int tile0 = (int)((int64_t)sp * alltiles / nsplit);
+    const int ntile = (int)((int64_t)(sp + 1) * alltiles / nsplit) - tile0;
+    const int nk = min(p.kv_tokens - 64 * tile0, 64 * ntile);
 
-    const char* kg = (const char*)(kp + (int64_t)b * p.k_stride[0] + (int64_t)h * p.k_stride[2]);
-    const char* vg = (const char*)(vp + (int64_t)b * p.v_stride[0] + (int64_t)h * p.v_stride[2]);
     const uint32_t krs = (uint32_t)p.k_stride[1] * 2, vrs = (uint32_t)p.v_stride[1] * 2;     // row strides in bytes
+    const char* kg = (const char*)(kp + (int64_t)b * p.k_stride[0] + (int64_t)h * p.k_stride[2]) + (size_t)tile0 * 64 * krs;
+    const char* vg = (const char*)(vp + (int64_t)b * p.v_stride[0] + (int64_t)h * p.v_stride[2]) + (size_t)tile0 * 64 * vrs;
 
     // query operand (B of the logits MFMA): lane (m, hf) holds Q[q0 + m][16 ds + 8 hf + 0..7]
     u32x4 qb[DS];
@@ -139,7 +149,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
         for (int v = 0; v < 16; ++v) oacc[dt][v] = 0.f;
     float mrun = -INFINITY, lrun = 0.f;            // running max (scaled, base-2 units) and sum
     const float sc2 = p.sm_scale * kLog2e;
-    const int ntile = (nk + 63) / 64;
     const int lrem = nk - 64 * (ntile - 1);        // valid keys of the last tile (1..64)
 
     // Both phases of an iteration are sequences of steps, one MFMA each, with the step's A operand read from
@@ -191,7 +200,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
         float mx = sbuf[0][0][0];
 #pragma unroll
         for (int i = 1; i < 32; ++i) mx = fmaxf(mx, DN_SVAL(sbuf[0], i));
-        mrun = xhalf_max(mx) * sc2;
+        mrun = fmaxf(xhalf_max(mx) * sc2, -3.0e38f);       // finite also where every key so far is at -inf: their weights are 0
     }
 
     // One iteration consumes tile n (logits in sbuf[n & 1], maximum already folded into mrun) and, unless it is
@@ -301,6 +310,24 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #undef DN_SVAL
 
     const float ltot = xhalf_sum(lrun);
+    if (nsplit > 1) {
+        // partial [split][unit][q]: D floats of O, then, behind all of them, (maximum, sum)
+        const int64_t row = ((int64_t)sp * p.B * p.H + unit) * nq + q0 + m, rows = (int64_t)nsplit * p.B * p.H * nq;
+        if (q0 + m < nq) {
+            float* const po = part + row * D + 4 * hf;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    *(f32x4*)(po + 32 * dt + 8 * g) = f32x4{oacc[dt][4 * g], oacc[dt][4 * g + 1], oacc[dt][4 * g + 2], oacc[dt][4 * g + 3]};
+            if (hf == 0) {
+                float* const ml = part + rows * D + row * 2;
+                ml[0] = mrun;
+                ml[1] = ltot;
+            }
+        }
+        return;
+    }
     const float inv = 1.f / ltot;
     if (lse != nullptr && hf == 0 && q0 + m < nq)
         lse[((int64_t)b * p.H + h) * nq + q0 + m] = (mrun + log2f(ltot)) * kLn2;
@@ -329,6 +356,38 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
             }
         }
     }
+}
+
+// Combines the partials of a query row: D / 4 lanes hold four elements each, and as many groups of them as there are
+// partials (a power of two, up to the workgroup's 256 lanes) take the partials in turn and add up through LDS.  Bound by
+// reading the partials once.
+template <class E, int D>
+__global__ __launch_bounds__(256) void dense_merge_kernel(sfm_dense_desc p, const float* __restrict__ part, uint16_t* __restrict__ out,
+                                                          float* __restrict__ lse, int nsplit, int groups) {
+    constexpr int CH = D / 4, NSUB = 256 / CH;
+    __shared__ f32x4 red[256];
+    const int tid = threadIdx.x, ch = tid % CH, sub = tid / CH;
+    const int g = sub % groups, per_wg = NSUB / groups;
+    const int nq = p.q_tokens;
+    const int64_t units = (int64_t)p.B * p.H, rows = units * nq;
+    const int64_t row = (int64_t)blockIdx.x * per_wg + sub / groups;
+    const bool ok = row < rows;
+    const float* const ml = part + (int64_t)nsplit * rows * D + (ok ? row : rows - 1) * 2;
+    float M = -INFINITY, sum = 0.f;
+    for (int s = 0; s < nsplit; ++s) M = fmaxf(M, ml[s * rows * 2]);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < nsplit; ++s) sum += ml[s * rows * 2 + 1] * fast_exp2(ml[s * rows * 2] - M);
+    const float* const po = part + (ok ? row : rows - 1) * D + 4 * ch;
+    for (int s = g; s < nsplit; s += groups) acc += *(const f32x4*)(po + s * rows * D) * fast_exp2(ml[s * rows * 2] - M);
+    red[tid] = acc;
+    __syncthreads();
+    if (g != 0 || !ok) return;
+    for (int x = 1; x < groups; ++x) acc += red[tid + x * CH];
+    const float inv = 1.f / sum;
+    const int64_t unit = row / nq, q = row % nq;
+    const u32x2 w = {pack2<E>(acc.x * inv, acc.y * inv), pack2<E>(acc.z * inv, acc.w * inv)};
+    *(u32x2*)(out + (unit / p.H) * p.o_stride[0] + q * p.o_stride[1] + (unit % p.H) * p.o_stride[2] + 4 * ch) = w;
+    if (lse != nullptr && ch == 0) lse[row] = (M + log2f(sum)) * kLn2;
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -404,13 +463,56 @@ __global__ __launch_bounds__(256) void dense_generic_kernel(sfm_dense_desc p, co
     if (lse != nullptr && tid == 0) lse[((int64_t)b * p.H + h) * p.q_tokens + qi] = (mrun + log2f(lrun)) * kLn2;
 }
 
-int launch_dense(const sfm_dense_desc& d, const void* q, const void* k, const void* v, void* out, float* lse,
-                 hipStream_t stream) {
+// 256 queries per workgroup (8 waves, one workgroup per compute unit) stream every K / V tile once per compute
+// unit instead of twice; short query ranges keep 128 so that more compute units get a workgroup
+static bool dense_wide(const sfm_dense_desc& d) { return (int64_t)((d.q_tokens + 255) / 256) * d.B * d.H >= cu_count() / 2; }
+
+// Ranges of key tiles a query block is split into: the number that a model of the call's time says is fastest, if it saves a
+// tenth.  The model, in ns at head_dim 128 (64: 0.6 of it): 5000 for the ends of a workgroup, and per 64-key tile
+//     narrow  1100 with at most one workgroup on a compute unit, 1900 with two   (930 measured on an empty chip, 1250, 1900)
+//     wide    1460 on half the compute units or fewer, 1830 on all
+// and, when split, 6000 for the second launch plus writing and reading the fp32 partials at 3.5 TB/s.  A range keeps four tiles
+// or more, and calls of less than 16 tiles are left alone (they are as long as their launch).  Measured, us, 128-wide heads:
+//     heads x queries x keys        unsplit  split          heads x queries x keys      unsplit  split
+//     1 x 64 x 32760                    477     38           8 x 4096 x 32760 (wide)        746    505
+//     2 x 1000 x 32760                  498     64           4 x 4096 x 32760               505    290
+//     3 x 500 x 10000                   163     36           17 x 805 x 8356                147     95
+//     2 x 108 x 3093                     56     17           30 x 500 x 1100 (left whole)    27     40 in four ranges
+static int dense_split(const sfm_dense_desc& d) {
+    if ((d.dtype != SFM_BF16 && d.dtype != SFM_F16) || (d.D != 64 && d.D != 128)) return 1;
+    const bool wide = dense_wide(d);
+    const int qrows = wide ? 256 : 128;
+    const int64_t items = (int64_t)((d.q_tokens + qrows - 1) / qrows) * d.B * d.H, cu = cu_count();
+    const int64_t tiles = (d.kv_tokens + 63) / 64;
+    if (tiles < 16) return 1;
+    const double scale = d.D == 64 ? 0.6 : 1.0, partial_ns = (double)d.B * d.H * d.q_tokens * (d.D + 2) * 8 / 3500;
+    int best = 1;
+    double t1 = 0, tbest = 0;
+    for (int s = 1; s <= 64 && s <= tiles / 4 && (s == 1 || items * s <= cu * (wide ? 1 : 2)); ++s) {
+        const double tile_ns = wide ? (items * s <= cu / 2 ? 1460 : 1830) : (items * s <= cu ? 1100 : 1900);
+        double t = 5000 + (double)((tiles + s - 1) / s) * tile_ns * scale;
+        if (s == 1) t1 = tbest = t;
+        else t += 6000 + s * partial_ns;
+        if (t < tbest && t < 0.9 * t1) {
+            best = s;
+            tbest = t;
+        }
+    }
+    return best;
+}
+
+size_t dense_workspace_bytes(const sfm_dense_desc& d) {
+    const int s = dense_split(d);
+    return s < 2 ? 0 : (size_t)s * d.B * d.H * d.q_tokens * (d.D + 2) * sizeof(float);
+}
+
+int launch_dense(const sfm_dense_desc& d, const void* q, const void* k, const void* v, void* out, float* lse, void* workspace,
+                 size_t workspace_bytes, hipStream_t stream) {
     const bool mfma = (d.dtype == SFM_BF16 || d.dtype == SFM_F16) && (d.D == 64 || d.D == 128);
     if (mfma) {
-        // 256 queries per workgroup (8 waves, one workgroup per compute unit) stream every K / V tile once per compute
-        // unit instead of twice; short query ranges keep 128 so that more compute units get a workgroup
-        const bool wide = (int64_t)((d.q_tokens + 255) / 256) * d.B * d.H >= cu_count() / 2;
+        const bool wide = dense_wide(d);
+        const int nsplit = workspace && workspace_bytes >= dense_workspace_bytes(d) ? dense_split(d) : 1;
+        float* const part = (float*)workspace;
         const uint16_t* qq = (const uint16_t*)q;
         const uint16_t* kk = (const uint16_t*)k;
         const uint16_t* vv = (const uint16_t*)v;
@@ -421,9 +523,9 @@ int launch_dense(const sfm_dense_desc& d, const void* q, const void* k, const vo
                 set_error("hipFuncSetAttribute failed: %s", hipGetErrorString(e));
                 return SFM_ERR_HIP;
             }
-            const int total = (d.q_tokens + 32 * nw - 1) / (32 * nw) * d.B * d.H;
+            const int total = (d.q_tokens + 32 * nw - 1) / (32 * nw) * d.B * d.H * nsplit;
             dim3 grid(xcd_grid(total));
-            hipLaunchKernelGGL(kern, grid, dim3(64 * nw), ldsb, stream, d, qq, kk, vv, oo, lse);
+            hipLaunchKernelGGL(kern, grid, dim3(64 * nw), ldsb, stream, d, qq, kk, vv, oo, lse, nsplit, part);
             return SFM_OK;
         };
         int rc;
@@ -435,6 +537,15 @@ int launch_dense(const sfm_dense_desc& d, const void* q, const void* k, const vo
             else rc = wide ? go(dense_fwd_kernel<F16, 64, 8>, 8, DnLds<64, 8>::kTotal) : go(dense_fwd_kernel<F16, 64, 4>, 4, DnLds<64, 4>::kTotal);
         }
         if (rc) return rc;
+        if (nsplit > 1) {
+            const int nsub = 1024 / d.D;
+            int groups = 1;
+            while (groups * 2 <= nsplit && groups * 2 <= nsub) groups *= 2;
+            const dim3 mg((unsigned)(((int64_t)d.B * d.H * d.q_tokens + nsub / groups - 1) / (nsub / groups)));
+            auto merge = d.dtype == SFM_BF16 ? (d.D == 128 ? dense_merge_kernel<BF16, 128> : dense_merge_kernel<BF16, 64>)
+                                             : (d.D == 128 ? dense_merge_kernel<F16, 128> : dense_merge_kernel<F16, 64>);
+            hipLaunchKernelGGL(merge, mg, dim3(256), 0, stream, d, (const float*)part, oo, lse, nsplit, groups);
+        }
     } else {
         dim3 grid(d.q_tokens, d.B * d.H);
         if (d.dtype == SFM_F32) hipLaunchKernelGGL((dense_generic_kernel<float>), grid, dim3(256), 0, stream, d, q, k, v, out, lse);

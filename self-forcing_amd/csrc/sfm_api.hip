@@ -54,8 +54,9 @@ void set_error(const char* fmt, ...) {
 int launch_kv_cache_write(int esz, int B, int H, int D, const TokMap& map, int nbf, const void* nk, const void* nv,
                           const int64_t ns[3], void* kc, void* vc, const int64_t cs[3], int64_t start,
                           hipStream_t stream);
-int launch_dense(const sfm_dense_desc& d, const void* q, const void* k, const void* v, void* out, float* lse,
-                 hipStream_t stream);
+size_t dense_workspace_bytes(const sfm_dense_desc& d);
+int launch_dense(const sfm_dense_desc& d, const void* q, const void* k, const void* v, void* out, float* lse, void* workspace,
+                 size_t workspace_bytes, hipStream_t stream);
 int launch_prologue(const sfm_prologue_desc& d, const TokMap& map, const void* xq, const void* xk, const void* xv,
                     const void* wq, const void* wk, const double* rope, void* q_out, void* kc, void* vc,
                     hipStream_t stream);
@@ -868,24 +869,48 @@ static int check_dense(const sfm_dense_desc* d) {
     return SFM_OK;
 }
 
+int sfm_dense_workspace_bytes(const sfm_dense_desc* desc, size_t* bytes) {
+    if (!bytes) {
+        set_error("bytes is NULL");
+        return SFM_ERR_NULL;
+    }
+    const int rc = check_dense(desc);
+    if (rc) return rc;
+    *bytes = dense_workspace_bytes(*desc);
+    return SFM_OK;
+}
+
 int sfm_dense_fwd(const sfm_dense_desc* desc, const void* q, const void* k, const void* v, void* out, float* lse,
                   void* stream) {
+    return sfm_dense_fwd_ws(desc, q, k, v, out, lse, nullptr, 0, stream);
+}
+
+int sfm_dense_fwd_ws(const sfm_dense_desc* desc, const void* q, const void* k, const void* v, void* out, float* lse,
+                     void* workspace, size_t workspace_bytes, void* stream) {
     int rc = check_dense(desc);
     if (rc) return rc;
     if (!q || !k || !v || !out) {
         set_error("q, k, v and out must be non-NULL");
         return SFM_ERR_NULL;
     }
-    if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out)) {
-        set_error("q, k, v and out must be 16-byte aligned");
+    if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out) || !aligned16(workspace)) {
+        set_error("q, k, v, out and the workspace must be 16-byte aligned");
         return SFM_ERR_ALIGN;
     }
-    return launch_dense(*desc, q, k, v, out, lse, (hipStream_t)stream);
+    return launch_dense(*desc, q, k, v, out, lse, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 int sfm_full_attention_with_kv_cache(const sfm_dense_desc* desc, const void* q, void* k_cache, void* v_cache,
                                      const void* new_k, const void* new_v, const int64_t new_stride[3],
                                      int64_t start_idx, int64_t end_idx, void* out, float* lse, void* stream) {
+    return sfm_full_attention_with_kv_cache_ws(desc, q, k_cache, v_cache, new_k, new_v, new_stride, start_idx, end_idx, out, lse,
+                                               nullptr, 0, stream);
+}
+
+int sfm_full_attention_with_kv_cache_ws(const sfm_dense_desc* desc, const void* q, void* k_cache, void* v_cache,
+                                        const void* new_k, const void* new_v, const int64_t new_stride[3],
+                                        int64_t start_idx, int64_t end_idx, void* out, float* lse, void* workspace,
+                                        size_t workspace_bytes, void* stream) {
     int rc = check_dense(desc);
     if (rc) return rc;
     if (!q || !k_cache || !v_cache || !out || !new_k || !new_v || !new_stride) {
@@ -902,7 +927,7 @@ int sfm_full_attention_with_kv_cache(const sfm_dense_desc* desc, const void* q, 
         return SFM_ERR_STRIDE;
     }
     if (!aligned16(q) || !aligned16(k_cache) || !aligned16(v_cache) || !aligned16(out) || !aligned16(new_k) ||
-        !aligned16(new_v)) {
+        !aligned16(new_v) || !aligned16(workspace)) {
         set_error("tensors must be 16-byte aligned");
         return SFM_ERR_ALIGN;
     }
@@ -914,7 +939,7 @@ int sfm_full_attention_with_kv_cache(const sfm_dense_desc* desc, const void* q, 
                                 v_cache, desc->k_stride, desc->kv_tokens, start_idx, end_idx, stream);
         if (rc) return rc;
     }
-    return launch_dense(*desc, q, k_cache, v_cache, out, lse, (hipStream_t)stream);
+    return launch_dense(*desc, q, k_cache, v_cache, out, lse, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 static int check_dense_bwd(const sfm_dense_bwd_desc* bd) {

@@ -24,6 +24,7 @@ ERR_NAMES = {
 SYMBOLS = [
     "sfm_monarch_workspace_bytes", "sfm_monarch_fwd", "sfm_monarch_fwd_timed", "sfm_kv_cache_write", "sfm_monarch_attn_with_kv_cache",
     "sfm_monarch_attn_with_kv_cache_static",
+    "sfm_dense_workspace_bytes", "sfm_dense_fwd_ws", "sfm_full_attention_with_kv_cache_ws",
     "sfm_dense_fwd", "sfm_full_attention_with_kv_cache", "sfm_qk_prologue", "sfm_ln_modulate", "sfm_gate_residual",
     "sfm_rms_norm", "sfm_gate_residual_ln", "sfm_linear", "sfm_monarch_bwd_workspace_bytes", "sfm_monarch_bwd", "sfm_monarch_bwd_uses_gemm",
     "sfm_monarch_stats_bytes", "sfm_monarch_fwd_stats", "sfm_monarch_bwd_saved", "sfm_dense_bwd_workspace_bytes", "sfm_dense_bwd", "sfm_probe_mfma_bf16", "sfm_probe_tile_traffic", "sfm_probe_row_stream", "sfm_probe_l2_read", "sfm_conv3d_cl", "sfm_vae_norm_act", "sfm_set_switches", "sfm_get_switches", "sfm_last_error", "sfm_version",
@@ -120,6 +121,9 @@ def load():
                                                    C.c_size_t, P]
     lib.sfm_monarch_attn_with_kv_cache_static.argtypes = [C.POINTER(MonarchDesc), P, P, P, P, P, S3, I64, I64, P, P]
     lib.sfm_dense_fwd.argtypes = [C.POINTER(DenseDesc), P, P, P, P, P, P]
+    lib.sfm_dense_workspace_bytes.argtypes = [C.POINTER(DenseDesc), C.POINTER(C.c_size_t)]
+    lib.sfm_dense_fwd_ws.argtypes = [C.POINTER(DenseDesc), P, P, P, P, P, P, C.c_size_t, P]
+    lib.sfm_full_attention_with_kv_cache_ws.argtypes = [C.POINTER(DenseDesc), P, P, P, P, P, S3, I64, I64, P, P, P, C.c_size_t, P]
     lib.sfm_full_attention_with_kv_cache.argtypes = [C.POINTER(DenseDesc), P, P, P, P, P, S3, I64, I64, P, P, P]
     lib.sfm_qk_prologue.argtypes = [C.POINTER(PrologueDesc), P, P, P, P, P, P, C.c_int32, P, P, P, P]
     lib.sfm_ln_modulate.argtypes = [C.c_int32, I64, C.c_int32, C.c_float, P, I64, P, I64, P, P, I64, C.c_int32, P, P, P]

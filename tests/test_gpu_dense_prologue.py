@@ -1,4 +1,6 @@
 """GPU parity of the dense-attention and fused-prologue kernels against the CPU oracle."""
+import ctypes as C
+
 import pytest
 import torch
 
@@ -207,3 +209,36 @@ def test_traffic_probe_moves_the_bytes_and_reports_a_duration():
         got = o0[:, t].reshape(-1, 16)          # piece c of the item's output comes from thread c % 320
         idx = torch.arange(got.shape[0], device="cuda") % 320
         assert torch.equal(got, want[idx])
+
+
+# few queries against many keys are split over the keys: 2 to 64 ranges of four tiles or more, ragged last tiles, query blocks of
+# one row up to two blocks; 8 heads x 2048 queries run the 256-query kernel in two ranges
+@pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (64, torch.bfloat16), (128, torch.float16), (64, torch.float16)])
+@pytest.mark.parametrize("B,H,nq,nk", [(1, 1, 1, 960), (1, 1, 1, 1600), (1, 2, 129, 2049), (2, 3, 128, 2112), (1, 1, 64, 16384),
+                                       (1, 1, 200, 16449), (1, 5, 255, 2500), (1, 16, 2048, 8000), (1, 25, 300, 5000)])
+def test_queries_split_over_the_keys(B, H, nq, nk, D, dtype):
+    q, k, v = (randn((B, n, H, D), 70 + i, dtype).to(DEV) for i, n in enumerate((nq, nk, nk)))
+    lib = sfa.lib.load()
+    out, lse = sfa.attention.attention(q, k, v, return_lse=True)
+    n = C.c_size_t(0)
+    d = sfa.attention._dense_desc(q, k, v, out, D ** -0.5)
+    sfa.lib.check(lib.sfm_dense_workspace_bytes(C.byref(d), C.byref(n)))
+    assert (n.value > 0) == (nk > 960)
+    whole, wlse = torch.empty_like(out), torch.empty_like(lse)
+    sfa.lib.check(lib.sfm_dense_fwd(C.byref(d), q.data_ptr(), k.data_ptr(), v.data_ptr(), whole.data_ptr(), wlse.data_ptr(),
+                                    C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    qd, kd, vd = (t.transpose(1, 2).double() for t in (q, k, v))
+    ref, rl = torch.empty_like(qd), []
+    for b in range(B):
+        for h in range(H):
+            z = qd[b, h] @ kd[b, h].T.contiguous() * D ** -0.5
+            ref[b, h] = torch.softmax(z, -1) @ vd[b, h]
+            rl.append(torch.logsumexp(z, -1))
+    ref, rl = ref.transpose(1, 2), torch.stack(rl).reshape(B, H, nq)
+    err = lambda x: ((x.double() - ref).norm() / ref.norm()).item()
+    # one rounding of P and of the output each (2^-9 for bfloat16, rms about 0.4 of it); no worse than the unsplit kernel, up to four times the
+    # spread 1 / sqrt(n) of the ratio of two such errors over n elements
+    unit = 2 ** -8 if dtype == torch.bfloat16 else 2 ** -11
+    assert err(out) < unit and err(out) < (1.02 + 4 / ref.numel() ** 0.5) * err(whole)
+    # float32 sums of nk terms around 1, logits of size about ten: 2^-24 (log2 nk + 10) rounded up
+    assert (lse.double() - rl).abs().max() < 1e-5 and (wlse.double() - rl).abs().max() < 1e-5
