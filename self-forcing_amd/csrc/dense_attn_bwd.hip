@@ -15,6 +15,8 @@
 //   dq kernel:  own = 32 queries per wave (4 waves, 128 queries per workgroup), streamed = K and V tiles.
 //   dkv kernel: own = 32 keys per wave (4 waves, 128 keys per workgroup), streamed = q and dO tiles plus the tile's
 //               log-sum-exp and delta values; three tiles in LDS, one wave per SIMD.
+// The workgroups of the last, partly filled round over the compute units (all of them for a small call) split the streamed
+// side into ranges, leave fp32 partials and a small kernel adds them; see split_last_round.
 
 #include <hip/hip_runtime.h>
 
@@ -25,6 +27,13 @@
 
 namespace sfm {
 namespace {
+
+// A grid of `items` workgroups: the first `full` fill whole rounds of the compute units, each of the others is split into
+// `ranges` workgroups.
+struct Rounds {
+    int items, full, ranges;
+    __host__ __device__ int grid() const { return full + xcd_grid((items - full) * ranges); }
+};
 
 struct DenseBwdArgs {
     const char *q, *k, *v, *out, *dout;
@@ -37,6 +46,8 @@ struct DenseBwdArgs {
     int B, H, Sq, Skv;
     int kv0, kv1;            // keys whose dK / dV are produced
     float scale;
+    Rounds rq, rkv;          // of the dq and the dkv grid
+    float* part;             // partials of the grid that is running: [last-round item][range][(dk, dv: 2)][128 rows][D]
 };
 
 typedef short db_s16x4 __attribute__((ext_vector_type(4)));
@@ -125,6 +136,20 @@ __device__ __forceinline__ u32x4 tile_tr(const char* tile, uint32_t tr_lo, uint3
     return u32x4{lo.x, lo.y, hi.x, hi.y};
 }
 
+// Workgroup -> (item, range), item < 0: nothing to do.  Either part of the grid gives each XCD one contiguous run of items
+// (`full` is a multiple of 8), so that the blocks of one (batch, head) meet in one L2.
+struct WorkItem {
+    int item, range;
+};
+__device__ __forceinline__ WorkItem work_item(const Rounds& r) {
+    const int rest = r.items - r.full, blk = (int)blockIdx.x;
+    if (blk < r.full) return {(blk % 8) * (r.full / 8) + blk / 8, 0};
+    const int total = rest * r.ranges, x = (blk % 8) * ((total + 7) / 8) + (blk - r.full) / 8;
+    if (x >= total) return {-1, 0};
+    const int range = __builtin_amdgcn_readfirstlane(x / rest);
+    return {r.full + x - range * rest, range};
+}
+
 template <class E, int D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void dense_bwd_dq_kernel(DenseBwdArgs p) {
     using T = Tile<D>;
@@ -134,8 +159,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // the query blocks of one (batch, head) go to one XCD, which then fetches that head's K / V rows once
     const int nblk = (p.Sq + 127) / 128;
-    const int item = xcd_item(nblk * p.B * p.H);
-    if (item >= nblk * p.B * p.H) return;
+    const auto [item, range] = work_item(p.rq);
+    if (item < 0) return;
     const int bh = item / nblk, b = bh / p.H, h = bh % p.H;
     const int i = (item - bh * nblk) * 128 + wave * 32 + m;
     const int ic = min(i, p.Sq - 1);
@@ -186,7 +211,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[dt][v] = 0.f;
 
-    const int nt = (p.Skv + 63) / 64;
+    const int alltiles = (p.Skv + 63) / 64;
+    const bool split = item >= p.rq.full && p.rq.ranges > 1;          // uniform
+    const int t0 = split ? __builtin_amdgcn_readfirstlane(range * alltiles / p.rq.ranges) : 0;        // this workgroup's tiles: t0 .. nt - 1
+    const int nt = split ? __builtin_amdgcn_readfirstlane((range + 1) * alltiles / p.rq.ranges) : alltiles;
     // one tile; RAGGED (only the last tile can be) masks the keys past the end
     auto tile = [&](int t, auto ragged_c) {
         constexpr bool ragged = decltype(ragged_c)::value;
@@ -251,10 +279,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    stage(0);
-    for (int t = 0; t + 1 < nt; ++t) tile(t, std::false_type{});
-    if (p.Skv % 64) tile(nt - 1, std::true_type{});
+    stage(t0);
+    for (int t = t0; t + 1 < nt; ++t) tile(t, std::false_type{});
+    if (p.Skv % 64 && nt == alltiles) tile(nt - 1, std::true_type{});
     else tile(nt - 1, std::false_type{});
+    if (split) {
+        float* const row = p.part + (((int64_t)(item - p.rq.full) * p.rq.ranges + range) * 128 + wave * 32 + m) * D + 4 * hf;
+#pragma unroll
+        for (int dt = 0; dt < T::DT; ++dt)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                *(f32x4*)(row + 32 * dt + 8 * g) = f32x4{acc[dt][4 * g], acc[dt][4 * g + 1], acc[dt][4 * g + 2], acc[dt][4 * g + 3]};
+        return;
+    }
     if (i < p.Sq) {
         float* row = p.dq + (int64_t)b * p.dqs[0] + (int64_t)i * p.dqs[1] + (int64_t)h * p.dqs[2] + 4 * hf;
 #pragma unroll
@@ -282,8 +319,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // the key blocks of one (batch, head) go to one XCD, which then fetches that head's q / dO rows once
     const int nblk = (p.kv1 - p.kv0 + 127) / 128;
-    const int item = xcd_item(nblk * p.B * p.H);
-    if (item >= nblk * p.B * p.H) return;
+    const auto [item, range] = work_item(p.rkv);
+    if (item < 0) return;
     const int bh = item / nblk, b = bh / p.H, h = bh % p.H;
     const int l = p.kv0 + (item - bh * nblk) * 128 + wave * 32 + m;
     const int lc = min(l, p.kv1 - 1);
@@ -337,7 +374,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 #pragma unroll
         for (int v = 0; v < 16; ++v) dka[dt][v] = dva[dt][v] = 0.f;
 
-    const int nt = (p.Sq + 63) / 64;
+    const int alltiles = (p.Sq + 63) / 64;
+    const bool split = item >= p.rkv.full && p.rkv.ranges > 1;        // uniform
+    const int t0 = split ? __builtin_amdgcn_readfirstlane(range * alltiles / p.rkv.ranges) : 0;       // this workgroup's tiles: t0 .. nt - 1
+    const int nt = split ? __builtin_amdgcn_readfirstlane((range + 1) * alltiles / p.rkv.ranges) : alltiles;
     // one tile; RAGGED (only the last tile can be) masks the queries past the end
     auto tile = [&](int t, auto ragged_c) {
         constexpr bool ragged = decltype(ragged_c)::value;
@@ -429,11 +469,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    stage(0);
-    if (nt > 1) stage(1);
-    for (int t = 0; t + 1 < nt; ++t) tile(t, std::false_type{});
-    if (p.Sq % 64) tile(nt - 1, std::true_type{});
+    stage(t0);
+    if (t0 + 1 < nt) stage(t0 + 1);
+    for (int t = t0; t + 1 < nt; ++t) tile(t, std::false_type{});
+    if (p.Sq % 64 && nt == alltiles) tile(nt - 1, std::true_type{});
     else tile(nt - 1, std::false_type{});
+    if (split) {
+        float* const row = p.part + (((int64_t)(item - p.rkv.full) * p.rkv.ranges + range) * 256 + wave * 32 + m) * D + 4 * hf;
+#pragma unroll
+        for (int dt = 0; dt < T::DT; ++dt)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                *(f32x4*)(row + 32 * dt + 8 * g) = f32x4{dka[dt][4 * g], dka[dt][4 * g + 1], dka[dt][4 * g + 2], dka[dt][4 * g + 3]};
+                *(f32x4*)(row + 128 * D + 32 * dt + 8 * g) = f32x4{dva[dt][4 * g], dva[dt][4 * g + 1], dva[dt][4 * g + 2], dva[dt][4 * g + 3]};
+            }
+        return;
+    }
     // lane (key, hf) holds head-dim 32 dt + 8 g + 4 hf + 0..3; the half swap leaves 8 consecutive ones per lane
     const int64_t obase = ((int64_t)b * p.dks[0] + (int64_t)(lc - p.kv0) * p.dks[1] + (int64_t)h * p.dks[2]) * 2;
     auto store = [&](char* dst, const f32x16& a, int dt, float sc) {
@@ -453,6 +504,80 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     }
 }
 
+// Adds the partials of the last round: eight values per thread.  KV: dK and dV in the tensor dtype, else dq in float.
+template <class E, int D, bool KV>
+__global__ __launch_bounds__(256) void dense_bwd_sum_kernel(DenseBwdArgs p) {
+    constexpr int CH = D / 8, ROWS = KV ? 256 : 128;       // rows of a partial (dK's 128, then dV's)
+    const Rounds& r = KV ? p.rkv : p.rq;
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int ch = (int)(t % CH), prow = (int)(t / CH % ROWS), rest = (int)(t / CH / ROWS);
+    if (rest >= r.items - r.full) return;
+    const int nblk = ((KV ? p.kv1 - p.kv0 : p.Sq) + 127) / 128;
+    const int item = r.full + rest, bh = item / nblk, b = bh / p.H, h = bh % p.H;
+    const int row = (item - bh * nblk) * 128 + prow % 128;
+    if (row >= (KV ? p.kv1 - p.kv0 : p.Sq)) return;
+    const float* src = p.part + ((int64_t)rest * r.ranges * ROWS + prow) * D + 8 * ch;
+    f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;
+    for (int x = 0; x < r.ranges; ++x, src += (int64_t)ROWS * D) {
+        lo += *(const f32x4*)src;
+        hi += *(const f32x4*)(src + 4);
+    }
+    const float sc = KV && prow >= 128 ? 1.f : p.scale;
+    lo *= sc;
+    hi *= sc;
+    if constexpr (KV) {
+        char* const dst = (prow < 128 ? p.dk : p.dv) + ((int64_t)b * p.dks[0] + (int64_t)row * p.dks[1] + (int64_t)h * p.dks[2]) * 2 + 16 * ch;
+        *(u32x4*)dst = u32x4{pack2<E>(lo.x, lo.y), pack2<E>(lo.z, lo.w), pack2<E>(hi.x, hi.y), pack2<E>(hi.z, hi.w)};
+    } else {
+        float* const dst = p.dq + (int64_t)b * p.dqs[0] + (int64_t)row * p.dqs[1] + (int64_t)h * p.dqs[2] + 8 * ch;
+        *(f32x4*)dst = lo;
+        *(f32x4*)(dst + 4) = hi;
+    }
+}
+
+// The rounds of a grid of `items` workgroups over `tiles` streamed tiles each, of which the chip holds `slots` at once.  The
+// last, partly filled round (1320 key blocks on 256 compute units: 40 blocks in a sixth round) is split into ranges where a
+// model of its time in ns says that saves a tenth: a tile takes `tile_ns` with the chip full, `half_ns` on half of the slots
+// or fewer; the sum's launch 5000, and the partials (`floats` each) are written and read at 3.5 TB/s.  Measured:
+//     heads x queries x keys, us    before  now           heads x queries x keys, new keys' gradients only    before  now
+//     12 x 4680 x 14040 (dkv)         1132  1028           9 x 1000 x 5000                                       154   94
+//     1 x 500 x 16000                  365    64           21 x 202 x 2804                                        84   46
+//     1 x 4000 x 500                   153    46           3 x 4680 x 4680                                       267  177
+Rounds split_last_round(int64_t items, int tiles, int slots, double tile_ns, double half_ns, int floats) {
+    Rounds r;
+    r.items = (int)items;
+    r.full = (int)(items / slots * slots);
+    r.ranges = 1;
+    const int64_t rest = items - r.full;
+    if (rest == 0 || r.full % 8) {                         // (a chip whose slots are no multiple of 8: nothing is split)
+        r.full = r.full % 8 ? 0 : r.full;
+        return r;
+    }
+    double best = 0;
+    for (int n = 1; n <= 64 && n <= tiles / 2 + 1 && rest * n <= slots; ++n) {
+        double t = (double)((tiles + n - 1) / n) * (rest * n <= slots / 2 ? half_ns : tile_ns);
+        if (n == 1) best = 0.9 * t;
+        else if ((t += 5000 + (double)rest * n * floats * 8 / 3500) < best) {
+            best = t;
+            r.ranges = n;
+        }
+    }
+    return r;
+}
+
+void plan_rounds(int64_t units, int Sq, int Skv, int nkv, int D, Rounds* rq, Rounds* rkv) {
+    const double f = D == 64 ? 0.55 : 1.0;
+    *rq = split_last_round((Sq + 127) / 128 * units, (Skv + 63) / 64, 2 * cu_count(), 2640 * f, 1500 * f, 128 * D);
+    *rkv = split_last_round((nkv + 127) / 128 * units, (Sq + 63) / 64, cu_count(), 2550 * f, 2100 * f, 256 * D);
+}
+
+// floats of the partials (the two grids run one after the other and share them)
+int64_t part_floats(const Rounds& rq, const Rounds& rkv, int D) {
+    const int64_t q = rq.ranges > 1 ? (int64_t)(rq.items - rq.full) * rq.ranges * 128 * D : 0;
+    const int64_t kv = rkv.ranges > 1 ? (int64_t)(rkv.items - rkv.full) * rkv.ranges * 256 * D : 0;
+    return q > kv ? q : kv;
+}
+
 template <class E, int D>
 int launch_t(const DenseBwdArgs& a, hipStream_t stream) {
     using T = Tile<D>;
@@ -469,9 +594,13 @@ int launch_t(const DenseBwdArgs& a, hipStream_t stream) {
             return SFM_ERR_HIP;
         }
     }
-    hipLaunchKernelGGL((dense_bwd_dq_kernel<E, D>), dim3(xcd_grid((a.Sq + 127) / 128 * a.B * a.H)), dim3(256), lds_dq, stream, a);
-    if (a.kv1 > a.kv0)
-        hipLaunchKernelGGL((dense_bwd_dkv_kernel<E, D>), dim3(xcd_grid((a.kv1 - a.kv0 + 127) / 128 * a.B * a.H)), dim3(256), lds_dkv, stream, a);
+    auto sum_grid = [&](const Rounds& r, int rows) { return dim3((unsigned)(((int64_t)(r.items - r.full) * rows * (D / 8) + 255) / 256)); };
+    hipLaunchKernelGGL((dense_bwd_dq_kernel<E, D>), dim3(a.rq.grid()), dim3(256), lds_dq, stream, a);
+    if (a.rq.ranges > 1) hipLaunchKernelGGL((dense_bwd_sum_kernel<E, D, false>), sum_grid(a.rq, 128), dim3(256), 0, stream, a);
+    if (a.kv1 > a.kv0) {
+        hipLaunchKernelGGL((dense_bwd_dkv_kernel<E, D>), dim3(a.rkv.grid()), dim3(256), lds_dkv, stream, a);
+        if (a.rkv.ranges > 1) hipLaunchKernelGGL((dense_bwd_sum_kernel<E, D, true>), sum_grid(a.rkv, 256), dim3(256), 0, stream, a);
+    }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         set_error("dense backward: launch failed: %s", hipGetErrorString(e));
@@ -484,9 +613,18 @@ int launch_t(const DenseBwdArgs& a, hipStream_t stream) {
 
 bool dense_bwd_supported(int dtype, int D) { return (dtype == SFM_BF16 || dtype == SFM_F16) && (D == 64 || D == 128); }
 
+// two floats per (batch, head, query), then the partials
+static size_t row_values_bytes(const sfm_dense_desc& d) { return ((size_t)2 * d.B * d.H * d.q_tokens * sizeof(float) + 255) / 256 * 256; }
+
+size_t dense_bwd_workspace_bytes(const sfm_dense_desc& d, int64_t kv0, int64_t kv1) {
+    Rounds rq, rkv;
+    plan_rounds((int64_t)d.B * d.H, d.q_tokens, d.kv_tokens, (int)(kv1 - kv0), d.D, &rq, &rkv);
+    return row_values_bytes(d) + (size_t)part_floats(rq, rkv, d.D) * sizeof(float);
+}
+
 int launch_dense_bwd(const sfm_dense_desc& d, const int64_t* dq_stride, const int64_t* dkv_stride, int64_t kv0, int64_t kv1,
                      const void* q, const void* k, const void* v, const void* out, const float* lse, const void* dout, float* dq,
-                     void* dk, void* dv, float* scratch, hipStream_t stream) {
+                     void* dk, void* dv, float* scratch, size_t scratch_bytes, hipStream_t stream) {
     if (!dense_bwd_supported(d.dtype, d.D)) {
         set_error("dense backward: bf16 / fp16 tensors with head_dim 64 or 128 only");
         return SFM_ERR_UNSUPPORTED;
@@ -513,6 +651,9 @@ int launch_dense_bwd(const sfm_dense_desc& d, const int64_t* dq_stride, const in
     a.B = d.B; a.H = d.H; a.Sq = d.q_tokens; a.Skv = d.kv_tokens;
     a.kv0 = (int)kv0; a.kv1 = (int)kv1;
     a.scale = d.sm_scale;
+    plan_rounds((int64_t)a.B * a.H, a.Sq, a.Skv, a.kv1 - a.kv0, d.D, &a.rq, &a.rkv);
+    a.part = (float*)((char*)scratch + row_values_bytes(d));
+    if (scratch_bytes < dense_bwd_workspace_bytes(d, kv0, kv1)) a.rq.ranges = a.rkv.ranges = 1;      // no room for partials
     if (d.dtype == SFM_BF16) return d.D == 128 ? launch_t<BF16, 128>(a, stream) : launch_t<BF16, 64>(a, stream);
     return d.D == 128 ? launch_t<F16, 128>(a, stream) : launch_t<F16, 64>(a, stream);
 }

@@ -972,7 +972,7 @@ int sfm_dense_bwd_workspace_bytes(const sfm_dense_bwd_desc* desc, size_t* bytes)
     }
     int rc = check_dense_bwd(desc);
     if (rc) return rc;
-    *bytes = ((size_t)2 * desc->fwd.B * desc->fwd.H * desc->fwd.q_tokens * sizeof(float) + 255) / 256 * 256;
+    *bytes = dense_bwd_workspace_bytes(desc->fwd, desc->kv_grad_start, desc->kv_grad_end);
     return SFM_OK;
 }
 
@@ -996,7 +996,7 @@ int sfm_dense_bwd(const sfm_dense_bwd_desc* desc, const void* q, const void* k, 
         return SFM_ERR_WORKSPACE;
     }
     return launch_dense_bwd(desc->fwd, desc->dq_stride, desc->dkv_stride, desc->kv_grad_start, desc->kv_grad_end, q, k, v, out, lse,
-                            dout, dq, dk, dv, (float*)workspace, (hipStream_t)stream);
+                            dout, dq, dk, dv, (float*)workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 int sfm_qk_prologue(const sfm_prologue_desc* d, const void* xq, const void* xk, const void* xv, const void* wq,

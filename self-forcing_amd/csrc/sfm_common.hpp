@@ -246,11 +246,13 @@ int launch_monarch_bwd_dqk(int dtype, int D, int64_t nuk, int b1, int b2, int AJ
                            const TokMap& kmap, const void* ds1, float* dqk, const int64_t* dqs, const TokMap& qmap, int H, int unit0,
                            hipStream_t stream);
 
-// backward of the dense attention (dense_attn_bwd.hip); scratch is 2*B*H*q_tokens floats
+// backward of the dense attention (dense_attn_bwd.hip); with less scratch than this (2*B*H*q_tokens floats at least) no
+// workgroup is split
+size_t dense_bwd_workspace_bytes(const sfm_dense_desc& d, int64_t kv0, int64_t kv1);
 bool dense_bwd_supported(int dtype, int D);
 int launch_dense_bwd(const sfm_dense_desc& d, const int64_t* dq_stride, const int64_t* dkv_stride, int64_t kv0, int64_t kv1,
                      const void* q, const void* k, const void* v, const void* out, const float* lse, const void* dout, float* dq,
-                     void* dk, void* dv, float* scratch, hipStream_t stream);
+                     void* dk, void* dv, float* scratch, size_t scratch_bytes, hipStream_t stream);
 
 void set_error(const char* fmt, ...);
 int cu_count();                                  // compute units of the current device (cached per thread)

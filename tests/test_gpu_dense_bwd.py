@@ -2,6 +2,8 @@
 through the float64 oracle.  The oracle's dense attention is a plain softmax(q k^T s) v in torch (oracle/dense.py),
 pinned by the golden vectors and closed forms of tests/test_oracle_dense_prologue.py; its autograd gradient is the
 mathematical one."""
+import ctypes as C
+
 import pytest
 import torch
 
@@ -82,3 +84,56 @@ def test_dense_backward_argument_checks():
     out = sfa.attention.attention(q, q, q)
     with pytest.raises(Exception):
         out.sum().backward()
+
+
+@pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (64, torch.float16)])
+@pytest.mark.parametrize("B,H,Lq,Lk,kv0", [
+    (1, 1, 1, 64, 0),              # one tile on either side: nothing to split
+    (1, 1, 130, 4001, 0),          # two query blocks against 63 key tiles; ragged last tile in the last range
+    (2, 3, 2001, 100, 0),          # one key block per head against 32 query tiles
+    (1, 5, 3000, 6600, 0),         # 260 key blocks: one whole round of 256 compute units and four blocks of a second
+    (1, 7, 700, 2500, 1801),       # gradients of the last keys only, from an odd key on
+    (1, 2, 500, 900, 900),         # dq only
+])
+def test_last_round_split_into_ranges(B, H, Lq, Lk, kv0, D, dtype):
+    """sfm_dense_bwd with the queried workspace, which lets the last round's workgroups be split, and with the smallest one,
+    which does not: the split gradients are as close to float64 as the unsplit ones, and nothing is written behind the
+    workspace."""
+    q, do = (randn((B, Lq, H, D), 600 + i, dtype).to(DEV) for i in range(2))
+    k, v = (randn((B, Lk, H, D), 602 + i, dtype).to(DEV) for i in range(2))
+    s = D ** -0.5
+    out, lse = sfa.attention.attention(q, k, v, return_lse=True)
+    lib, stream = sfa.lib.load(), C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    got = []
+    for smallest in (False, True):
+        dq = torch.full((B, Lq, H, D), float("nan"), device=DEV)
+        dk, dv = (torch.full((B, Lk - kv0, H, D), float("nan"), dtype=dtype, device=DEV) for _ in range(2))
+        bd = sfa.lib.DenseBwdDesc()
+        bd.fwd = sfa.attention._dense_desc(q, k, v, out, s)
+        bd.dq_stride, bd.dkv_stride = sfa.lib.strides3(dq), sfa.lib.strides3(dk)
+        bd.kv_grad_start, bd.kv_grad_end = kv0, Lk
+        n = C.c_size_t(0)
+        sfa.lib.check(lib.sfm_dense_bwd_workspace_bytes(C.byref(bd), C.byref(n)))
+        nbytes = 2 * B * H * Lq * 4 if smallest else n.value
+        ws = torch.full((nbytes + 1024,), 0x5a, dtype=torch.uint8, device=DEV)
+        sfa.lib.check(lib.sfm_dense_bwd(C.byref(bd), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(), do.data_ptr(),
+                                        dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), nbytes, stream))
+        assert bool((ws[nbytes:] == 0x5a).all())
+        got.append((dq, dk, dv))
+    f = lambda t, b, h: t[b, :, h].double()
+    num, den = torch.zeros(2, 3), torch.zeros(3)
+    for b in range(B):
+        for h in range(H):
+            p = torch.softmax(f(q, b, h) @ f(k, b, h).T.contiguous() * s, -1)
+            dp = f(do, b, h) @ f(v, b, h).T.contiguous()
+            ds = p * (dp - (p * dp).sum(-1, keepdim=True)) * s
+            ref = (ds @ f(k, b, h), (ds.T.contiguous() @ f(q, b, h))[kv0:], (p.T.contiguous() @ f(do, b, h))[kv0:])
+            for x, r in enumerate(ref):
+                den[x] += r.square().sum().cpu()
+                for y in range(2):
+                    num[y, x] += (f(got[y][x], b, h) - r).square().sum().cpu()
+    # P, dS and a 16-bit gradient are rounded once each, delta comes from a rounded output: two units of the last place
+    unit = 2 ** -7 if dtype == torch.bfloat16 else 2 ** -10
+    for x in range(3 if Lk > kv0 else 1):
+        split, whole = ((num[y, x] / den[x]).sqrt() for y in range(2))
+        assert split < unit and split < 1.02 * whole + 1e-6
