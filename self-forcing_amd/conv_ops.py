@@ -79,7 +79,18 @@ def release_padded():
     _PADDED.clear()
 
 
-def conv_cl(x, conv, history=None, up2x=False, norm=None, want_tail=False, res=None):
+def padded_input(T, H, W, conv, dtype, device):
+    """(padded buffer, its interior [T, H, W, Cin]) for conv_cl of T frames without history: who fills the whole interior
+    passes it as `x` with the buffer as `padded`, and no copy is left."""
+    _, _, kt, k, _, cin, cin_p, _ = prepared(conv, dtype, device)
+    pad = (k - 1) // 2
+    xp, new = _padded((T + kt - 1, H + 2 * pad, W + 2 * pad, cin_p), cin, dtype, device)
+    if kt > 1 and not new:
+        xp[:kt - 1].zero_()
+    return xp, xp[kt - 1:, pad:pad + H, pad:pad + W, :cin]
+
+
+def conv_cl(x, conv, history=None, up2x=False, norm=None, want_tail=False, res=None, padded=None):
     """x [T, H, W, Cin] -> [T, H', W', Cout] for a causal Conv3d (kt - 1 frames of `history`, zeros where it is
     shorter) or a Conv2d applied per frame; with up2x the nearest x2 upsampling in front of a 3x3 Conv2d is folded
     into the convolution (H' = 2 H, W' = 2 W).  With norm = (gamma, act) the convolution's input is
@@ -92,7 +103,9 @@ def conv_cl(x, conv, history=None, up2x=False, norm=None, want_tail=False, res=N
     T, H, W, _ = x.shape
     past = kt - 1
     pad = (k - 1) // 2
-    if past == 0 and pad == 0 and cin_p == cin and x.is_contiguous() and norm is None:
+    if padded is not None:
+        xp = padded
+    elif past == 0 and pad == 0 and cin_p == cin and x.is_contiguous() and norm is None:
         xp = x
     else:
         xp, new = _padded((T + past, H + 2 * pad, W + 2 * pad, cin_p), cin, x.dtype, x.device)

@@ -121,3 +121,21 @@ def test_hip_convolution_path_reproduces_the_reference_output(dtype, split):
     err = (torch.cat(outs, 1).cpu().double() - want).abs()
     bar = (6e-2, 8e-3) if dtype == torch.bfloat16 else (1e-2, 1.5e-3)
     assert err.max() < bar[0] and err.mean() < bar[1], (err.max().item(), err.mean().item())
+
+
+@pytest.mark.parametrize("splits", [(1,), (2,), (1, 1), (2, 1, 2), (1, 3), (4, 1), (5,)])
+def test_first_frame_of_a_stream_goes_with_any_others(splits):
+    """The temporal upsamplers treat a stream's first frame apart from whatever else the call carries: every way to cut a
+    stream gives the pixels of a one-shot decode, which keeps no tails, and of the frame-by-frame oracle."""
+    m = _decoder(torch.float16, seed=18)
+    n = sum(splits)
+    lat = torch.randn(1, n, 16, 6, 5, generator=torch.Generator().manual_seed(19)).to(torch.float16)
+    want = ov.decode_to_pixel(lat.double(), {k: v.cpu() for k, v in m.state_dict().items()})
+    st, outs, t0 = m.new_state(), [], 0
+    for c in splits:
+        outs.append(m.decode_to_pixel(lat[:, t0:t0 + c].cuda(), use_cache=True, state=st))
+        t0 += c
+    whole = m.decode_to_pixel(lat.cuda())
+    for got in (torch.cat(outs, 1), whole):
+        err = (got.cpu().double() - want).abs()
+        assert got.shape == want.shape and err.max() < 1.5e-2 and err.mean() < 2e-3      # the float16 stream's bar above
