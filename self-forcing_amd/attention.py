@@ -9,27 +9,20 @@ import warnings
 import torch
 
 from . import lib as _l
-from .monarch_attn import _DT, _check4, _stream, scratch as _scratch
+from .monarch_attn import _DT, _check4, _on_device, _stream, scratch as _scratch
 
 
 def _dense_desc(q, k, v, out, sm_scale):
-    d = _l.DenseDesc()
-    d.dtype = _DT[q.dtype]
-    d.B, d.q_tokens, d.H, d.D = q.shape
-    d.kv_tokens = k.shape[1]
-    d.sm_scale = float(sm_scale)
-    d.q_stride = _l.strides3(q)
-    d.k_stride = _l.strides3(k)
-    d.v_stride = _l.strides3(v)
-    d.o_stride = _l.strides3(out)
-    return d
+    B, q_tokens, H, D = q.shape
+    return _l.DenseDesc(_DT[q.dtype], B, H, D, q_tokens, k.shape[1], float(sm_scale), q.stride()[:3], k.stride()[:3], v.stride()[:3],
+                        out.stride()[:3])
 
 
 def _dense_fwd(q, k, v, sm_scale, want_lse):
     out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     lse = torch.empty((q.shape[0], q.shape[2], q.shape[1]), dtype=torch.float32, device=q.device) if want_lse else None
     d = _dense_desc(q, k, v, out, sm_scale)
-    with torch.cuda.device(q.device):
+    with _on_device(q.device):
         ws, nbytes = _dense_workspace(d, q.device)
         _l.check(_l.load().sfm_dense_fwd_ws(C.byref(d), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
                                             lse.data_ptr() if want_lse else None, ws.data_ptr() if nbytes else None, nbytes, _stream(q)))
@@ -62,7 +55,7 @@ def _dense_bwd(q, k, v, out, lse, dout, sm_scale, kv0=0, kv1=None):
     n = C.c_size_t(0)
     _l.check(_l.load().sfm_dense_bwd_workspace_bytes(C.byref(bd), C.byref(n)))
     ws = _scratch(n.value, q.device)
-    with torch.cuda.device(q.device):
+    with _on_device(q.device):
         _l.check(_l.load().sfm_dense_bwd(C.byref(bd), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
                                          dout.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), n.value,
                                          _stream(q)))
@@ -170,7 +163,7 @@ def _dense_cache_fwd(q, k_cache, v_cache, new_k, new_v, start_idx, end_idx, sm_s
     out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     lse = torch.empty((q.shape[0], q.shape[2], q.shape[1]), dtype=torch.float32, device=q.device) if want_lse else None
     d = _dense_desc(q, k_cache, v_cache, out, sm_scale)
-    with torch.cuda.device(q.device):
+    with _on_device(q.device):
         ws, nbytes = _dense_workspace(d, q.device)
         _l.check(_l.load().sfm_full_attention_with_kv_cache_ws(
             C.byref(d), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), new_k.data_ptr(), new_v.data_ptr(),

@@ -11,6 +11,7 @@ num_iters > 1 runs the alternating refinement the reference implements in pure t
 kernels and its backward differentiates a torch restatement of the passes on the GPU (the reference's own refinement is
 differentiable torch and has no backward kernels either).
 """
+import contextlib
 import ctypes as C
 
 import torch
@@ -37,21 +38,20 @@ def _desc(q, k, v, out, f_tied, h_reduce, w_reduce, h, w, sm_scale, kv_block_ord
           one_kernel=False):
     if q.dtype not in _DT:
         raise ValueError(f"unsupported dtype {q.dtype}")
-    d = _l.MonarchDesc()
-    d.dtype = _DT[q.dtype]
-    d.B, d.q_tokens, d.H, d.D = q.shape
-    d.kv_tokens = k.shape[1]
-    d.tiling = _l.Tiling(f_tied, h_reduce, w_reduce, h, w)
-    d.kv_block_order = kv_block_order
-    d.causal_block_frames = causal_block_frames
-    d.sm_scale = float(sm_scale)
-    d.num_iters = int(num_iters)
-    d.flags = _l.SFM_MONARCH_ONE_KERNEL if one_kernel else 0
-    d.q_stride = _l.strides3(q)
-    d.k_stride = _l.strides3(k)
-    d.v_stride = _l.strides3(v)
-    d.o_stride = _l.strides3(out)
-    return d
+    B, q_tokens, H, D = q.shape
+    # all fields in one call: one by one they take twice as long, a seventh of a small call's host time
+    return _l.MonarchDesc(_DT[q.dtype], B, H, D, q_tokens, k.shape[1], (f_tied, h_reduce, w_reduce, h, w), kv_block_order,
+                          causal_block_frames, float(sm_scale), int(num_iters), _l.SFM_MONARCH_ONE_KERNEL if one_kernel else 0,
+                          q.stride()[:3], k.stride()[:3], v.stride()[:3], out.stride()[:3])
+
+
+_raw_stream = torch._C._cuda_getCurrentRawStream      # torch.cuda.current_stream(device).cuda_stream without the Stream object
+_HERE = contextlib.nullcontext()
+
+
+def _on_device(device):
+    """torch.cuda.device(device), or nothing where it is the current device already."""
+    return _HERE if torch.cuda.current_device() == device.index else torch.cuda.device(device)
 
 
 _SCRATCH = {}
@@ -61,7 +61,8 @@ def scratch(nbytes, device):
     """The library's workspace for a call on `device`'s current stream: one grow-only byte buffer per (device, stream),
     so that steady-state calls allocate nothing (a caller recording a HIP graph warms the buffer up with one eager
     call first).  Calls on one stream are ordered, so they can share it; `release_scratch()` gives the memory back."""
-    key = (device.index if device.index is not None else torch.cuda.current_device(), torch.cuda.current_stream(device).cuda_stream)
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    key = (index, _raw_stream(index))
     buf = _SCRATCH.get(key)
     if buf is None or buf.numel() < nbytes:
         buf = _SCRATCH[key] = torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
@@ -79,7 +80,7 @@ def monarch_workspace_bytes(desc, heads_per_pass=0):
 
 
 def _stream(t):
-    return C.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return C.c_void_p(_raw_stream(t.device.index))
 
 
 def _from_block_order(x, f_tied, h_reduce, w_reduce, h, w):
@@ -116,7 +117,7 @@ def kv_cache_write(new_k, new_v, k_cache, v_cache, start_idx, end_idx, f_tied, h
     if k_cache.stride() != v_cache.stride():
         raise ValueError("k_cache and v_cache must share their strides")
     B, _, H, D = new_k.shape
-    with torch.cuda.device(new_k.device):
+    with _on_device(new_k.device):
         _l.check(_l.load().sfm_kv_cache_write(_DT[new_k.dtype], B, H, D, C.byref(_l.Tiling(f_tied, h_reduce, w_reduce, h, w)),
                                               new_k.data_ptr(), new_v.data_ptr(), _l.strides3(new_k), k_cache.data_ptr(),
                                               v_cache.data_ptr(), _l.strides3(k_cache), k_cache.shape[1], start_idx, end_idx,
@@ -134,7 +135,7 @@ def _monarch_fwd_stats(q, k, v, tiling, sm_scale, kv_block_order, cbf, heads_per
     nbytes = monarch_workspace_bytes(d, heads_per_pass)
     ws = scratch(nbytes, q.device)
     stats = torch.empty(n.value // 4, dtype=torch.float32, device=q.device) if n.value else None
-    with torch.cuda.device(q.device):
+    with _on_device(q.device):
         if stats is None:
             _l.check(_l.load().sfm_monarch_fwd(C.byref(d), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
                                                ws.data_ptr(), nbytes, _stream(q)))
@@ -168,7 +169,7 @@ def _monarch_bwd(q, k, v, dout, tiling, sm_scale, kv_block_order, cbf, kv_f0=0, 
     n = C.c_size_t(0)
     _l.check(_l.load().sfm_monarch_bwd_workspace_bytes(C.byref(bd), heads_per_pass, C.byref(n)))
     ws = scratch(n.value, q.device)
-    with torch.cuda.device(q.device):
+    with _on_device(q.device):
         if out is None or stats is None:
             _l.check(_l.load().sfm_monarch_bwd(C.byref(bd), q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(),
                                                dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), n.value,
@@ -388,7 +389,7 @@ def monarch_attn_with_kv_cache(q, k_cache, v_cache, new_k, new_v, start_idx, end
     d = _desc(q, k_cache, v_cache, out, f_tied, h_reduce, w_reduce, h, w, sm_scale, 1, 0, num_iters, one_kernel)
     nbytes = monarch_workspace_bytes(d, heads_per_pass)
     ws = scratch(nbytes, q.device)
-    with torch.cuda.device(q.device):
+    with _on_device(q.device):
         _l.check(_l.load().sfm_monarch_attn_with_kv_cache(
             C.byref(d), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), new_k.data_ptr(), new_v.data_ptr(),
             _l.strides3(new_k), start_idx, end_idx, out.data_ptr(), ws.data_ptr(), nbytes, _stream(q)))
@@ -416,7 +417,7 @@ def monarch_attn_with_kv_cache_static(q, k_cache, v_cache, new_k, new_v, start_i
         if out.shape != q.shape:
             raise ValueError("out must have q's shape")
     d = _desc(q, k_cache, v_cache, out, f_tied, h_reduce, w_reduce, h, w, sm_scale, 1, 0, num_iters)
-    with torch.cuda.device(q.device):
+    with _on_device(q.device):
         _l.check(_l.load().sfm_monarch_attn_with_kv_cache_static(
             C.byref(d), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), new_k.data_ptr(), new_v.data_ptr(),
             _l.strides3(new_k), start_idx, end_idx, out.data_ptr(), _stream(q)))
@@ -451,7 +452,7 @@ def monarch_attn(q, k, v, f_tied, h_reduce, w_reduce, h, w, sm_scale=None, block
     d = _desc(q, k, v, out, f_tied, h_reduce, w_reduce, h, w, sm_scale, 1 if kv_block_order else 0, cbf, num_iters, one_kernel)
     nbytes = monarch_workspace_bytes(d, heads_per_pass)
     ws = scratch(nbytes, q.device)
-    with torch.cuda.device(q.device):
+    with _on_device(q.device):
         _l.check(_l.load().sfm_monarch_fwd(C.byref(d), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
                                            ws.data_ptr(), nbytes, _stream(q)))
     return out
