@@ -516,6 +516,7 @@ int run(const MonarchBwdArgs& g, int n, void* workspace, hipStream_t stream) {
 
     const int64_t nseg = (int64_t)n * b1 * AJ * nf;
     const bool fused_left = parts.left, fused_fwd = parts.fwd, fused_dqa = parts.dqa, fused_right = parts.right;
+    const bool skip = p.causal && parts.left && parts.fwd && parts.dqa && parts.right && parts.dqk;     // masked pairs are left out
     const bool dq_direct = parts.dqa && parts.dqk;       // both parts of dq go to the caller's rows
     const int ds2_ld = fused_left ? (RR + 7) / 8 * 8 : RR;
     const int rb_ld = fused_fwd ? 64 : b2;
@@ -566,6 +567,7 @@ int run(const MonarchBwdArgs& g, int n, void* workspace, hipStream_t stream) {
         f1.y = ws + lay.Y;
         f1.cl = (float*)(ws + lay.c);
         f1.rb = ws + lay.Rb;
+        f1.skip_masked = skip;
         f1.ws_unit = (uint32_t)((int64_t)RR * AJ);
         f1.ws_aj = 1;
         f1.ws_row = (uint32_t)(nf * AJ);
@@ -590,7 +592,7 @@ int run(const MonarchBwdArgs& g, int n, void* workspace, hipStream_t stream) {
                                                 g.dos, p.qmap, H, p.unit0, ws + lay.Kbar, ws + lay.Y, (const float*)(ws + lay.c),
                                                 fused_fwd ? 1 : 0, ws + lay.dKbar, ws + lay.dY, (float*)(ws + lay.dc),
                                                 fused_dqa ? nullptr : ws + lay.dS2, ds2_ld,
-                                                !fused_dqa ? nullptr : dq_direct ? g.dq : (float*)(ws + lay.dQa), dq_direct ? g.dqs : nullptr, saved ? g.fstats : nullptr, (b1 + 31) / 32 * 32, stream);
+                                                !fused_dqa ? nullptr : dq_direct ? g.dq : (float*)(ws + lay.dQa), dq_direct ? g.dqs : nullptr, saved ? g.fstats : nullptr, (b1 + 31) / 32 * 32, skip, stream);
     } else {
         // 4, 5. per unit and (a, j): S2 = q_i . Kbar_r, dLm = dO_i . Y_r; the [RR x D] matrix of column aj is every AJ-th row
         for (int u = 0; u < n && !cx.status; ++u) {
@@ -630,7 +632,7 @@ int run(const MonarchBwdArgs& g, int n, void* workspace, hipStream_t stream) {
         if (!cx.status)
             cx.status = launch_monarch_bwd_right(left_dtype<E>(), D, nt, b1, b2, AJ, nf, s, p.k, p.ks, p.v, p.vs, ws + lay.Rb,
                                                  ws + lay.dKbar, ws + lay.dY, (const float*)(ws + lay.dc), p.q, p.qs, p.qmap, ws + lay.dS1, g.dk,
-                                                 g.dv, g.dks, g.dk_row0, p.kmap, H, p.unit0, g.kv_f0, g.kv_f1, stream);
+                                                 g.dv, g.dks, g.dk_row0, p.kmap, H, p.unit0, g.kv_f0, g.kv_f1, skip ? p.causal : 0, stream);
     } else {
         // 9. dR block = dKbar block . K block^T + dY block . V block^T per t
         gemm(cx, false, true, AJ, b2, D, 1.f, 0.f, dKbar_t, Kk_t, dRb_t, tE, tF, nt);
@@ -648,7 +650,7 @@ int run(const MonarchBwdArgs& g, int n, void* workspace, hipStream_t stream) {
     if (parts.dqk) {
         if (!cx.status)
             cx.status = launch_monarch_bwd_dqk(left_dtype<E>(), D, nuk, b1, b2, AJ, nf, s, p.k, p.ks, p.kmap, ws + lay.dS1,
-                                               dq_direct ? g.dq : (float*)(ws + lay.dQk), dq_direct ? g.dqs : nullptr, p.qmap, H, p.unit0, stream);
+                                               dq_direct ? g.dq : (float*)(ws + lay.dQk), dq_direct ? g.dqs : nullptr, p.qmap, H, p.unit0, skip ? p.causal : 0, stream);
     } else {
         gemm(cx, false, false, AJ, D, NL, s, 0.f, dS1_uk, Kk_uk, dQk_uk, tE, tF, nuk);
     }

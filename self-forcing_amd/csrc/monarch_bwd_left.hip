@@ -24,7 +24,7 @@
 //
 // Bound by HBM: Kbar, Y read and dKbar, dY written once.  At 12 heads, a = 3, f = 21, b1 = 30, b2 = 52, 1.3 GB in 283 us,
 // where the kernel without dQ took 306 and a second one that read Kbar again for dQ 117.  With three frames tied (a = 3,
-// f = 3, b1 = 90, b2 = 52) 217 us; a grid slice per 32 query rows, which read the rows three times and wrote partial
+// f = 3, b1 = 90, b2 = 52) 217 us, block-causal over single block-frames, where a third of the rows is left out, 183; a grid slice per 32 query rows, which read the rows three times and wrote partial
 // sums, took 352, the kernel that added them 179 and dQ 175.
 
 #include <hip/hip_runtime.h>
@@ -61,6 +61,7 @@ struct LeftArgs {
     int b1, b2, AJ, nf, RR, causal;
     float scale;
     int nunits;              // units of this launch
+    bool skip;               // only the rows r that a column sees are read and written (block-causal)
 };
 
 typedef short bl_s16x4 __attribute__((ext_vector_type(4)));
@@ -176,7 +177,11 @@ void monarch_bwd_left_kernel(LeftArgs p) {
     const char* const cpb = (const char*)(p.c_rows ? p.c + (int64_t)u * RR * p.AJ + aj : p.c + uaj * RR);
     const float cmul = p.c_rows ? 1.f : kLog2e;
     const float sc2 = p.scale * kLog2e;
-    const int nch = (RR + 31) / 32;
+    // The rows of a column, in order: all of them, or (skip) those of its flim visible block-frames
+    const bool skip = p.skip && flim < p.nf;              // uniform
+    const int RV = skip ? b1 * flim : RR;
+    const int nch = (RV + 31) / 32;
+    auto row_of = [&](int x) { return skip ? x / flim * p.nf + x % flim : x; };
 
     // A chunk of 32 rows r goes from global memory into LDS (a row's 2 D bytes by consecutive lanes); there is one chunk
     // buffer.  A lone wave fills its operand registers from it and requests the next chunk at once; a team reads the operands
@@ -187,7 +192,7 @@ void monarch_bwd_left_kernel(LeftArgs p) {
     auto piece_off = [&](int n, int g) {
         const int P = g * 64 + lane;
         const int r = P / CPR, c = (P % CPR) ^ bl_swz<CPR>(r);
-        return (uint32_t)min(32 * n + r, RR - 1) * rsb + (uint32_t)c * 16;
+        return (uint32_t)row_of(min(32 * n + r, RV - 1)) * rsb + (uint32_t)c * 16;
     };
     auto request_piece = [&](int n, auto g_c) {
         constexpr int g = decltype(g_c)::value;
@@ -214,7 +219,7 @@ void monarch_bwd_left_kernel(LeftArgs p) {
                 if (q < 2 * NG) bl_load_lds16(q < NG ? kbb : ybb, piece_off(n, q % NG), kt0 + (uint32_t)q * 1024);
             }
         }
-        if (wave == (SOLO ? wave : TEAM - 1)) bl_load_lds4_at<2 * kTile>(cpb, (uint32_t)min(32 * n + m, RR - 1) * csb, kt0);
+        if (wave == (SOLO ? wave : TEAM - 1)) bl_load_lds4_at<2 * kTile>(cpb, (uint32_t)row_of(min(32 * n + m, RV - 1)) * csb, kt0);
     };
     const uint32_t b_off = (uint32_t)m * kPitch + (uint32_t)((hf ^ bl_swz<CPR>(m)) << 4);     // row m of a tile as an operand
     // transposing reads of a tile: lane (m, hf) gets, for head-dim column 32 dt + m, rows 16 ks + 4 hf + {0..3} and + 8 +
@@ -292,7 +297,7 @@ void monarch_bwd_left_kernel(LeftArgs p) {
     };
     auto row_ok = [&](int n) {
         const int r = 32 * n + m;
-        return r < RR && (r % p.nf) < flim;
+        return r < RV && (skip || (r % p.nf) < flim);
     };
 
     float lse[16], delta[16];
@@ -368,8 +373,8 @@ void monarch_bwd_left_kernel(LeftArgs p) {
         products(s, d);
         const float cl2 = ccur;
         const bool ok = row_ok(n);
-        const int r = 32 * n + m;
-        const bool r_in = r < RR;
+        const bool r_in = 32 * n + m < RV;
+        const int r = row_of(32 * n + m);
         float dsum = 0.f;
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
@@ -440,8 +445,8 @@ void monarch_bwd_left_kernel(LeftArgs p) {
 #pragma unroll
         for (int rb = 0; rb < 4; ++rb) {
             const int rr = 32 * n + (m & 7) + 8 * rb;
-            row_in[rb] = rr < RR;
-            rowoff[rb] = (int64_t)min(rr, RR - 1) * rstride + (4 * ((m >> 3) & 1) + 2 * ((m >> 4) & 1) + hf) * 8;
+            row_in[rb] = rr < RV;
+            rowoff[rb] = (int64_t)row_of(min(rr, RV - 1)) * rstride + (4 * ((m >> 3) & 1) + 2 * ((m >> 4) & 1) + hf) * 8;
         }
         auto half_rows = [&](int which, int dp) {
             const char* src = which == 0 ? dot_t : qt;
@@ -563,7 +568,8 @@ bool monarch_bwd_left_supported(int dtype, int D, int b1) {
 int launch_monarch_bwd_left(int dtype, int D, int n, int b1, int b2, int AJ, int nf, int causal, float scale, const void* q,
                             const int64_t* qs, const void* dout, const void* out, const int64_t* os, const TokMap& qmap, int H,
                             int unit0, const void* kbar, const void* y, const float* c, int c_rows, void* dkbar, void* dy, float* dc,
-                            void* ds2, int ds2_ld, float* dq, const int64_t* dqs, const float* stats, int stats_ld, hipStream_t stream) {
+                            void* ds2, int ds2_ld, float* dq, const int64_t* dqs, const float* stats, int stats_ld, bool skip_masked,
+                            hipStream_t stream) {
     LeftArgs a;
     a.ds2_ld = ds2_ld;
     a.q = (const char*)q; a.dout = (const char*)dout; a.out = (const char*)out;
@@ -586,6 +592,7 @@ int launch_monarch_bwd_left(int dtype, int D, int n, int b1, int b2, int AJ, int
     a.b1 = b1; a.b2 = b2; a.AJ = AJ; a.nf = nf; a.RR = nf * b1; a.causal = causal;
     a.scale = scale;
     a.nunits = n;
+    a.skip = skip_masked && causal && !ds2;
     if (dtype == SFM_BF16) return D == 128 ? launch_left<BF16, 128>(a, stream) : launch_left<BF16, 64>(a, stream);
     return D == 128 ? launch_left<F16, 128>(a, stream) : launch_left<F16, 64>(a, stream);
 }

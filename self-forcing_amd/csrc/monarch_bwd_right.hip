@@ -53,6 +53,7 @@ struct RightArgs {
     int64_t s0, s1, s2, row0;
     TokMap kmap;
     int b1, b2, AJ, nf, H, unit0, f0, f1;
+    int causal;              // block-causal size: the columns before a tile's first visible one are left out; 0 = none
     float scale;
 };
 
@@ -166,19 +167,21 @@ __global__ __launch_bounds__(kThreads) void monarch_bwd_right_kernel(RightArgs p
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[v] = accq[v] = 0.f;
 
-    // the tile's columns (a, j), up to 160 per pass
+    // the tile's columns (a, j), up to 160 per pass, from the first that sees key block-frame f on
+    const int cfirst = p.causal ? f / p.causal * p.causal * b2 : 0;
     auto pass = [&](auto pi_c) {
     constexpr int pi = decltype(pi_c)::value;
-    constexpr int c0 = pi * kMaxAJ;
-    const int nrows = MULTI ? min(kMaxAJ, AJ - c0) : AJ;
+    const int c0 = cfirst + pi * kMaxAJ;
+    const int nrows = MULTI ? min(kMaxAJ, AJ - c0) : AJ - c0;
+    if (MULTI && nrows <= 0) return;                                     // uniform
     stage(p.dkbar + (t * AJ + c0) * kPitch, kPitch, nrows * CPR, oG, c_d{});
     stage(p.dy + (t * AJ + c0) * kPitch, kPitch, nrows * CPR, oH, c_d{});
     stage(p.rb + (t * AJ + c0) * 128, 128, nrows * 8, oR, c_r{});
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (nrows < kMaxAJ || c0 == 0) {                                     // rows past the end are zero: they add nothing to any contraction
+    if (nrows < kMaxAJ || pi == 0) {                                     // rows past the end are zero: they add nothing to any contraction
         const u32x4 z = {0u, 0u, 0u, 0u};
-        if (c0 == 0)                                                     // K, V rows past b2: what the logits pick up there is masked, but must be finite
+        if (pi == 0)                                                     // K, V rows past b2: what the logits pick up there is masked, but must be finite
             for (int i = tid; i < (64 - b2) * CPR; i += kThreads) {
                 *(u32x4*)(lds + oK + b2 * kPitch + i * 16) = z;
                 *(u32x4*)(lds + oV + b2 * kPitch + i * 16) = z;
@@ -321,6 +324,7 @@ struct DqkArgs {
     int64_t dqs0, dqs1, dqs2;
     TokMap qmap;
     bool add;
+    int causal;              // block-causal size: dS1 beyond a column's visible block-frames is not there; 0 = none
     int b1, b2, AJ, nf, H, unit0;
     float scale;
 };
@@ -341,6 +345,7 @@ __global__ __launch_bounds__(1024) void monarch_bwd_dqk_kernel(DqkArgs p) {
     const int unit = p.unit0 + (int)(uk / p.b1);
     const int b2 = p.b2, AJ = p.AJ, NL = p.nf * b2;
     const int nt = (NL + 63) / 64;
+    auto visible = [&](int aj) { return p.causal ? min(p.nf, (aj / b2 / p.causal + 1) * p.causal) * b2 : NL; };      // elements of dS1 row aj
 
     const char* kbase = p.k + ((int64_t)(unit / p.H) * p.ks0 + (int64_t)(unit % p.H) * p.ks2) * 2;
     const uint32_t krb = (uint32_t)(p.ks1 * 2);
@@ -358,13 +363,15 @@ __global__ __launch_bounds__(1024) void monarch_bwd_dqk_kernel(DqkArgs p) {
     // dS1 pieces of row aj = 32 wave + m: x = 64 t + 16 ks + 4 hf + {0..3} and + 8 + {0..3}
     const int aj = min(32 * wave + m, AJ - 1);
     const uint16_t* arow = p.ds1 + (uk * AJ + aj) * (int64_t)NL + 4 * hf;
+    const int na = visible(aj);
+    const int nwave = __builtin_amdgcn_readfirstlane(visible(min(32 * wave + 31, AJ - 1)));      // of the wave's longest row
     auto load_a = [&](int t, u32x4 (&a)[4]) {
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
             const int x0 = 64 * t + 16 * ks + 4 * hf;
             u32x2 lo = {0u, 0u}, hi = {0u, 0u};
-            if (x0 + 4 <= NL) lo = *(const u32x2*)(arow + 64 * t + 16 * ks);           // NL is a multiple of 4: whole pieces
-            if (x0 + 12 <= NL) hi = *(const u32x2*)(arow + 64 * t + 16 * ks + 8);
+            if (x0 + 4 <= na) lo = *(const u32x2*)(arow + 64 * t + 16 * ks);           // a multiple of 4: whole pieces
+            if (x0 + 12 <= na) hi = *(const u32x2*)(arow + 64 * t + 16 * ks + 8);
             a[ks] = u32x4{lo.x, lo.y, hi.x, hi.y};
         }
     };
@@ -398,15 +405,17 @@ __global__ __launch_bounds__(1024) void monarch_bwd_dqk_kernel(DqkArgs p) {
             load_a(t + 1, anext);
         }
         const char* tile = lds + (t & 1) * kTile;
+        if (64 * t < nwave) {
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks)
+            for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt) {
-                const u32x2 lo = br_read_tr(tile, tr[dt][0] + ks * 16 * kPitch);
-                const u32x2 hi = br_read_tr(tile, tr[dt][1] + ks * 16 * kPitch);
-                const u32x4 bop = {lo.x, lo.y, hi.x, hi.y};
-                acc[dt] = E::mfma32(acur[ks], bop, acc[dt]);
-            }
+                for (int dt = 0; dt < DT; ++dt) {
+                    const u32x2 lo = br_read_tr(tile, tr[dt][0] + ks * 16 * kPitch);
+                    const u32x2 hi = br_read_tr(tile, tr[dt][1] + ks * 16 * kPitch);
+                    const u32x4 bop = {lo.x, lo.y, hi.x, hi.y};
+                    acc[dt] = E::mfma32(acur[ks], bop, acc[dt]);
+                }
+        }
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) acur[ks] = anext[ks];
     }
@@ -456,7 +465,7 @@ bool monarch_bwd_right_supported(int dtype, int D, int b2, int AJ) {
 int launch_monarch_bwd_right(int dtype, int D, int64_t ntiles, int b1, int b2, int AJ, int nf, float scale, const void* kk,
                              const int64_t* ks, const void* v, const int64_t* vs, const void* rb, const void* dkbar, const void* dy, const float* dc, const void* q,
                              const int64_t* qs, const TokMap& qmap, void* ds1, void* dk, void* dv, const int64_t* dks, int64_t row0,
-                             const TokMap& kmap, int H, int unit0, int f0, int f1, hipStream_t stream) {
+                             const TokMap& kmap, int H, int unit0, int f0, int f1, int skip_causal, hipStream_t stream) {
     if ((dks[0] | dks[1] | dks[2] | vs[0] | vs[1] | vs[2] | ks[0] | ks[1] | ks[2]) % 8 ||
         ((uintptr_t)dk | (uintptr_t)dv | (uintptr_t)v | (uintptr_t)kk) % 16 || (int64_t)(b2 - 1) * vs[1] * 2 + 2 * D > 0xffffffffll ||
         (int64_t)(b2 - 1) * ks[1] * 2 + 2 * D > 0xffffffffll) {
@@ -476,6 +485,7 @@ int launch_monarch_bwd_right(int dtype, int D, int64_t ntiles, int b1, int b2, i
     a.s0 = dks[0]; a.s1 = dks[1]; a.s2 = dks[2]; a.row0 = row0;
     a.kmap = kmap;
     a.b1 = b1; a.b2 = b2; a.AJ = AJ; a.nf = nf; a.H = H; a.unit0 = unit0; a.f0 = f0; a.f1 = f1;
+    a.causal = skip_causal;
     a.scale = scale;
     const size_t kv = (size_t)2 * 64 * 2 * D, rt = (size_t)kMaxAJ * 128;
     const size_t ldsb = kv + (size_t)2 * kMaxAJ * 2 * D + rt + (rt <= kv && AJ <= kMaxAJ ? 0 : rt) + 2 * kMaxAJ * 4;
@@ -515,7 +525,7 @@ bool monarch_bwd_dqk_supported(int dtype, int D, int b2, int AJ) {
 
 int launch_monarch_bwd_dqk(int dtype, int D, int64_t nuk, int b1, int b2, int AJ, int nf, float scale, const void* k, const int64_t* ks,
                            const TokMap& kmap, const void* ds1, float* dqk, const int64_t* dqs, const TokMap& qmap, int H, int unit0,
-                           hipStream_t stream) {
+                           int skip_causal, hipStream_t stream) {
     if ((ks[0] | ks[1] | ks[2]) % 8 || ((uintptr_t)k) % 16 || (int64_t)nf * b1 * b2 * ks[1] * 2 > 0xffffffffll) {
         set_error("monarch backward (dQ of the right factor): k rows must be 16-byte aligned and a (batch, head) slice under 4 GiB");
         return SFM_ERR_STRIDE;
@@ -526,6 +536,7 @@ int launch_monarch_bwd_dqk(int dtype, int D, int64_t nuk, int b1, int b2, int AJ
     a.ds1 = (const uint16_t*)ds1;
     a.dqk = dqk;
     a.add = dqs != nullptr;
+    a.causal = skip_causal;
     a.dqs0 = dqs ? dqs[0] : 0; a.dqs1 = dqs ? dqs[1] : 0; a.dqs2 = dqs ? dqs[2] : 0;
     a.qmap = qmap;
     a.b1 = b1; a.b2 = b2; a.AJ = AJ; a.nf = nf; a.H = H; a.unit0 = unit0;

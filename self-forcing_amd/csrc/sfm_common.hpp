@@ -164,6 +164,7 @@ struct MonarchArgs {
     uint32_t stats_ld;   // at ((b*H + h) * na*b2 + a*b2 + j) * stats_ld + i
     int unit0;       // first (b*H + h) unit of this pass
     int causal;      // block-causal size in block-frames, 0 = none
+    int skip_masked; // MFMA step 1 only: the scratch rows of masked (query, key) block-frame pairs are not read: do not form them
     float scale;
     TokMap qmap, kmap;
     int64_t qs[3], ks[3], vs[3], os[3];
@@ -230,21 +231,24 @@ bool monarch_bwd_left_supported(int dtype, int D, int b1);
 int launch_monarch_bwd_left(int dtype, int D, int n, int b1, int b2, int AJ, int nf, int causal, float scale, const void* q,
                             const int64_t* qs, const void* dout, const void* out, const int64_t* os, const TokMap& qmap, int H,
                             int unit0, const void* kbar, const void* y, const float* c, int c_rows, void* dkbar, void* dy, float* dc,
-                            void* ds2, int ds2_ld, float* dq, const int64_t* dqs, const float* stats, int stats_ld, hipStream_t stream);
+                            void* ds2, int ds2_ld, float* dq, const int64_t* dqs, const float* stats, int stats_ld, bool skip_masked,
+                            hipStream_t stream);
 // fused right-factor part of the backward (monarch_bwd_right.hip): per tile t = (unit, k, f) the dS1 block (scratch, for
 // dQ = s dS1 K) and the finished dK / dV rows of kv block-frames [f0, f1) in the caller's tensors; q, k and v are the caller's tensors too
 bool monarch_bwd_right_supported(int dtype, int D, int b2, int AJ);
 int launch_monarch_bwd_right(int dtype, int D, int64_t ntiles, int b1, int b2, int AJ, int nf, float scale, const void* kk,
                              const int64_t* ks, const void* v, const int64_t* vs, const void* rb, const void* dkbar, const void* dy, const float* dc, const void* q,
                              const int64_t* qs, const TokMap& qmap, void* ds1, void* dk, void* dv, const int64_t* dks, int64_t row0,
-                             const TokMap& kmap, int H, int unit0, int f0, int f1, hipStream_t stream);
+                             const TokMap& kmap, int H, int unit0, int f0, int f1, int skip_causal, hipStream_t stream);
 
+// With `skip_masked` / `skip_causal` (the block-causal size) the three parts neither read nor write the scratch rows of masked
+// (query, key) block-frame pairs; the caller passes it when all of them (and step 1) run.
 // dQ of the right factor (monarch_bwd_right.hip): dqk[(u, k)][aj][:] = s sum_{f, l} dS1 K, float, or, with dqs given, added
 // to the caller's rows; k is the caller's tensor
 bool monarch_bwd_dqk_supported(int dtype, int D, int b2, int AJ);
 int launch_monarch_bwd_dqk(int dtype, int D, int64_t nuk, int b1, int b2, int AJ, int nf, float scale, const void* k, const int64_t* ks,
                            const TokMap& kmap, const void* ds1, float* dqk, const int64_t* dqs, const TokMap& qmap, int H, int unit0,
-                           hipStream_t stream);
+                           int skip_causal, hipStream_t stream);
 
 // backward of the dense attention (dense_attn_bwd.hip); with less scratch than this (2*B*H*q_tokens floats at least) no
 // workgroup is split

@@ -203,6 +203,35 @@ def test_gradients_around_the_left_factors_query_tiles(b1, Fk, part, D, switches
         _close(dv, vr.grad, dtype)
 
 
+@pytest.mark.parametrize("h,w,F,chunk,D,dtype", [
+    (4, 52, 3, 1, 128, torch.bfloat16),       # waves of step 1 with both masked and visible columns
+    (6, 20, 6, 2, 64, torch.float16),         # chunks of two block-frames
+    (5, 52, 9, 3, 128, torch.bfloat16),       # several query chunks in step 1, three passes of the right factor over a tile
+    (70, 8, 3, 1, 64, torch.bfloat16),        # three query tiles
+    (30, 80, 3, 1, 64, torch.bfloat16),       # b2 > 64: the library chain, for which nothing is left out
+    (40, 12, 6, 6, 128, torch.float16),       # one chunk: nothing is masked
+])
+def test_masked_pairs_are_left_out_of_a_block_causal_call(h, w, F, chunk, D, dtype):
+    """The scratch rows of masked (query, key) block-frame pairs are neither formed nor read: forward and gradients on a
+    scratch full of NaN."""
+    H = 2
+    mattn.scratch(256 << 20, torch.device(DEV)).fill_(0xff)
+    q0, do = (randn((1, F * h * w, H, D), 700 + i, dtype) for i in range(2))
+    k0, v0 = (randn((1, F * h * w, H, D), 702 + i, dtype) for i in range(2))
+    kw = {"block_causal_size": chunk * h * w}
+    qr, kr, vr = _leaf(q0.double()), _leaf(k0.double()), _leaf(v0.double())
+    ref = monarch.monarch_attn(qr, kr, vr, 1, 1, 1, h, w, **kw)
+    ref.backward(do.double())
+    qd, kd, vd = _leaf(q0, DEV), _leaf(k0, DEV), _leaf(v0, DEV)
+    out = mattn.monarch_attn(qd, kd, vd, 1, 1, 1, h, w, **kw)
+    _close(out, ref, dtype)
+    mattn.scratch(256 << 20, torch.device(DEV)).fill_(0xff)
+    out.backward(do.to(DEV))
+    _close(qd.grad, qr.grad, dtype)
+    _close(kd.grad, kr.grad, dtype)
+    _close(vd.grad, vr.grad, dtype)
+
+
 @pytest.mark.parametrize("causal", [False, True])
 def test_backward_with_and_without_the_forwards_saved_tensors(causal):
     """sfm_monarch_bwd recomputes the left factor's row statistics; sfm_monarch_bwd_saved takes them (and the output)
