@@ -56,8 +56,8 @@ __device__ __forceinline__ void cv_wait_stage() { asm volatile("s_waitcnt vmcnt(
 
 // Epilogue of one voxel (t, h, w) of a lane: residual and bias added in fp32, one rounding, CB blocks of 32 channels
 // from channel cbase0 on.  Lane half hf of block cb holds channels 8 g + 4 hf + (e & 3) in acc[cb][vb][4 g + (e & 3)].
-template <class E, int CB>
-__device__ __forceinline__ void store_voxel(const ConvArgs& p, f32x16 (&acc)[CB][2], int vb, bool vok, int t, int h, int w,
+template <class E, int CB, int VB>
+__device__ __forceinline__ void store_voxel(const ConvArgs& p, f32x16 (&acc)[CB][VB], int vb, bool vok, int t, int h, int w,
                                             int cbase0, int hf) {
     const int64_t yoff = ((int64_t)t * p.ys_t + (int64_t)h * p.ys_h + (int64_t)w * p.ys_w) * 2;
     char* yrow = p.y + yoff;
@@ -254,7 +254,7 @@ __global__ __launch_bounds__(256, 2) void conv3d_cl_kernel(ConvArgs p) {
         const int64_t vc = vok ? v : 0;
         const int w = (int)(vc % p.W);
         const int64_t r = vc / p.W;
-        store_voxel<E, CB>(p, acc, vb, vok, (int)(r / p.H), (int)(r % p.H), w, co0 + 32 * CB * wn, hf);
+        store_voxel<E, CB, 2>(p, acc, vb, vok, (int)(r / p.H), (int)(r % p.H), w, co0 + 32 * CB * wn, hf);
     }
 }
 
@@ -380,8 +380,168 @@ __global__ __launch_bounds__(256, 2) void conv3d_row3_kernel(ConvArgs p) {
         const int rem = (int)(uc - (int64_t)t * FS);
         const int hp = rem / WP, wp = rem - hp * WP;
         const bool vok = u <= u_last && hp >= 1 && hp <= p.H && wp >= 1 && wp <= p.W;
-        store_voxel<E, CB>(p, acc, vb, vok, vok ? t : 0, vok ? hp - 1 : 0, vok ? wp - 1 : 0, co0, hf);
+        store_voxel<E, CB, 2>(p, acc, vb, vok, vok ? t : 0, vok ? hp - 1 : 0, vok ? wp - 1 : 0, co0, hf);
     }
+}
+
+// The same for 96 output channels per workgroup (every 3x3x3 convolution of the decoder but its head), where the kernel above
+// is bound by its LDS: per stage and compute unit its two workgroups read 240 KB and fetch 70 KB for 288 matrix instructions,
+// 2480 cycles of LDS against 2320 of the matrix pipes.  Here one workgroup of four waves, one per SIMD, takes 512 positions,
+// a wave 96 channels x 128 positions (192 accumulators): 168 KB and 51 KB for the same instructions.  With a single wave per
+// SIMD nothing else hides its latencies, so a wave reads each step's operands one step ahead, a read beside a matrix
+// instruction; three stage buffers, and the one barrier of a stage sits before its last step, when the operands of that
+// step have been read: it hands over the next stage and frees this one's buffer for the stage after the next two.
+// TFLOP/s of one convolution, before -> now: 384 channels 7 x 120 x 208 1154 -> 1239, 192 channels 13 x 240 x 416 1155 -> 1233,
+// 96 channels 13 x 480 x 832 1061 -> 1098 (27 stages: the ends of a workgroup, which nothing overlaps, weigh more).
+template <class E>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void conv3d_row3_wide_kernel(ConvArgs p) {
+    constexpr int CB = 3, VB = 4, kVox = 512, kCo = 32 * CB;
+    constexpr int kWRows = 3 * kCo;                       // weights of the three taps
+    constexpr int kNWG = kWRows / 16, kNXG = 33;          // 16-row groups: weights, input run (514 rows -> 528)
+    constexpr int kNG = kNWG + kNXG;
+    constexpr int kPer = (kNG + 3) / 4;                   // groups a wave stages (the last one may repeat group kNG - 1)
+    constexpr int kStage = kNG * 1024, kBufs = 3;
+    extern __shared__ __attribute__((aligned(256))) char lds[];
+    const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)lds;
+
+    const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, hf = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int WP = p.W + 2;
+    const int64_t FS = (int64_t)(p.H + 2) * WP;
+    const int64_t u_first = WP + 1, u_last = (int64_t)(p.T - 1) * FS + (int64_t)p.H * WP + p.W;
+    const int ny = p.Cout_pad / kCo;
+    const int per_xcd = (int)gridDim.x / 8;               // as in conv3d_cl_kernel
+    const int seq = (int)(blockIdx.x >> 3);
+    const int64_t u0 = u_first + ((int64_t)(blockIdx.x & 7) * (per_xcd / ny) + seq / ny) * kVox;
+    if (u0 > u_last) return;
+    const int co0 = (seq % ny) * kCo;
+
+    const int g_line = lane >> 4, g_row = lane >> 2, g_c = (lane & 3) ^ g_line;      // as in conv3d_row3_kernel
+    uint32_t src[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        const int g = min(wave + 4 * i, kNG - 1);
+        const int j = g * 16 + g_row;
+        if (g < kNWG) {
+            const int dw = j / kCo, r = j - dw * kCo;
+            src[i] = (uint32_t)(((int64_t)dw * p.Cout_pad + co0 + r) * p.Cin * 2 + g_c * 16);
+        } else {
+            const int64_t u = min(u0 + (j - kWRows), u_last + 2) - WP - 1;
+            src[i] = (uint32_t)(u * p.Cin * 2 + g_c * 16);
+        }
+    }
+
+    const int cin_steps = p.Cin / kKC;
+    const int nstage = p.kt * 3 * cin_steps;
+    const char* f_w = p.wt;
+    const char* f_x = p.x;
+    const int64_t w_next_row = 3 * (int64_t)p.Cout_pad * p.Cin * 2 - (int64_t)p.Cin * 2;      // next kernel row: three taps on
+    const int64_t x_next_row = ((int64_t)WP - 1) * p.Cin * 2;
+    const int64_t x_next_frame = (FS - 3 * (int64_t)WP) * p.Cin * 2;
+    int f_cs = 0, f_dh = 0;
+    auto load = [&](uint32_t buf, int i) {                 // one of the kPer loads of a stage, which the partial waits count
+        const int g = min(wave + 4 * i, kNG - 1);
+        cv_load_lds16(g < kNWG ? f_w : f_x, src[i], lds0 + buf + (uint32_t)g * 1024);
+    };
+    auto advance = [&]() {
+        f_w += kKC * 2;
+        f_x += kKC * 2;
+        if (++f_cs == cin_steps) {
+            f_cs = 0;
+            f_w += w_next_row;
+            f_x += x_next_row;
+            if (++f_dh == 3) {
+                f_dh = 0;
+                f_x += x_next_frame;
+            }
+        }
+    };
+
+    f32x16 acc[CB][VB];
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int vb = 0; vb < VB; ++vb)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[cb][vb][v] = 0.f;
+
+    uint32_t a_off[2], b_off[3][2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+        a_off[ks] = tile_off(m, 2 * ks + hf);
+#pragma unroll
+        for (int dw = 0; dw < 3; ++dw) b_off[dw][ks] = tile_off(kWRows + 32 * VB * wave + m + dw, 2 * ks + hf);
+    }
+    // operand i (0..2 weights, 3..6 input rows) of step j = (dw, ks) of the stage in buffer `buf`
+    u32x4 op[2][CB + VB];
+    auto read = [&](uint32_t buf, int j, int i) {
+        const int dw = j >> 1, ks = j & 1;
+        return i < CB ? *(const u32x4*)(lds + buf + a_off[ks] + (dw * kCo + 32 * i) * kRowBytes)
+                      : *(const u32x4*)(lds + buf + b_off[dw][ks] + (i - CB) * (32 * kRowBytes));
+    };
+
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) load(0, i);
+    if (nstage > 1) advance();
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) load(kStage, i);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kPer) : "memory");
+#pragma unroll
+    for (int i = 0; i < CB + VB; ++i) op[0][i] = read(0, 0, i);
+    uint32_t buf = 0, free = 2 * kStage;
+    for (int s = 0; s < nstage; ++s) {
+        // Stage s + 2 goes where stage s - 1 was, a load at a time between the matrix instructions (all of them at once kept the
+        // wave from issuing: all of a decode's wide convolutions 42.4 ms, this way 36.7).  Behind the last stage its loads are repeated into a free buffer.
+        if (s + 2 < nstage) advance();
+        const uint32_t next = buf == (kBufs - 1) * kStage ? 0 : buf + kStage;
+#pragma unroll
+        for (int j = 0; j < 6; ++j) {
+            // stage s + 1 has landed when only the loads of stage s + 2 are outstanding; this stage's operands are read
+            if (j == 5) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kPer) : "memory");
+#pragma unroll
+            for (int i = 0; i < CB * VB; ++i) {
+                // the reads behind the last stage take what lies in the next buffer and are not used
+                if (i < CB + VB) op[(j + 1) & 1][i] = j < 5 ? read(buf, j + 1, i) : read(next, 0, i);
+                else if (j < 5 && (i & 1) && 3 * j + (i - 7) / 2 < kPer) load(free, 3 * j + (i - 7) / 2);
+                acc[i / VB][i % VB] = E::mfma32(op[j & 1][i / VB], op[j & 1][CB + i % VB], acc[i / VB][i % VB]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        free = buf;
+        buf = next;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // no load into this workgroup's LDS outlives it
+
+#pragma unroll
+    for (int vb = 0; vb < VB; ++vb) {
+        const int64_t u = u0 + 32 * VB * wave + 32 * vb + m;
+        const int64_t uc = min(u, u_last);
+        const int t = (int)(uc / FS);
+        const int rem = (int)(uc - (int64_t)t * FS);
+        const int hp = rem / WP, wp = rem - hp * WP;
+        const bool vok = u <= u_last && hp >= 1 && hp <= p.H && wp >= 1 && wp <= p.W;
+        store_voxel<E, CB, VB>(p, acc, vb, vok, vok ? t : 0, vok ? hp - 1 : 0, vok ? wp - 1 : 0, co0, hf);
+    }
+}
+
+template <class E>
+int launch_row3_wide(const ConvArgs& a, hipStream_t st) {
+    constexpr int ldsb = 3 * 51 * 1024;
+    hipError_t e = hipFuncSetAttribute((const void*)conv3d_row3_wide_kernel<E>, hipFuncAttributeMaxDynamicSharedMemorySize, ldsb);
+    if (e != hipSuccess) {
+        set_error("sfm_conv3d_cl: hipFuncSetAttribute failed: %s", hipGetErrorString(e));
+        return SFM_ERR_HIP;
+    }
+    const int64_t WP = a.W + 2, FS = (int64_t)(a.H + 2) * WP;
+    const int64_t positions = (int64_t)(a.T - 1) * FS + (int64_t)(a.H - 1) * WP + a.W;     // first to last interior voxel
+    const unsigned tiles = (unsigned)((positions + 511) / 512);
+    hipLaunchKernelGGL((conv3d_row3_wide_kernel<E>), dim3((tiles + 7) / 8 * 8 * (unsigned)(a.Cout_pad / 96)), dim3(256), ldsb, st, a);
+    e = hipGetLastError();
+    if (e != hipSuccess) {
+        set_error("sfm_conv3d_cl: launch failed: %s", hipGetErrorString(e));
+        return SFM_ERR_HIP;
+    }
+    return SFM_OK;
 }
 
 template <class E, int CB>
@@ -429,7 +589,15 @@ template <class E>
 int launch_dtype(const ConvArgs& a, hipStream_t st) {
     const bool run = a.kh == 3 && !a.up2x && a.xs_w == a.Cin && a.xs_h == (int64_t)(a.W + 2) * a.Cin &&
                      a.xs_t == (int64_t)(a.H + 2) * (a.W + 2) * a.Cin && 3 * (int64_t)a.Cout_pad * a.Cin * 2 < ((int64_t)1 << 32);
-    if (run && a.Cout_pad % 96 == 0) return launch_row3<E, 3>(a, st);
+    if (run && a.Cout_pad % 96 == 0) {
+        // The wide kernel puts one workgroup on a compute unit, so its rounds have to be well filled: with 192 or more input
+        // channels (54 stages) three quarters full, with fewer eight whole rounds.  Measured with the narrow and the wide one,
+        // us: 204 workgroups (384 channels, 4 x 60 x 104) 224, 196; 84 (2 x 64 x 80) 125, 143; 782 of 96 channels 216, 226.
+        const int64_t positions = (int64_t)(a.T - 1) * (a.H + 2) * (a.W + 2) + (int64_t)(a.H - 1) * (a.W + 2) + a.W;
+        const int64_t wgs = (positions + 511) / 512 * (a.Cout_pad / 96), cu = cu_count(), rounds = (wgs + cu - 1) / cu;
+        if (a.Cin >= 192 ? 4 * wgs >= 3 * rounds * cu : wgs >= 8 * cu) return launch_row3_wide<E>(a, st);
+        return launch_row3<E, 3>(a, st);
+    }
     if (run && a.Cout_pad == 32) return launch_row3<E, 1>(a, st);
     if (a.Cout_pad % 192 == 0) return launch_cfg<E, 3, 2>(a, st);
     if (a.Cout_pad % 96 == 0) return launch_cfg<E, 3, 1>(a, st);

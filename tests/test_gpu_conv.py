@@ -174,3 +174,29 @@ def test_conv_cl_at_the_decoders_full_sizes(cin, cout, T, H, W):
         worst = max(worst, (y[t].float() - ref[t]).abs().max().item())
     assert worst <= tol
     co.release_padded()
+
+
+# enough positions for the 512-position workgroups: one round three quarters full, a ragged last tile, the fewest stages
+# (a per-frame 3x3 convolution of 32 channels), residual input, both types
+@pytest.mark.parametrize("cin,cout,kt,T,H,W,dt,with_res", [
+    (192, 384, 3, 3, 91, 89, torch.bfloat16, True), (384, 192, 3, 2, 160, 163, torch.float16, False),
+    (192, 192, 3, 1, 225, 225, torch.float16, True), (96, 96, 3, 5, 480, 441, torch.bfloat16, True),
+    (32, 96, 1, 5, 470, 457, torch.bfloat16, False)])
+def test_wide_workgroups(cin, cout, kt, T, H, W, dt, with_res):
+    torch.manual_seed(cin + W)
+    conv = (nn.Conv2d(cin, cout, 3, padding=1) if kt == 1 else nn.Conv3d(cin, cout, 3)).cuda().to(dt)
+    x = torch.randn(T, H, W, cin, device="cuda").to(dt)
+    res = torch.randn(T, H, W, cout, device="cuda").to(dt) if with_res else None
+    y = co.conv_cl(x, conv, None, res=res)
+    # reference: the 27 (9) taps as fp32 matrix products of the shifted input
+    pad = F.pad(x, (0, 0, 1, 1, 1, 1, kt - 1, 0))
+    w = conv.weight.float().reshape(cout, cin, kt, 3, 3)
+    ref = conv.bias.float().expand(T, H, W, cout).clone()
+    for i in range(kt):
+        for j in range(3):
+            for k in range(3):
+                ref += pad[i:i + T, j:j + H, k:k + W].float() @ w[:, :, i, j, k].T.contiguous()
+    if with_res:
+        ref += res.float()
+    tol = (2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11) * max(1.0, ref.abs().max().item()) * 1.01      # as above
+    assert (y.float() - ref).abs().max().item() <= tol
