@@ -56,17 +56,18 @@ __device__ __forceinline__ void dn_load_lds16(const char* base, uint32_t off, ui
 }
 __device__ __forceinline__ void dn_wait_tiles() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-template <class E, int D, int NW>
+template <class E, int D, int NW, bool SPLIT>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void dense_fwd_kernel(sfm_dense_desc p, const uint16_t* __restrict__ q,
                                                         const uint16_t* __restrict__ kp,
                                                         const uint16_t* __restrict__ vp, uint16_t* __restrict__ out,
-                                                        float* __restrict__ lse, int nsplit, float* __restrict__ part) {
+                                                        float* __restrict__ lse, int ranges, float* __restrict__ part) {
     using L = DnLds<D, NW>;
     constexpr int DS = D / 16, DT = D / 32;
     constexpr int NTH = 64 * NW;
     extern __shared__ __attribute__((aligned(256))) char lds[];
     const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)lds;
 
+    const int nsplit = SPLIT ? ranges : 1;
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, hf = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // the query blocks of one (batch, head) go to one XCD: its K / V rows are fetched from memory once, not once per XCD
@@ -81,9 +82,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     const int q0 = (item - us * nqb) * (32 * NW) + wave * 32;
     // this workgroup's keys: tiles [tile0, tile0 + ntile) of 64, nk keys in all
     const int alltiles = (p.kv_tokens + 63) / 64;
-    const int tile0 = (int)((int64_t)sp * alltiles / nsplit);
-    const int ntile = (int)((int64_t)(sp + 1) * alltiles / nsplit) - tile0;
-    const int nk = min(p.kv_tokens - 64 * tile0, 64 * ntile);
+    const int tile0 = SPLIT ? (int)((int64_t)sp * alltiles / nsplit) : 0;
+    const int ntile = SPLIT ? (int)((int64_t)(sp + 1) * alltiles / nsplit) - tile0 : alltiles;
+    const int nk = SPLIT ? min(p.kv_tokens - 64 * tile0, 64 * ntile) : p.kv_tokens;
 
     const uint32_t krs = (uint32_t)p.k_stride[1] * 2, vrs = (uint32_t)p.v_stride[1] * 2;     // row strides in bytes
     const char* kg = (const char*)(kp + (int64_t)b * p.k_stride[0] + (int64_t)h * p.k_stride[2]) + (size_t)tile0 * 64 * krs;
@@ -310,7 +311,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #undef DN_SVAL
 
     const float ltot = xhalf_sum(lrun);
-    if (nsplit > 1) {
+    if constexpr (SPLIT) {
         // partial [split][unit][q]: D floats of O, then, behind all of them, (maximum, sum)
         const int64_t row = ((int64_t)sp * p.B * p.H + unit) * nq + q0 + m, rows = (int64_t)nsplit * p.B * p.H * nq;
         if (q0 + m < nq) {
@@ -506,6 +507,11 @@ size_t dense_workspace_bytes(const sfm_dense_desc& d) {
     return s < 2 ? 0 : (size_t)s * d.B * d.H * d.q_tokens * (d.D + 2) * sizeof(float);
 }
 
+// The whole call has a kernel of its own: with the ranges as arguments of one kernel for both, 4680 queries x 32760 keys of
+// 12 heads took 890 us instead of 883.
+template <class E, int D, int NW>
+static auto dense_kernel(bool split) { return split ? dense_fwd_kernel<E, D, NW, true> : dense_fwd_kernel<E, D, NW, false>; }
+
 int launch_dense(const sfm_dense_desc& d, const void* q, const void* k, const void* v, void* out, float* lse, void* workspace,
                  size_t workspace_bytes, hipStream_t stream) {
     const bool mfma = (d.dtype == SFM_BF16 || d.dtype == SFM_F16) && (d.D == 64 || d.D == 128);
@@ -530,11 +536,11 @@ int launch_dense(const sfm_dense_desc& d, const void* q, const void* k, const vo
         };
         int rc;
         if (d.dtype == SFM_BF16) {
-            if (d.D == 128) rc = wide ? go(dense_fwd_kernel<BF16, 128, 8>, 8, DnLds<128, 8>::kTotal) : go(dense_fwd_kernel<BF16, 128, 4>, 4, DnLds<128, 4>::kTotal);
-            else rc = wide ? go(dense_fwd_kernel<BF16, 64, 8>, 8, DnLds<64, 8>::kTotal) : go(dense_fwd_kernel<BF16, 64, 4>, 4, DnLds<64, 4>::kTotal);
+            if (d.D == 128) rc = wide ? go(dense_kernel<BF16, 128, 8>(nsplit > 1), 8, DnLds<128, 8>::kTotal) : go(dense_kernel<BF16, 128, 4>(nsplit > 1), 4, DnLds<128, 4>::kTotal);
+            else rc = wide ? go(dense_kernel<BF16, 64, 8>(nsplit > 1), 8, DnLds<64, 8>::kTotal) : go(dense_kernel<BF16, 64, 4>(nsplit > 1), 4, DnLds<64, 4>::kTotal);
         } else {
-            if (d.D == 128) rc = wide ? go(dense_fwd_kernel<F16, 128, 8>, 8, DnLds<128, 8>::kTotal) : go(dense_fwd_kernel<F16, 128, 4>, 4, DnLds<128, 4>::kTotal);
-            else rc = wide ? go(dense_fwd_kernel<F16, 64, 8>, 8, DnLds<64, 8>::kTotal) : go(dense_fwd_kernel<F16, 64, 4>, 4, DnLds<64, 4>::kTotal);
+            if (d.D == 128) rc = wide ? go(dense_kernel<F16, 128, 8>(nsplit > 1), 8, DnLds<128, 8>::kTotal) : go(dense_kernel<F16, 128, 4>(nsplit > 1), 4, DnLds<128, 4>::kTotal);
+            else rc = wide ? go(dense_kernel<F16, 64, 8>(nsplit > 1), 8, DnLds<64, 8>::kTotal) : go(dense_kernel<F16, 64, 4>(nsplit > 1), 4, DnLds<64, 4>::kTotal);
         }
         if (rc) return rc;
         if (nsplit > 1) {
