@@ -418,12 +418,12 @@ void monarch_step2_kernel(MonarchArgs p) {
     const int hf = lane >> 5;
 
     const int b2 = p.b2;
-    const int split = SOLO ? p.s2_split : 1;
-    const int per_wg = SOLO ? 4 / split : 1;               // columns of a workgroup
+    const int split = SOLO ? p.s2_split : 1, lsplit = split >> 1;          // 1, 2 or 4 and its logarithm
+    const int per_wg = SOLO ? 4 >> lsplit : 1;             // columns of a workgroup
     const int sp = SOLO ? wave & (split - 1) : 0;
     const int njg = (b2 + per_wg - 1) / per_wg;
     const int a = blockIdx.x / njg;
-    const int jraw = (blockIdx.x % njg) * per_wg + (SOLO ? wave / split : 0);
+    const int jraw = (blockIdx.x % njg) * per_wg + (SOLO ? wave >> lsplit : 0);
     const bool j_ok = jraw < b2;
     const int j = j_ok ? jraw : b2 - 1;
     const int ul = blockIdx.y;
@@ -638,7 +638,7 @@ void monarch_step2_kernel(MonarchArgs p) {
                 *(f32x4*)(wl + m * (4 * D) + (((8 * dt + 2 * g + hf) ^ m) & (D / 4 - 1)) * 16) = w;
             }
         lds_barrier();
-        const int rows = 32 / split;                                      // this wave's share of the rows
+        const int rows = 32 >> lsplit;                                    // this wave's share of the rows
         for (int c = lane; c < rows * CPR; c += 64) {
             const int r = sp * rows + c / CPR, ch = c % CPR;
             f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;
@@ -688,12 +688,12 @@ void monarch_left_stats_kernel(MonarchArgs p) {
     const int hf = lane >> 5;
 
     const int b2 = p.b2;
-    const int split = SOLO ? p.s2_split : 1;
-    const int per_wg = SOLO ? 4 / split : 1;               // columns of a workgroup
+    const int split = SOLO ? p.s2_split : 1, lsplit = split >> 1;          // 1, 2 or 4 and its logarithm
+    const int per_wg = SOLO ? 4 >> lsplit : 1;             // columns of a workgroup
     const int sp = SOLO ? wave & (split - 1) : 0;
     const int njg = (b2 + per_wg - 1) / per_wg;
     const int a = blockIdx.x / njg;
-    const int jraw = (blockIdx.x % njg) * per_wg + (SOLO ? wave / split : 0);
+    const int jraw = (blockIdx.x % njg) * per_wg + (SOLO ? wave >> lsplit : 0);
     const bool j_ok = jraw < b2;
     const int j = j_ok ? jraw : b2 - 1;
     const int ul = blockIdx.y;
