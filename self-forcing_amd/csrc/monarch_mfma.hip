@@ -398,10 +398,12 @@ __device__ __forceinline__ void wait_vm() {
 //       buffers per matrix, one barrier before the logits and one before the output products.  (A pass over the rows for
 //       every 32 query rows, as before, took 518 us at the 720p grid, b1 = 45, and 96 us at three frames tied, b1 = 90;
 //       this form 299 and 70.  Two query tiles in one wave need 290 registers and spill.)
-// split (TEAM = 1): 1, 2 or 4 waves of a workgroup share a column's rows, 32-row chunks dealt in turn, and merge (maximum,
-// sum, output) through LDS at the end: with few (a, j) columns the chip is otherwise idle and a wave's chain of dependent
-// chunks (about 2.5 us each) is the whole time.
-template <class E, int D, int TEAM>
+// SHARE (TEAM = 1): 2 or 4 (p.s2_split) waves of a workgroup share a column's rows, 32-row chunks dealt in turn, and merge
+// (maximum, sum, output) through LDS at the end: with few (a, j) columns the chip is otherwise idle and a wave's chain of
+// dependent chunks (about 2.5 us each) is the whole time.  A kernel of its own: with the number of waves an argument of one
+// kernel for both, a call of three 480p frames against themselves (12 heads), whose columns are not shared, took 76.2 us
+// instead of 75.4 (two runs differ by 0.1).
+template <class E, int D, int TEAM, bool SHARE = false>
 __global__ __launch_bounds__(TEAM == 1 ? 256 : 64 * TEAM) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void monarch_step2_kernel(MonarchArgs p) {
     using L = S2Lds<D>;
@@ -418,9 +420,9 @@ void monarch_step2_kernel(MonarchArgs p) {
     const int hf = lane >> 5;
 
     const int b2 = p.b2;
-    const int split = SOLO ? p.s2_split : 1, lsplit = split >> 1;          // 1, 2 or 4 and its logarithm
+    const int split = SHARE ? p.s2_split : 1, lsplit = split >> 1;         // 1, 2 or 4 and its logarithm
     const int per_wg = SOLO ? 4 >> lsplit : 1;             // columns of a workgroup
-    const int sp = SOLO ? wave & (split - 1) : 0;
+    const int sp = SHARE ? wave & (split - 1) : 0;
     const int njg = (b2 + per_wg - 1) / per_wg;
     const int a = blockIdx.x / njg;
     const int jraw = (blockIdx.x % njg) * per_wg + (SOLO ? wave >> lsplit : 0);
@@ -588,7 +590,7 @@ void monarch_step2_kernel(MonarchArgs p) {
     uint16_t* const og = (uint16_t*)p.out + (int64_t)b * p.os[0] + (int64_t)h * p.os[2];
     float* const stats = p.stats ? p.stats + ((int64_t)unit * (p.na * b2) + a * b2 + j) * p.stats_ld : nullptr;
     float ltot = xhalf_sum(lrun);
-    if (split == 1) {
+    if constexpr (!SHARE) {
         if (!SOLO) lds_barrier();
         char* const ol = SOLO ? wl : lds_s2 + wave * L::kTile;
         const float inv = 1.f / ltot;
@@ -611,9 +613,7 @@ void monarch_step2_kernel(MonarchArgs p) {
                 *(u32x4*)(og + (p.qmap.row(a, i) + j) * p.os[1] + ch * 8) = w;
             }
         }
-        return;
-    }
-    if constexpr (SOLO) {
+    } else {
         // merge of the `split` waves of a column: statistics through the (dead) cl buffers, outputs through the waves' tile
         // buffers as fp32 rows of 4 D bytes, 16-byte pieces XOR-ed with the row
         char* const col = lds_s2 + (wave - sp) * L::kWave;                // the column's first wave
@@ -1111,6 +1111,7 @@ static int enqueue_step2(const MonarchArgs& a, int nunits, hipStream_t stream, b
         const int64_t columns = (int64_t)a.B * a.H * a.na * a.b2;
         const int nch = (a.nf * a.b1 + 31) / 32;
         if (columns <= 2 * (int64_t)cu_count()) a2.s2_split = nch >= 8 ? 4 : nch >= 4 ? 2 : 1;
+        if (!stats_only && a2.s2_split > 1) fn = (const void*)monarch_step2_kernel<E, D, 1, true>;
     }
     const int per_wg = team > 1 ? 1 : 4 / a2.s2_split;
     if (lds > 64 * 1024) {

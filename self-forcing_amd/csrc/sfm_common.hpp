@@ -164,7 +164,6 @@ struct MonarchArgs {
     uint32_t stats_ld;   // at ((b*H + h) * na*b2 + a*b2 + j) * stats_ld + i
     int unit0;       // first (b*H + h) unit of this pass
     int causal;      // block-causal size in block-frames, 0 = none
-    int skip_masked; // MFMA step 1 only: the scratch rows of masked (query, key) block-frame pairs are not read: do not form them
     float scale;
     TokMap qmap, kmap;
     int64_t qs[3], ks[3], vs[3], os[3];
@@ -172,8 +171,10 @@ struct MonarchArgs {
     int n_achunks;
     int s1_wgs;      // step-1 workgroups, 0 = one per CU (tuning override)
     int s1_groups;   // wave groups per step-1 workgroup
-    int s2_split;    // step-2 waves that share the rows of one (a, j) column: 1, 2 or 4
     int s1_total;    // step-1 work items: (unit, k, a-chunk, f) tiles
+    // kept behind the fields that every step-1 kernel reads, whose places decide how the compiler fetches and keeps them
+    int s2_split;    // step-2 waves that share the rows of one (a, j) column: 1, 2 or 4
+    int skip_masked; // MFMA step 1 only: the scratch rows of masked (query, key) block-frame pairs are not read: do not form them
 };
 
 // Backward: the forward arguments (scratch matrices in float) plus the gradient tensors.
