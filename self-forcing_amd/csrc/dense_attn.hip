@@ -169,13 +169,15 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
         const u32x2 hi = dn_read_tr(lds + (trA[1] ^ (uint32_t)((j >> 2) << 6)), vbuf + (j & 3) * 16 * L::kPitch);
         return u32x4{lo.x, lo.y, hi.x, hi.y};
     };
-    auto mask_tail = [&](f32x16* s) {              // logits of the keys past the end of a ragged last tile
+    // logits of the keys past the end of a ragged last tile: -inf, which weighs nothing against the finite running maximum
+    // however low the row's own logits are
+    auto mask_tail = [&](f32x16* s) {
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const int l = 32 * t + 8 * (v >> 2) + 4 * hf + (v & 3);
-                s[t][v] = l < lrem ? s[t][v] : kMaskLogit;
+                s[t][v] = l < lrem ? s[t][v] : -INFINITY;
             }
     };
     // value i (0..31) of a lane's logits, in the order the P^T operands take them
@@ -201,7 +203,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
         float mx = sbuf[0][0][0];
 #pragma unroll
         for (int i = 1; i < 32; ++i) mx = fmaxf(mx, DN_SVAL(sbuf[0], i));
-        mrun = fmaxf(xhalf_max(mx) * sc2, -3.0e38f);       // finite also where every key so far is at -inf: their weights are 0
+        mrun = fmaxf(xhalf_max(mx) * sc2, -__FLT_MAX__);   // finite also where every key so far is at -inf: their weights are 0
     }
 
     // One iteration consumes tile n (logits in sbuf[n & 1], maximum already folded into mrun) and, unless it is

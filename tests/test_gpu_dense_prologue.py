@@ -242,3 +242,32 @@ def test_queries_split_over_the_keys(B, H, nq, nk, D, dtype):
     assert err(out) < unit and err(out) < (1.02 + 4 / ref.numel() ** 0.5) * err(whole)
     # float32 sums of nk terms around 1, logits of size about ten: 2^-24 (log2 nk + 10) rounded up
     assert (lse.double() - rl).abs().max() < 1e-5 and (wlse.double() - rl).abs().max() < 1e-5
+
+
+# tiles of 64 keys with and without a ragged tail, one workgroup over all keys and split over the keys
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("nk", [7, 64, 200, 256, 3000, 3072])
+def test_logits_at_minus_infinity_and_at_the_lowest_floats(nk, D):
+    """softmax as torch takes it: a key at -inf weighs nothing, a row of nothing but such keys is NaN, and a row whose logits are
+    all alike is the mean of v however low they are.  Logits are the products with one element of k, exactly."""
+    H, nq, ln2 = 2, 3, 0.6931471805599453          # sm_scale = ln 2: the kernel's base-2 factor is 1 and rounds nothing
+    q = torch.zeros(1, nq, H, D, dtype=torch.bfloat16, device=DEV)
+    q[..., 0] = 1
+    k = torch.zeros(1, nk, H, D, dtype=torch.bfloat16, device=DEV)
+    v = randn((1, nk, H, D), 81, torch.bfloat16).to(DEV)
+    mean = v.double().mean(1, keepdim=True)
+
+    def run(column):
+        k[..., 0] = column
+        return sfa.attention.attention(q, k, v, softmax_scale=ln2, return_lse=True)
+
+    for low in (-2.0e30, -3.2e38):
+        out, _ = run(low)
+        assert ((out.double() - mean).abs().max() < 2 ** -8 * v.abs().max()), low
+    out, lse = run(float("-inf"))
+    assert bool(out.isnan().all()) and bool((lse == float("-inf")).all())
+    column = torch.full((1, nk, 1), float("-inf"), device=DEV)
+    column[:, nk // 2] = 3.0                          # one key of all has the whole weight, whichever tile or range it is in
+    out, lse = run(column)
+    assert torch.equal(out, v[:, nk // 2:nk // 2 + 1].expand_as(out))
+    assert (lse - 3 * ln2).abs().max() < 1e-6
