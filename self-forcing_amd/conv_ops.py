@@ -12,6 +12,13 @@ from . import lib as L
 
 _DT = {torch.bfloat16: L.SFM_BF16, torch.float16: L.SFM_F16}
 
+INPUT_LIMIT = 1 << 32       # bytes: the padded input of one sfm_conv3d_cl call stays below
+
+
+def padded_channels(cin):
+    """Input channels as the convolution kernels take them: whole blocks of 32."""
+    return (cin + 31) // 32 * 32
+
 
 def prepared(conv, dtype, device):
     """(wt [kt,kh,kw,Cout_pad,Cin_pad], bias fp32 or None, kt, k) of an nn.Conv3d / nn.Conv2d, cached on the module.
@@ -24,7 +31,7 @@ def prepared(conv, dtype, device):
     if w.dim() == 4:                                   # Conv2d: one frame
         w = w.unsqueeze(2)
     cout, cin, kt, kh, kw = w.shape
-    cin_p, cout_p = (cin + 31) // 32 * 32, (cout + 31) // 32 * 32
+    cin_p, cout_p = padded_channels(cin), (cout + 31) // 32 * 32
     wt = torch.zeros(kt, kh, kw, cout_p, cin_p, dtype=dtype, device=device)
     wt[:, :, :, :cout, :cin] = w.permute(2, 3, 4, 0, 1).to(device=device, dtype=dtype)
     bias = conv.bias.detach().to(device=device, dtype=torch.float32).contiguous() if conv.bias is not None else None

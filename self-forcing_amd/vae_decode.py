@@ -341,11 +341,13 @@ class WanVAEDecoder(nn.Module):
             run, cat_dim = self.decoder, 2
             pick = lambda a, b: x[:, :, a:b]
         n = z.shape[2]
-        # channels-last the first frame goes with the others, unless only without it the largest convolution's input (at the
-        # head, which the frames reach four times as many) stays below the 4 GiB that one call takes
+        # channels-last the first frame goes with the others, unless only without it the largest convolution's input (the
+        # head's, which the frames reach four times as many) stays below what one call takes
         alone = state.frames_in == 0 and n > 1
         if alone and state.layout == "cl":
-            alone = (4 * n - 3 + TAIL) * (8 * z.shape[3] + 2) * (8 * z.shape[4] + 2) * self.decoder.head[2].in_channels * 2 >= 1 << 32
+            from . import conv_ops
+            voxels = (4 * n - 3 + TAIL) * (8 * z.shape[3] + 2) * (8 * z.shape[4] + 2)
+            alone = voxels * conv_ops.padded_channels(self.decoder.head[2].in_channels) * 2 >= conv_ops.INPUT_LIMIT
         keep, outs = state.keep_tails, []
         if alone:
             state.keep_tails = True

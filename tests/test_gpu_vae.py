@@ -139,3 +139,30 @@ def test_first_frame_of_a_stream_goes_with_any_others(splits):
     for got in (torch.cat(outs, 1), whole):
         err = (got.cpu().double() - want).abs()
         assert got.shape == want.shape and err.max() < 1.5e-2 and err.mean() < 2e-3      # the float16 stream's bar above
+
+
+def test_first_frame_alone_equals_all_frames_together(monkeypatch):
+    """The frame count at which only the frames behind the first fit one call, at a lowered limit: the same pixels, in a
+    one-shot decode, whose last run keeps no tails, and in a stream that goes on."""
+    co = sfa.conv_ops
+    m = _decoder(torch.float16, seed=20)
+    h, w, n = 6, 5, 4
+    lat = torch.randn(1, n + 2, 16, h, w, generator=torch.Generator().manual_seed(21)).to(torch.float16).cuda()
+    runs, forward = [], m.decoder.forward_cl
+    monkeypatch.setattr(m.decoder, "forward_cl", lambda x, state: runs.append(x.shape[0]) or forward(x, state))
+
+    def decode():
+        whole = m.decode_to_pixel(lat[:, :n])
+        st = m.new_state()
+        parts = [m.decode_to_pixel(lat[:, a:b], use_cache=True, state=st) for a, b in ((0, n), (n, n + 2))]
+        return whole, torch.cat(parts, 1)
+
+    together = decode()
+    assert runs == [n, n, 2]
+    runs.clear()
+    monkeypatch.setattr(co, "INPUT_LIMIT", (4 * n - 1) * (8 * h + 2) * (8 * w + 2) * 96 * 2)
+    alone = decode()
+    assert runs == [1, n - 1, 1, n - 1, 2]
+    for a, b in zip(alone, together):
+        err = (a.double() - b.double()).abs()
+        assert a.shape == b.shape and err.max() < 1.5e-2 and err.mean() < 2e-3       # the float16 stream's bar above

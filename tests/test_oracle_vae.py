@@ -170,3 +170,32 @@ def test_parameter_names_follow_the_reference_layout():
     del extra["decoder.head.2.weight"]
     with pytest.raises(KeyError):
         m.load_reference_state_dict(extra)
+
+
+@pytest.mark.parametrize("dim,cin_p", [(96, 96), (80, 96), (8, 32)])
+def test_a_streams_first_frame_goes_alone_only_where_the_rest_alone_fits(dim, cin_p):
+    """Channels-last, a stream's first frames go through the decoder together while the head's input, channels padded to whole
+    blocks of 32 as the convolution takes them, stays below 4 GiB; past that the first goes alone, without which the rest
+    may still fit."""
+    vd = sfa.vae_decode
+    with torch.device("meta"):
+        m = vd.WanVAEDecoder(dim=dim)
+    runs = []
+
+    def decoder(x, state):
+        runs.append((x.shape[0], state.keep_tails))
+        return x.new_zeros(4 * x.shape[0] - 3 if not state.frames_in and len(runs) == 1 else 4 * x.shape[0], 1, 1, 3)
+
+    m.decoder.forward_cl = decoder
+    h, w = 60, 104
+    frame = (8 * h + 2) * (8 * w + 2) * cin_p * 2
+    most = (2 ** 32 - 1) // frame                      # padded frames below the limit: 4 n - 3 and two of history
+    joint = (most + 1) // 4
+    for n, want in ((1, [1]), (joint - 1, [joint - 1]), (joint, [joint]), (joint + 1, [1, joint])):
+        for keep in (True, False):
+            runs.clear()
+            st = m.new_state()
+            st.layout, st.keep_tails = "cl", keep
+            out = m._frames(torch.empty(1, 16, n, h, w, device="meta"), st)
+            assert [r[0] for r in runs] == want and out.shape[2] == 4 * n - 3
+            assert all(r[1] for r in runs[:-1]) and runs[-1][1] is keep and st.keep_tails is keep and st.frames_in == n
