@@ -244,7 +244,8 @@ class AttentionBlock(nn.Module):
         if x.is_cuda and x.dtype in (torch.bfloat16, torch.float16):
             # head_dim 384 is outside the fused attention kernels of the libraries: two plain matrix products with the
             # logits kept in fp32 (6240 x 6240 per frame) and the softmax between them
-            p = torch.bmm(q, k.transpose(1, 2), out_dtype=torch.float32).mul_(c ** -0.5)
+            # (k^T laid out in memory: the library's 16-bit batched products are not safe with a transposed view on the right)
+            p = torch.bmm(q, k.transpose(1, 2).contiguous(), out_dtype=torch.float32).mul_(c ** -0.5)
             o = torch.bmm(torch.softmax(p, dim=-1, out=p).to(x.dtype), v)
         else:
             o = F.scaled_dot_product_attention(q.unsqueeze(1), k.unsqueeze(1), v.unsqueeze(1))[:, 0]
