@@ -183,6 +183,10 @@ def test_conv_cl_at_the_decoders_full_sizes(cin, cout, T, H, W):
     (192, 192, 3, 1, 225, 225, torch.float16, True), (96, 96, 3, 5, 480, 441, torch.bfloat16, True),
     (32, 96, 1, 5, 470, 457, torch.bfloat16, False)])
 def test_wide_workgroups(cin, cout, kt, T, H, W, dt, with_res):
+    # the rule that these sizes are chosen by: workgroups of 512 positions x 96 channels, one to a compute unit
+    cu = torch.cuda.get_device_properties(0).multi_processor_count
+    wgs = (((T - 1) * (H + 2) + H - 1) * (W + 2) + W + 511) // 512 * (cout // 96)
+    assert 4 * wgs >= 3 * -(-wgs // cu) * cu if cin >= 192 else wgs >= 8 * cu
     torch.manual_seed(cin + W)
     conv = (nn.Conv2d(cin, cout, 3, padding=1) if kt == 1 else nn.Conv3d(cin, cout, 3)).cuda().to(dt)
     x = torch.randn(T, H, W, cin, device="cuda").to(dt)

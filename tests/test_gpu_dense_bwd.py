@@ -87,15 +87,17 @@ def test_dense_backward_argument_checks():
 
 
 @pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (64, torch.float16)])
-@pytest.mark.parametrize("B,H,Lq,Lk,kv0", [
-    (1, 1, 1, 64, 0),              # one tile on either side: nothing to split
-    (1, 1, 130, 4001, 0),          # two query blocks against 63 key tiles; ragged last tile in the last range
-    (2, 3, 2001, 100, 0),          # one key block per head against 32 query tiles
-    (1, 5, 3000, 6600, 0),         # 260 key blocks: one whole round of 256 compute units and four blocks of a second
-    (1, 7, 700, 2500, 1801),       # gradients of the last keys only, from an odd key on
-    (1, 2, 500, 900, 900),         # dq only
+@pytest.mark.parametrize("B,H,Lq,Lk,kv0,grids", [              # grids that are split on 256 compute units
+    (1, 1, 1, 64, 0, ""),              # one tile on either side: nothing to split
+    (1, 1, 130, 4001, 0, "dq"),        # two query blocks against 63 key tiles; ragged last tile in the last range
+    (2, 3, 2001, 100, 0, "dkv"),       # one key block per head against 32 query tiles
+    (1, 5, 3000, 6600, 0, "dq dkv"),   # 260 key blocks: one whole round of 256 compute units and four blocks of a second
+    (1, 7, 700, 2500, 1801, "dq"),     # gradients of the last keys only, from an odd key on
+    (1, 1, 3000, 300, 1, "dkv"),       # the same with those of the keys in ranges
+    (1, 2, 500, 900, 900, "dq"),       # dq only
+    (1, 40, 1700, 1290, 1290, "dq"),   # dq only: 560 query blocks, 512 in the whole round and 48 in ranges
 ])
-def test_last_round_split_into_ranges(B, H, Lq, Lk, kv0, D, dtype):
+def test_last_round_split_into_ranges(B, H, Lq, Lk, kv0, grids, D, dtype):
     """sfm_dense_bwd with the queried workspace, which lets the last round's workgroups be split, and with the smallest one,
     which does not: the split gradients are as close to float64 as the unsplit ones, and nothing is written behind the
     workspace."""
@@ -115,6 +117,8 @@ def test_last_round_split_into_ranges(B, H, Lq, Lk, kv0, D, dtype):
         n = C.c_size_t(0)
         sfa.lib.check(lib.sfm_dense_bwd_workspace_bytes(C.byref(bd), C.byref(n)))
         nbytes = 2 * B * H * Lq * 4 if smallest else n.value
+        if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+            assert (n.value > (2 * B * H * Lq * 4 + 255) // 256 * 256) == bool(grids)
         ws = torch.full((nbytes + 1024,), 0x5a, dtype=torch.uint8, device=DEV)
         sfa.lib.check(lib.sfm_dense_bwd(C.byref(bd), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(), do.data_ptr(),
                                         dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), nbytes, stream))

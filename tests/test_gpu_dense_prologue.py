@@ -212,7 +212,7 @@ def test_traffic_probe_moves_the_bytes_and_reports_a_duration():
 
 
 # few queries against many keys are split over the keys: 2 to 64 ranges of four tiles or more, ragged last tiles, query blocks of
-# one row up to two blocks; 8 heads x 2048 queries run the 256-query kernel in two ranges
+# one row up to two blocks; 16 heads x 2048 queries run the 256-query kernel in two ranges
 @pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (64, torch.bfloat16), (128, torch.float16), (64, torch.float16)])
 @pytest.mark.parametrize("B,H,nq,nk", [(1, 1, 1, 960), (1, 1, 1, 1600), (1, 2, 129, 2049), (2, 3, 128, 2112), (1, 1, 64, 16384),
                                        (1, 1, 200, 16449), (1, 5, 255, 2500), (1, 16, 2048, 8000), (1, 25, 300, 5000)])

@@ -24,7 +24,7 @@ def test_block_rows_around_query_tiles(b1, D):
     _check(2, D, b1, 3, 1, 2, torch.bfloat16, 900 + b1)
 
 
-# (block rows, key frames): 1, 2, 4, 5, 8 and 13 chunks of 32 rows; two columns keep the chip empty, so that the rows are shared
+# (block rows, key frames): 1, 2, 4, 5, 8 and 13 chunks of 32 rows; five columns keep the chip empty, so that the rows are shared
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("b1,fk", [(5, 4), (11, 4), (32, 4), (30, 5), (31, 8), (32, 8), (9, 45)])
 @pytest.mark.parametrize("D", [64, 128])
