@@ -490,8 +490,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     for (int i = 0; i < CB + VB; ++i) op[0][i] = read(0, 0, i);
     uint32_t buf = 0, free = 2 * kStage;
     for (int s = 0; s < nstage; ++s) {
-        // Stage s + 2 goes where stage s - 1 was, a load at a time between the matrix instructions (all of them at once kept the
-        // wave from issuing: all of a decode's wide convolutions 42.4 ms, this way 36.7).  Behind the last stage its loads are repeated into a free buffer.
+        // Stage s + 2 goes where stage s - 1 was, a load at a time between the matrix instructions (all of them at once kept
+        // the wave from issuing: all of a decode's wide convolutions 42.4 ms, this way 36.7).  Behind the last stage its loads
+        // are repeated into a free buffer.
         if (s + 2 < nstage) advance();
         const uint32_t next = buf == (kBufs - 1) * kStage ? 0 : buf + kStage;
 #pragma unroll

@@ -6,7 +6,8 @@
 //
 // MFMA kernel (bf16 / fp16, head_dim 64 or 128): workgroup = 256 or 128 queries of one (batch, head) in 8 or 4 waves,
 // wave = 32 queries; with 8 waves a compute unit holds one workgroup and streams every K / V tile once instead of
-// twice (3 % faster at 4680 x 32760 on random operands, 6 % on zeros: the chip's power limit takes the rest).  Per 64-key tile (K and V rows in LDS, row-major, 16-byte chunks XOR-swizzled):
+// twice (3 % faster at 4680 x 32760 on random operands, 6 % on zeros: the chip's power limit takes the rest).  Per 64-key
+// tile (K and V rows in LDS, row-major, 16-byte chunks XOR-swizzled):
 //     S^T[l, q] = K[l,:] . Q[q,:]          online softmax per query column (lane)
 //     O^T[d, q] += V^T[d, l] P^T[l, q]     V^T comes from transposing LDS reads (ds_read_tr16_b64), P^T from the
 //                                          accumulator layout (perm_row)
@@ -537,13 +538,15 @@ int launch_dense(const sfm_dense_desc& d, const void* q, const void* k, const vo
             return SFM_OK;
         };
         int rc;
-        if (d.dtype == SFM_BF16) {
-            if (d.D == 128) rc = wide ? go(dense_kernel<BF16, 128, 8>(nsplit > 1), 8, DnLds<128, 8>::kTotal) : go(dense_kernel<BF16, 128, 4>(nsplit > 1), 4, DnLds<128, 4>::kTotal);
-            else rc = wide ? go(dense_kernel<BF16, 64, 8>(nsplit > 1), 8, DnLds<64, 8>::kTotal) : go(dense_kernel<BF16, 64, 4>(nsplit > 1), 4, DnLds<64, 4>::kTotal);
-        } else {
-            if (d.D == 128) rc = wide ? go(dense_kernel<F16, 128, 8>(nsplit > 1), 8, DnLds<128, 8>::kTotal) : go(dense_kernel<F16, 128, 4>(nsplit > 1), 4, DnLds<128, 4>::kTotal);
-            else rc = wide ? go(dense_kernel<F16, 64, 8>(nsplit > 1), 8, DnLds<64, 8>::kTotal) : go(dense_kernel<F16, 64, 4>(nsplit > 1), 4, DnLds<64, 4>::kTotal);
-        }
+        auto pick = [&](auto e_c, auto d_c) {
+            using E = decltype(e_c);
+            constexpr int D = decltype(d_c)::value;
+            return wide ? go(dense_kernel<E, D, 8>(nsplit > 1), 8, DnLds<D, 8>::kTotal) : go(dense_kernel<E, D, 4>(nsplit > 1), 4, DnLds<D, 4>::kTotal);
+        };
+        using d64 = std::integral_constant<int, 64>;
+        using d128 = std::integral_constant<int, 128>;
+        if (d.dtype == SFM_BF16) rc = d.D == 128 ? pick(BF16{}, d128{}) : pick(BF16{}, d64{});
+        else rc = d.D == 128 ? pick(F16{}, d128{}) : pick(F16{}, d64{});
         if (rc) return rc;
         if (nsplit > 1) {
             const int nsub = 1024 / d.D;

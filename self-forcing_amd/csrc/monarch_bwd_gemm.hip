@@ -592,7 +592,11 @@ int run(const MonarchBwdArgs& g, int n, void* workspace, hipStream_t stream) {
                                                 g.dos, p.qmap, H, p.unit0, ws + lay.Kbar, ws + lay.Y, (const float*)(ws + lay.c),
                                                 fused_fwd ? 1 : 0, ws + lay.dKbar, ws + lay.dY, (float*)(ws + lay.dc),
                                                 fused_dqa ? nullptr : ws + lay.dS2, ds2_ld,
-                                                !fused_dqa ? nullptr : dq_direct ? g.dq : (float*)(ws + lay.dQa), dq_direct ? g.dqs : nullptr, saved ? g.fstats : nullptr, (b1 + 31) / 32 * 32, skip, stream);
+                                                !fused_dqa  ? nullptr
+                                                : dq_direct ? g.dq
+                                                            : (float*)(ws + lay.dQa),
+                                                dq_direct ? g.dqs : nullptr, saved ? g.fstats : nullptr, (b1 + 31) / 32 * 32, skip,
+                                                stream);
     } else {
         // 4, 5. per unit and (a, j): S2 = q_i . Kbar_r, dLm = dO_i . Y_r; the [RR x D] matrix of column aj is every AJ-th row
         for (int u = 0; u < n && !cx.status; ++u) {
@@ -650,7 +654,8 @@ int run(const MonarchBwdArgs& g, int n, void* workspace, hipStream_t stream) {
     if (parts.dqk) {
         if (!cx.status)
             cx.status = launch_monarch_bwd_dqk(left_dtype<E>(), D, nuk, b1, b2, AJ, nf, s, p.k, p.ks, p.kmap, ws + lay.dS1,
-                                               dq_direct ? g.dq : (float*)(ws + lay.dQk), dq_direct ? g.dqs : nullptr, p.qmap, H, p.unit0, skip ? p.causal : 0, stream);
+                                               dq_direct ? g.dq : (float*)(ws + lay.dQk), dq_direct ? g.dqs : nullptr, p.qmap, H,
+                                               p.unit0, skip ? p.causal : 0, stream);
     } else {
         gemm(cx, false, false, AJ, D, NL, s, 0.f, dS1_uk, Kk_uk, dQk_uk, tE, tF, nuk);
     }

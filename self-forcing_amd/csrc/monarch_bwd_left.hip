@@ -24,8 +24,9 @@
 //
 // Bound by HBM: Kbar, Y read and dKbar, dY written once.  At 12 heads, a = 3, f = 21, b1 = 30, b2 = 52, 1.3 GB in 283 us,
 // where the kernel without dQ took 306 and a second one that read Kbar again for dQ 117.  With three frames tied (a = 3,
-// f = 3, b1 = 90, b2 = 52) 217 us, block-causal over single block-frames, where a third of the rows is left out, 183; a grid slice per 32 query rows, which read the rows three times and wrote partial
-// sums, took 352, the kernel that added them 179 and dQ 175.
+// f = 3, b1 = 90, b2 = 52) 217 us, block-causal over single block-frames, where a third of the rows is left out, 183; a
+// grid slice per 32 query rows, which read the rows three times and wrote partial sums, took 352, the kernel that added
+// them 179 and dQ 175.
 
 #include <hip/hip_runtime.h>
 

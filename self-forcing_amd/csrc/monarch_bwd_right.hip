@@ -311,10 +311,11 @@ __global__ __launch_bounds__(kThreads) void monarch_bwd_right_kernel(RightArgs p
 
 // ---------------------------------------------------------------------------------------------------------------
 // dQ of the right factor: dQk[(u, k)][aj, :] = s sum_{f, l} dS1[(u, k)][aj, (f, l)] K[(f, k, l), :], float, added to the
-// caller's dq rows, where the left factor's part is, or written to a scratch matrix.  One workgroup per (unit, k), one wave per 32 columns (a, j); the K rows of the nf
-// block-frames stream through LDS 64 at a time straight from the caller's tensor (global_load_lds_dwordx4, double
-// buffered, chunk swizzle) and come back transposed as the B operand [n = d, k = (f, l)]; the A operand is dS1 straight
-// from memory, two 8-byte pieces per step in the order in which the transposing reads deliver the rows.
+// caller's dq rows, where the left factor's part is, or written to a scratch matrix.  One workgroup per (unit, k), one
+// wave per 32 columns (a, j); the K rows of the nf block-frames stream through LDS 64 at a time straight from the
+// caller's tensor (global_load_lds_dwordx4, double buffered, chunk swizzle) and come back transposed as the B operand
+// [n = d, k = (f, l)]; the A operand is dS1 straight from memory, two 8-byte pieces per step in the order in which the
+// transposing reads deliver the rows.
 struct DqkArgs {
     const char* k;           // caller's tensor: row kmap.row(f, k) + l, strides ks0 (batch), ks1 (row), ks2 (head), in elements
     int64_t ks0, ks1, ks2;

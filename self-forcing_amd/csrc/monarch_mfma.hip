@@ -15,8 +15,10 @@
 //      v_permlane32_swap per dword pair leaves 8 consecutive head-dim elements per lane (16-byte stores).
 //
 //  step 2 (left factor; replaces _z_fwd, monarch_attn.py:698-842)
-//      wave = (unit, a, j): streams its contiguous Kbar / Y rows once, 32 rows at a time, through its own part of
-//      LDS (global_load_lds_dwordx4, one chunk ahead; no barriers: a wave waits for its own loads only),
+//      per (unit, a, j) its contiguous Kbar / Y rows once, 32 rows at a time, through LDS (global_load_lds_dwordx4, one
+//      chunk ahead): by one wave that waits for its own loads only (b1 <= 32), by a team of two to four waves with two
+//      barriers per chunk (b1 > 32), or, where columns are few, by two or four waves that take the chunks in turn and
+//      merge at the end,
 //          S2^T[(f,k), i] = Kbar[(f,k),:] . Q[a,i,j,:]  - cl       online softmax over (f,k)
 //          O^T[d, i]     += Y^T[d,(f,k)] P^T[(f,k), i]
 //      with the Y^T operands from transposing LDS reads and the query rows in registers.
@@ -1062,8 +1064,10 @@ static int enqueue_step1(const MonarchArgs& a, int nunits, hipStream_t stream, c
     const void* fn = fn_override ? fn_override
                      : skip && nt == 4 ? (const void*)monarch_step1_kernel<E, D, 4, false, false, false, true>
                      : skip && nt == 3 ? (const void*)monarch_step1_kernel<E, D, 3, false, false, false, true>
-                     : skip && nt == 2 ? (a.rb ? (const void*)monarch_step1_kernel<E, D, 2, true, false, false, true> : (const void*)monarch_step1_kernel<E, D, 2, false, false, false, true>)
-                     : skip ? (a.rb ? (const void*)monarch_step1_kernel<E, D, 1, true, false, false, true> : (const void*)monarch_step1_kernel<E, D, 1, false, false, false, true>)
+                     : skip && nt == 2 ? (a.rb ? (const void*)monarch_step1_kernel<E, D, 2, true, false, false, true>
+                                               : (const void*)monarch_step1_kernel<E, D, 2, false, false, false, true>)
+                     : skip ? (a.rb ? (const void*)monarch_step1_kernel<E, D, 1, true, false, false, true>
+                                    : (const void*)monarch_step1_kernel<E, D, 1, false, false, false, true>)
                      : nt == 4 ? (const void*)monarch_step1_kernel<E, D, 4, false>
                      : nt == 3 ? (const void*)monarch_step1_kernel<E, D, 3, false>
                      : nt == 2 ? (a.rb ? (const void*)monarch_step1_kernel<E, D, 2, true> : (const void*)monarch_step1_kernel<E, D, 2, false>)
@@ -1095,11 +1099,16 @@ static int enqueue_step1(const MonarchArgs& a, int nunits, hipStream_t stream, c
 template <class E, int D>
 static int enqueue_step2(const MonarchArgs& a, int nunits, hipStream_t stream, bool stats_only = false) {
     const int team = a.b1 > 96 ? 4 : (a.b1 + 31) / 32;
-    const void* fn = stats_only ? (team == 4 ? (const void*)monarch_left_stats_kernel<E, D, 4> : team == 3 ? (const void*)monarch_left_stats_kernel<E, D, 3>
-                                   : team == 2 ? (const void*)monarch_left_stats_kernel<E, D, 2> : (const void*)monarch_left_stats_kernel<E, D, 1>)
+    const void* fn = stats_only ? (team == 4   ? (const void*)monarch_left_stats_kernel<E, D, 4>
+                                   : team == 3 ? (const void*)monarch_left_stats_kernel<E, D, 3>
+                                   : team == 2 ? (const void*)monarch_left_stats_kernel<E, D, 2>
+                                               : (const void*)monarch_left_stats_kernel<E, D, 1>)
                    : team == 4 ? (const void*)monarch_step2_kernel<E, D, 4> : team == 3 ? (const void*)monarch_step2_kernel<E, D, 3>
                    : team == 2 ? (const void*)monarch_step2_kernel<E, D, 2> : (const void*)monarch_step2_kernel<E, D, 1>;
-    const size_t lds = stats_only ? (team == 4 ? StLds<D, 4>::bytes() : team == 3 ? StLds<D, 3>::bytes() : team == 2 ? StLds<D, 2>::bytes() : StLds<D, 1>::bytes())
+    const size_t lds = stats_only ? (team == 4   ? StLds<D, 4>::bytes()
+                                     : team == 3 ? StLds<D, 3>::bytes()
+                                     : team == 2 ? StLds<D, 2>::bytes()
+                                                 : StLds<D, 1>::bytes())
                        : team > 1 ? S2Lds<D>::team_bytes(team) : S2Lds<D>::bytes();
     MonarchArgs a2 = a;
     a2.s2_split = 1;
