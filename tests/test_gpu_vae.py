@@ -144,7 +144,7 @@ def test_first_frame_of_a_stream_goes_with_any_others(splits):
 def test_first_frame_alone_equals_all_frames_together(monkeypatch):
     """The frame count at which only the frames behind the first fit one call, at a lowered limit: the same pixels, in a
     one-shot decode, whose last run keeps no tails, and in a stream that goes on."""
-    co = sfa.conv_ops
+    from self_forcing_amd import conv_ops as co
     m = _decoder(torch.float16, seed=20)
     h, w, n = 6, 5, 4
     lat = torch.randn(1, n + 2, 16, h, w, generator=torch.Generator().manual_seed(21)).to(torch.float16).cuda()
