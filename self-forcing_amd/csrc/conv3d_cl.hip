@@ -386,8 +386,9 @@ __global__ __launch_bounds__(256, 2) void conv3d_row3_kernel(ConvArgs p) {
 
 // The same for 96 output channels per workgroup (every 3x3x3 convolution of the decoder but its head), where the kernel above
 // is bound by its LDS: per stage and compute unit its two workgroups read 240 KB and fetch 70 KB for 288 matrix instructions,
-// 2480 cycles of LDS against 2320 of the matrix pipes.  Here one workgroup of four waves, one per SIMD, takes 512 positions,
-// a wave 96 channels x 128 positions (192 accumulators): 168 KB and 51 KB for the same instructions.  With a single wave per
+// reckoned at 128 bytes a cycle 2480 cycles against 2320 of the matrix pipes (SQ_INSTS_LDS 0.83 per matrix instruction).
+// Here one workgroup of four waves, one per SIMD, takes 512 positions, a wave 96 channels x 128 positions (192
+// accumulators): 168 KB and 51 KB for the same instructions (0.59, without bank conflicts).  With a single wave per
 // SIMD nothing else hides its latencies, so a wave reads each step's operands one step ahead, a read beside a matrix
 // instruction; three stage buffers, and the one barrier of a stage sits before its last step, when the operands of that
 // step have been read: it hands over the next stage and frees this one's buffer for the stage after the next two.
