@@ -145,12 +145,19 @@ int sfm_kv_cache_write(int32_t dtype, int32_t B, int32_t H, int32_t D, const sfm
                        int64_t cache_tokens, int64_t start_idx, int64_t end_idx, void* stream);
 
 /* monarch_attn_with_kv_cache (monarch_attn.py:1778-1796): cache write at [start_idx,end_idx)
- * followed by sfm_monarch_fwd over the whole cache view (desc->kv_tokens tokens,
+ * and sfm_monarch_fwd over the whole cache view (desc->kv_tokens tokens,
  * desc->kv_block_order must be 1). */
 int sfm_monarch_attn_with_kv_cache(const sfm_monarch_desc* desc, const void* q, void* k_cache, void* v_cache,
                                    const void* new_k, const void* new_v, const int64_t new_stride[3],
                                    int64_t start_idx, int64_t end_idx, void* out,
                                    void* workspace, size_t workspace_bytes, void* stream);
+
+/* The same with the row statistics of sfm_monarch_fwd_stats (which see for their size and where they exist), for a backward
+ * to come.  start_idx / end_idx as for sfm_kv_cache_write: the chunk need not start at a block. */
+int sfm_monarch_attn_with_kv_cache_stats(const sfm_monarch_desc* desc, const void* q, void* k_cache, void* v_cache,
+                                         const void* new_k, const void* new_v, const int64_t new_stride[3],
+                                         int64_t start_idx, int64_t end_idx, void* out, float* stats,
+                                         void* workspace, size_t workspace_bytes, void* stream);
 
 /* sfm_monarch_attn_with_kv_cache for callers that cannot allocate or hand over a workspace (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  The scratch is a

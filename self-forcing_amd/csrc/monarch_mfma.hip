@@ -130,6 +130,9 @@ void monarch_step1_kernel(MonarchArgs p) {
         return x;
     };
 
+    // tile x is of the new chunk, whose rows are not in the cache yet
+    auto is_new = [&](const Tile& x) { return !WR && !CS && p.new_kv && x.f >= p.new_f0 && x.f < p.new_f1; };
+
     // Tile x into buffer `buf`: LDS position P (in 16-byte units) holds chunk (P % CPR) ^ swz(row) of row P / CPR.
     // Rows past the end of a short tile (l >= b2) load row b2 - 1 again; their logits are masked below.  Every wave
     // issues the same number of loads for every tile, which the partial wait at the top of a round relies on.
@@ -138,14 +141,46 @@ void monarch_step1_kernel(MonarchArgs p) {
         const int b = unit / p.H, h = unit % p.H;
         const char* kg = (const char*)p.k + ((int64_t)b * p.ks[0] + (int64_t)h * p.ks[2]) * 2;
         const char* vg = (const char*)p.v + ((int64_t)b * p.vs[0] + (int64_t)h * p.vs[2]) * 2;
-        const uint32_t krow0 = (uint32_t)p.kmap.row(x.f, x.k);        // uniform
+        uint32_t row0 = (uint32_t)p.kmap.row(x.f, x.k), rs = ks1 * 2;      // uniform
+        uint32_t vrow0 = row0, vrs = rs;                                   // V's, where they are not K's
+        if (is_new(x)) {               // a refinement's last pass finds K in the cache
+            const int64_t n0 = ((int64_t)b * p.ns[0] + (int64_t)h * p.ns[2]) * 2;
+            vrow0 = (uint32_t)p.qmap.row(x.f - p.new_f0, x.k);
+            vrs = (uint32_t)p.ns[1] * 2;
+            if (!IT || KO) {
+                kg = (const char*)p.new_k + n0;
+                row0 = vrow0;
+                rs = vrs;
+            }
+            vg = (const char*)p.new_v + n0;
+        }
         const uint32_t dst = lds0 + (uint32_t)buf * 2 * L::kTile;
         for (int g = wave; g < NT * (CPR / 2); g += nwaves) {         // 1 KB (64 / CPR rows) per step
             const int P = g * 64 + lane;
             const int r = P / CPR, c = (P % CPR) ^ s1_swz<CPR>(r);
-            const uint32_t off = (krow0 + (uint32_t)min(r, b2 - 1)) * ks1 * 2 + (uint32_t)c * 16;
+            const uint32_t off = (row0 + (uint32_t)min(r, b2 - 1)) * rs + (uint32_t)c * 16;
             s1_load_lds16(kg, off, dst + (uint32_t)g * 1024);
-            if (!KO) s1_load_lds16(vg, off, dst + L::kTile + (uint32_t)g * 1024);
+            if (!KO) s1_load_lds16(vg, IT ? (vrow0 + (uint32_t)min(r, b2 - 1)) * vrs + (uint32_t)c * 16 : off, dst + L::kTile + (uint32_t)g * 1024);
+        }
+    };
+    // The new chunk's rows of tile x from LDS to the cache: K and V, or K in a refinement's first pass and V in its last.
+    // The write is at the end of a tile's round, behind the stores that the next round's wait leaves in flight, and
+    // non-temporal.  Whole call against a write kernel in front (12 heads x 128, 480p): 3 frames against themselves 75.7 -> 63.2
+    // us (71.1 with ordinary stores, 74.3 with the write before the next tile's loads), 21 frames 329.8 -> 324.9, 720p 727 ->
+    // 716, 2 heads x 64 of 8 x 8 tokens 22.0 -> 18.4.
+    auto write_new = [&](const Tile& x, const char* tile) {
+        const int unit = p.unit0 + x.ul;
+        const int64_t c0 = ((int64_t)(unit / p.H) * p.ks[0] + (int64_t)(unit % p.H) * p.ks[2]) * 2;
+        char* kg = (char*)p.k + c0;
+        char* vg = (char*)p.v + c0;
+        const uint32_t row0 = (uint32_t)p.kmap.row(x.f, x.k);
+        for (int g = wave; g < NT * (CPR / 2); g += nwaves) {
+            const int P = g * 64 + lane;
+            const int r = P / CPR, c = (P % CPR) ^ s1_swz<CPR>(r);
+            if (r >= b2) continue;
+            const uint32_t off = (row0 + (uint32_t)r) * ks1 * 2 + (uint32_t)c * 16;
+            if (!IT || KO) __builtin_nontemporal_store(*(const u32x4*)(tile + P * 16), (u32x4*)(kg + off));
+            if (!KO) __builtin_nontemporal_store(*(const u32x4*)(tile + L::kTile + P * 16), (u32x4*)(vg + off));
         }
     };
     // K rows 32 t + m as the logits' A operand
@@ -174,55 +209,74 @@ void monarch_step1_kernel(MonarchArgs p) {
     // addresses).  The number of stores after a tile's loads is then the same on every path, so that the
     // wait for the loads can leave those stores in flight instead of draining them.
     u32x4 qb[DS];                                          // logits operand (B): this lane's query row
+    u32x4 qn[DS];                                          // the next tile's, requested a tile ahead where it is another one
+    float wn = 1.f;                                        // IT: the weight of the next tile's representative
     uint32_t crow[4] = {0, 0, 0, 0};                       // byte offsets in the (f, k) slab of the four scratch rows this lane stores to
     uint32_t cloff = 0;                                    // same for cl
     int qkey = -1;
     float wsc = 1.f;                                       // IT: the column's logits factor
 
+    auto scratch_row = [&](const Tile& x) { return (uint32_t)x.ul * p.ws_unit + (uint32_t)x.k * p.ws_row + (uint32_t)x.f * fstep; };
+    auto query_key = [&](const Tile& x) { return (x.ul * p.b1 + x.k) * p.n_achunks + x.ac; };     // one value per (unit, k, query chunk)
+    // Query rows of tile x.  They are asked for after the tile's own loads and before this round's stores, and so have landed
+    // with them: fetched where they are used, they are waited for behind all the stores of the tile before (3 refinement
+    // passes at three frames tied, which fetch them for every tile, 547 -> 534 us).  CS fetches them there all the same: a
+    // wave that skips a tile has no stores to count, and the whole clip's step 1 took 86.3 us this way, 83.6 that.
+    auto fetch_query = [&](const Tile& x, u32x4* to) {
+        const int unit = p.unit0 + x.ul;
+        const int b = unit / p.H, h = unit % p.H;
+        const uint16_t* qg = (const uint16_t*)p.q + (int64_t)b * p.qs[0] + (int64_t)h * p.qs[2];
+        const int cg = min(wave * 32 + m, x.ncols - 1);
+        const int ca = cg / b2;
+        const uint16_t* qrow = qg + ((uint32_t)(p.qmap.row(x.a0 + ca, x.k) + cg - ca * b2) * qs1 + 8 * hf);
+        if (IT && p.iter_mode == 2) {
+            const size_t rrow = (size_t)scratch_row(x) + (size_t)(x.a0 * b2 + cg) * p.ws_aj;
+            qrow = (const uint16_t*)p.rep + rrow * D + 8 * hf;
+            wn = p.wgt[rrow];
+        }
+#pragma unroll
+        for (int ds = 0; ds < DS; ++ds) to[ds] = *(const u32x4*)(qrow + 16 * ds);
+    };
+
     Tile cur = decode(t0 + grp), nxt = cur;
     bool stored = true;                                    // CS: this wave stored rows in the round before
+    if (!CS) fetch_query(cur, qn);
     stage(cur, 0);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (!CS) {                                             // landed: a wait in the loop counts the loop's operations only
+#pragma unroll
+        for (int ds = 0; ds < DS; ++ds) asm volatile("" : "+v"(qn[ds]));
+        if (IT) asm volatile("" : "+v"(wn));
+    }
     for (int r = 0; r < rounds; ++r) {
         const bool fresh = r < mine;     // in its last round a group may have no tile left: it repeats its previous one
         // Vector memory operations complete in order: this wave's part of tile r has landed when only the Kbar / Y
-        // stores of the round before (the last 8 * D / 64 operations it issued, half as many without Y) are outstanding.
+        // stores of the round before (8 * D / 64 operations, half as many without Y; a new chunk's cache rows come behind
+        // them) are outstanding.
         if (!CS || stored) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((KO ? 4 : 8) * D / 64) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         lds_barrier();                   // tile r is in LDS; every wave has finished reading the tile before it
         if (fresh) cur = nxt;
         const char* kt = lds + (r & 1) * 2 * L::kTile;
         const char* vt = kt + L::kTile;
-        const int key = (cur.ul * p.b1 + cur.k) * p.n_achunks + cur.ac;       // one value per (unit, k, query chunk)
-        const uint32_t srow = (uint32_t)cur.ul * p.ws_unit + (uint32_t)cur.k * p.ws_row + (uint32_t)cur.f * fstep;
-        if ((IT && p.iter_mode == 2) || key != qkey) {
-            qkey = key;
-            const int unit = p.unit0 + cur.ul;
-            const int b = unit / p.H, h = unit % p.H;
-            const uint16_t* qg = (const uint16_t*)p.q + (int64_t)b * p.qs[0] + (int64_t)h * p.qs[2];
-            const int cg = min(wave * 32 + m, cur.ncols - 1);
-            const int cl_a = cg / b2;
-            const int cj = cg - cl_a * b2;
-            const int ca = cur.a0 + cl_a;
-            const uint16_t* qrow = qg + ((uint32_t)(p.qmap.row(ca, cur.k) + cj) * qs1 + 8 * hf);
-            if (IT) {
-                wsc = 1.0f / (1.0f + 1e-6f);
-                if (p.iter_mode == 2) {
-                    const size_t rrow = (size_t)srow + (size_t)(ca * b2 + cj) * p.ws_aj;
-                    qrow = (const uint16_t*)p.rep + rrow * D + 8 * hf;
-                    wsc = fminf(1.0f / (p.wgt[rrow] + 1e-6f), 1e4f);
-                }
+        const uint32_t srow = scratch_row(cur);
+        if ((IT && p.iter_mode == 2) || query_key(cur) != qkey) {
+            qkey = query_key(cur);
+            if (CS) {
+                fetch_query(cur, qb);
+#pragma unroll
+                for (int ds = 0; ds < DS; ++ds) asm volatile("" : "+v"(qb[ds]));      // waited for here, before the tile loads below
+            } else {
+#pragma unroll
+                for (int ds = 0; ds < DS; ++ds) qb[ds] = qn[ds];
             }
-#pragma unroll
-            for (int ds = 0; ds < DS; ++ds) qb[ds] = *(const u32x4*)(qrow + 16 * ds);
-#pragma unroll
-            for (int ds = 0; ds < DS; ++ds) asm volatile("" : "+v"(qb[ds]));      // waited for here, before the tile loads below
-            cloff = (uint32_t)(ca * b2 + cj) * p.cl_aj * 4;
+            if (IT) wsc = p.iter_mode == 2 ? fminf(1.0f / (wn + 1e-6f), 1e4f) : 1.0f / (1.0f + 1e-6f);
+            const int cg = min(wave * 32 + m, cur.ncols - 1);
+            cloff = (uint32_t)(cur.a0 * b2 + cg) * p.cl_aj * 4;
 #pragma unroll
             for (int rb = 0; rb < 4; ++rb) {
                 const int sg = min(wave * 32 + (m & 7) + 8 * rb, cur.ncols - 1);
-                const int sa = sg / b2;
-                crow[rb] = (uint32_t)((cur.a0 + sa) * b2 + (sg - sa * b2)) * p.ws_aj * (D * 2) + piece;
+                crow[rb] = (uint32_t)(cur.a0 * b2 + sg) * p.ws_aj * (D * 2) + piece;
             }
         }
         if (r + 1 < rounds) {
@@ -230,6 +284,7 @@ void monarch_step1_kernel(MonarchArgs p) {
             const int tn = t0 + grp + (r + 1) * G;
             nxt = decode(tn < t1 ? tn : t0 + grp + (mine - 1) * G);
             stage(nxt, (r + 1) & 1);
+            if (!CS && ((IT && p.iter_mode == 2) || query_key(nxt) != qkey)) fetch_query(nxt, qn);
         }
 
         if (CS) {
@@ -361,6 +416,7 @@ void monarch_step1_kernel(MonarchArgs p) {
                 }
             }
         }
+        if (!WR && !CS && fresh && cur.ac == 0 && is_new(cur)) write_new(cur, kt);
     }
 }
 
@@ -1206,6 +1262,7 @@ static int launch_iter_t(const MonarchArgs& a, int nunits, int num_iters, hipStr
         MonarchArgs a1 = a;
         a1.rb = nullptr;
         a1.iter_mode = it == 0 ? 1 : 2;
+        a1.new_kv = it == 0 || last ? a.new_kv : 0;      // K in the first pass, V in the last
         if (int rc = enqueue_step1<E, D>(a1, nunits, stream, last ? fn1 : fnk)) return rc;
         MonarchArgs a2 = a;
         if (last) a2.stats = nullptr;

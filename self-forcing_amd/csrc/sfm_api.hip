@@ -341,8 +341,16 @@ static void init_args(const sfm_monarch_desc* desc, const MonarchPlan& pl, Monar
     a.s1_wgs = step1_wgs_override();            // tuning override: step-1 workgroups (default 0: one per CU)
 }
 
+// The new chunk of a KV-cache call: token-order rows for cache rows [start, end) in block order.
+struct NewChunk {
+    const void *k, *v;
+    const int64_t* stride;
+    int64_t start, end;
+};
+
 static int monarch_fwd_impl(const sfm_monarch_desc* desc, const void* q, const void* k, const void* v, void* out,
-                            void* workspace, size_t workspace_bytes, void* stream, float* step_ms, float* stats = nullptr) {
+                            void* workspace, size_t workspace_bytes, void* stream, float* step_ms, float* stats = nullptr,
+                            const NewChunk* nc = nullptr) {
     MonarchPlan pl;
     int rc = plan_monarch(desc, &pl);
     if (rc) return rc;
@@ -367,6 +375,22 @@ static int monarch_fwd_impl(const sfm_monarch_desc* desc, const void* q, const v
     a.q = q; a.k = k; a.v = v; a.out = out;
     a.stats = stats;
     a.stats_ld = (uint32_t)((pl.b1 + 31) / 32 * 32);
+    if (nc && nc->end > nc->start) {
+        const int64_t blk = (int64_t)pl.b1 * pl.b2;
+        if ((pl.mfma || pl.iter_mfma) && !pl.fused && nc->start % blk == 0) {
+            // step 1 loads the chunk's tiles from it and writes the cache itself: no launch in front, the chunk read once
+            a.new_kv = 1;
+            a.new_f0 = (int)(nc->start / blk);
+            a.new_f1 = (int)(nc->end / blk);
+            a.new_k = nc->k; a.new_v = nc->v;
+            for (int i = 0; i < 3; ++i) a.ns[i] = nc->stride[i];
+        } else {
+            const int nbf = (int)((nc->end - nc->start) / blk);
+            rc = launch_kv_cache_write(elem_size(desc->dtype), desc->B, desc->H, desc->D, a.qmap, nbf, nc->k, nc->v, nc->stride,
+                                       const_cast<void*>(k), const_cast<void*>(v), desc->k_stride, nc->start, (hipStream_t)stream);
+            if (rc) return rc;
+        }
+    }
     if (pl.fused) {
         // as many units per pass as the workspace holds (the scratch of a pass is not linear in its units)
         int upp = pl.units;
@@ -694,10 +718,9 @@ static int monarch_bwd_impl(const sfm_monarch_bwd_desc* desc, const void* q, con
     return SFM_OK;
 }
 
-int sfm_kv_cache_write(int32_t dtype, int32_t B, int32_t H, int32_t D, const sfm_tiling* tiling, const void* new_k,
-                       const void* new_v, const int64_t new_stride[3], void* k_cache, void* v_cache,
-                       const int64_t cache_stride[3], int64_t cache_tokens, int64_t start_idx, int64_t end_idx,
-                       void* stream) {
+static int check_cache_write(int32_t dtype, int32_t B, int32_t H, int32_t D, const sfm_tiling* tiling, const void* new_k,
+                             const void* new_v, const int64_t new_stride[3], void* k_cache, void* v_cache,
+                             const int64_t cache_stride[3], int64_t cache_tokens, int64_t start_idx, int64_t end_idx) {
     if (!tiling || !new_k || !new_v || !new_stride || !k_cache || !v_cache || !cache_stride) {
         set_error("NULL argument");
         return SFM_ERR_NULL;
@@ -730,17 +753,28 @@ int sfm_kv_cache_write(int32_t dtype, int32_t B, int32_t H, int32_t D, const sfm
         set_error("tensors must be 16-byte aligned");
         return SFM_ERR_ALIGN;
     }
-    if (n == 0) return SFM_OK;
+    return SFM_OK;
+}
+
+int sfm_kv_cache_write(int32_t dtype, int32_t B, int32_t H, int32_t D, const sfm_tiling* tiling, const void* new_k,
+                       const void* new_v, const int64_t new_stride[3], void* k_cache, void* v_cache,
+                       const int64_t cache_stride[3], int64_t cache_tokens, int64_t start_idx, int64_t end_idx,
+                       void* stream) {
+    const int rc = check_cache_write(dtype, B, H, D, tiling, new_k, new_v, new_stride, k_cache, v_cache, cache_stride, cache_tokens,
+                                     start_idx, end_idx);
+    if (rc) return rc;
+    if (end_idx == start_idx) return SFM_OK;
     TokMap map = make_map(*tiling, 1);
-    const int nbf = (int)(n / group) * tiling->h_reduce * tiling->w_reduce;
-    return launch_kv_cache_write(esz, B, H, D, map, nbf, new_k, new_v, new_stride, k_cache, v_cache, cache_stride,
+    const int nbf = (int)((end_idx - start_idx) / ((int64_t)map.b1 * map.b2));
+    return launch_kv_cache_write(elem_size(dtype), B, H, D, map, nbf, new_k, new_v, new_stride, k_cache, v_cache, cache_stride,
                                  start_idx, (hipStream_t)stream);
 }
 
-int sfm_monarch_attn_with_kv_cache(const sfm_monarch_desc* desc, const void* q, void* k_cache, void* v_cache,
-                                   const void* new_k, const void* new_v, const int64_t new_stride[3],
-                                   int64_t start_idx, int64_t end_idx, void* out, void* workspace,
-                                   size_t workspace_bytes, void* stream) {
+// `stats` (optional): row statistics as sfm_monarch_fwd_stats leaves them; the chunk may then start anywhere in the cache, as
+// sfm_kv_cache_write takes it
+static int with_kv_cache_impl(const sfm_monarch_desc* desc, const void* q, void* k_cache, void* v_cache, const void* new_k,
+                              const void* new_v, const int64_t new_stride[3], int64_t start_idx, int64_t end_idx, void* out,
+                              float* stats, void* workspace, size_t workspace_bytes, void* stream) {
     MonarchPlan pl;
     int rc = plan_monarch(desc, &pl);
     if (rc) return rc;
@@ -753,12 +787,12 @@ int sfm_monarch_attn_with_kv_cache(const sfm_monarch_desc* desc, const void* q, 
         return SFM_ERR_UNSUPPORTED;
     }
     const int64_t blk = (int64_t)pl.b1 * pl.b2;
-    if (start_idx < 0 || end_idx < start_idx || end_idx > desc->kv_tokens) {
+    if (!stats && (start_idx < 0 || end_idx < start_idx || end_idx > desc->kv_tokens)) {
         set_error("start_idx=%lld, end_idx=%lld outside the cache view of %d tokens", (long long)start_idx,
                   (long long)end_idx, desc->kv_tokens);
         return SFM_ERR_RANGE;
     }
-    if (start_idx % blk || end_idx % blk) {
+    if (!stats && (start_idx % blk || end_idx % blk)) {
         set_error("start_idx=%lld / end_idx=%lld must be multiples of b1*b2=%lld", (long long)start_idx,
                   (long long)end_idx, (long long)blk);
         return SFM_ERR_RANGE;
@@ -776,10 +810,31 @@ int sfm_monarch_attn_with_kv_cache(const sfm_monarch_desc* desc, const void* q, 
         set_error("workspace must be non-NULL, 256-byte aligned and hold at least %zu bytes (one unit)", pl.per_unit);
         return SFM_ERR_WORKSPACE;
     }
-    rc = sfm_kv_cache_write(desc->dtype, desc->B, desc->H, desc->D, &desc->tiling, new_k, new_v, new_stride, k_cache,
-                            v_cache, desc->k_stride, desc->kv_tokens, start_idx, end_idx, stream);
+    rc = check_cache_write(desc->dtype, desc->B, desc->H, desc->D, &desc->tiling, new_k, new_v, new_stride, k_cache, v_cache,
+                           desc->k_stride, desc->kv_tokens, start_idx, end_idx);
     if (rc) return rc;
-    return sfm_monarch_fwd(desc, q, k_cache, v_cache, out, workspace, workspace_bytes, stream);
+    const NewChunk nc = {new_k, new_v, new_stride, start_idx, end_idx};
+    return monarch_fwd_impl(desc, q, k_cache, v_cache, out, workspace, workspace_bytes, stream, nullptr, stats, &nc);
+}
+
+int sfm_monarch_attn_with_kv_cache(const sfm_monarch_desc* desc, const void* q, void* k_cache, void* v_cache,
+                                   const void* new_k, const void* new_v, const int64_t new_stride[3],
+                                   int64_t start_idx, int64_t end_idx, void* out, void* workspace,
+                                   size_t workspace_bytes, void* stream) {
+    return with_kv_cache_impl(desc, q, k_cache, v_cache, new_k, new_v, new_stride, start_idx, end_idx, out, nullptr, workspace,
+                              workspace_bytes, stream);
+}
+
+int sfm_monarch_attn_with_kv_cache_stats(const sfm_monarch_desc* desc, const void* q, void* k_cache, void* v_cache,
+                                         const void* new_k, const void* new_v, const int64_t new_stride[3],
+                                         int64_t start_idx, int64_t end_idx, void* out, float* stats, void* workspace,
+                                         size_t workspace_bytes, void* stream) {
+    if (!stats) {
+        set_error("stats is NULL");
+        return SFM_ERR_NULL;
+    }
+    return with_kv_cache_impl(desc, q, k_cache, v_cache, new_k, new_v, new_stride, start_idx, end_idx, out, stats, workspace,
+                              workspace_bytes, stream);
 }
 
 }  // extern "C"

@@ -175,6 +175,12 @@ struct MonarchArgs {
     // kept behind the fields that every step-1 kernel reads, whose places decide how the compiler fetches and keeps them
     int s2_split;    // step-2 waves that share the rows of one (a, j) column: 1, 2 or 4
     int skip_masked; // MFMA step 1 only: the scratch rows of masked (query, key) block-frame pairs are not read: do not form them
+    // MFMA step 1 only, with new_kv: kv block-frames [new_f0, new_f1) come from the new chunk's token-order tensors, tiled
+    // like q, and are written to their cache rows by the workgroups that load them
+    int new_kv, new_f0, new_f1;
+    const void* new_k;
+    const void* new_v;
+    int64_t ns[3];
 };
 
 // Backward: the forward arguments (scratch matrices in float) plus the gradient tensors.

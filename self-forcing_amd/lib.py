@@ -23,7 +23,7 @@ ERR_NAMES = {
 # every symbol include/sfm_attn.h declares
 SYMBOLS = [
     "sfm_monarch_workspace_bytes", "sfm_monarch_fwd", "sfm_monarch_fwd_timed", "sfm_kv_cache_write", "sfm_monarch_attn_with_kv_cache",
-    "sfm_monarch_attn_with_kv_cache_static",
+    "sfm_monarch_attn_with_kv_cache_static", "sfm_monarch_attn_with_kv_cache_stats",
     "sfm_dense_workspace_bytes", "sfm_dense_fwd_ws", "sfm_full_attention_with_kv_cache_ws",
     "sfm_dense_fwd", "sfm_full_attention_with_kv_cache", "sfm_qk_prologue", "sfm_ln_modulate", "sfm_gate_residual",
     "sfm_rms_norm", "sfm_gate_residual_ln", "sfm_linear", "sfm_monarch_bwd_workspace_bytes", "sfm_monarch_bwd", "sfm_monarch_bwd_uses_gemm",
@@ -119,6 +119,8 @@ def load():
                                        S3, I64, I64, I64, P]
     lib.sfm_monarch_attn_with_kv_cache.argtypes = [C.POINTER(MonarchDesc), P, P, P, P, P, S3, I64, I64, P, P,
                                                    C.c_size_t, P]
+    lib.sfm_monarch_attn_with_kv_cache_stats.argtypes = [C.POINTER(MonarchDesc), P, P, P, P, P, S3, I64, I64, P, P, P,
+                                                         C.c_size_t, P]
     lib.sfm_monarch_attn_with_kv_cache_static.argtypes = [C.POINTER(MonarchDesc), P, P, P, P, P, S3, I64, I64, P, P]
     lib.sfm_dense_fwd.argtypes = [C.POINTER(DenseDesc), P, P, P, P, P, P]
     lib.sfm_dense_workspace_bytes.argtypes = [C.POINTER(DenseDesc), C.POINTER(C.c_size_t)]

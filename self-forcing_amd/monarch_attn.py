@@ -124,8 +124,8 @@ def kv_cache_write(new_k, new_v, k_cache, v_cache, start_idx, end_idx, f_tied, h
                                               _stream(new_k)))
 
 
-def _monarch_fwd_stats(q, k, v, tiling, sm_scale, kv_block_order, cbf, heads_per_pass=0):
-    """Forward for autograd: returns (out, stats) where stats is the opaque row-statistics tensor that
+def _monarch_fwd_stats(q, k, v, tiling, sm_scale, kv_block_order, cbf, heads_per_pass=0, new=None):
+    """Forward for autograd, with new = (new_k, new_v, start_idx, end_idx) of the KV-cache operator: returns (out, stats) where stats is the opaque row-statistics tensor that
     sfm_monarch_bwd_saved takes, or None when the forward that runs for these tensors produces none (the
     reference's forward keeps z and z_lse the same way, monarch_attn.py:1309-1317)."""
     out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
@@ -135,8 +135,19 @@ def _monarch_fwd_stats(q, k, v, tiling, sm_scale, kv_block_order, cbf, heads_per
     nbytes = monarch_workspace_bytes(d, heads_per_pass)
     ws = scratch(nbytes, q.device)
     stats = torch.empty(n.value // 4, dtype=torch.float32, device=q.device) if n.value else None
+    if new is not None and stats is None:
+        kv_cache_write(*new[:2], k, v, *new[2:], *tiling)
     with _on_device(q.device):
-        if stats is None:
+        if new is not None and stats is not None:
+            new_k, new_v, start_idx, end_idx = new
+            if new_k.stride() != new_v.stride():
+                new_k, new_v = new_k.contiguous(), new_v.contiguous()
+            if k.stride() != v.stride():
+                raise ValueError("k_cache and v_cache must share their strides")
+            _l.check(_l.load().sfm_monarch_attn_with_kv_cache_stats(
+                C.byref(d), q.data_ptr(), k.data_ptr(), v.data_ptr(), new_k.data_ptr(), new_v.data_ptr(), _l.strides3(new_k),
+                start_idx, end_idx, out.data_ptr(), stats.data_ptr(), ws.data_ptr(), nbytes, _stream(q)))
+        elif stats is None:
             _l.check(_l.load().sfm_monarch_fwd(C.byref(d), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
                                                ws.data_ptr(), nbytes, _stream(q)))
         else:
@@ -225,8 +236,8 @@ class _MonarchCacheFn(torch.autograd.Function):
             raise ValueError("k/v shapes differ")
         if new_k.shape[1] != end_idx - start_idx:
             raise ValueError(f"new_k holds {new_k.shape[1]} tokens but end_idx - start_idx = {end_idx - start_idx}")
-        kv_cache_write(new_k, new_v, k_cache, v_cache, start_idx, end_idx, *tiling)
-        out, stats = _monarch_fwd_stats(q, k_cache, v_cache, tiling, sm_scale, 1, 0, heads_per_pass)
+        out, stats = _monarch_fwd_stats(q, k_cache, v_cache, tiling, sm_scale, 1, 0, heads_per_pass,
+                                        new=(new_k, new_v, start_idx, end_idx))
         ctx.has_stats = stats is not None
         if stats is not None:
             ctx.save_for_backward(q, k_cache, v_cache, out, stats)

@@ -131,6 +131,54 @@ def test_kv_cache_op_tilings(f_tied, h_reduce, w_reduce):
     assert_close_16bit(out, ref, dtype)
 
 
+@pytest.mark.parametrize("B,H,D,tiling,q_frames,first,last,frames,num_iters", [
+    (1, 2, 128, (1, 1, 1, 5, 52), 3, 2, 5, 5, 1),        # the last frames
+    (2, 3, 64, (1, 1, 1, 7, 9), 1, 1, 2, 4, 1),          # rows in the middle of the cache, short blocks
+    (1, 1, 128, (1, 2, 2, 6, 14), 2, 0, 2, 3, 1),        # block columns and rows apart in the frame
+    (1, 2, 128, (3, 1, 1, 4, 33), 3, 3, 6, 6, 1),        # tied frames, 33 columns
+    (1, 2, 128, (1, 1, 1, 3, 100), 6, 0, 6, 6, 1),       # four key tiles, several chunks of query block-frames
+    (1, 1, 64, (1, 1, 1, 2, 80), 1, 1, 2, 2, 1),         # three key tiles
+    (1, 2, 128, (1, 1, 1, 5, 20), 3, 3, 6, 6, 3),        # refinement: K in the first pass, V in the last
+    (2, 2, 64, (3, 2, 1, 4, 10), 3, 0, 3, 6, 2),
+    (1, 1, 128, (1, 1, 1, 4, 70), 3, 1, 4, 4, 2),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_step_1_writes_the_new_chunk_to_the_cache(dtype, B, H, D, tiling, q_frames, first, last, frames, num_iters):
+    """The kernels that read the new chunk where it is and write its cache rows beside the right factor give, bit for bit,
+    what the cache write in front of the no-cache operator gives: output, written rows and all the others.  The chunk is a view with strides
+    of its own; passes over one head at a time and the call with row statistics included."""
+    per = tiling[3] * tiling[4]
+    n = (last - first) * per
+    q = randn((B, q_frames * per, H, D), 1, dtype).to(DEV)
+    caches = [randn((B, frames * per + 3, H, D), 2 + i, dtype).to(DEV)[:, 3:] for i in range(2)]
+    news = [randn((B, n, H + 1, D), 4 + i, dtype).to(DEV)[:, :, 1:] for i in range(2)]
+    ref = [c.clone(memory_format=torch.preserve_format) for c in caches]
+    mattn.kv_cache_write(*news, *ref, first * per, last * per, *tiling)
+    want = mattn.monarch_attn(q, *ref, *tiling, num_iters=num_iters, kv_block_order=True)
+    for heads_per_pass in (0, 1):
+        got = [c.clone(memory_format=torch.preserve_format) for c in caches]
+        out = mattn.monarch_attn_with_kv_cache(q, *got, *news, first * per, last * per, *tiling, num_iters=num_iters, heads_per_pass=heads_per_pass)
+        assert torch.equal(out, want) and all(torch.equal(a, b) for a, b in zip(got, ref))
+    if num_iters == 1:
+        out, stats = mattn._monarch_fwd_stats(q, *ref, tiling, D ** -0.5, 1, 0)
+        got = [c.clone(memory_format=torch.preserve_format) for c in caches]
+        out2, stats2 = mattn._monarch_fwd_stats(q, *got, tiling, D ** -0.5, 1, 0, new=(*news, first * per, last * per))
+        b1 = tiling[0] * tiling[3] // tiling[1]
+        rows = lambda s: s.view(-1, (b1 + 31) // 32 * 32)[:, :b1]
+        assert torch.equal(out2, out) and torch.equal(rows(stats2), rows(stats)) and all(torch.equal(a, b) for a, b in zip(got, ref))
+
+
+def test_cache_call_under_autograd_takes_a_chunk_that_starts_within_a_block():
+    per = 4 * 20
+    q, nk, nv = (randn((1, per, 2, 64), i, torch.bfloat16).to(DEV) for i in range(3))
+    kc, vc = (randn((1, 3 * per, 2, 64), 3 + i, torch.bfloat16).to(DEV) for i in range(2))
+    ref = kc.clone(), vc.clone()
+    mattn.kv_cache_write(nk, nv, *ref, 30, 30 + per, 1, 1, 1, 4, 20)
+    want = mattn.monarch_attn(q, *ref, 1, 1, 1, 4, 20, kv_block_order=True)
+    out = mattn.monarch_attn_with_kv_cache(q.requires_grad_(True), kc, vc, nk, nv, 30, 30 + per, 1, 1, 1, 4, 20)
+    assert torch.equal(out.detach(), want) and torch.equal(kc, ref[0]) and torch.equal(vc, ref[1])
+
+
 def test_kv_cache_view_with_batch_stride_and_prefix():
     """B=2, the op sees kv_cache[:, :local_end] of a longer allocation (batch stride = full cache)."""
     h, w, H, D = 4, 20, 2, 64
