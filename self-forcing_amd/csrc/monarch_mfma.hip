@@ -28,6 +28,8 @@
 
 #include "sfm_common.hpp"
 
+#include <algorithm>
+
 namespace sfm {
 
 // ------------------------------------------------------------------------------------------------
@@ -49,17 +51,16 @@ template <int CPR>
 __device__ __forceinline__ int s1_swz(int r) {
     return CPR >= 16 ? (((r & 3) << 2) | ((r >> 2) & 3)) : ((((r >> 1) & 1) << 2) | ((r >> 2) & 3));
 }
-template <int D, int NT>
+template <int D, int NT, bool KO>
 struct S1Lds {
-    static constexpr int kRows = NT <= 2 ? 64 : 32 * NT;     // rows of a K / V tile
-    static constexpr int kPitch = 2 * D, kTile = kRows * kPitch;
-    static constexpr int kGroup = 4 * kTile;                 // [buffer][K tile | V tile]
-    static __host__ __device__ constexpr size_t bytes() { return (size_t)kGroup; }
+    static constexpr int kPitch = 2 * D, kTile = 32 * NT * kPitch;
+    static constexpr int kBuf = (KO ? 1 : 2) * kTile;        // [K tile | V tile]
+    static constexpr int kGroup = 2 * kBuf;
 };
 
-// NT: 32-row tiles of the key axis l (b2 <= 32 NT).  Up to two tiles a workgroup is two wave groups of at most 5 waves
-//     (170 registers per wave); three and four tiles (b2 up to 128: the 720p and 1080p grids) run one group of up to 8
-//     waves with 256 registers, whose tile buffers take 96 / 128 KB of LDS.
+// NT: 32-row tiles of the key axis l (b2 <= 32 NT).  Up to two tiles a wave has 170 registers and a workgroup is several
+//     wave groups: two of 5 waves at 156 columns.  Three and four tiles (b2 up to 128: the 720p and
+//     1080p grids) have 256 registers for up to 8 waves, and their tile buffers take 96 / 128 KB of LDS.
 // WR: also write the right factor R (16 bit, 64 values per scratch row) to p.rb; the backward uses it.
 // IT: a pass of the iterated refinement (wan/modules/monarch_attn.py:1716-1722): the logits are scaled per (a, f, k, j)
 //     column and, after the first pass, the query operand of tile (f, k) is the column's representative p.rep[a, j, (f, k)]
@@ -70,9 +71,9 @@ struct S1Lds {
 //     training clip of three chunks (a = f = 3, b1 = 90, b2 = 52, 12 heads) has a third of its pairs masked: 99 -> 85 us,
 //     with R written 119 -> 98.
 template <class E, int D, int NT, bool WR = false, bool IT = false, bool KO = false, bool CS = false>
-__global__ __launch_bounds__(NT > 2 ? 512 : 640) __attribute__((amdgpu_waves_per_eu(NT > 2 ? 2 : 3, NT > 2 ? 2 : 3)))
+__global__ __launch_bounds__(NT > 2 ? 512 : 768) __attribute__((amdgpu_waves_per_eu(NT > 2 ? 2 : 3, NT > 2 ? 2 : 3)))
 void monarch_step1_kernel(MonarchArgs p) {
-    using L = S1Lds<D, NT>;
+    using L = S1Lds<D, NT, KO>;
     constexpr int CPR = D / 8;   // 16-byte chunks of a K/V row
     constexpr int DS = D / 16;   // contraction steps of the logits
     extern __shared__ __attribute__((aligned(256))) char lds_s1[];
@@ -154,7 +155,7 @@ void monarch_step1_kernel(MonarchArgs p) {
             }
             vg = (const char*)p.new_v + n0;
         }
-        const uint32_t dst = lds0 + (uint32_t)buf * 2 * L::kTile;
+        const uint32_t dst = lds0 + (uint32_t)buf * L::kBuf;
         for (int g = wave; g < NT * (CPR / 2); g += nwaves) {         // 1 KB (64 / CPR rows) per step
             const int P = g * 64 + lane;
             const int r = P / CPR, c = (P % CPR) ^ s1_swz<CPR>(r);
@@ -257,7 +258,7 @@ void monarch_step1_kernel(MonarchArgs p) {
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         lds_barrier();                   // tile r is in LDS; every wave has finished reading the tile before it
         if (fresh) cur = nxt;
-        const char* kt = lds + (r & 1) * 2 * L::kTile;
+        const char* kt = lds + (r & 1) * L::kBuf;
         const char* vt = kt + L::kTile;
         const uint32_t srow = scratch_row(cur);
         if ((IT && p.iter_mode == 2) || query_key(cur) != qkey) {
@@ -1099,50 +1100,68 @@ int cu_count() {
     return cached;
 }
 
+enum class Step1 { kWhole, kIter, kIterKbar };           // the forward's (or the backward's), a refinement's last pass, its earlier ones
+
+struct Step1Kernel {
+    const void* fn;
+    size_t group;      // bytes of LDS of a wave group
+};
+
+template <class E, int D, int NT>
+static Step1Kernel step1_kernel(const MonarchArgs& a, Step1 kind) {
+    constexpr size_t whole = S1Lds<D, NT, false>::kGroup;
+    if (kind == Step1::kIterKbar) return {(const void*)monarch_step1_kernel<E, D, NT, false, true, true>, S1Lds<D, NT, true>::kGroup};
+    if (kind == Step1::kIter) return {(const void*)monarch_step1_kernel<E, D, NT, false, true>, whole};
+    const bool skip = a.causal && a.skip_masked;
+    if constexpr (NT <= 2) {
+        if (a.rb) return {skip ? (const void*)monarch_step1_kernel<E, D, NT, true, false, false, true> : (const void*)monarch_step1_kernel<E, D, NT, true>, whole};
+    }
+    return {skip ? (const void*)monarch_step1_kernel<E, D, NT, false, false, false, true> : (const void*)monarch_step1_kernel<E, D, NT, false>, whole};
+}
+
 // Enqueues step 1 (with the right factor written too when a.rb is set).
 template <class E, int D>
-static int enqueue_step1(const MonarchArgs& a, int nunits, hipStream_t stream, const void* fn_override = nullptr) {
+static int enqueue_step1(const MonarchArgs& a, int nunits, hipStream_t stream, Step1 kind = Step1::kWhole) {
     const int ncols = a.a_chunk * a.b2;
-    const int ntiles = (ncols + 31) / 32;
-    const int nwaves = ntiles < 4 ? 4 : ntiles;   // a wave per 32 (a, j) columns, at least 4 to share the tile loads
-    if (ntiles < 1 || nwaves > 8) {
+    const int nwaves = (ncols + 31) / 32;                 // a wave per 32 (a, j) columns
+    if (nwaves < 1 || nwaves > 8) {
         set_error("internal: step-1 launch shape (a_chunk=%d, b2=%d)", a.a_chunk, a.b2);
         return SFM_ERR_UNSUPPORTED;
     }
     const int nt = (a.b2 + 31) / 32;
-    const int groups = nwaves <= 5 && nt <= 2 ? 2 : 1;  // wave groups per workgroup (<= 10 waves in all)
-    const size_t lds1 = (nt == 4 ? S1Lds<D, 4>::bytes() : nt == 3 ? S1Lds<D, 3>::bytes() : S1Lds<D, 2>::bytes()) * groups;
     if (nt > 2 && a.rb) {
         set_error("internal: the right factor is written for b2 <= 64 only");
         return SFM_ERR_UNSUPPORTED;
     }
-    const bool skip = a.causal && a.skip_masked;
-    const void* fn = fn_override ? fn_override
-                     : skip && nt == 4 ? (const void*)monarch_step1_kernel<E, D, 4, false, false, false, true>
-                     : skip && nt == 3 ? (const void*)monarch_step1_kernel<E, D, 3, false, false, false, true>
-                     : skip && nt == 2 ? (a.rb ? (const void*)monarch_step1_kernel<E, D, 2, true, false, false, true>
-                                               : (const void*)monarch_step1_kernel<E, D, 2, false, false, false, true>)
-                     : skip ? (a.rb ? (const void*)monarch_step1_kernel<E, D, 1, true, false, false, true>
-                                    : (const void*)monarch_step1_kernel<E, D, 1, false, false, false, true>)
-                     : nt == 4 ? (const void*)monarch_step1_kernel<E, D, 4, false>
-                     : nt == 3 ? (const void*)monarch_step1_kernel<E, D, 3, false>
-                     : nt == 2 ? (a.rb ? (const void*)monarch_step1_kernel<E, D, 2, true> : (const void*)monarch_step1_kernel<E, D, 2, false>)
-                               : (a.rb ? (const void*)monarch_step1_kernel<E, D, 1, true> : (const void*)monarch_step1_kernel<E, D, 1, false>);
+    const Step1Kernel k = nt == 4   ? step1_kernel<E, D, 4>(a, kind)
+                          : nt == 3 ? step1_kernel<E, D, 3>(a, kind)
+                          : nt == 2 ? step1_kernel<E, D, 2>(a, kind)
+                                    : step1_kernel<E, D, 1>(a, kind);
+    MonarchArgs a1 = a;
+    a1.s1_total = a.nf * a.b1 * nunits * a.n_achunks;
+    // One workgroup per CU, of as many wave groups as its LDS holds up to 8 waves, or two of 5 or 6 (8 waves in all where one has
+    // 256 registers): a group's loads, logits, softmax and stores follow each other, and the other groups fill the gaps.  A
+    // group has the waves that its columns need and no more.  With at least four, the others of which formed and stored the last
+    // column again and again, and never more than two groups, three refinement passes at three frames tied (52 columns, 12
+    // heads x 128, 480p, 21 frames) took 529 us, now 499 (Kbar alone, four groups: 92 -> 73 a pass); one pass 176 -> 164; three
+    // tied frames against themselves 50 -> 46; 24 columns of nine 30 x 24 frames 52 -> 39.  Four groups of three waves: 50 us
+    // at 7 heads of nine 23 x 31 frames, two 44.5.  Two or four waves for 32 columns, each with its part of the output, took
+    // the refinement to 505 and 541 us: they fetch the query rows as often.
+    const int cus = a.s1_wgs > 0 ? a.s1_wgs : cu_count();
+    const int by_waves = nt > 2 ? 8 / nwaves : std::min(12 / nwaves, std::max(2, 8 / nwaves));      // within the launch bounds
+    const int room = std::min(by_waves, (int)(160 * 1024 / k.group));
+    a1.s1_groups = std::max(1, std::min(room, (a1.s1_total + cus - 1) / cus));
+    const int wgs = std::min(cus, (a1.s1_total + a1.s1_groups - 1) / a1.s1_groups);
+    const size_t lds1 = k.group * a1.s1_groups;
     if (lds1 > 64 * 1024) {
-        hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds1);
+        hipError_t e = hipFuncSetAttribute(k.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds1);
         if (e != hipSuccess) {
             set_error("hipFuncSetAttribute failed: %s", hipGetErrorString(e));
             return SFM_ERR_HIP;
         }
     }
-    MonarchArgs a1 = a;
-    a1.s1_total = a.nf * a.b1 * nunits * a.n_achunks;
-    a1.s1_groups = groups;
-    // one workgroup per CU (a CU holds one: 3 waves per SIMD), fewer when there are not two tiles for each
-    int wgs = a.s1_wgs > 0 ? a.s1_wgs : cu_count();
-    if (wgs > (a1.s1_total + groups - 1) / groups) wgs = (a1.s1_total + groups - 1) / groups;
     void* args[] = {&a1};
-    hipError_t e = hipLaunchKernel(fn, dim3(wgs), dim3(nwaves * 64 * groups), args, lds1, stream);
+    hipError_t e = hipLaunchKernel(k.fn, dim3(wgs), dim3(nwaves * 64 * a1.s1_groups), args, lds1, stream);
     if (e != hipSuccess) {
         set_error("hip launch failed: %s", hipGetErrorString(e));
         return SFM_ERR_HIP;
@@ -1248,22 +1267,13 @@ static int launch_rep_t(const MonarchArgs& a, int nunits, hipStream_t stream) {
 template <class E, int D>
 static int launch_iter_t(const MonarchArgs& a, int nunits, int num_iters, hipStream_t stream) {
     const int nq = (a.b1 + 31) / 32;
-    const int nt = (a.b2 + 31) / 32;
-    const void* fnk = nt == 4 ? (const void*)monarch_step1_kernel<E, D, 4, false, true, true>
-                    : nt == 3 ? (const void*)monarch_step1_kernel<E, D, 3, false, true, true>
-                    : nt == 2 ? (const void*)monarch_step1_kernel<E, D, 2, false, true, true>
-                              : (const void*)monarch_step1_kernel<E, D, 1, false, true, true>;
-    const void* fn1 = nt == 4 ? (const void*)monarch_step1_kernel<E, D, 4, false, true>
-                    : nt == 3 ? (const void*)monarch_step1_kernel<E, D, 3, false, true>
-                    : nt == 2 ? (const void*)monarch_step1_kernel<E, D, 2, false, true>
-                              : (const void*)monarch_step1_kernel<E, D, 1, false, true>;
     for (int it = 0; it < num_iters; ++it) {
         const bool last = it + 1 == num_iters;
         MonarchArgs a1 = a;
         a1.rb = nullptr;
         a1.iter_mode = it == 0 ? 1 : 2;
         a1.new_kv = it == 0 || last ? a.new_kv : 0;      // K in the first pass, V in the last
-        if (int rc = enqueue_step1<E, D>(a1, nunits, stream, last ? fn1 : fnk)) return rc;
+        if (int rc = enqueue_step1<E, D>(a1, nunits, stream, last ? Step1::kIter : Step1::kIterKbar)) return rc;
         MonarchArgs a2 = a;
         if (last) a2.stats = nullptr;
         if (int rc = enqueue_step2<E, D>(a2, nunits, stream, !last)) return rc;

@@ -168,6 +168,26 @@ def test_step_1_writes_the_new_chunk_to_the_cache(dtype, B, H, D, tiling, q_fram
         assert torch.equal(out2, out) and torch.equal(rows(stats2), rows(stats)) and all(torch.equal(a, b) for a, b in zip(got, ref))
 
 
+@pytest.mark.parametrize("D,w,q_frames,H,num_iters", [
+    (128, 5, 1, 5, 1),          # one wave to a group, five groups of 32 KB
+    (64, 32, 1, 6, 1),          # one wave, a whole key tile; eight groups
+    (128, 33, 1, 5, 1),         # two waves, two key tiles
+    (64, 21, 2, 6, 1),          # two waves, one key tile; four groups
+    (128, 31, 3, 4, 1),         # three waves
+    (128, 52, 1, 5, 3),         # two waves; Kbar alone with four groups, the last pass with two
+    (64, 9, 3, 6, 2),
+    (128, 70, 1, 4, 2),         # three key tiles: one group, two of Kbar alone at most
+])
+def test_step_1_wave_groups(D, w, q_frames, H, num_iters):
+    """More tiles than two wave groups of every compute unit take, few columns: every number of waves and of groups."""
+    h, frames, dtype = 32, 9, torch.bfloat16
+    q = randn((1, q_frames * h * w, H, D), 11, dtype)
+    k, v = (randn((1, frames * h * w, H, D), 12 + i, dtype) for i in range(2))
+    ref = monarch.monarch_attn(q, k, v, 1, 1, 1, h, w, num_iters=num_iters, dtype=torch.float32)
+    out = mattn.monarch_attn(q.to(DEV), k.to(DEV), v.to(DEV), 1, 1, 1, h, w, num_iters=num_iters)
+    assert_close_16bit(out, ref, dtype)
+
+
 def test_cache_call_under_autograd_takes_a_chunk_that_starts_within_a_block():
     per = 4 * 20
     q, nk, nv = (randn((1, per, 2, 64), i, torch.bfloat16).to(DEV) for i in range(3))
