@@ -1081,6 +1081,280 @@ __global__ __launch_bounds__(64 * (RepLds<D, NQ>::kWaves)) void monarch_rep_kern
 }
 
 // ------------------------------------------------------------------------------------------------
+// The two kernels above in one, for columns whose logits fit the registers of the waves that share them: W waves of a
+// workgroup deal the column's 32-row chunks of Kbar in turn and keep their logits S[i, r] (C chunks x NQ query tiles x 16
+// registers), reduce each row's maximum and sum over their lanes, merge them through LDS and scale:
+//   L[i, r] = exp2(z - max_wave) * exp2(max_wave - stats_i),   z = s log2e <Q_i, Kbar_r> - cl_r
+// so that Kbar is read, and its logits and exponentials are formed, once.  At one query tile (framewise 480p, 21 frames, 12
+// heads x 128: 604 MB) 148 us where the two kernels took 69 + 150, bound by that traffic; at three (three frames tied: 201
+// MB) 75 for 46 + 62, where one workgroup fills a compute unit and its loads, logits, reductions and stores follow each
+// other.  (98 with every value's maximum and sum reduced in all lanes, and with exp2f.)
+// ------------------------------------------------------------------------------------------------
+template <int D, int NQ, int W>
+struct WtLds {
+    static constexpr int kPitch = 2 * D, kTile = 32 * kPitch;
+    static constexpr int kBuf = kTile + 256;               // [Kbar chunk | cl values]
+    static constexpr int kWave = 2 * kBuf;                 // reused: the wave's rows' maxima, sums and scales
+    static constexpr int kWaves = W == 1 ? 4 : W;          // waves of a workgroup
+    static constexpr int kCols = kWaves / W;               // and its columns
+    static __host__ __device__ constexpr size_t bytes() { return (size_t)kWaves * kWave + (size_t)kCols * NQ * kTile; }
+};
+
+// Maximum / sum of each of 16 values over the 32 lanes of a half wave: a lane ends with value half_reduce_at(m), and its
+// neighbour m ^ 1 with the same.  Lanes trade half of their values at every step, so that it takes 38 operations for the 16.
+__device__ __forceinline__ int half_reduce_at(int m) { return 8 * ((m >> 4) & 1) + 4 * ((m >> 3) & 1) + 2 * ((m >> 2) & 1) + ((m >> 1) & 1); }
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+}
+
+template <bool MAX>
+__device__ __forceinline__ float half_reduce(float* x, int m) {
+    auto op = [](float a, float b) { return MAX ? fmaxf(a, b) : a + b; };
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        auto y = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, x[i]), __builtin_bit_cast(uint32_t, x[i + 8]), false, false);
+        x[i] = op(__builtin_bit_cast(float, (uint32_t)y[0]), __builtin_bit_cast(float, (uint32_t)y[1]));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const bool up = m & 8;
+        x[i] = op(up ? x[i + 4] : x[i], dpp_move<0x128>(up ? x[i] : x[i + 4]));          // row_ror:8
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const bool up = m & 4;
+        x[i] = op(up ? x[i + 2] : x[i], dpp_move<0x141>(up ? x[i] : x[i + 2]));          // row_half_mirror: lane 7 - l of eight
+    }
+    const bool up = m & 2;
+    x[0] = op(up ? x[1] : x[0], dpp_move<0x4e>(up ? x[0] : x[1]));                       // quad_perm:[2,3,0,1]
+    return op(x[0], dpp_move<0xb1>(x[0]));                                               // quad_perm:[1,0,3,2]
+}
+
+template <class E, int D, int NQ, int W, int C>
+__global__ __launch_bounds__(64 * (WtLds<D, NQ, W>::kWaves)) __attribute__((amdgpu_waves_per_eu(2, 2))) void monarch_weights_kernel(MonarchArgs p) {
+    using L = WtLds<D, NQ, W>;
+    constexpr int DS = D / 16, DT = D / 32, CPR = D / 8;
+    constexpr int NG = CPR / 2;                            // 1 KB pieces of a chunk
+    extern __shared__ __attribute__((aligned(256))) char lds_s2[];
+
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63;
+    const int m = lane & 31;
+    const int hf = lane >> 5;
+
+    const int b2 = p.b2;
+    const int njg = (b2 + L::kCols - 1) / L::kCols;
+    const int a = blockIdx.x / njg;
+    const int col = W == 1 ? wave : 0;                     // this wave's column of the workgroup's
+    const int j = min((int)(blockIdx.x % njg) * L::kCols + col, b2 - 1);      // past the last column: that one again, with the same results
+    const int w = W == 1 ? 0 : wave;                       // its chunks: w, w + W, ...
+    const int ul = blockIdx.y;
+    const int unit = p.unit0 + ul;
+    const int b = unit / p.H, h = unit % p.H;
+
+    const int r_lim = p.nf * p.b1;
+    const int nch = (r_lim + 31) / 32;
+    const int64_t blk = (int64_t)ul * p.ws_unit + (int64_t)(a * b2 + j) * p.ws_aj;
+    const char* kb = (const char*)p.kbar + blk * (2 * D);
+    const char* clp = (const char*)(p.cl + (int64_t)ul * p.cl_unit + (int64_t)(a * b2 + j) * p.cl_aj);
+    const uint32_t cl_ld = p.cl_row * 4;
+    char* repb = (char*)p.rep + blk * (2 * D);
+    float* wgt = p.wgt + blk;
+
+    char* const wl = lds_s2 + wave * L::kWave;
+    const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)wl;
+    char* const qt = lds_s2 + L::kWaves * L::kWave + col * NQ * L::kTile;     // the column's query rows, laid out like chunks of scratch rows
+    const uint32_t qt0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)qt;
+
+    // query rows into LDS (rows past b1 repeat the last one; their scale is zero)
+    const uint16_t* qg = (const uint16_t*)p.q + (int64_t)b * p.qs[0] + (int64_t)h * p.qs[2];
+    for (int g = w; g < NQ * NG; g += W) {
+        const int P = g * 64 + lane;
+        const int r = P / CPR, c = (P % CPR) ^ s1_swz<CPR>(r);
+        const uint32_t off = (uint32_t)((p.qmap.row(a, min(r, p.b1 - 1)) + j) * p.qs[1] * 2) + (uint32_t)c * 16;
+        s1_load_lds16((const char*)qg, off, qt0 + (uint32_t)g * 1024);
+    }
+    auto issue = [&](int n, int buf) {
+        const uint32_t dst = lds0 + (uint32_t)buf * L::kBuf;
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            const int P = g * 64 + lane;
+            const int r = P / CPR, c = (P % CPR) ^ s1_swz<CPR>(r);
+            const uint32_t off = (uint32_t)min(32 * n + r, r_lim - 1) * (2 * D) + (uint32_t)c * 16;
+            s1_load_lds16(kb, off, dst + (uint32_t)g * 1024);
+        }
+        s2_load_lds4(clp, (uint32_t)(32 * n + m) * cl_ld, dst + L::kTile);
+    };
+    if (w < nch) issue(w, 0);
+    if (w + W < nch) issue(w + W, 1);
+    const uint32_t b_off = (uint32_t)m * L::kPitch + (uint32_t)((hf ^ s1_swz<CPR>(m)) << 4);   // row m of a 32-row tile as an MFMA operand
+    uint32_t tr[DT][2];            // Q^T as the representatives' A operand: transposing reads
+    {
+        const int s16 = lane & 15, g16 = lane >> 4;
+        const int rl = 4 * hf + (s16 >> 2);
+        const int cl = 2 * (g16 & 1) + ((s16 & 3) >> 1);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+                const int r = rl + 8 * half;
+                tr[dt][half] = (uint32_t)(r * L::kPitch + (((4 * dt + cl) ^ s1_swz<CPR>(r)) << 4) + (s16 & 1) * 8);
+            }
+    }
+    const float sc2 = p.scale * kLog2e;
+    const f32x16 kZero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+
+    // this wave's share of the query rows has landed when only its first two chunks are outstanding
+    if (w + W < nch) wait_vm<2 * (NG + 1)>();
+    else if (w < nch) wait_vm<NG + 1>();
+    else wait_vm<0>();
+    lds_barrier();
+
+    f32x16 z[C][NQ];               // S[i = 32 qi + 8 g + 4 hf + e, r = 32 n + m], then its exponentials
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int n = w + c * W;
+        if (n >= nch) {
+#pragma unroll
+            for (int qi = 0; qi < NQ; ++qi)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) z[c][qi][v] = -INFINITY;
+            continue;
+        }
+        // chunk n has landed when only the one requested after it is outstanding
+        if (n + W < nch) wait_vm<NG + 1>();
+        else wait_vm<0>();
+        const char* kt = wl + (c & 1) * L::kBuf;
+        const float cc = *(const float*)(kt + L::kTile + m * 4);
+        const bool rok = 32 * n + m < r_lim;
+#pragma unroll
+        for (int qi = 0; qi < NQ; ++qi) {
+            f32x16 t;
+#pragma unroll
+            for (int ds = 0; ds < DS; ++ds) {
+                const u32x4 bk = *(const u32x4*)(kt + (b_off ^ (uint32_t)(ds << 5)));
+                const u32x4 aq = *(const u32x4*)(qt + qi * L::kTile + (b_off ^ (uint32_t)(ds << 5)));
+                t = E::mfma32(aq, bk, ds ? t : kZero);
+            }
+#pragma unroll
+            for (int v = 0; v < 16; ++v) z[c][qi][v] = rok ? t[v] * sc2 - cc : -INFINITY;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // the chunk has been read: the next but one may land on it
+        if (n + 2 * W < nch) issue(n + 2 * W, c & 1);
+    }
+
+    // Rows' maxima and sums over this wave's chunks, to the (dead) front of its chunk buffers: [NQ * 32] maxima, sums
+    float* const own = (float*)wl;
+    const int at = half_reduce_at(m), myrow = 8 * (at >> 2) + 4 * hf + (at & 3);
+#pragma unroll
+    for (int qi = 0; qi < NQ; ++qi) {
+        float t[16];
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            t[v] = z[0][qi][v];
+#pragma unroll
+            for (int c = 1; c < C; ++c) t[v] = fmaxf(t[v], z[c][qi][v]);
+        }
+        own[32 * qi + myrow] = half_reduce<true>(t, m);
+    }
+    lds_wave_sync();
+#pragma unroll
+    for (int qi = 0; qi < NQ; ++qi) {
+        float t[16];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const f32x4 mx = *(const f32x4*)(own + 32 * qi + 8 * g + 4 * hf);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float base = mx[e] == -INFINITY ? 0.f : mx[e];       // a wave without chunks
+                t[4 * g + e] = 0.f;
+#pragma unroll
+                for (int c = 0; c < C; ++c) {
+                    z[c][qi][4 * g + e] = fast_exp2(z[c][qi][4 * g + e] - base);
+                    t[4 * g + e] += z[c][qi][4 * g + e];
+                }
+            }
+        }
+        own[NQ * 32 + 32 * qi + myrow] = half_reduce<false>(t, m);
+    }
+    if (W > 1) lds_barrier();
+    else lds_wave_sync();
+    // scale of row i for this wave: exp2(max_wave - max) / sum, behind the maxima and sums that other waves still read
+    for (int i = lane; i < NQ * 32; i += 64) {
+        float M = -INFINITY, sum = 0.f;
+#pragma unroll
+        for (int x = 0; x < W; ++x) M = fmaxf(M, *(const float*)((W == 1 ? wl : lds_s2 + x * L::kWave) + i * 4));
+#pragma unroll
+        for (int x = 0; x < W; ++x) {
+            const float* o = (const float*)(W == 1 ? wl : lds_s2 + x * L::kWave);
+            sum += o[NQ * 32 + i] * exp2f(o[i] - M);             // a wave without chunks: 0 * exp2(-inf)
+        }
+        own[2 * NQ * 32 + i] = i < p.b1 ? exp2f(own[i] - M) / sum : 0.f;
+    }
+    lds_wave_sync();
+
+#pragma unroll
+    for (int qi = 0; qi < NQ; ++qi)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const f32x4 fac = *(const f32x4*)(own + 2 * NQ * 32 + 32 * qi + 8 * g + 4 * hf);
+#pragma unroll
+            for (int c = 0; c < C; ++c)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) z[c][qi][4 * g + e] *= fac[e];
+        }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int n = w + c * W;
+        if (n >= nch) break;
+        float wsum = 0.f;
+        u32x4 pb[NQ][2];
+#pragma unroll
+        for (int qi = 0; qi < NQ; ++qi) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) wsum += z[c][qi][v];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                pb[qi][q].x = pack2<E>(z[c][qi][8 * q + 0], z[c][qi][8 * q + 1]);
+                pb[qi][q].y = pack2<E>(z[c][qi][8 * q + 2], z[c][qi][8 * q + 3]);
+                pb[qi][q].z = pack2<E>(z[c][qi][8 * q + 4], z[c][qi][8 * q + 5]);
+                pb[qi][q].w = pack2<E>(z[c][qi][8 * q + 6], z[c][qi][8 * q + 7]);
+            }
+        }
+        wsum = xhalf_sum(wsum);
+        if (hf == 0) wgt[32 * n + m] = wsum;
+        char* rrow = repb + (size_t)(32 * n + m) * (2 * D);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+            f32x16 acc;
+#pragma unroll
+            for (int qi = 0; qi < NQ; ++qi)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const u32x2 lo = s1_read_tr(qt + qi * L::kTile, tr[dt][0] + q * 16 * L::kPitch);
+                    const u32x2 hi = s1_read_tr(qt + qi * L::kTile, tr[dt][1] + q * 16 * L::kPitch);
+                    const u32x4 aq = {lo.x, lo.y, hi.x, hi.y};
+                    acc = E::mfma32(aq, pb[qi][q], (qi | q) ? acc : kZero);
+                }
+            // rep^T[d = 32 dt + 8 g + 4 hf + e, r]: the half-swap leaves 8 consecutive d per lane
+#pragma unroll
+            for (int gp = 0; gp < 2; ++gp) {
+                const int g0 = 2 * gp, g1 = 2 * gp + 1;
+                auto rx = __builtin_amdgcn_permlane32_swap(pack2<E>(acc[4 * g0 + 0], acc[4 * g0 + 1]),
+                                                           pack2<E>(acc[4 * g1 + 0], acc[4 * g1 + 1]), false, false);
+                auto ry = __builtin_amdgcn_permlane32_swap(pack2<E>(acc[4 * g0 + 2], acc[4 * g0 + 3]),
+                                                           pack2<E>(acc[4 * g1 + 2], acc[4 * g1 + 3]), false, false);
+                const u32x4 o = {(uint32_t)rx[0], (uint32_t)ry[0], (uint32_t)rx[1], (uint32_t)ry[1]};
+                *(u32x4*)(rrow + (32 * dt + 16 * gp + 8 * hf) * 2) = o;
+            }
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------------------
 // host launch
 // ------------------------------------------------------------------------------------------------
 bool monarch_mfma_supported(int dtype, int D, int b2) {
@@ -1261,6 +1535,33 @@ static int launch_rep_t(const MonarchArgs& a, int nunits, hipStream_t stream) {
     return SFM_OK;
 }
 
+// Representatives and weights in one kernel; false where the logits of a column do not fit its waves' registers (C chunks of
+// NQ tiles are 16 C NQ of them, and four query tiles spill at two chunks).  Up to four chunks a wave has a column of its own:
+// three passes of 2 heads x 64 over 24 rows took 41.0 us with the two kernels, now 34.0; three frames of 480p 134 -> 123.
+template <class E, int D, int NQ, int W, int C>
+static bool launch_weights_t(const MonarchArgs& a, int nunits, hipStream_t stream, int* rc) {
+    using L = WtLds<D, NQ, W>;
+    if ((a.nf * a.b1 + 31) / 32 > W * C) return false;
+    const void* fn = (const void*)monarch_weights_kernel<E, D, NQ, W, C>;
+    hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)L::bytes());
+    MonarchArgs a1 = a;
+    void* args[] = {&a1};
+    if (e == hipSuccess) e = hipLaunchKernel(fn, dim3(a.na * ((a.b2 + L::kCols - 1) / L::kCols), nunits), dim3(64 * L::kWaves), args, L::bytes(), stream);
+    if (e != hipSuccess) set_error("hip launch failed: %s", hipGetErrorString(e));
+    *rc = e == hipSuccess ? SFM_OK : SFM_ERR_HIP;
+    return true;
+}
+
+template <class E, int D>
+static bool launch_weights(const MonarchArgs& a, int nunits, hipStream_t stream, int* rc) {
+    switch ((a.b1 + 31) / 32) {
+        case 1: return launch_weights_t<E, D, 1, 1, 4>(a, nunits, stream, rc) || launch_weights_t<E, D, 1, 4, 8>(a, nunits, stream, rc);
+        case 2: return launch_weights_t<E, D, 2, 8, 4>(a, nunits, stream, rc);
+        case 3: return launch_weights_t<E, D, 3, 8, 3>(a, nunits, stream, rc);
+        default: return false;
+    }
+}
+
 // num_iters - 1 passes of [step 1 with the pass's query operands, Kbar only | row statistics of the left factor |
 // representatives for the next pass], then a whole forward with the last representatives.  (With whole forwards in every
 // pass a three-pass call at three frames tied took 696 us.)
@@ -1276,6 +1577,11 @@ static int launch_iter_t(const MonarchArgs& a, int nunits, int num_iters, hipStr
         if (int rc = enqueue_step1<E, D>(a1, nunits, stream, last ? Step1::kIter : Step1::kIterKbar)) return rc;
         MonarchArgs a2 = a;
         if (last) a2.stats = nullptr;
+        int wrc = SFM_OK;
+        if (!last && launch_weights<E, D>(a, nunits, stream, &wrc)) {
+            if (wrc) return wrc;
+            continue;
+        }
         if (int rc = enqueue_step2<E, D>(a2, nunits, stream, !last)) return rc;
         if (!last) {
             const int rc = nq == 1 ? launch_rep_t<E, D, 1>(a, nunits, stream) : nq == 2 ? launch_rep_t<E, D, 2>(a, nunits, stream)

@@ -51,6 +51,38 @@ def test_fp32_tilings_against_oracle(tiling, h, w, n):
     assert max_abs(out, ref) < 2e-5
 
 
+@pytest.mark.parametrize("D,h,w,frames", [
+    (64, 1, 3, 1),        # one row, one column short of a workgroup's four
+    (128, 32, 5, 4),      # four chunks of 32 rows: a wave per column, its last chunk full
+    (128, 31, 6, 5),      # five chunks, the last of them ragged: four waves per column
+    (64, 32, 4, 32),      # 32 chunks: the most that four waves hold
+    (64, 32, 4, 33),      # 33: two kernels
+    (128, 33, 3, 1),      # two query tiles, the second with one row; waves without chunks
+    (64, 64, 3, 16),      # 32 chunks, the most for two tiles
+    (64, 43, 3, 24),      # 33
+    (128, 90, 3, 7),      # three tiles
+    (64, 96, 2, 8),       # 24 chunks, the most for three tiles
+    (128, 65, 3, 12),     # 25
+    (64, 100, 2, 3),      # four tiles: two kernels
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_representatives_from_logits_in_registers(dtype, D, h, w, frames):
+    """Columns around the numbers of 32-row chunks and of query tiles where the kernel that forms the left factor's weights once
+    takes another shape or leaves the column to two kernels.  Again with logits of up to 30, whose rows differ in their
+    maxima: a representative rounded to 16 bit moves such a logit by 30 / 2^9 (2^12), the weights and with them the
+    output by as large a part."""
+    q = randn((1, h * w, 2, D), 60, dtype)
+    k, v = (randn((1, frames * h * w, 2, D), 61 + i, dtype) for i in range(2))
+    for sharp in (1, 6):
+        scale = sharp * D ** -0.5
+        ref = monarch.monarch_attn(q, k, v, 1, 1, 1, h, w, sm_scale=scale, num_iters=2, dtype=torch.float32)
+        out = mattn.monarch_attn(q.to(DEV), k.to(DEV), v.to(DEV), 1, 1, 1, h, w, sm_scale=scale, num_iters=2)
+        if sharp == 1:
+            assert_close_16bit(out, ref, dtype)
+        else:
+            assert ((out.float().cpu() - ref).norm() / ref.norm()).item() < 30 / 2 ** (9 if dtype == torch.bfloat16 else 12)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_16bit_inputs_and_cache_entry_point(dtype):
     """Cache holds 2 of 3 frames, the third arrives with the call; rows are in block order (h_reduce = 2)."""
