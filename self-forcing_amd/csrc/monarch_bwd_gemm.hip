@@ -425,9 +425,11 @@ Parts make_parts(const MonarchArgs& p, int dtype, const int64_t* dks) {
     f.dqa = f.left && !(sw & SFM_SW_BWD_DQA_GEMM);
     const bool direct_ok = (dks[0] | dks[1] | dks[2] | p.vs[0] | p.vs[1] | p.vs[2] | p.ks[0] | p.ks[1] | p.ks[2]) % 8 == 0 &&      // 16-byte rows of k, v, dk, dv
                            (int64_t)p.nf * p.b1 * p.b2 * p.ks[1] * 2 < ((int64_t)1 << 32);
-    f.right = f.fwd && direct_ok && monarch_bwd_right_supported(dtype, p.D, p.b2, p.na * p.b2) &&
+    f.dqk = monarch_bwd_dqk_supported(dtype, p.D, p.b2, p.na * p.b2) && !(sw & SFM_SW_BWD_DQK_GEMM);
+    // the rows of dS1 are padded to whole 8-byte pieces, which the library product of part 10 does not know
+    f.right = f.fwd && direct_ok && monarch_bwd_right_supported(dtype, p.D, p.b2, p.na * p.b2) && (f.dqk || p.b2 % 4 == 0) &&
               !(sw & SFM_SW_BWD_RIGHT_GEMM);
-    f.dqk = f.right && monarch_bwd_dqk_supported(dtype, p.D, p.b2, p.na * p.b2) && !(sw & SFM_SW_BWD_DQK_GEMM);
+    f.dqk = f.dqk && f.right;
     return f;
 }
 
@@ -445,7 +447,7 @@ Layout make_layout(const MonarchArgs& p, int n, size_t e, const Parts& f) {
     l.S1f = take(!f.fwd, n * p.b1 * AJ * NL * 4);
     l.dRb = take(!f.right, n * p.b1 * AJ * NL * 4);
     l.Rb = take(true, n * p.b1 * AJ * p.nf * (size_t)(p.b2 > 64 ? p.b2 : 64) * e);      // row pitch 64 when step 1 of the forward writes it
-    l.dS1 = take(true, n * p.b1 * AJ * NL * e);
+    l.dS1 = take(true, n * p.b1 * AJ * p.nf * (size_t)(f.right ? (p.b2 + 3) / 4 * 4 : p.b2) * e);
     l.Kbar = take(true, n * AJ * RR * D * e);
     l.Y = take(true, n * AJ * RR * D * e);
     l.dKbar = take(true, n * AJ * RR * D * e);

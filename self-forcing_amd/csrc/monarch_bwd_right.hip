@@ -1,4 +1,4 @@
-// Right-factor part of the Monarch backward on gfx950 MFMA (bf16 / fp16, head_dim 64 or 128, b2 <= 64 a multiple of 4;
+// Right-factor part of the Monarch backward on gfx950 MFMA (bf16 / fp16, head_dim 64 or 128, b2 <= 64;
 // at most 480 (a, j) columns, taken 160 at a time).
 //
 // Replaces, per tile t = (unit, k, f), the small batched products and the row kernel of the GEMM chain
@@ -47,7 +47,7 @@ struct RightArgs {
     const char* q;           // caller's tensor: row (a, j) of (unit, k) is token qmap.row(a, k) + j, strides qs0, qs1, qs2
     int64_t qs0, qs1, qs2;
     TokMap qmap;
-    uint16_t* ds1;           // [(u, k)][AJ][nf * b2]
+    uint16_t* ds1;           // [(u, k)][AJ][nf * b2p], b2p = b2 rounded up to 4; the padding is zero
     uint16_t* dk;            // caller's tensors: row kmap.row(f, k) + l - row0, strides s0 (batch), s1 (row), s2 (head)
     uint16_t* dv;
     int64_t s0, s1, s2, row0;
@@ -243,8 +243,8 @@ __global__ __launch_bounds__(kThreads) void monarch_bwd_right_kernel(RightArgs p
             const u32x2 w = *(const u32x2*)(lds + oR + col * 128 + ((c ^ br_swz<8>(col)) << 4) + 8 * hf);
             const float r0 = E::to_float((uint16_t)(w.x & 0xffffu)), r1 = E::to_float((uint16_t)(w.x >> 16));
             const float r2 = E::to_float((uint16_t)(w.y & 0xffffu)), r3 = E::to_float((uint16_t)(w.y >> 16));
-            const bool live = 32 * tl + 8 * g + 4 * hf < b2;            // b2 is a multiple of 4: whole pieces
-            const float rr[4] = {live ? r0 : 0.f, live ? r1 : 0.f, live ? r2 : 0.f, live ? r3 : 0.f};
+            const int left = b2 - (32 * tl + 8 * g + 4 * hf);            // rows l of this piece that exist
+            const float rr[4] = {left > 0 ? r0 : 0.f, left > 1 ? r1 : 0.f, left > 2 ? r2 : 0.f, left > 3 ? r3 : 0.f};
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int v = 4 * g + e;
@@ -273,14 +273,14 @@ __global__ __launch_bounds__(kThreads) void monarch_bwd_right_kernel(RightArgs p
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                     // the query rows have landed
     __syncthreads();                                                     // the dS1 tile is complete
-    // dS1 to memory for dQ = s dS1 K: row aj is b2 consecutive elements, 8-byte pieces, consecutive lanes along a row
+    // dS1 to memory for dQ = s dS1 K: row aj is b2p consecutive elements, 8-byte pieces, consecutive lanes along a row
     {
-        const int ppr = b2 / 4;                                          // pieces per row
-        uint16_t* out = p.ds1 + (uk * AJ + c0) * ((int64_t)nf * b2) + (int64_t)f * b2;
+        const int ppr = (b2 + 3) / 4, b2p = 4 * ppr;                     // pieces per row
+        uint16_t* out = p.ds1 + (uk * AJ + c0) * ((int64_t)nf * b2p) + (int64_t)f * b2p;
         for (int i = tid; i < nrows * ppr; i += kThreads) {
             const int row = i / ppr, pc = i % ppr;
             const u32x2 w = *(const u32x2*)(lds + oS + row * 128 + (((pc >> 1) ^ br_swz<8>(row)) << 4) + 8 * (pc & 1));
-            *(u32x2*)(out + (int64_t)row * nf * b2 + 4 * pc) = w;
+            *(u32x2*)(out + (int64_t)row * nf * b2p + 4 * pc) = w;
         }
     }
     if (want) {
@@ -320,7 +320,7 @@ struct DqkArgs {
     const char* k;           // caller's tensor: row kmap.row(f, k) + l, strides ks0 (batch), ks1 (row), ks2 (head), in elements
     int64_t ks0, ks1, ks2;
     TokMap kmap;
-    const uint16_t* ds1;     // [(u, k)][AJ][nf * b2]
+    const uint16_t* ds1;     // [(u, k)][AJ][nf * b2p] as the kernel above writes it
     float* dqk;              // [(u, k)][AJ][D], or the caller's rows to add to: token qmap.row(a, k) + j, strides dqs
     int64_t dqs0, dqs1, dqs2;
     TokMap qmap;
@@ -344,20 +344,20 @@ __global__ __launch_bounds__(1024) void monarch_bwd_dqk_kernel(DqkArgs p) {
     const int64_t uk = blockIdx.x;
     const int k = (int)(uk % p.b1);
     const int unit = p.unit0 + (int)(uk / p.b1);
-    const int b2 = p.b2, AJ = p.AJ, NL = p.nf * b2;
+    const int b2 = p.b2, b2p = (b2 + 3) & ~3, AJ = p.AJ, NL = p.nf * b2p;
     const int nt = (NL + 63) / 64;
-    auto visible = [&](int aj) { return p.causal ? min(p.nf, (aj / b2 / p.causal + 1) * p.causal) * b2 : NL; };      // elements of dS1 row aj
+    auto visible = [&](int aj) { return p.causal ? min(p.nf, (aj / b2 / p.causal + 1) * p.causal) * b2p : NL; };      // elements of dS1 row aj
 
     const char* kbase = p.k + ((int64_t)(unit / p.H) * p.ks0 + (int64_t)(unit % p.H) * p.ks2) * 2;
     const uint32_t krb = (uint32_t)(p.ks1 * 2);
     // LDS position P (16-byte units) of a tile holds chunk (P % CPR) ^ swz(row) of row P / CPR; row x of the flat (f, l)
-    // axis is token kmap.row(x / b2, k) + x % b2 (rows past the end repeat the last one; dS1 is zero there)
+    // axis is token kmap.row(x / b2p, k) + x % b2p (rows past a block's or the whole end repeat its last one; dS1 is zero there)
     auto stage = [&](int t) {
         for (int g = wave; g < CPR; g += nwaves) {
             const int P = g * 64 + lane;
             const int r = P / CPR, c = (P % CPR) ^ br_swz<CPR>(r);
             const int x = min(64 * t + r, NL - 1);
-            const uint32_t tok = (uint32_t)(p.kmap.row(x / b2, k) + x % b2);
+            const uint32_t tok = (uint32_t)(p.kmap.row(x / b2p, k) + min(x % b2p, b2 - 1));
             br_load_lds16(kbase, tok * krb + (uint32_t)(c * 16), lds0 + (uint32_t)(t & 1) * kTile + (uint32_t)g * 1024);
         }
     };
@@ -460,7 +460,7 @@ __global__ __launch_bounds__(1024) void monarch_bwd_dqk_kernel(DqkArgs p) {
 
 bool monarch_bwd_right_supported(int dtype, int D, int b2, int AJ) {
     // up to three passes of 160 columns over a tile
-    return (dtype == SFM_BF16 || dtype == SFM_F16) && (D == 64 || D == 128) && b2 >= 4 && b2 <= 64 && b2 % 4 == 0 && AJ <= 3 * kMaxAJ;
+    return (dtype == SFM_BF16 || dtype == SFM_F16) && (D == 64 || D == 128) && b2 >= 1 && b2 <= 64 && AJ <= 3 * kMaxAJ;
 }
 
 int launch_monarch_bwd_right(int dtype, int D, int64_t ntiles, int b1, int b2, int AJ, int nf, float scale, const void* kk,
@@ -521,7 +521,7 @@ int launch_monarch_bwd_right(int dtype, int D, int64_t ntiles, int b1, int b2, i
 
 // at most 16 waves of 32 columns each
 bool monarch_bwd_dqk_supported(int dtype, int D, int b2, int AJ) {
-    return (dtype == SFM_BF16 || dtype == SFM_F16) && (D == 64 || D == 128) && b2 % 4 == 0 && AJ <= 512;
+    return (dtype == SFM_BF16 || dtype == SFM_F16) && (D == 64 || D == 128) && AJ <= 512;
 }
 
 int launch_monarch_bwd_dqk(int dtype, int D, int64_t nuk, int b1, int b2, int AJ, int nf, float scale, const void* k, const int64_t* ks,

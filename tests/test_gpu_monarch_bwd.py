@@ -158,7 +158,7 @@ def test_480p_block_shape_bf16_one_head(bwd_path):
     (4, 52, 3, 5, 64, False, torch.float16),
     (4, 52, 4, 4, 64, True, torch.bfloat16),       # 208 columns: two passes of the right-factor kernel over each tile
     (4, 52, 7, 7, 128, False, torch.float16),      # 364 columns: three passes
-    (5, 6, 2, 3, 64, False, torch.bfloat16),       # b2 = 6, not a multiple of 4: likewise
+    (5, 6, 2, 3, 64, False, torch.bfloat16),       # b2 = 6, not a multiple of 4
     (4, 20, 3, 9, 128, False, torch.bfloat16),     # 36 rows (f, k) per column: two chunks of the left factor, the second with 4 rows
     (8, 12, 2, 8, 64, False, torch.float16),       # 64 rows: two full chunks
     (6, 10, 6, 6, 128, True, torch.bfloat16),      # block-causal with two chunks: the visible rows end inside a chunk
@@ -178,6 +178,26 @@ def test_16bit_gradients_across_the_fused_kernels_limits(h, w, Fq, Fk, D, causal
     _close(qd.grad, qr.grad, dtype)
     _close(kd.grad, kr.grad, dtype)
     _close(vd.grad, vr.grad, dtype)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("b2", [1, 2, 3, 5, 26, 31, 33, 39, 63])
+def test_block_columns_that_are_no_multiple_of_four(b2, D):
+    """The rows of dS1 hold whole pieces of four: gradients at block widths between them, block-causal and not, on a scratch
+    full of NaN, and from the fused chain, whose workspace is smaller than the library chain's."""
+    h, F, H, dtype = 5, 4, 2, torch.bfloat16
+    q0, do = (randn((1, F * h * b2, H, D), 800 + b2 + i, dtype) for i in range(2))
+    k0, v0 = (randn((1, F * h * b2, H, D), 802 + b2 + i, dtype) for i in range(2))
+    for kw in ({}, {"block_causal_size": 2 * h * b2}):
+        qr, kr, vr = _leaf(q0.double()), _leaf(k0.double()), _leaf(v0.double())
+        monarch.monarch_attn(qr, kr, vr, 1, 1, 1, h, b2, **kw).backward(do.double())
+        qd, kd, vd = _leaf(q0, DEV), _leaf(k0, DEV), _leaf(v0, DEV)
+        out = mattn.monarch_attn(qd, kd, vd, 1, 1, 1, h, b2, **kw)
+        mattn.scratch(256 << 20, torch.device(DEV)).fill_(0xff)
+        out.backward(do.to(DEV))
+        _close(qd.grad, qr.grad, dtype)
+        _close(kd.grad, kr.grad, dtype)
+        _close(vd.grad, vr.grad, dtype)
 
 
 @pytest.mark.parametrize("D", [64, 128])
