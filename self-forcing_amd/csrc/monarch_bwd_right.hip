@@ -34,8 +34,6 @@
 namespace sfm {
 namespace {
 
-constexpr int kMaxAJ = 160;
-
 struct RightArgs {
     const char* kk;          // callers' tensors: row kmap.row(f, k) + l, strides (batch, row, head) in elements
     const char* v;
@@ -52,6 +50,7 @@ struct RightArgs {
     uint16_t* dv;
     int64_t s0, s1, s2, row0;
     TokMap kmap;
+    int64_t ntiles;
     int b1, b2, AJ, nf, H, unit0, f0, f1;
     int causal;              // block-causal size: the columns before a tile's first visible one are left out; 0 = none
     float scale;
@@ -72,80 +71,229 @@ __device__ __forceinline__ int br_swz(int r) {
     return CPR >= 16 ? (((r & 3) << 2) | ((r >> 2) & 3)) : ((((r >> 1) & 1) << 2) | ((r >> 2) & 3));
 }
 
-constexpr int kWaves = 16, kThreads = 64 * kWaves;
+constexpr int kCols = 64;                                  // columns per chunk
+constexpr int kWaves = 8, kThreads = 64 * kWaves;
 
-// NP: passes over the tile, 160 columns each (with more than one the dS1 tile has LDS of its own).  The passes are
-// written out one after the other: as a loop, the invariant LDS addresses of all the transposing reads get hoisted
-// out of it and spill.
-template <class E, int D, int NP>
-__global__ __launch_bounds__(kThreads) void monarch_bwd_right_kernel(RightArgs p) {
+template <int D>
+struct RightLds {
+    static constexpr int kPitch = 2 * D, kTile = 64 * kPitch;             // K, V, dKbar, dY: 64 rows
+    static constexpr int oK = 0, oV = kTile, oG = 2 * kTile, oH = 3 * kTile, oR = 4 * kTile, oDot = oR + kCols * 128;
+    static constexpr int kBytes = oDot + 2 * kCols * 4;
+};
+
+template <class E, int D>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void monarch_bwd_right_kernel(RightArgs p) {
+    using L = RightLds<D>;
     constexpr int DS = D / 16, DT = D / 32;
     constexpr int CPR = D / 8;                            // chunks per row of the D-wide tiles
-    constexpr int kPitch = 2 * D;
-    constexpr int kKV = 64 * kPitch;                      // K or V tile, 64 rows
-    constexpr int kG = kMaxAJ * kPitch;                   // dKbar or dY tile, 160 rows
-    constexpr int kR = kMaxAJ * 128;                      // R tile, 160 rows of 64
-    constexpr int oK = 0, oV = kKV, oG = 2 * kKV, oH = 2 * kKV + kG, oR = 2 * kKV + 2 * kG;
-    // dS1 tile (like R): over the K / V tiles after phase 1 where it fits there and they are not needed again (head_dim
-    // 128, all columns in one pass), else behind the R tile
-    constexpr bool MULTI = NP > 1;
-    constexpr bool s_over_kv = kR <= 2 * kKV && !MULTI;
-    constexpr uint32_t oS = s_over_kv ? 0 : oR + kR;
-    constexpr uint32_t oDot = oR + kR + (s_over_kv ? 0 : kR);             // float [2][160]: per-column partial sums of the two l halves
+    constexpr int kPitch = L::kPitch;
+    constexpr int LBW = DT / 2;                           // 32-row blocks of key rows that a gradient wave owns
     extern __shared__ __attribute__((aligned(256))) char lds[];
     const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)lds;
 
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, hf = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int64_t t = blockIdx.x;
+    // neighbouring tiles (block-frames of one block row) run on one XCD: their query rows and the lines of their dS1 rows meet in its L2
+    const int64_t t = (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    if (t >= p.ntiles) return;
     const int b2 = p.b2, AJ = p.AJ, nf = p.nf;
     const int f = (int)(t % nf);
     const int64_t uk = t / nf;
     const int k = (int)(uk % p.b1);
     const int64_t u = uk / p.b1;
+    const int unit = p.unit0 + (int)u;
 
-    // ---- stage the five tiles: LDS position P (16-byte units) of a tile holds chunk (P % CPR) ^ swz(row) of row P / CPR
-    auto stage = [&](const char* src, uint32_t row_bytes, int nchunks, uint32_t dst, auto cpr_c) {
+    // LDS position P (16-byte units) of a tile holds chunk (P % C) ^ swz(row) of row P / C; 64 rows, those past the end repeat
+    // the last one: what they add is multiplied by zeros of R and dS1 or lands in key rows that are not stored
+    auto stage = [&](const char* src, uint32_t row_bytes, int nrows, uint32_t dst, auto cpr_c) {
         constexpr int C = decltype(cpr_c)::value;
-        for (int g = wave; g * 64 < nchunks; g += kWaves) {
-            const int P = min(g * 64 + lane, nchunks - 1);             // lanes past the end repeat the last chunk (into a pad row, zeroed below)
+#pragma unroll
+        for (int g = 0; g < C / kWaves; ++g) {
+            const int P = (wave + g * kWaves) * 64 + lane;
             const int r = P / C, c = (P % C) ^ br_swz<C>(r);
-            br_load_lds16(src, (uint32_t)r * row_bytes + (uint32_t)(c * 16), lds0 + dst + (uint32_t)g * 1024);
+            br_load_lds16(src, (uint32_t)min(r, nrows - 1) * row_bytes + (uint32_t)(c * 16), lds0 + dst + (uint32_t)(wave + g * kWaves) * 1024);
         }
     };
     using c_d = std::integral_constant<int, CPR>;
     using c_r = std::integral_constant<int, 8>;
-    const int unit = p.unit0 + (int)u;
-    stage(p.kk + ((int64_t)(unit / p.H) * p.ks0 + (int64_t)(unit % p.H) * p.ks2 + p.kmap.row(f, k) * p.ks1) * 2, (uint32_t)(p.ks1 * 2),
-          b2 * CPR, oK, c_d{});
-    stage(p.v + ((int64_t)(unit / p.H) * p.vs0 + (int64_t)(unit % p.H) * p.vs2 + p.kmap.row(f, k) * p.vs1) * 2, (uint32_t)(p.vs1 * 2),
-          b2 * CPR, oV, c_d{});
+    stage(p.kk + ((int64_t)(unit / p.H) * p.ks0 + (int64_t)(unit % p.H) * p.ks2 + p.kmap.row(f, k) * p.ks1) * 2, (uint32_t)(p.ks1 * 2), b2,
+          L::oK, c_d{});
+    stage(p.v + ((int64_t)(unit / p.H) * p.vs0 + (int64_t)(unit % p.H) * p.vs2 + p.kmap.row(f, k) * p.vs1) * 2, (uint32_t)(p.vs1 * 2), b2,
+          L::oV, c_d{});
     const bool want = f >= p.f0 && f < p.f1;                             // uniform: dK / dV of this kv block-frame are asked for
 
-    // phase 2 operands: C^T[d, l] = sum_aj A^T[d, aj] B[aj, l]; a wave owns 32 head-dim rows x 32 key rows of dV (waves
-    // 0 .. 2 DT - 1) or of dK (the next 2 DT waves)
-    const int s16 = lane & 15, g16 = lane >> 4;
-    const int rl = 4 * hf + (s16 >> 2);
-    const int cl = 2 * (g16 & 1) + ((s16 & 3) >> 1);
-    const uint32_t sub = (uint32_t)(s16 & 1) * 8;
-    const int dt = wave % DT, lb = (wave / DT) & 1, which = wave / (2 * DT);      // which: 0 dV, 1 dK, else idle
-    auto product = [&](uint32_t oA, uint32_t oB, f32x16& acc) {      // acc += ...
-        const int ca = 4 * dt + cl, cb = 4 * lb + cl;
-#pragma unroll
-        for (int ks = 0; ks < kMaxAJ / 16; ++ks) {
-            const int r0 = 16 * ks + rl, r1 = r0 + 8;                     // rows aj of the two halves of the operands
-            const u32x2 alo = br_read_tr(lds, oA + (uint32_t)r0 * kPitch + (uint32_t)((ca ^ br_swz<CPR>(r0)) << 4) + sub);
-            const u32x2 ahi = br_read_tr(lds, oA + (uint32_t)r1 * kPitch + (uint32_t)((ca ^ br_swz<CPR>(r1)) << 4) + sub);
-            const u32x2 blo = br_read_tr(lds, oB + (uint32_t)r0 * 128 + (uint32_t)((cb ^ br_swz<8>(r0)) << 4) + sub);
-            const u32x2 bhi = br_read_tr(lds, oB + (uint32_t)r1 * 128 + (uint32_t)((cb ^ br_swz<8>(r1)) << 4) + sub);
-            const u32x4 aop = {alo.x, alo.y, ahi.x, ahi.y};
-            const u32x4 bop = {blo.x, blo.y, bhi.x, bhi.y};
-            acc = E::mfma32(aop, bop, acc);
+    const char* qbase = p.q + ((int64_t)(unit / p.H) * p.qs0 + (int64_t)(unit % p.H) * p.qs2) * 2;
+    const uint32_t qrb = (uint32_t)(p.qs1 * 2);
+    const int ppr = (b2 + 3) / 4, b2p = 4 * ppr;                         // 8-byte pieces of a dS1 row
+    const int cfirst = p.causal ? f / p.causal * p.causal * b2 : 0;      // the first column (a, j) that sees key block-frame f
+
+    // What every wave does in a chunk; the two kinds of waves meet in the same four barriers.
+    auto begin = [&](int c0, int nrows) {
+        stage(p.dkbar + (t * AJ + c0) * kPitch, kPitch, nrows, L::oG, c_d{});
+        stage(p.dy + (t * AJ + c0) * kPitch, kPitch, nrows, L::oH, c_d{});
+        stage(p.rb + (t * AJ + c0) * 128, 128, nrows, L::oR, c_r{});
+    };
+    auto loaded = [&](int nrows) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (nrows < kCols) {                                             // columns past the end have no weight
+            const u32x4 z = {0u, 0u, 0u, 0u};
+            for (int i = tid; i < (kCols - nrows) * 8; i += kThreads) *(u32x4*)(lds + L::oR + nrows * 128 + i * 16) = z;
+            __syncthreads();
         }
     };
+    auto queries = [&](int c0, int nrows) {                              // the query rows of (unit, k) take the place of the dY tile
+        if (!want) return;
+#pragma unroll
+        for (int g = 0; g < CPR / kWaves; ++g) {
+            const int P = (wave + g * kWaves) * 64 + lane;
+            const int r = P / CPR, c = (P % CPR) ^ br_swz<CPR>(r);
+            const int aj = c0 + min(r, nrows - 1);
+            const uint32_t tok = (uint32_t)(p.qmap.row(aj / b2, k) + aj % b2);
+            br_load_lds16(qbase, tok * qrb + (uint32_t)(c * 16), lds0 + L::oH + (uint32_t)(wave + g * kWaves) * 1024);
+        }
+    };
+    auto complete = [&](int c0, int nrows) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                 // the query rows have landed
+        __syncthreads();                                                 // the dS1 tile is complete
+        // dS1 to memory for dQ = s dS1 K: row aj is b2p consecutive elements, 8-byte pieces, consecutive lanes along a row
+        uint16_t* out = p.ds1 + (uk * AJ + c0) * ((int64_t)nf * b2p) + (int64_t)f * b2p;
+        for (int i = tid; i < nrows * ppr; i += kThreads) {
+            const int row = i / ppr, pc = i - row * ppr;
+            const u32x2 w = *(const u32x2*)(lds + L::oR + row * 128 + (((pc >> 1) ^ br_swz<8>(row)) << 4) + 8 * (pc & 1));
+            *(u32x2*)(out + (int64_t)row * nf * b2p + 4 * pc) = w;
+        }
+    };
+
+    if (wave < 4) {
+        // ---- softmax waves: 32 columns x 32 key rows
+        const int tl = wave >> 1, col = 32 * (wave & 1) + m;
+        const uint32_t a_off = (uint32_t)(32 * tl + m) * kPitch + (uint32_t)((hf ^ br_swz<CPR>(m)) << 4);
+        const uint32_t b_off = (uint32_t)col * kPitch + (uint32_t)((hf ^ br_swz<CPR>(m)) << 4);
+        for (int c0 = cfirst; c0 < AJ; c0 += kCols) {
+            const int nrows = min(kCols, AJ - c0);
+            begin(c0, nrows);
+            const float dcv = col < nrows ? p.dc[(u * AJ + c0 + col) * ((int64_t)nf * p.b1) + (int64_t)k * nf + f] : 0.f;
+            loaded(nrows);
+            // dR^T[l, aj] = K dKbar^T + V dY^T, then R (16 bit) of the l this lane holds: l = 32 tl + 8 g + 4 hf + 0..3
+            f32x16 dr;
+            float rv[16];
+            float dot = 0.f;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) dr[v] = 0.f;
+#pragma unroll
+            for (int ds = 0; ds < DS; ++ds) {
+                const u32x4 bg = *(const u32x4*)(lds + L::oG + (b_off ^ (uint32_t)(ds << 5)));
+                const u32x4 bh = *(const u32x4*)(lds + L::oH + (b_off ^ (uint32_t)(ds << 5)));
+                const u32x4 ak = *(const u32x4*)(lds + L::oK + (a_off ^ (uint32_t)(ds << 5)));
+                const u32x4 av = *(const u32x4*)(lds + L::oV + (a_off ^ (uint32_t)(ds << 5)));
+                dr = E::mfma32(ak, bg, dr);
+                dr = E::mfma32(av, bh, dr);
+            }
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const u32x2 w = *(const u32x2*)(lds + L::oR + col * 128 + (((4 * tl + g) ^ br_swz<8>(m)) << 4) + 8 * hf);
+                const float r4[4] = {E::to_float((uint16_t)(w.x & 0xffffu)), E::to_float((uint16_t)(w.x >> 16)),
+                                     E::to_float((uint16_t)(w.y & 0xffffu)), E::to_float((uint16_t)(w.y >> 16))};
+                const int left = b2 - (32 * tl + 8 * g + 4 * hf);        // rows l of this piece that exist
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int v = 4 * g + e;
+                    const float r = e < left ? r4[e] : 0.f;
+                    const float gv = r > 0.f ? dr[v] + dcv * __logf(r) : 0.f;        // dR + dc ln R
+                    rv[v] = r;
+                    dr[v] = gv;
+                    dot += r * gv;
+                }
+            }
+            dot = xhalf_sum(dot);
+            if (hf == 0) *(float*)(lds + L::oDot + (tl * kCols + col) * 4) = dot;
+            __syncthreads();                                             // the dKbar, dY and R tiles are free, the sums complete
+            queries(c0, nrows);
+            // dS1 over the R tile, laid out like it (columns past the end and l >= b2 come out as zeros)
+            dot = *(const float*)(lds + L::oDot + col * 4) + *(const float*)(lds + L::oDot + (kCols + col) * 4);
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                u32x2 w;
+                w.x = pack2<E>(rv[4 * g + 0] * (dr[4 * g + 0] - dot), rv[4 * g + 1] * (dr[4 * g + 1] - dot));
+                w.y = pack2<E>(rv[4 * g + 2] * (dr[4 * g + 2] - dot), rv[4 * g + 3] * (dr[4 * g + 3] - dot));
+                *(u32x2*)(lds + L::oR + col * 128 + (((4 * tl + g) ^ br_swz<8>(m)) << 4) + 8 * hf) = w;
+            }
+            complete(c0, nrows);
+            __syncthreads();                                             // every wave is done with this chunk
+        }
+        return;
+    }
+
+    // ---- gradient waves: 32 head-dim rows (block dt) x LBW blocks of 32 key rows of dV and of dK, C^T[d, l] = sum_aj A^T[d, aj] B[aj, l]
+    const int dt = wave % DT, lb0 = DT == 4 ? 0 : (wave >> 1) & 1;
+    uint32_t atr[2], btr[LBW][2];
+    {
+        const int s16 = lane & 15, g16 = lane >> 4;
+        const int rl = 4 * hf + (s16 >> 2);
+        const int cl = 2 * (g16 & 1) + ((s16 & 3) >> 1);
+        const uint32_t sub = (uint32_t)(s16 & 1) * 8;
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            const int r = rl + 8 * half;                                 // swz depends on r mod 16 only
+            atr[half] = (uint32_t)(r * kPitch + (((4 * dt + cl) ^ br_swz<CPR>(r)) << 4)) + sub;
+#pragma unroll
+            for (int lb = 0; lb < LBW; ++lb)
+                btr[lb][half] = (uint32_t)(L::oR + r * 128 + (((4 * (lb0 + lb) + cl) ^ br_swz<8>(r)) << 4)) + sub;
+        }
+    }
+    auto read_a = [&](int tile, int ks) {
+        const u32x2 lo = br_read_tr(lds, atr[0] + tile + ks * 16 * kPitch), hi = br_read_tr(lds, atr[1] + tile + ks * 16 * kPitch);
+        return u32x4{lo.x, lo.y, hi.x, hi.y};
+    };
+    auto read_b = [&](int lb, int ks) {
+        const u32x2 lo = br_read_tr(lds, btr[lb][0] + ks * 16 * 128), hi = br_read_tr(lds, btr[lb][1] + ks * 16 * 128);
+        return u32x4{lo.x, lo.y, hi.x, hi.y};
+    };
+    f32x16 dva[LBW], dka[LBW];
+#pragma unroll
+    for (int lb = 0; lb < LBW; ++lb)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) dva[lb][v] = dka[lb][v] = 0.f;
+    for (int c0 = cfirst; c0 < AJ; c0 += kCols) {
+        const int nrows = min(kCols, AJ - c0);
+        begin(c0, nrows);
+        loaded(nrows);
+        if (want) {
+            // dV += R^T dY, dK += R^T dKbar
+#pragma unroll
+            for (int ks = 0; ks < kCols / 16; ++ks) {
+                const u32x4 ah = read_a(L::oH, ks), ag = read_a(L::oG, ks);
+#pragma unroll
+                for (int lb = 0; lb < LBW; ++lb) {
+                    const u32x4 b = read_b(lb, ks);
+                    dva[lb] = E::mfma32(ah, b, dva[lb]);
+                    dka[lb] = E::mfma32(ag, b, dka[lb]);
+                }
+            }
+        }
+        __syncthreads();                                                 // the dKbar, dY and R tiles are free, the sums complete
+        queries(c0, nrows);
+        complete(c0, nrows);
+        if (want) {
+            // dK += s dS1^T q
+#pragma unroll
+            for (int lb = 0; lb < LBW; ++lb) {
+                f32x16 x;
+#pragma unroll
+                for (int v = 0; v < 16; ++v) x[v] = 0.f;
+#pragma unroll
+                for (int ks = 0; ks < kCols / 16; ++ks) x = E::mfma32(read_a(L::oH, ks), read_b(lb, ks), x);
+#pragma unroll
+                for (int v = 0; v < 16; ++v) dka[lb][v] = fmaf(p.scale, x[v], dka[lb][v]);
+            }
+        }
+        __syncthreads();                                                 // every wave is done with this chunk
+    }
+    if (!want) return;
     // lane (l, hf) holds head-dim 32 dt + 8 g + 4 hf + 0..3 of key row l; the half swap leaves 8 consecutive ones per lane
     const int64_t obase = (int64_t)(unit / p.H) * p.s0 + (int64_t)(unit % p.H) * p.s2 + (p.kmap.row(f, k) - p.row0) * p.s1;
-    auto store = [&](uint16_t* dst, const f32x16& acc) {
+    auto store = [&](uint16_t* dst, const f32x16& acc, int lb) {
         const int l = 32 * lb + m;
         uint16_t* row = dst + obase + min(l, b2 - 1) * p.s1 + 32 * dt + 8 * hf;
 #pragma unroll
@@ -157,154 +305,10 @@ __global__ __launch_bounds__(kThreads) void monarch_bwd_right_kernel(RightArgs p
             if (l < b2) *(u32x4*)(row + 16 * gp) = w;
         }
     };
-
-    const bool active = wave < 10;                                       // phase 1: waves 0..9 = (32 columns, 32 rows l) blocks of dS1
-    const int cblk = wave % 5, tl = (wave / 5) & 1;
-    const int col = 32 * cblk + m;                                       // column within the pass, < 160
-    const char* qbase = p.q + ((int64_t)(unit / p.H) * p.qs0 + (int64_t)(unit % p.H) * p.qs2) * 2;
-    const uint32_t qrb = (uint32_t)(p.qs1 * 2);
-    f32x16 acc, accq;                                                    // dV^T, or R^T dKbar and dS1^T q of dK^T
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[v] = accq[v] = 0.f;
-
-    // the tile's columns (a, j), up to 160 per pass, from the first that sees key block-frame f on
-    const int cfirst = p.causal ? f / p.causal * p.causal * b2 : 0;
-    auto pass = [&](auto pi_c) {
-    constexpr int pi = decltype(pi_c)::value;
-    const int c0 = cfirst + pi * kMaxAJ;
-    const int nrows = MULTI ? min(kMaxAJ, AJ - c0) : AJ - c0;
-    if (MULTI && nrows <= 0) return;                                     // uniform
-    stage(p.dkbar + (t * AJ + c0) * kPitch, kPitch, nrows * CPR, oG, c_d{});
-    stage(p.dy + (t * AJ + c0) * kPitch, kPitch, nrows * CPR, oH, c_d{});
-    stage(p.rb + (t * AJ + c0) * 128, 128, nrows * 8, oR, c_r{});
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (nrows < kMaxAJ || pi == 0) {                                     // rows past the end are zero: they add nothing to any contraction
-        const u32x4 z = {0u, 0u, 0u, 0u};
-        if (pi == 0)                                                     // K, V rows past b2: what the logits pick up there is masked, but must be finite
-            for (int i = tid; i < (64 - b2) * CPR; i += kThreads) {
-                *(u32x4*)(lds + oK + b2 * kPitch + i * 16) = z;
-                *(u32x4*)(lds + oV + b2 * kPitch + i * 16) = z;
-            }
-        for (int i = tid; i < (kMaxAJ - nrows) * CPR; i += kThreads) {
-            *(u32x4*)(lds + oG + nrows * kPitch + i * 16) = z;
-            *(u32x4*)(lds + oH + nrows * kPitch + i * 16) = z;
-        }
-        for (int i = tid; i < (kMaxAJ - nrows) * 8; i += kThreads) *(u32x4*)(lds + oR + nrows * 128 + i * 16) = z;
-        __syncthreads();
-    }
-
-    // ---- phase 1, products: dR^T
-    f32x16 dr;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) dr[v] = 0.f;
-    if (active) {
-        const uint32_t a_off = (uint32_t)(32 * tl + m) * kPitch + (uint32_t)((hf ^ br_swz<CPR>(m)) << 4);   // swz depends on r mod 16
-        const uint32_t b_off = (uint32_t)col * kPitch + (uint32_t)((hf ^ br_swz<CPR>(col)) << 4);
-#pragma unroll
-        for (int ds = 0; ds < DS; ++ds) {
-            const u32x4 bg = *(const u32x4*)(lds + oG + (b_off ^ (uint32_t)(ds << 5)));
-            const u32x4 bh = *(const u32x4*)(lds + oH + (b_off ^ (uint32_t)(ds << 5)));
-            const u32x4 ak = *(const u32x4*)(lds + oK + (a_off ^ (uint32_t)(ds << 5)));
-            const u32x4 av = *(const u32x4*)(lds + oV + (a_off ^ (uint32_t)(ds << 5)));
-            dr = E::mfma32(ak, bg, dr);
-            dr = E::mfma32(av, bh, dr);
-        }
-    }
-    // ---- phase 2, the products that only need the loaded tiles: dV += R^T dY, dK += R^T dKbar
-    if (want) {
-        if (which == 0) {
-            product(oH, oR, acc);
-        } else if (which == 1) {
-            product(oG, oR, acc);
-        }
-    }
-    __syncthreads();                                                     // K, V, dKbar, dY tiles are free
-    // the query rows of (unit, k) take the place of the dY tile while the softmax backward runs
-    if (want) {
-        const int nchunks = nrows * CPR;
-        for (int g = wave; g * 64 < nchunks; g += kWaves) {
-            const int P = min(g * 64 + lane, nchunks - 1);
-            const int r = P / CPR, c = (P % CPR) ^ br_swz<CPR>(r);
-            const int aj = c0 + r;
-            const uint32_t tok = (uint32_t)(p.qmap.row(aj / b2, k) + aj % b2);
-            br_load_lds16(qbase, tok * qrb + (uint32_t)(c * 16), lds0 + oH + (uint32_t)g * 1024);
-        }
-    }
-
-    // ---- phase 1, softmax backward.  R[col][l] for the l this lane holds: l = 32 tl + 8 g + 4 hf + 0..3, 8 bytes of chunk 4 tl + g
-    float rv[16];
-    float dot = 0.f;
-    if (active) {
-        const float dcv = c0 + col < AJ ? p.dc[(u * AJ + c0 + col) * ((int64_t)nf * p.b1) + (int64_t)k * nf + f] : 0.f;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const int c = 4 * tl + g;
-            const u32x2 w = *(const u32x2*)(lds + oR + col * 128 + ((c ^ br_swz<8>(col)) << 4) + 8 * hf);
-            const float r0 = E::to_float((uint16_t)(w.x & 0xffffu)), r1 = E::to_float((uint16_t)(w.x >> 16));
-            const float r2 = E::to_float((uint16_t)(w.y & 0xffffu)), r3 = E::to_float((uint16_t)(w.y >> 16));
-            const int left = b2 - (32 * tl + 8 * g + 4 * hf);            // rows l of this piece that exist
-            const float rr[4] = {left > 0 ? r0 : 0.f, left > 1 ? r1 : 0.f, left > 2 ? r2 : 0.f, left > 3 ? r3 : 0.f};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int v = 4 * g + e;
-                float gv = dr[v];
-                if (rr[e] > 0.f) gv += dcv * __logf(rr[e]);              // dR + dc ln R
-                else gv = 0.f;
-                rv[v] = rr[e];
-                dr[v] = gv;
-                dot += rr[e] * gv;
-            }
-        }
-        dot = xhalf_sum(dot);
-        if (hf == 0) *(float*)(lds + oDot + (tl * kMaxAJ + col) * 4) = dot;
-    }
-    lds_barrier();                                                       // (the query rows stay in flight)
-    if (active) {
-        dot = *(const float*)(lds + oDot + col * 4) + *(const float*)(lds + oDot + (kMaxAJ + col) * 4);
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            u32x2 w;
-            w.x = pack2<E>(rv[4 * g + 0] * (dr[4 * g + 0] - dot), rv[4 * g + 1] * (dr[4 * g + 1] - dot));
-            w.y = pack2<E>(rv[4 * g + 2] * (dr[4 * g + 2] - dot), rv[4 * g + 3] * (dr[4 * g + 3] - dot));
-            // into the dS1 tile, laid out like R's (columns past the end and l >= b2 come out as zeros)
-            *(u32x2*)(lds + oS + col * 128 + (((4 * tl + g) ^ br_swz<8>(col)) << 4) + 8 * hf) = w;
-        }
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                     // the query rows have landed
-    __syncthreads();                                                     // the dS1 tile is complete
-    // dS1 to memory for dQ = s dS1 K: row aj is b2p consecutive elements, 8-byte pieces, consecutive lanes along a row
-    {
-        const int ppr = (b2 + 3) / 4, b2p = 4 * ppr;                     // pieces per row
-        uint16_t* out = p.ds1 + (uk * AJ + c0) * ((int64_t)nf * b2p) + (int64_t)f * b2p;
-        for (int i = tid; i < nrows * ppr; i += kThreads) {
-            const int row = i / ppr, pc = i % ppr;
-            const u32x2 w = *(const u32x2*)(lds + oS + row * 128 + (((pc >> 1) ^ br_swz<8>(row)) << 4) + 8 * (pc & 1));
-            *(u32x2*)(out + (int64_t)row * nf * b2p + 4 * pc) = w;
-        }
-    }
-    if (want) {
-        if ((nrows * CPR) % 64) {                                        // the last load spilled copies of a chunk into the zero rows
-            const u32x4 z = {0u, 0u, 0u, 0u};
-            for (int i = tid; i < (kMaxAJ - nrows) * CPR; i += kThreads) *(u32x4*)(lds + oH + nrows * kPitch + i * 16) = z;
-            __syncthreads();
-        }
-        // ---- phase 2, the product that needs dS1: dS1^T q
-        if (which == 1) product(oH, oS, accq);
-    }
-    if (pi + 1 < NP) __syncthreads();                                    // every wave is done with this pass's rows
-    };
-    pass(std::integral_constant<int, 0>{});
-    if constexpr (NP > 1) pass(std::integral_constant<int, 1>{});
-    if constexpr (NP > 2) pass(std::integral_constant<int, 2>{});
-    if (!want) return;
-    // dK = R^T dKbar + s dS1^T q
-    if (which == 1) {
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[v] += p.scale * accq[v];
-        store(p.dk, acc);
-    } else if (which == 0) {
-        store(p.dv, acc);
+    for (int lb = 0; lb < LBW; ++lb) {
+        store(p.dv, dva[lb], lb0 + lb);
+        store(p.dk, dka[lb], lb0 + lb);
     }
 }
 
@@ -460,7 +464,7 @@ __global__ __launch_bounds__(1024) void monarch_bwd_dqk_kernel(DqkArgs p) {
 
 bool monarch_bwd_right_supported(int dtype, int D, int b2, int AJ) {
     // up to three passes of 160 columns over a tile
-    return (dtype == SFM_BF16 || dtype == SFM_F16) && (D == 64 || D == 128) && b2 >= 1 && b2 <= 64 && AJ <= 3 * kMaxAJ;
+    return (dtype == SFM_BF16 || dtype == SFM_F16) && (D == 64 || D == 128) && b2 >= 1 && b2 <= 64 && AJ <= 480;
 }
 
 int launch_monarch_bwd_right(int dtype, int D, int64_t ntiles, int b1, int b2, int AJ, int nf, float scale, const void* kk,
@@ -488,15 +492,11 @@ int launch_monarch_bwd_right(int dtype, int D, int64_t ntiles, int b1, int b2, i
     a.b1 = b1; a.b2 = b2; a.AJ = AJ; a.nf = nf; a.H = H; a.unit0 = unit0; a.f0 = f0; a.f1 = f1;
     a.causal = skip_causal;
     a.scale = scale;
-    const size_t kv = (size_t)2 * 64 * 2 * D, rt = (size_t)kMaxAJ * 128;
-    const size_t ldsb = kv + (size_t)2 * kMaxAJ * 2 * D + rt + (rt <= kv && AJ <= kMaxAJ ? 0 : rt) + 2 * kMaxAJ * 4;
-    const int np = (AJ + kMaxAJ - 1) / kMaxAJ;                         // 1, 2 or 3 (monarch_bwd_right_supported)
+    a.ntiles = ntiles;
+    const size_t ldsb = D == 128 ? RightLds<128>::kBytes : RightLds<64>::kBytes;
     const void* fn = nullptr;
-#define SFM_RIGHT_FN(E, D) \
-    (np == 1 ? (const void*)monarch_bwd_right_kernel<E, D, 1> : np == 2 ? (const void*)monarch_bwd_right_kernel<E, D, 2> : (const void*)monarch_bwd_right_kernel<E, D, 3>)
-    if (dtype == SFM_BF16) fn = D == 128 ? SFM_RIGHT_FN(BF16, 128) : SFM_RIGHT_FN(BF16, 64);
-    else fn = D == 128 ? SFM_RIGHT_FN(F16, 128) : SFM_RIGHT_FN(F16, 64);
-#undef SFM_RIGHT_FN
+    if (dtype == SFM_BF16) fn = D == 128 ? (const void*)monarch_bwd_right_kernel<BF16, 128> : (const void*)monarch_bwd_right_kernel<BF16, 64>;
+    else fn = D == 128 ? (const void*)monarch_bwd_right_kernel<F16, 128> : (const void*)monarch_bwd_right_kernel<F16, 64>;
     if (ldsb > 48 * 1024) {
         hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsb);
         if (e != hipSuccess) {
@@ -504,7 +504,7 @@ int launch_monarch_bwd_right(int dtype, int D, int64_t ntiles, int b1, int b2, i
             return SFM_ERR_HIP;
         }
     }
-    const dim3 grid((unsigned)ntiles);
+    const dim3 grid((unsigned)((ntiles + 7) / 8 * 8));
     void* kargs[] = {(void*)&a};
     hipError_t le = hipLaunchKernel(fn, grid, dim3(kThreads), kargs, ldsb, stream);
     if (le != hipSuccess) {
