@@ -637,7 +637,7 @@ int run(const MonarchBwdArgs& g, int n, void* workspace, hipStream_t stream) {
     if (fused_right) {
         if (!cx.status)
             cx.status = launch_monarch_bwd_right(left_dtype<E>(), D, nt, b1, b2, AJ, nf, s, p.k, p.ks, p.v, p.vs, ws + lay.Rb,
-                                                 ws + lay.dKbar, ws + lay.dY, (const float*)(ws + lay.dc), p.q, p.qs, p.qmap, ws + lay.dS1, g.dk,
+                                                 ws + lay.dKbar, ws + lay.dY, (const float*)(ws + lay.dc), p.q, p.qs, p.qmap, ws + lay.dS1, parts.dqk, g.dk,
                                                  g.dv, g.dks, g.dk_row0, p.kmap, H, p.unit0, g.kv_f0, g.kv_f1, skip ? p.causal : 0, stream);
     } else {
         // 9. dR block = dKbar block . K block^T + dY block . V block^T per t

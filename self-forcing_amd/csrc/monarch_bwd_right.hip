@@ -45,7 +45,8 @@ struct RightArgs {
     const char* q;           // caller's tensor: row (a, j) of (unit, k) is token qmap.row(a, k) + j, strides qs0, qs1, qs2
     int64_t qs0, qs1, qs2;
     TokMap qmap;
-    uint16_t* ds1;           // [(u, k)][AJ][nf * b2p], b2p = b2 rounded up to 4; the padding is zero
+    uint16_t* ds1;           // row (a, j) of tile t at u k AJ nf b2p + f ds1_f + aj ds1_aj, b2p = b2 rounded up to 4; the padding is zero
+    int64_t ds1_f, ds1_aj;
     uint16_t* dk;            // caller's tensors: row kmap.row(f, k) + l - row0, strides s0 (batch), s1 (row), s2 (head)
     uint16_t* dv;
     int64_t s0, s1, s2, row0;
@@ -157,11 +158,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                 // the query rows have landed
         __syncthreads();                                                 // the dS1 tile is complete
         // dS1 to memory for dQ = s dS1 K: row aj is b2p consecutive elements, 8-byte pieces, consecutive lanes along a row
-        uint16_t* out = p.ds1 + (uk * AJ + c0) * ((int64_t)nf * b2p) + (int64_t)f * b2p;
+        uint16_t* out = p.ds1 + uk * AJ * ((int64_t)nf * b2p) + f * p.ds1_f + c0 * p.ds1_aj;
         for (int i = tid; i < nrows * ppr; i += kThreads) {
             const int row = i / ppr, pc = i - row * ppr;
             const u32x2 w = *(const u32x2*)(lds + L::oR + row * 128 + (((pc >> 1) ^ br_swz<8>(row)) << 4) + 8 * (pc & 1));
-            *(u32x2*)(out + (int64_t)row * nf * b2p + 4 * pc) = w;
+            *(u32x2*)(out + row * p.ds1_aj + 4 * pc) = w;
         }
     };
 
@@ -324,7 +325,8 @@ struct DqkArgs {
     const char* k;           // caller's tensor: row kmap.row(f, k) + l, strides ks0 (batch), ks1 (row), ks2 (head), in elements
     int64_t ks0, ks1, ks2;
     TokMap kmap;
-    const uint16_t* ds1;     // [(u, k)][AJ][nf * b2p] as the kernel above writes it
+    const uint16_t* ds1;     // [(u, k)][f][AJ][b2p] as the kernel above writes it
+    uint32_t b2p_inv;        // 2^32 / b2p, rounded up: x / b2p is the upper half of the product for every x below 2^26
     float* dqk;              // [(u, k)][AJ][D], or the caller's rows to add to: token qmap.row(a, k) + j, strides dqs
     int64_t dqs0, dqs1, dqs2;
     TokMap qmap;
@@ -367,7 +369,9 @@ __global__ __launch_bounds__(1024) void monarch_bwd_dqk_kernel(DqkArgs p) {
     };
     // dS1 pieces of row aj = 32 wave + m: x = 64 t + 16 ks + 4 hf + {0..3} and + 8 + {0..3}
     const int aj = min(32 * wave + m, AJ - 1);
-    const uint16_t* arow = p.ds1 + (uk * AJ + aj) * (int64_t)NL + 4 * hf;
+    const uint16_t* arow = p.ds1 + uk * AJ * (int64_t)NL + aj * b2p;
+    const uint32_t fstep = (uint32_t)((AJ - 1) * b2p);                  // from a row's end in one block-frame to its start in the next
+    auto piece = [&](int x) { return *(const u32x2*)(arow + (uint32_t)x + __umulhi((uint32_t)x, p.b2p_inv) * fstep); };
     const int na = visible(aj);
     const int nwave = __builtin_amdgcn_readfirstlane(visible(min(32 * wave + 31, AJ - 1)));      // of the wave's longest row
     auto load_a = [&](int t, u32x4 (&a)[4]) {
@@ -375,8 +379,8 @@ __global__ __launch_bounds__(1024) void monarch_bwd_dqk_kernel(DqkArgs p) {
         for (int ks = 0; ks < 4; ++ks) {
             const int x0 = 64 * t + 16 * ks + 4 * hf;
             u32x2 lo = {0u, 0u}, hi = {0u, 0u};
-            if (x0 + 4 <= na) lo = *(const u32x2*)(arow + 64 * t + 16 * ks);           // a multiple of 4: whole pieces
-            if (x0 + 12 <= na) hi = *(const u32x2*)(arow + 64 * t + 16 * ks + 8);
+            if (x0 + 4 <= na) lo = piece(x0);                            // a multiple of 4: whole pieces
+            if (x0 + 12 <= na) hi = piece(x0 + 8);
             a[ks] = u32x4{lo.x, lo.y, hi.x, hi.y};
         }
     };
@@ -469,7 +473,7 @@ bool monarch_bwd_right_supported(int dtype, int D, int b2, int AJ) {
 
 int launch_monarch_bwd_right(int dtype, int D, int64_t ntiles, int b1, int b2, int AJ, int nf, float scale, const void* kk,
                              const int64_t* ks, const void* v, const int64_t* vs, const void* rb, const void* dkbar, const void* dy, const float* dc, const void* q,
-                             const int64_t* qs, const TokMap& qmap, void* ds1, void* dk, void* dv, const int64_t* dks, int64_t row0,
+                             const int64_t* qs, const TokMap& qmap, void* ds1, bool ds1_tiles, void* dk, void* dv, const int64_t* dks, int64_t row0,
                              const TokMap& kmap, int H, int unit0, int f0, int f1, int skip_causal, hipStream_t stream) {
     if ((dks[0] | dks[1] | dks[2] | vs[0] | vs[1] | vs[2] | ks[0] | ks[1] | ks[2]) % 8 ||
         ((uintptr_t)dk | (uintptr_t)dv | (uintptr_t)v | (uintptr_t)kk) % 16 || (int64_t)(b2 - 1) * vs[1] * 2 + 2 * D > 0xffffffffll ||
@@ -486,6 +490,9 @@ int launch_monarch_bwd_right(int dtype, int D, int64_t ntiles, int b1, int b2, i
     a.q = (const char*)q; a.qs0 = qs[0]; a.qs1 = qs[1]; a.qs2 = qs[2];
     a.qmap = qmap;
     a.ds1 = (uint16_t*)ds1;
+    const int b2p = (b2 + 3) / 4 * 4;
+    a.ds1_f = ds1_tiles ? (int64_t)AJ * b2p : b2p;
+    a.ds1_aj = ds1_tiles ? b2p : (int64_t)nf * b2p;
     a.dk = (uint16_t*)dk; a.dv = (uint16_t*)dv;
     a.s0 = dks[0]; a.s1 = dks[1]; a.s2 = dks[2]; a.row0 = row0;
     a.kmap = kmap;
@@ -535,6 +542,7 @@ int launch_monarch_bwd_dqk(int dtype, int D, int64_t nuk, int b1, int b2, int AJ
     a.k = (const char*)k; a.ks0 = ks[0]; a.ks1 = ks[1]; a.ks2 = ks[2];
     a.kmap = kmap;
     a.ds1 = (const uint16_t*)ds1;
+    a.b2p_inv = (uint32_t)((((uint64_t)1 << 32) + (b2 + 3) / 4 * 4 - 1) / (uint64_t)((b2 + 3) / 4 * 4));
     a.dqk = dqk;
     a.add = dqs != nullptr;
     a.causal = skip_causal;

@@ -241,11 +241,12 @@ int launch_monarch_bwd_left(int dtype, int D, int n, int b1, int b2, int AJ, int
                             void* ds2, int ds2_ld, float* dq, const int64_t* dqs, const float* stats, int stats_ld, bool skip_masked,
                             hipStream_t stream);
 // fused right-factor part of the backward (monarch_bwd_right.hip): per tile t = (unit, k, f) the dS1 block (scratch, for
-// dQ = s dS1 K) and the finished dK / dV rows of kv block-frames [f0, f1) in the caller's tensors; q, k and v are the caller's tensors too
+// dQ = s dS1 K; rows [f][(a, j)] per (unit, k) with ds1_tiles, as launch_monarch_bwd_dqk reads them, else [(a, j)][f]) and the
+// finished dK / dV rows of kv block-frames [f0, f1) in the caller's tensors; q, k and v are the caller's tensors too
 bool monarch_bwd_right_supported(int dtype, int D, int b2, int AJ);
 int launch_monarch_bwd_right(int dtype, int D, int64_t ntiles, int b1, int b2, int AJ, int nf, float scale, const void* kk,
                              const int64_t* ks, const void* v, const int64_t* vs, const void* rb, const void* dkbar, const void* dy, const float* dc, const void* q,
-                             const int64_t* qs, const TokMap& qmap, void* ds1, void* dk, void* dv, const int64_t* dks, int64_t row0,
+                             const int64_t* qs, const TokMap& qmap, void* ds1, bool ds1_tiles, void* dk, void* dv, const int64_t* dks, int64_t row0,
                              const TokMap& kmap, int H, int unit0, int f0, int f1, int skip_causal, hipStream_t stream);
 
 // With `skip_masked` / `skip_causal` (the block-causal size) the three parts neither read nor write the scratch rows of masked
