@@ -1,28 +1,26 @@
-// Right-factor part of the Monarch backward on gfx950 MFMA (bf16 / fp16, head_dim 64 or 128, b2 <= 64;
-// at most 480 (a, j) columns, taken 160 at a time).
+// Right-factor part of the Monarch backward on gfx950 MFMA (bf16 / fp16, head_dim 64 or 128, b2 <= 64, at most 480 (a, j)
+// columns).
 //
 // Replaces, per tile t = (unit, k, f), the small batched products and the row kernel of the GEMM chain
 //     dR[aj, l]  = dKbar[aj,:] . K[l,:] + dY[aj,:] . V[l,:]
 //     dS1[aj, l] = R (dR + dc ln R - sum_l R (dR + dc ln R))
 //     dK[l, :]   = sum_aj R[aj, l] dKbar[aj,:] + s sum_aj dS1[aj, l] q[aj,:]
 //     dV[l, :]   = sum_aj R[aj, l] dY[aj,:]
-// (wan/modules/monarch_attn.py:403-596 `_al_cl_y_bwd`).  One workgroup per tile: the K and V blocks (52 rows each, read
-// where the callers' tensors have them), and the tile's rows of R, dKbar and dY (contiguous in the backward's scratch)
-// go straight into LDS (global_load_lds_dwordx4, 16-byte chunks XOR-swizzled per row as in the dense attention
-// kernel); rows past the end are zeroed.  A tile with more than 160 columns is taken in passes of 160, the K and V
-// blocks and the accumulators of dK and dV staying where they are.
-// Sixteen waves per workgroup (one workgroup fills the LDS of a compute unit, so the waves have to come from it).
-//   phase 1: wave = 32 columns aj x 32 key rows l (ten waves busy).  dR^T[l, aj] with A = K / V rows, B = dKbar / dY
-//            rows, so that a lane owns one column and the softmax backward is in-lane plus one cross-half add and one
-//            exchange between the two waves of a column through LDS.
-//   phase 2: wave = 32 head-dim rows x 32 key rows of dV or of dK.  C^T[d, l] with both operands from transposing LDS
-//            reads (ds_read_tr16_b64): A = dY^T / dKbar^T / q^T, B = R or dS1 (kept in LDS, 16 bit; with a single pass
-//            over the K / V tiles once phase 1 is done with them), contraction over the columns aj.  The products
-//            with R run right after the logits of phase 1; the query rows of (unit, k) then load over the dY tile
-//            while the softmax backward runs.  dK and dV leave in the tensor dtype, straight to the caller's rows;
-//            tiles whose kv block-frame is outside the wanted range skip phase 2.
+// (wan/modules/monarch_attn.py:403-596 `_al_cl_y_bwd`).  One workgroup per tile: the K and V blocks (read where the callers'
+// tensors have them) stay in LDS, the tile's rows of R, dKbar and dY (contiguous in the backward's scratch) come 64
+// columns at a time (global_load_lds_dwordx4, 16-byte chunks XOR-swizzled per row as in the dense attention kernel).
+//   softmax waves (4): 32 columns aj x 32 key rows l.  dR^T[l, aj] with A = K / V rows, B = dKbar / dY rows, so that a lane
+//            owns one column and the softmax backward is in-lane plus one cross-half add and one exchange between the
+//            two waves of a column through LDS.  dS1 (16 bit) takes the place of R.
+//   gradient waves (4): 32 head-dim rows x 64 (head_dim 64: 32) key rows of dV and of dK, C^T[d, l] with both operands from
+//            transposing LDS reads (ds_read_tr16_b64): A = dY^T / dKbar^T / q^T, B = R or dS1, contraction over the columns
+//            aj.  The products with R run beside the softmax waves; the query rows of (unit, k) then load over the dY tile.
 // dS1 is also written to memory (16 bit) for dQ = s dS1 K, which contracts over f across tiles (monarch_bwd_dqk_kernel
 // below).
+//
+// Bound by HBM and its latency: dKbar, dY, R read and dS1 written once, 0.87 GB at 12 heads x 128, a = 3, f = 21, b1 = 30,
+// b2 = 52: 262 us.  64 columns because two workgroups then share a compute unit and one's loads run beside the other's
+// products: sixteen waves with 160 columns, which filled the LDS alone, took 336 us there, and as long for 52 columns as for 160.
 
 #include <hip/hip_runtime.h>
 
@@ -129,18 +127,29 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
     const int cfirst = p.causal ? f / p.causal * p.causal * b2 : 0;      // the first column (a, j) that sees key block-frame f
 
     // What every wave does in a chunk; the two kinds of waves meet in the same four barriers.
-    auto begin = [&](int c0, int nrows) {
-        stage(p.dkbar + (t * AJ + c0) * kPitch, kPitch, nrows, L::oG, c_d{});
-        stage(p.dy + (t * AJ + c0) * kPitch, kPitch, nrows, L::oH, c_d{});
-        stage(p.rb + (t * AJ + c0) * 128, 128, nrows, L::oR, c_r{});
+    auto load_g = [&](int c0) { stage(p.dkbar + (t * AJ + c0) * kPitch, kPitch, min(kCols, AJ - c0), L::oG, c_d{}); };
+    auto load_h = [&](int c0) { stage(p.dy + (t * AJ + c0) * kPitch, kPitch, min(kCols, AJ - c0), L::oH, c_d{}); };
+    auto load_r = [&](int c0) { stage(p.rb + (t * AJ + c0) * 128, 128, min(kCols, AJ - c0), L::oR, c_r{}); };
+    // the next chunk's rows are requested as soon as their tiles are free: dKbar (and dY, where no query rows take its place)
+    // behind the products, the others at the chunk's end
+    auto next_early = [&](int c1) {
+        if (c1 >= AJ) return;
+        load_g(c1);
+        if (!want) load_h(c1);
+    };
+    auto next_late = [&](int c1) {
+        lds_barrier();                                                   // every wave is done with this chunk
+        if (c1 >= AJ) return;
+        if (want) load_h(c1);
+        load_r(c1);
     };
     auto loaded = [&](int nrows) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
+        lds_barrier();  
         if (nrows < kCols) {                                             // columns past the end have no weight
             const u32x4 z = {0u, 0u, 0u, 0u};
             for (int i = tid; i < (kCols - nrows) * 8; i += kThreads) *(u32x4*)(lds + L::oR + nrows * 128 + i * 16) = z;
-            __syncthreads();
+            lds_barrier();  
         }
     };
     auto queries = [&](int c0, int nrows) {                              // the query rows of (unit, k) take the place of the dY tile
@@ -155,8 +164,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
         }
     };
     auto complete = [&](int c0, int nrows) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                 // the query rows have landed
-        __syncthreads();                                                 // the dS1 tile is complete
+        if (want) {                                                      // the query rows have landed (behind them the next dKbar rows)
+            if (c0 + kCols < AJ) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(CPR / kWaves) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
+        lds_barrier();                                                   // the dS1 tile is complete
         // dS1 to memory for dQ = s dS1 K: row aj is b2p consecutive elements, 8-byte pieces, consecutive lanes along a row
         uint16_t* out = p.ds1 + uk * AJ * ((int64_t)nf * b2p) + f * p.ds1_f + c0 * p.ds1_aj;
         for (int i = tid; i < nrows * ppr; i += kThreads) {
@@ -166,6 +178,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
         }
     };
 
+    load_g(cfirst);
+    load_h(cfirst);
+    load_r(cfirst);
     if (wave < 4) {
         // ---- softmax waves: 32 columns x 32 key rows
         const int tl = wave >> 1, col = 32 * (wave & 1) + m;
@@ -173,7 +188,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
         const uint32_t b_off = (uint32_t)col * kPitch + (uint32_t)((hf ^ br_swz<CPR>(m)) << 4);
         for (int c0 = cfirst; c0 < AJ; c0 += kCols) {
             const int nrows = min(kCols, AJ - c0);
-            begin(c0, nrows);
             const float dcv = col < nrows ? p.dc[(u * AJ + c0 + col) * ((int64_t)nf * p.b1) + (int64_t)k * nf + f] : 0.f;
             loaded(nrows);
             // dR^T[l, aj] = K dKbar^T + V dY^T, then R (16 bit) of the l this lane holds: l = 32 tl + 8 g + 4 hf + 0..3
@@ -209,8 +223,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
             }
             dot = xhalf_sum(dot);
             if (hf == 0) *(float*)(lds + L::oDot + (tl * kCols + col) * 4) = dot;
-            __syncthreads();                                             // the dKbar, dY and R tiles are free, the sums complete
+            lds_barrier();                                               // the dKbar, dY and R tiles are free, the sums complete
             queries(c0, nrows);
+            next_early(c0 + kCols);
             // dS1 over the R tile, laid out like it (columns past the end and l >= b2 come out as zeros)
             dot = *(const float*)(lds + L::oDot + col * 4) + *(const float*)(lds + L::oDot + (kCols + col) * 4);
 #pragma unroll
@@ -221,7 +236,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
                 *(u32x2*)(lds + L::oR + col * 128 + (((4 * tl + g) ^ br_swz<8>(m)) << 4) + 8 * hf) = w;
             }
             complete(c0, nrows);
-            __syncthreads();                                             // every wave is done with this chunk
+            next_late(c0 + kCols);
         }
         return;
     }
@@ -258,7 +273,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
         for (int v = 0; v < 16; ++v) dva[lb][v] = dka[lb][v] = 0.f;
     for (int c0 = cfirst; c0 < AJ; c0 += kCols) {
         const int nrows = min(kCols, AJ - c0);
-        begin(c0, nrows);
         loaded(nrows);
         if (want) {
             // dV += R^T dY, dK += R^T dKbar
@@ -273,8 +287,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
                 }
             }
         }
-        __syncthreads();                                                 // the dKbar, dY and R tiles are free, the sums complete
+        lds_barrier();                                                   // the dKbar, dY and R tiles are free, the sums complete
         queries(c0, nrows);
+        next_early(c0 + kCols);
         complete(c0, nrows);
         if (want) {
             // dK += s dS1^T q
@@ -289,7 +304,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
                 for (int v = 0; v < 16; ++v) dka[lb][v] = fmaf(p.scale, x[v], dka[lb][v]);
             }
         }
-        __syncthreads();                                                 // every wave is done with this chunk
+        next_late(c0 + kCols);
     }
     if (!want) return;
     // lane (l, hf) holds head-dim 32 dt + 8 g + 4 hf + 0..3 of key row l; the half swap leaves 8 consecutive ones per lane
@@ -467,7 +482,6 @@ __global__ __launch_bounds__(1024) void monarch_bwd_dqk_kernel(DqkArgs p) {
 }  // namespace
 
 bool monarch_bwd_right_supported(int dtype, int D, int b2, int AJ) {
-    // up to three passes of 160 columns over a tile
     return (dtype == SFM_BF16 || dtype == SFM_F16) && (D == 64 || D == 128) && b2 >= 1 && b2 <= 64 && AJ <= 480;
 }
 
