@@ -311,7 +311,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 template <class E, int D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void dense_bwd_dkv_kernel(DenseBwdArgs p) {
     using T = Tile<D>;
-    constexpr int kBuf = 3;                                // tiles in LDS: the one in use and two on their way
+    constexpr int kBuf = 3;                                // tiles in LDS: one ends, one begins, one on its way
     constexpr int oStat = kBuf * 2 * T::kBytes;            // [buffer][lse 64 floats | delta 64 floats | 128 unused]
     extern __shared__ __attribute__((aligned(256))) char lds[];          // [buffer][q tile | dO tile], then the row values
     const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)lds;
@@ -378,102 +378,107 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     const bool split = item >= p.rkv.full && p.rkv.ranges > 1;        // uniform
     const int t0 = split ? __builtin_amdgcn_readfirstlane(range * alltiles / p.rkv.ranges) : 0;       // this workgroup's tiles: t0 .. nt - 1
     const int nt = split ? __builtin_amdgcn_readfirstlane((range + 1) * alltiles / p.rkv.ranges) : alltiles;
-    // one tile; RAGGED (only the last tile can be) masks the queries past the end
-    auto tile = [&](int t, auto ragged_c) {
-        constexpr bool ragged = decltype(ragged_c)::value;
-        // tile t has landed when at most the loads of tile t + 1 are outstanding
-        if (t + 1 < nt) {
-            if (T::CPR == 16) asm volatile("s_waitcnt vmcnt(9)" ::: "memory");
-            else asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
-        } else {
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // Halves of 32 queries follow each other in a pipeline.  Step H of it, H = 2 t + tl, is the gradient products of half H - 1 and the
+    // logits and dP of half H + 1, with the softmax backward of half H spread over all of their MFMAs: a wave alone on its SIMD
+    // issues nothing else while it waits, and with the softmax beside every second run of MFMAs only, the other runs
+    // left the vector unit idle and these the matrix pipe: 12 heads x 4680 queries x 14040 keys took 1061 us where this takes 925
+    // (873 TFLOP/s; the clock is down to 1.95 GHz).  Two waves per SIMD, each with half of the head dim's sums, that hand
+    // their P and dS to each other through LDS: 1020.
+    constexpr int NO = 4 * T::DT, NA = 2 * T::DS, NS = NO + NA;         // MFMAs of a half's gradients, of its logits, of a step
+    constexpr int kAhead = 4, kRing = 8;                    // A operands are read this many MFMAs ahead, over the end of a step too
+    constexpr int kLag = 3;                                 // the last MFMAs of a step are behind this many of the next one
+    static_assert(NS % kRing == 0, "");
+    f32x16 s[2], dp[2];
+    u32x4 pb[2][2], sb[2][2], ring[kRing];                  // packed P, dS of a half: two steps of 16 queries each
+    auto buffer = [&](int t) { return (const char*)lds + (t % kBuf) * 2 * T::kBytes; };
+    auto read_prod = [&](const char* tile, int tl, int j) { // j even: q rows for S, odd: dO rows for dP
+        return *(const u32x4*)(tile + (j & 1) * T::kBytes + tl * 32 * T::kPitch + (a_off ^ (uint32_t)((j >> 1) << 5)));
+    };
+    // gradient MFMA j of a half: queries 16 (j / (2 DT)) + 0..15, head-dim block dt = (j / 2) % DT, j even: dV (dO^T), odd: dK (q^T)
+    auto read_out = [&](const char* tile, int tl, int j) {
+        const int dt = (j >> 1) % T::DT;
+        return tile_tr<D>(tile + ((j & 1) ? 0 : T::kBytes), tr[dt][0], tr[dt][1], 2 * tl + j / (2 * T::DT));
+    };
+    auto prod = [&](int tl, int j, const u32x4& a) {
+        f32x16& c = (j & 1) ? dp[tl] : s[tl];
+        c = E::mfma32(a, (j & 1) ? vb[j >> 1] : kb[j >> 1], j < 2 ? f32x16{} : c);
+    };
+    auto grad = [&](int tl, int j, const u32x4& a) {
+        const int dt = (j >> 1) % T::DT, x = j / (2 * T::DT);
+        if (j & 1) dka[dt] = E::mfma32(a, sb[tl][x], dka[dt]);
+        else dva[dt] = E::mfma32(a, pb[tl][x], dva[dt]);
+    };
+    // row values of four queries, read a group of four ahead: LDS reads return in order, so that one that is used at once waits
+    // for all operands on their way as well
+    f32x4 ls4[2], dl4[2];
+    auto read_rows = [&](const char* st, int tl, int g) {
+        ls4[g & 1] = *(const f32x4*)(st + (32 * tl + 8 * g + 4 * hf) * 4);
+        dl4[g & 1] = *(const f32x4*)(st + 256 + (32 * tl + 8 * g + 4 * hf) * 4);
+    };
+    auto soft = [&](const char* st, int tl, int v) {
+        const int g = v >> 2;
+        if ((v & 3) == 0 && g < 3) read_rows(st, tl, g + 1);
+        const float pv = fast_exp2(fmaf(s[tl][v], sc2, -ls4[g & 1][v & 3]));
+        s[tl][v] = pv;
+        dp[tl][v] = pv * (dp[tl][v] - dl4[g & 1][v & 3]);
+        if (v & 1) {
+            pb[tl][v >> 3][(v >> 1) & 3] = pack2<E>(s[tl][v - 1], s[tl][v]);
+            sb[tl][v >> 3][(v >> 1) & 3] = pack2<E>(dp[tl][v - 1], dp[tl][v]);
         }
-        __syncthreads();                                   // tile t is in LDS; every wave is done with tile t - 1
-        if (t + 2 < nt) stage(t + 2);
-        const char* qt = lds + (t % kBuf) * 2 * T::kBytes;
-        const char* gt = qt + T::kBytes;
-        const char* st_ = lds + oStat + (t % kBuf) * 1024;
-
-        // Four stages per tile as in the dq kernel; lane = key, registers = queries:
-        //   1  S, dP of queries 0..31            2  those of queries 32..63 | softmax backward of queries 0..31
-        //   3  dV^T += dO^T P, dK^T += q^T dS of queries 0..31 | softmax backward of queries 32..63      4  the same of queries 32..63
-        constexpr int NA = 2 * T::DS, NO = 4 * T::DT;
-        constexpr int VA = 16 / NA > 0 ? 16 / NA : 1, VO = 16 / NO > 0 ? 16 / NO : 1;
-        f32x16 s[2], dp[2];
-        constexpr int kAhead = 4, kRing = 8;                // A operands read this many MFMAs ahead
-        u32x4 pb[4], sb[4], ring[kRing];
-        auto read_prod = [&](int tl, int j) {               // j even: q rows for S, odd: dO rows for dP
-            return *(const u32x4*)(((j & 1) ? gt : qt) + tl * 32 * T::kPitch + (a_off ^ (uint32_t)((j >> 1) << 5)));
+    };
+    // Step of half tl of tile t.  OUT: there is a half before it, PROD: a half behind it.  The ring holds the step's first operands.
+    auto step = [&](int t, auto tl_c, auto out_c, auto prod_c) {
+        constexpr int tl = decltype(tl_c)::value, no = decltype(out_c)::value ? NO : 0, na = decltype(prod_c)::value ? NA : 0;
+        const char *own = buffer(t), *before = tl ? own : buffer(t + kBuf - 1), *behind = tl ? buffer(t + 1) : own;
+        const char* st = lds + oStat + (t % kBuf) * 1024;
+        auto operand = [&](int i) {
+            if (i < no) return read_out(before, 1 - tl, i);
+            if (i < no + na) return read_prod(behind, 1 - tl, i - no);
+            return read_out(own, tl, i - no - na);          // the next step's
         };
-        // output MFMA j of a half: step st = 2 tl + j / (2 DT), head-dim block dt = (j / 2) % DT, j even: dV (dO^T), odd: dK (q^T)
-        auto read_out = [&](int tl, int j) {
-            const int dt = (j >> 1) % T::DT;
-            return tile_tr<D>((j & 1) ? qt : gt, tr[dt][0], tr[dt][1], 2 * tl + j / (2 * T::DT));
-        };
-        f32x4 ls4, dl4;                                     // row values of the four queries v & ~3 .. + 3
-        auto soft = [&](int tl, int v) {
-            const int r = 32 * tl + 8 * (v >> 2) + 4 * hf + (v & 3);
-            if ((v & 3) == 0) {
-                ls4 = *(const f32x4*)(st_ + r * 4);
-                dl4 = *(const f32x4*)(st_ + 256 + r * 4);
-            }
-            float pv = fast_exp2(fmaf(s[tl][v], sc2, -ls4[v & 3]));
-            if (ragged) pv = 64 * t + r < p.Sq ? pv : 0.f;
-            s[tl][v] = pv;
-            dp[tl][v] = pv * (dp[tl][v] - dl4[v & 3]);
-            if (v & 1) {
-                pb[2 * tl + (v >> 3)][(v >> 1) & 3] = pack2<E>(s[tl][v - 1], s[tl][v]);
-                sb[2 * tl + (v >> 3)][(v >> 1) & 3] = pack2<E>(dp[tl][v - 1], dp[tl][v]);
-            }
-        };
-        auto out_mfma = [&](int tl, int j, const u32x4& a) {
-            const int dt = (j >> 1) % T::DT, st = 2 * tl + j / (2 * T::DT);
-            if (j & 1) dka[dt] = E::mfma32(a, sb[st], dka[dt]);
-            else dva[dt] = E::mfma32(a, pb[st], dva[dt]);
-        };
-#pragma unroll
-        for (int tl = 0; tl < 2; ++tl)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) s[tl][v] = dp[tl][v] = 0.f;
-#pragma unroll
-        for (int j = 0; j < kAhead; ++j) ring[j] = read_prod(0, j);
+        read_rows(st, tl, 0);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < NA; ++j) {                      // stage 1
-            ring[(j + kAhead) % kRing] = j + kAhead < NA ? read_prod(0, j + kAhead) : read_prod(1, j + kAhead - NA);
-            if (j & 1) dp[0] = E::mfma32(ring[j % kRing], vb[j >> 1], dp[0]);
-            else s[0] = E::mfma32(ring[j % kRing], kb[j >> 1], s[0]);
-            __builtin_amdgcn_sched_barrier(0);
-        }
+        for (int i = 0; i < no + na; ++i) {
+            ring[(NS - no - na + i + kAhead) % kRing] = operand(i + kAhead);
+            if (i < no) grad(1 - tl, i, ring[(NS - no - na + i) % kRing]);
+            else prod(1 - tl, i - no, ring[(NS - no - na + i) % kRing]);
 #pragma unroll
-        for (int j = 0; j < NA; ++j) {                      // stage 2
-            ring[(NA + j + kAhead) % kRing] = j + kAhead < NA ? read_prod(1, j + kAhead) : read_out(0, j + kAhead - NA);
-            if (j & 1) dp[1] = E::mfma32(ring[(NA + j) % kRing], vb[j >> 1], dp[1]);
-            else s[1] = E::mfma32(ring[(NA + j) % kRing], kb[j >> 1], s[1]);
-#pragma unroll
-            for (int v = VA * j; v < VA * (j + 1) && v < 16; ++v) soft(0, v);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int j = 0; j < NO; ++j) {                      // stage 3
-            ring[(2 * NA + j + kAhead) % kRing] = j + kAhead < NO ? read_out(0, j + kAhead) : read_out(1, j + kAhead - NO);
-            out_mfma(0, j, ring[(2 * NA + j) % kRing]);
-#pragma unroll
-            for (int v = VO * j; v < VO * (j + 1) && v < 16; ++v) soft(1, v);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int j = 0; j < NO; ++j) {                      // stage 4
-            if (j + kAhead < NO) ring[(2 * NA + NO + j + kAhead) % kRing] = read_out(1, j + kAhead);
-            out_mfma(1, j, ring[(2 * NA + NO + j) % kRing]);
+            for (int v = 0; v < 16; ++v) {
+                const int at = v * (no + na) / 16;
+                if ((at < kLag ? kLag : at) == i) soft(st, tl, v);
+            }
             __builtin_amdgcn_sched_barrier(0);
         }
     };
+    // Tile t has landed (`more`: the next one's loads are behind its own) and is there for all waves, which are done with tile t - 2.
+    // The queries past the end have no weight.
+    auto meet = [&](int t, bool more) {
+        if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(T::CPR / 2 + 1) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (p.Sq % 64 && t == alltiles - 1 && wave == 0 && 64 * t + lane >= p.Sq)
+            *(float*)(lds + oStat + (t % kBuf) * 1024 + lane * 4) = INFINITY;
+        lds_barrier();
+    };
+    using c0 = std::integral_constant<int, 0>;
+    using c1 = std::integral_constant<int, 1>;
     stage(t0);
     if (t0 + 1 < nt) stage(t0 + 1);
-    for (int t = t0; t + 1 < nt; ++t) tile(t, std::false_type{});
-    if (p.Sq % 64 && nt == alltiles) tile(nt - 1, std::true_type{});
-    else tile(nt - 1, std::false_type{});
+    meet(t0, t0 + 1 < nt);
+#pragma unroll
+    for (int j = 0; j < NA; ++j) prod(0, j, read_prod(buffer(t0), 0, j));
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) ring[(NS - NA + j) % kRing] = read_prod(buffer(t0), 1, j);
+    step(t0, c0{}, c0{}, c1{});
+    for (int t = t0; t + 1 < nt; ++t) {
+        meet(t + 1, false);
+        if (t + 2 < nt) stage(t + 2);
+        step(t, c1{}, c1{}, c1{});
+        step(t + 1, c0{}, c1{}, c1{});
+    }
+    step(nt - 1, c1{}, c1{}, c0{});
+#pragma unroll
+    for (int j = 0; j < NO; ++j) grad(1, j, j < kAhead ? ring[j] : read_out(buffer(nt - 1), 1, j));
     if (split) {
         float* const row = p.part + (((int64_t)(item - p.rkv.full) * p.rkv.ranges + range) * 256 + wave * 32 + m) * D + 4 * hf;
 #pragma unroll
@@ -540,7 +545,7 @@ __global__ __launch_bounds__(256) void dense_bwd_sum_kernel(DenseBwdArgs p) {
 // model of its time in ns says that saves a tenth: a tile takes `tile_ns` with the chip full, `half_ns` on half of the slots
 // or fewer; the sum's launch 5000, and the partials (`floats` each) are written and read at 3.5 TB/s.  Measured:
 //     heads x queries x keys, us    before  now           heads x queries x keys, new keys' gradients only    before  now
-//     12 x 4680 x 14040 (dkv)         1132  1028           9 x 1000 x 5000                                       154   94
+//     12 x 4680 x 14040 (dkv)         1132   925           9 x 1000 x 5000                                       154   94
 //     1 x 500 x 16000                  365    64           21 x 202 x 2804                                        84   46
 //     1 x 4000 x 500                   153    46           3 x 4680 x 4680                                       267  177
 Rounds split_last_round(int64_t items, int tiles, int slots, double tile_ns, double half_ns, int floats) {
@@ -568,7 +573,7 @@ Rounds split_last_round(int64_t items, int tiles, int slots, double tile_ns, dou
 void plan_rounds(int64_t units, int Sq, int Skv, int nkv, int D, Rounds* rq, Rounds* rkv) {
     const double f = D == 64 ? 0.55 : 1.0;
     *rq = split_last_round((Sq + 127) / 128 * units, (Skv + 63) / 64, 2 * cu_count(), 2640 * f, 1500 * f, 128 * D);
-    *rkv = split_last_round((nkv + 127) / 128 * units, (Sq + 63) / 64, cu_count(), 2550 * f, 2100 * f, 256 * D);
+    *rkv = split_last_round((nkv + 127) / 128 * units, (Sq + 63) / 64, cu_count(), 2220 * f, 1830 * f, 256 * D);
 }
 
 // floats of the partials (the two grids run one after the other and share them)

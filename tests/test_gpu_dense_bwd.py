@@ -48,6 +48,23 @@ def test_dense_gradients(dtype, B, Lq, Lk, H, D):
     _close(vd.grad, vr.grad, dtype)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Lq", [1, 32, 33, 64, 65, 97, 128, 161, 192, 257])
+def test_dense_gradients_around_the_halves_of_a_tile(Lq, D):
+    """The keys' gradients take the queries 32 at a time in a pipeline over tiles of 64: one, two and more tiles, the last of them
+    one query, a half, a half and one query, or whole."""
+    dtype = torch.bfloat16
+    q0, do = (randn((1, Lq, 2, D), 300 + Lq + i, dtype) for i in range(2))
+    k0, v0 = (randn((1, 150, 2, D), 302 + Lq + i, dtype) for i in range(2))
+    qr, kr, vr = _leaf(q0.double()), _leaf(k0.double()), _leaf(v0.double())
+    dense.attention(qr, kr, vr).backward(do.double())
+    qd, kd, vd = _leaf(q0, DEV), _leaf(k0, DEV), _leaf(v0, DEV)
+    sfa.attention.attention(qd, kd, vd, dtype=dtype).backward(do.to(DEV))
+    _close(qd.grad, qr.grad, dtype)
+    _close(kd.grad, kr.grad, dtype)
+    _close(vd.grad, vr.grad, dtype)
+
+
 @pytest.mark.parametrize("partial", [False, True])
 def test_dense_kv_cache_gradients(partial):
     """q against a cache of 5 x 48 keys of which keys 96..192 arrive with the call; partial = grad_only_new_kv."""
