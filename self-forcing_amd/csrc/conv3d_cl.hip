@@ -384,6 +384,132 @@ __global__ __launch_bounds__(256, 2) void conv3d_row3_kernel(ConvArgs p) {
     }
 }
 
+// The same for grids that leave compute units idle: tiles of 128 positions x CB x 32 channels (a wave takes 32 positions), four stage
+// buffers, so that two stages are on their way behind the next one, and a step's operands read under the step before it:
+// alone on its compute unit a workgroup of the kernel above waits out every stage's loads and every step's reads.  384
+// channels, 28 x 26: 108 -> 31 us; 60 x 104: 113 -> 64.  The sums are formed in the same order as above, so that
+// how many frames a call holds, which decides the kernel, changes no bit of them.
+constexpr int kSmallBufs = 4;
+template <class E, int CB>
+__global__ __launch_bounds__(256) void conv3d_row3_small_kernel(ConvArgs p) {
+    constexpr int PW = 4, kVox = 32 * PW, kCo = 32 * CB;  // PW waves
+    constexpr int NB = kSmallBufs;
+    constexpr int kWRows = 3 * kCo;                       // weights of the three taps
+    constexpr int kNWG = kWRows / 16, kNXG = (kVox + 2 + 15) / 16;
+    constexpr int kNG = kNWG + kNXG;
+    constexpr int kPer = (kNG + PW - 1) / PW;             // groups a wave stages (the last ones may repeat group kNG - 1)
+    constexpr int kStage = kNG * 1024;
+    extern __shared__ __attribute__((aligned(256))) char lds[];
+    const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)lds;
+
+    const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, hf = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int WP = p.W + 2;
+    const int64_t FS = (int64_t)(p.H + 2) * WP;
+    const int64_t u_first = WP + 1, u_last = (int64_t)(p.T - 1) * FS + (int64_t)p.H * WP + p.W;
+    const int ny = p.Cout_pad / kCo;
+    const int per_xcd = (int)gridDim.x / 8;               // as in conv3d_cl_kernel
+    const int seq = (int)(blockIdx.x >> 3);
+    const int64_t u0 = u_first + ((int64_t)(blockIdx.x & 7) * (per_xcd / ny) + seq / ny) * kVox;
+    if (u0 > u_last) return;
+    const int co0 = (seq % ny) * kCo;
+
+    const int g_line = lane >> 4, g_row = lane >> 2, g_c = (lane & 3) ^ g_line;      // as in conv3d_row3_kernel
+    uint32_t src[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        const int g = min(wave + PW * i, kNG - 1);
+        const int j = g * 16 + g_row;
+        if (g < kNWG) {
+            const int dw = j / kCo, r = j - dw * kCo;
+            src[i] = (uint32_t)(((int64_t)dw * p.Cout_pad + co0 + r) * p.Cin * 2 + g_c * 16);
+        } else {
+            const int64_t u = min(u0 + (j - kWRows), u_last + 2) - WP - 1;
+            src[i] = (uint32_t)(u * p.Cin * 2 + g_c * 16);
+        }
+    }
+
+    const int cin_steps = p.Cin / kKC;
+    const int nstage = p.kt * 3 * cin_steps;
+    const char* f_w = p.wt;
+    const char* f_x = p.x;
+    const int64_t w_next_row = 3 * (int64_t)p.Cout_pad * p.Cin * 2 - (int64_t)p.Cin * 2;      // next kernel row: three taps on
+    const int64_t x_next_row = ((int64_t)WP - 1) * p.Cin * 2;
+    const int64_t x_next_frame = (FS - 3 * (int64_t)WP) * p.Cin * 2;
+    int f_cs = 0, f_dh = 0, f_s = 0;
+    // the next stage; behind the last one its loads are repeated into a free buffer, so that the partial waits count the same
+    auto stage = [&](uint32_t buf) {
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            const int g = min(wave + PW * i, kNG - 1);
+            cv_load_lds16(g < kNWG ? f_w : f_x, src[i], lds0 + buf + (uint32_t)g * 1024);
+        }
+        if (++f_s >= nstage) return;
+        f_w += kKC * 2;
+        f_x += kKC * 2;
+        if (++f_cs == cin_steps) {
+            f_cs = 0;
+            f_w += w_next_row;
+            f_x += x_next_row;
+            if (++f_dh == 3) {
+                f_dh = 0;
+                f_x += x_next_frame;
+            }
+        }
+    };
+
+    f32x16 acc[CB][1];
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[cb][0][v] = 0.f;
+    uint32_t a_off[2], b_off[3][2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+        a_off[ks] = tile_off(m, 2 * ks + hf);
+#pragma unroll
+        for (int dw = 0; dw < 3; ++dw) b_off[dw][ks] = tile_off(kWRows + 32 * wave + m + dw, 2 * ks + hf);
+    }
+
+#pragma unroll
+    for (int b = 0; b < NB - 1; ++b) stage(b * kStage);
+    uint32_t buf = 0, free = (NB - 1) * kStage;
+    for (int s = 0; s < nstage; ++s) {
+        // stage s has landed when only the loads of NB - 2 later ones are outstanding; all waves are done with the one before it
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NB - 2) * kPer) : "memory");
+        // a step's operands are read while the one before it is in the matrix pipe
+        u32x4 op[2][CB + 1];
+        auto read = [&](int j) {
+            const int dw = j >> 1, ks = j & 1;
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) op[j & 1][cb] = *(const u32x4*)(lds + buf + a_off[ks] + (dw * kCo + 32 * cb) * kRowBytes);
+            op[j & 1][CB] = *(const u32x4*)(lds + buf + b_off[dw][ks]);
+        };
+        read(0);
+        read(1);
+        __builtin_amdgcn_sched_barrier(0);
+        stage(free);
+        free = buf;
+#pragma unroll
+        for (int j = 0; j < 6; ++j) {
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) acc[cb][0] = E::mfma32(op[j & 1][cb], op[j & 1][CB], acc[cb][0]);
+            if (j + 2 < 6) read(j + 2);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        buf = buf == (NB - 1) * kStage ? 0 : buf + kStage;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // no load into this workgroup's LDS outlives it
+
+    const int64_t u = u0 + 32 * wave + m;
+    const int64_t uc = min(u, u_last);
+    const int t = (int)(uc / FS);
+    const int rem = (int)(uc - (int64_t)t * FS);
+    const int hp = rem / WP, wp = rem - hp * WP;
+    const bool vok = u <= u_last && hp >= 1 && hp <= p.H && wp >= 1 && wp <= p.W;
+    store_voxel<E, CB, 1>(p, acc, 0, vok, vok ? t : 0, vok ? hp - 1 : 0, vok ? wp - 1 : 0, co0, hf);
+}
+
 // The same for 96 output channels per workgroup (every 3x3x3 convolution of the decoder but its head), where the kernel above
 // is bound by its LDS: per stage and compute unit its two workgroups read 240 KB and fetch 70 KB for 288 matrix instructions,
 // reckoned at 128 bytes a cycle 2480 cycles against 2320 of the matrix pipes (SQ_INSTS_LDS 0.83 per matrix instruction).
@@ -571,6 +697,27 @@ int launch_row3(const ConvArgs& a, hipStream_t st) {
     return SFM_OK;
 }
 
+template <class E, int CB>
+int launch_row3_small(const ConvArgs& a, hipStream_t st) {
+    constexpr int ldsb = kSmallBufs * (3 * 32 * CB / 16 + 9) * 1024;
+    hipError_t e = hipFuncSetAttribute((const void*)conv3d_row3_small_kernel<E, CB>, hipFuncAttributeMaxDynamicSharedMemorySize, ldsb);
+    if (e != hipSuccess) {
+        set_error("sfm_conv3d_cl: hipFuncSetAttribute failed: %s", hipGetErrorString(e));
+        return SFM_ERR_HIP;
+    }
+    const int64_t WP = a.W + 2, FS = (int64_t)(a.H + 2) * WP;
+    const int64_t positions = (int64_t)(a.T - 1) * FS + (int64_t)(a.H - 1) * WP + a.W;     // first to last interior voxel
+    const unsigned tiles = (unsigned)((positions + 127) / 128);
+    hipLaunchKernelGGL((conv3d_row3_small_kernel<E, CB>), dim3((tiles + 7) / 8 * 8 * (unsigned)(a.Cout_pad / (32 * CB))), dim3(256),
+                       ldsb, st, a);
+    e = hipGetLastError();
+    if (e != hipSuccess) {
+        set_error("sfm_conv3d_cl: launch failed: %s", hipGetErrorString(e));
+        return SFM_ERR_HIP;
+    }
+    return SFM_OK;
+}
+
 template <class E, int CB, int WN>
 int launch_cfg(const ConvArgs& a, hipStream_t st) {
     constexpr int kVox = 64 * (4 / WN), kCo = 32 * CB * WN, kCoRows = (kCo + 63) / 64 * 64;
@@ -598,6 +745,13 @@ int launch_dtype(const ConvArgs& a, hipStream_t st) {
         const int64_t positions = (int64_t)(a.T - 1) * (a.H + 2) * (a.W + 2) + (int64_t)(a.H - 1) * (a.W + 2) + a.W;
         const int64_t wgs = (positions + 511) / 512 * (a.Cout_pad / 96), cu = cu_count(), rounds = (wgs + cu - 1) / cu;
         if (a.Cin >= 192 ? 4 * wgs >= 3 * rounds * cu : wgs >= 8 * cu) return launch_row3_wide<E>(a, st);
+        // Half-empty grids take the small tiles: 128 positions x 32 channels where two of its workgroups to a compute unit hold them all,
+        // 128 x 96 where one does.  us with 256 x 96, 128 x 96 and 128 x 32 (384 channels, workgroups of the first):
+        // 28 x 26 (16) 108, 60, 31; 56 x 52 (52) 109, 60, 45; 3 x 32 x 44 (76) 108, 62, 62; 60 x 104 (100) 113, 64, 86; 192
+        // channels, 3 x 64 x 88 (140) 59, 66, 55; 96 channels, 224 x 208 (186) 34, 38, 39.
+        const int64_t narrow = (positions + 255) / 256 * (a.Cout_pad / 96);
+        if (3 * narrow <= cu) return launch_row3_small<E, 1>(a, st);
+        if (2 * narrow <= cu) return launch_row3_small<E, 3>(a, st);
         return launch_row3<E, 3>(a, st);
     }
     if (run && a.Cout_pad == 32) return launch_row3<E, 1>(a, st);

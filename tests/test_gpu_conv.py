@@ -52,6 +52,32 @@ def test_conv_cl_matches_fp32_convolution(cin, cout, kt, k, T, H, W, up2x, hist,
     assert (y.float() - ref).abs().max().item() <= tol
 
 
+@pytest.mark.parametrize("cin,cout,T,H,W,chunks", [
+    (96, 96, 9, 100, 120, (1, 2, 6)),             # 49, 98 and 292 tiles of 256 positions: every tile size but the wide one
+    (384, 384, 4, 60, 104, (1, 3)),               # all frames at once on the wide tiles
+    (64, 192, 3, 9, 13, (1, 2)),
+    (32, 96, 2, 1, 127, (1, 1)),                  # a tile ends at the last position, one before and one behind it
+    (32, 96, 2, 1, 128, (1, 1)),
+    (32, 96, 2, 1, 129, (1, 1)),
+])
+def test_how_many_frames_a_call_holds_changes_no_bit(cin, cout, T, H, W, chunks):
+    """The frame count decides the tile size of a 3x3x3 convolution; all of them form their sums in one order."""
+    torch.manual_seed(cin + cout + W)
+    conv = nn.Conv3d(cin, cout, 3).cuda().to(torch.bfloat16)
+    x = torch.randn(T, H, W, cin, device="cuda").to(torch.bfloat16)
+    res = torch.randn(T, H, W, cout, device="cuda").to(torch.bfloat16)
+    whole = co.conv_cl(x, conv, None, res=res)
+    parts, t = [], 0
+    for n in chunks:
+        parts.append(co.conv_cl(x[t:t + n], conv, x[max(t - 2, 0):t] if t else None, res=res[t:t + n]))
+        t += n
+    assert t == T and torch.equal(torch.cat(parts), whole)
+    xf = F.pad(x.float().permute(3, 0, 1, 2).unsqueeze(0), (1, 1, 1, 1, 2, 0))
+    ref = F.conv3d(xf, conv.weight.float(), conv.bias.float())[0].permute(1, 2, 3, 0) + res.float()
+    # fp32 accumulation of 16-bit products, one rounding of the result
+    assert (whole.float() - ref).abs().max().item() <= 2.0 ** -8 * max(1.0, ref.abs().max().item()) * 1.01
+
+
 def test_conv_cl_rejects_bad_arguments():
     import ctypes as C
     from self_forcing_amd import lib as L
