@@ -457,13 +457,17 @@ __device__ __forceinline__ void wait_vm() {
 //       buffers per matrix, one barrier before the logits and one before the output products.  (A pass over the rows for
 //       every 32 query rows, as before, took 518 us at the 720p grid, b1 = 45, and 96 us at three frames tied, b1 = 90;
 //       this form 299 and 70.  Two query tiles in one wave need 290 registers and spill.)
+// A chunk is a chain, barrier to barrier: with the full exp2f and a row mask in every chunk a team's chunk took 1.2 us however
+// few columns there were, now 1.0 (2 heads x 30 columns of 1332 rows 50 -> 42 us).  Teams of three and four have three
+// waves per SIMD (168 registers), so that the 624 columns of 12 heads with three frames tied are one round: 69 -> 60 us,
+// head_dim 64 46 -> 31; a team of two gains nothing from a third wave.  A third chunk pair in LDS: 72.
 // SHARE (TEAM = 1): 2 or 4 (p.s2_split) waves of a workgroup share a column's rows, 32-row chunks dealt in turn, and merge
 // (maximum, sum, output) through LDS at the end: with few (a, j) columns the chip is otherwise idle and a wave's chain of
 // dependent chunks (about 2.5 us each) is the whole time.  A kernel of its own: with the number of waves an argument of one
 // kernel for both, a call of three 480p frames against themselves (12 heads), whose columns are not shared, took 76.2 us
 // instead of 75.4 (two runs differ by 0.1).
 template <class E, int D, int TEAM, bool SHARE = false>
-__global__ __launch_bounds__(TEAM == 1 ? 256 : 64 * TEAM) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ __launch_bounds__(TEAM == 1 ? 256 : 64 * TEAM) __attribute__((amdgpu_waves_per_eu(TEAM >= 3 ? 3 : 2, TEAM >= 3 ? 3 : 2)))
 void monarch_step2_kernel(MonarchArgs p) {
     using L = S2Lds<D>;
     constexpr int DS = D / 16, DT = D / 32, CPR = D / 8;
@@ -597,24 +601,32 @@ void monarch_step2_kernel(MonarchArgs p) {
 
         float mx = -INFINITY;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            int r = 32 * n + 8 * (v >> 2) + 4 * hf + (v & 3);
-            float z = r < r_lim ? s[v] * sc2 - cc[v >> 2][v & 3] : -INFINITY;
-            s[v] = z;
-            mx = fmaxf(mx, z);
+        for (int v = 0; v < 16; ++v) s[v] = fmaf(s[v], sc2, -cc[v >> 2][v & 3]);
+        if (!more && r_lim % 32) {                 // a column's last chunk: rows past its end
+#pragma unroll
+            for (int v = 0; v < 16; ++v) s[v] = 32 * n + 8 * (v >> 2) + 4 * hf + (v & 3) < r_lim ? s[v] : -INFINITY;
         }
-        mx = xhalf_max(mx);
-        const float mnew = fmaxf(mrun, mx);        // finite: chunk n has at least one valid row
-        const float alpha = exp2f(mrun - mnew);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) mx = fmaxf(mx, s[v]);
+        // The sums so far are rescaled only where a row's maximum moves.  (A reference point that may lag behind the maximum, so
+        // that this is rare, takes another 3 us of 60 off, but then a row's largest weight is no longer an exact 1: the
+        // output's error against float64 grows by 1 %.)
+        const bool moves = __any(mx > mrun);
+        float alpha = 1.f;
+        if (moves) {
+            const float mnew = fmaxf(mrun, xhalf_max(mx));       // finite: chunk n has at least one valid row
+            alpha = fast_exp2(mrun - mnew);
+            lrun *= alpha;
+            mrun = mnew;
+        }
         float psum = 0.f;
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-            float e = exp2f(s[v] - mnew);
+            const float e = fast_exp2(s[v] - mrun);
             psum += e;
             s[v] = e;
         }
-        lrun = lrun * alpha + psum;
-        mrun = mnew;
+        lrun += psum;
         u32x4 pb[2];
 #pragma unroll
         for (int st = 0; st < 2; ++st) {
@@ -627,10 +639,14 @@ void monarch_step2_kernel(MonarchArgs p) {
         if (more) wait_vm<SOLO ? MYG + 1 : 2 * MYG + 1>();
         else wait_vm<0>();
         if (!SOLO) lds_barrier();
+        if (moves) {
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) oacc[dt][v] *= alpha;
+        }
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
-#pragma unroll
-            for (int v = 0; v < 16; ++v) oacc[dt][v] *= alpha;
 #pragma unroll
             for (int st = 0; st < 2; ++st) {
                 const u32x2 lo = s1_read_tr(yt, tr[dt][0] + st * 16 * L::kPitch);

@@ -57,6 +57,22 @@ def test_mfma_path_small_shapes(dtype, B, H, D, a, f, b1, b2):
     assert_close_16bit(out, ref, dtype)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,b1", [(2, 30), (520, 30), (2, 45), (2, 90), (2, 128)])      # shared columns, a wave each, teams of 2, 3 and 4
+@pytest.mark.parametrize("grow", [0.2, 1.5, -1.5])
+def test_step_2_rescales_where_a_maximum_moves(H, b1, grow, dtype):
+    """Logits that grow slowly from chunk to chunk, that grow fast, and that fall, so that the first chunk's maxima stay.  One column per block: the right factor is 1 and Kbar, Y are the rows themselves, so that the logits are exact."""
+    f, D = 8, 128
+    q = randn((1, b1, H, D), 40, dtype)
+    k, v = (randn((1, f * b1, H, D), 41 + i, dtype) for i in range(2))
+    scale = torch.linspace(1.0, 1.0 + abs(grow) * f, f * b1)
+    k = (k * (scale if grow > 0 else scale.flip(0)).view(1, -1, 1, 1)).to(dtype)
+    v = v / 4      # near one-hot weights hand v out as it is: bf16 rounds |v| <= 5 by 2^-7, a quarter of it by 2^-9, inside the bar of 2e-2
+    ref = monarch.monarch_attn(q, k, v, 1, 1, 1, b1, 1, dtype=torch.float32)
+    out = mattn.monarch_attn(q.to(DEV), k.to(DEV), v.to(DEV), 1, 1, 1, b1, 1)
+    assert_close_16bit(out, ref, dtype)
+
+
 @pytest.mark.parametrize("heads_per_pass", [1, 2, 5])
 def test_head_passes_give_identical_results(heads_per_pass):
     """Passes over fewer heads give the same bits.  The one-kernel forward is the exception: the tile ranges of its
