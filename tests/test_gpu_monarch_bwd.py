@@ -226,7 +226,7 @@ def test_gradients_around_the_left_factors_query_tiles(b1, Fk, part, D, switches
 @pytest.mark.parametrize("h,w,F,chunk,D,dtype", [
     (4, 52, 3, 1, 128, torch.bfloat16),       # waves of step 1 with both masked and visible columns
     (6, 20, 6, 2, 64, torch.float16),         # chunks of two block-frames
-    (5, 52, 9, 3, 128, torch.bfloat16),       # several query chunks in step 1, three passes of the right factor over a tile
+    (5, 52, 9, 3, 128, torch.bfloat16),       # several query chunks in step 1, several chunks of the right factor over a tile
     (70, 8, 3, 1, 64, torch.bfloat16),        # three query tiles
     (30, 80, 3, 1, 64, torch.bfloat16),       # b2 > 64: the library chain, for which nothing is left out
     (40, 12, 6, 6, 128, torch.float16),       # one chunk: nothing is masked
@@ -388,7 +388,7 @@ def test_three_frames_tied_480p_blocks_on_the_fused_kernels(saved):
     (4, 52, 3, 5, 3, 0),        # one slab: every fused part, all heads in one pass
     (40, 12, 2, 3, 3, 2),       # b1 = 40: two query-row slices (two slabs of partial sums), a shorter last pass
     (90, 8, 1, 2, 2, 1),        # three slices, one head per pass
-    (5, 6, 2, 3, 2, 0),         # b2 = 6: the right factor on the library chain, whose scratch is laid out differently
+    (5, 6, 2, 3, 2, 0),         # b2 = 6: dS1 rows padded to whole pieces of four
 ])
 def test_backward_stays_inside_an_exactly_sized_workspace(h, w, Fq, Fk, H, hpp):
     """sfm_monarch_bwd with a workspace of exactly the queried size and canary bytes behind it; the gradients equal the
