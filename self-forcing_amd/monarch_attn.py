@@ -117,6 +117,8 @@ def kv_cache_write(new_k, new_v, k_cache, v_cache, start_idx, end_idx, f_tied, h
     if k_cache.stride() != v_cache.stride():
         raise ValueError("k_cache and v_cache must share their strides")
     B, _, H, D = new_k.shape
+    if B > k_cache.shape[0] or H > k_cache.shape[2] or D > k_cache.shape[3]:
+        raise ValueError(f"new_k {tuple(new_k.shape)} holds more batches, heads or channels than the cache {tuple(k_cache.shape)}")
     with _on_device(new_k.device):
         _l.check(_l.load().sfm_kv_cache_write(_DT[new_k.dtype], B, H, D, C.byref(_l.Tiling(f_tied, h_reduce, w_reduce, h, w)),
                                               new_k.data_ptr(), new_v.data_ptr(), _l.strides3(new_k), k_cache.data_ptr(),
@@ -124,10 +126,16 @@ def kv_cache_write(new_k, new_v, k_cache, v_cache, start_idx, end_idx, f_tied, h
                                               _stream(new_k)))
 
 
+def _like_q(q, new_k):
+    """The operators with a cache write take the new chunk's batches, heads and head_dim from q.  A chunk of other sizes is
+    written by itself (kv_cache_write takes them from the chunk)."""
+    return new_k.shape[0] == q.shape[0] and new_k.shape[2:] == q.shape[2:]
+
+
 def _monarch_fwd_stats(q, k, v, tiling, sm_scale, kv_block_order, cbf, heads_per_pass=0, new=None):
-    """Forward for autograd, with new = (new_k, new_v, start_idx, end_idx) of the KV-cache operator: returns (out, stats) where stats is the opaque row-statistics tensor that
-    sfm_monarch_bwd_saved takes, or None when the forward that runs for these tensors produces none (the
-    reference's forward keeps z and z_lse the same way, monarch_attn.py:1309-1317)."""
+    """Forward for autograd, with new = (new_k, new_v, start_idx, end_idx) of the KV-cache operator: returns (out, stats)
+    where stats is the opaque row-statistics tensor that sfm_monarch_bwd_saved takes, or None when the forward that runs for
+    these tensors produces none (the reference's forward keeps z and z_lse the same way, monarch_attn.py:1309-1317)."""
     out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     d = _desc(q, k, v, out, *tiling, sm_scale, kv_block_order, cbf, 1)
     n = C.c_size_t(0)
@@ -135,10 +143,11 @@ def _monarch_fwd_stats(q, k, v, tiling, sm_scale, kv_block_order, cbf, heads_per
     nbytes = monarch_workspace_bytes(d, heads_per_pass)
     ws = scratch(nbytes, q.device)
     stats = torch.empty(n.value // 4, dtype=torch.float32, device=q.device) if n.value else None
-    if new is not None and stats is None:
+    if new is not None and (stats is None or not _like_q(q, new[0])):
         kv_cache_write(*new[:2], k, v, *new[2:], *tiling)
+        new = None
     with _on_device(q.device):
-        if new is not None and stats is not None:
+        if new is not None:
             new_k, new_v, start_idx, end_idx = new
             if new_k.stride() != new_v.stride():
                 new_k, new_v = new_k.contiguous(), new_v.contiguous()
@@ -396,6 +405,10 @@ def monarch_attn_with_kv_cache(q, k_cache, v_cache, new_k, new_v, start_idx, end
         raise ValueError(f"new_k holds {new_k.shape[1]} tokens but end_idx - start_idx = {end_idx - start_idx}")
     if sm_scale is None:
         sm_scale = q.shape[-1] ** -0.5
+    if not _like_q(q, new_k):
+        kv_cache_write(new_k, new_v, k_cache, v_cache, start_idx, end_idx, f_tied, h_reduce, w_reduce, h, w)
+        return monarch_attn(q, k_cache, v_cache, f_tied, h_reduce, w_reduce, h, w, sm_scale=sm_scale, num_iters=num_iters,
+                            heads_per_pass=heads_per_pass, kv_block_order=True, one_kernel=one_kernel)
     out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     d = _desc(q, k_cache, v_cache, out, f_tied, h_reduce, w_reduce, h, w, sm_scale, 1, 0, num_iters, one_kernel)
     nbytes = monarch_workspace_bytes(d, heads_per_pass)
@@ -417,6 +430,8 @@ def monarch_attn_with_kv_cache_static(q, k_cache, v_cache, new_k, new_v, start_i
         _check4(name, t, q.dtype, q.device)
     if k_cache.shape != v_cache.shape or new_k.shape != new_v.shape or new_k.stride() != new_v.stride():
         raise ValueError("k/v shapes or strides differ")
+    if not _like_q(q, new_k):
+        raise ValueError(f"new_k {tuple(new_k.shape)} must have q's batches, heads and head_dim {tuple(q.shape)}")
     if new_k.shape[1] != end_idx - start_idx:
         raise ValueError(f"new_k holds {new_k.shape[1]} tokens but end_idx - start_idx = {end_idx - start_idx}")
     if sm_scale is None:

@@ -215,6 +215,35 @@ def test_cache_call_under_autograd_takes_a_chunk_that_starts_within_a_block():
     assert torch.equal(out.detach(), want) and torch.equal(kc, ref[0]) and torch.equal(vc, ref[1])
 
 
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])        # with row statistics under autograd, and without
+@pytest.mark.parametrize("batches,heads", [(1, 2), (2, 1), (1, 1)])
+def test_a_chunk_of_fewer_batches_or_heads_than_q(batches, heads, dtype, grad):
+    """The chunk's own rows go to the cache, no others, and nothing past the chunk's end is read: the rest of the storage behind it holds NaN."""
+    per, tiling = 4 * 20, (1, 1, 1, 4, 20)
+    q = randn((2, per, 2, 64), 0, dtype).to(DEV)
+    kc, vc = (randn((2, 3 * per, 2, 64), 1 + i, dtype).to(DEV) for i in range(2))
+    behind = [torch.full((4 * q.numel(),), float("nan"), dtype=dtype, device=DEV) for _ in range(2)]
+    new = []
+    for i, b in enumerate(behind):
+        n = batches * per * heads * 64
+        b[:n] = randn((n,), 3 + i, dtype).to(DEV)
+        new.append(b[:n].view(batches, per, heads, 64))
+    ref = kc.clone(), vc.clone()
+    for c, n in zip(ref, new):
+        c[:batches, per:2 * per, :heads] = n
+    want = mattn.monarch_attn(q, *ref, *tiling, kv_block_order=True)
+    out = mattn.monarch_attn_with_kv_cache(q.requires_grad_(grad), kc, vc, *new, per, 2 * per, *tiling)
+    assert torch.equal(out.detach(), want) and torch.equal(kc, ref[0]) and torch.equal(vc, ref[1])
+    if grad:
+        out.sum().backward()
+        assert torch.isfinite(q.grad).all()
+    with pytest.raises(ValueError):
+        mattn.monarch_attn_with_kv_cache_static(q.detach(), kc, vc, *new, per, 2 * per, *tiling)
+    with pytest.raises(ValueError):        # more than the cache holds
+        mattn.kv_cache_write(*new, kc[:batches, :, :heads, :32], vc[:batches, :, :heads, :32], per, 2 * per, *tiling)
+
+
 def test_kv_cache_view_with_batch_stride_and_prefix():
     """B=2, the op sees kv_cache[:, :local_end] of a longer allocation (batch stride = full cache)."""
     h, w, H, D = 4, 20, 2, 64
