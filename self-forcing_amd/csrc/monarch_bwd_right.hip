@@ -103,7 +103,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
     const int unit = p.unit0 + (int)u;
 
     // LDS position P (16-byte units) of a tile holds chunk (P % C) ^ swz(row) of row P / C; 64 rows, those past the end repeat
-    // the last one: what they add is multiplied by zeros of R and dS1 or lands in key rows that are not stored
+    // the last one.  Key rows past the end land in rows of dK and dV that are not stored; columns are cleared below; a query
+    // row that is not finite has made its column's dS1, and with it all of dK, NaN already
     auto stage = [&](const char* src, uint32_t row_bytes, int nrows, uint32_t dst, auto cpr_c) {
         constexpr int C = decltype(cpr_c)::value;
 #pragma unroll
@@ -145,11 +146,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
     };
     auto loaded = [&](int nrows) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        lds_barrier();  
-        if (nrows < kCols) {                                             // columns past the end have no weight
+        lds_barrier();
+        if (nrows < kCols) {
+            // Columns past the end have no weight, and nothing to weigh: what is loaded there is the last column again, and an
+            // infinity of it times a weight of zero would make every row of dV and dK NaN.
             const u32x4 z = {0u, 0u, 0u, 0u};
             for (int i = tid; i < (kCols - nrows) * 8; i += kThreads) *(u32x4*)(lds + L::oR + nrows * 128 + i * 16) = z;
-            lds_barrier();  
+            for (int i = tid; i < (kCols - nrows) * CPR; i += kThreads) {
+                *(u32x4*)(lds + L::oG + nrows * kPitch + i * 16) = z;
+                *(u32x4*)(lds + L::oH + nrows * kPitch + i * 16) = z;
+            }
+            lds_barrier();
         }
     };
     auto queries = [&](int c0, int nrows) {                              // the query rows of (unit, k) take the place of the dY tile

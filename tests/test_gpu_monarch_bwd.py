@@ -200,6 +200,27 @@ def test_block_columns_that_are_no_multiple_of_four(b2, D):
         _close(vd.grad, vr.grad, dtype)
 
 
+@pytest.mark.parametrize("dtype,D,h,w,F", [
+    (torch.bfloat16, 128, 5, 52, 3),      # 156 columns: the last chunk of 64 holds 28
+    (torch.float16, 64, 5, 39, 2),        # 78: 14; rows of dS1 padded to whole pieces
+    (torch.bfloat16, 128, 4, 20, 3),      # 60: one chunk
+    (torch.bfloat16, 64, 4, 32, 2),       # 64: nothing past the end
+])
+@pytest.mark.parametrize("row", [0, -1])
+def test_an_infinite_gradient_stays_in_its_channel(row, dtype, D, h, w, F):
+    """dV of an infinite output gradient is infinite in that channel of the keys that the query sees, and finite in all others.
+    The last query's column is the one that stands in for those past the end of a chunk."""
+    q0, k0, v0, do = (randn((1, F * h * w, 2, D), 900 + i, dtype) for i in range(4))
+    do[0, row, 1, 5] = float("inf")
+    q, k, v = (_leaf(t, DEV) for t in (q0, k0, v0))
+    out = mattn.monarch_attn(q, k, v, 1, 1, 1, h, w)
+    dv = torch.autograd.grad(out, v, do.to(DEV))[0][0]
+    # the weights of each query block row reach every key block row, and within it the keys that its columns' right factors see
+    assert torch.isinf(dv[:, 1, 5]).all() and not torch.isnan(dv).any()
+    dv[:, 1, 5] = 0
+    assert torch.isfinite(dv).all()
+
+
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("b1,Fk,part", [(1, 3, 0), (31, 2, 0), (32, 1, 0), (33, 2, 0), (64, 1, 0), (65, 2, 0), (96, 1, 0), (97, 2, 0), (128, 1, 0),
                                         (32, 2, "SW_BWD_DQA_GEMM"), (70, 2, "SW_BWD_DQA_GEMM"), (70, 2, "SW_BWD_DQK_GEMM")])
