@@ -129,7 +129,8 @@ def kv_cache_write(new_k, new_v, k_cache, v_cache, start_idx, end_idx, f_tied, h
 def _like_q(q, new_k):
     """The operators with a cache write take the new chunk's batches, heads and head_dim from q.  A chunk of other sizes is
     written by itself (kv_cache_write takes them from the chunk)."""
-    return new_k.shape[0] == q.shape[0] and new_k.shape[2:] == q.shape[2:]
+    n, s = new_k.shape, q.shape
+    return n[0] == s[0] and n[2] == s[2] and n[3] == s[3]
 
 
 def _monarch_fwd_stats(q, k, v, tiling, sm_scale, kv_block_order, cbf, heads_per_pass=0, new=None):
@@ -401,15 +402,16 @@ def monarch_attn_with_kv_cache(q, k_cache, v_cache, new_k, new_v, start_idx, end
     if new_k.stride() != new_v.stride():
         new_v = new_v.contiguous()
         new_k = new_k.contiguous()
-    if new_k.shape[1] != end_idx - start_idx:
-        raise ValueError(f"new_k holds {new_k.shape[1]} tokens but end_idx - start_idx = {end_idx - start_idx}")
+    n, size = new_k.shape, q.shape           # once: the smallest calls are host work
+    if n[1] != end_idx - start_idx:
+        raise ValueError(f"new_k holds {n[1]} tokens but end_idx - start_idx = {end_idx - start_idx}")
     if sm_scale is None:
-        sm_scale = q.shape[-1] ** -0.5
-    if not _like_q(q, new_k):
+        sm_scale = size[3] ** -0.5
+    if n[0] != size[0] or n[2] != size[2] or n[3] != size[3]:      # not _like_q
         kv_cache_write(new_k, new_v, k_cache, v_cache, start_idx, end_idx, f_tied, h_reduce, w_reduce, h, w)
         return monarch_attn(q, k_cache, v_cache, f_tied, h_reduce, w_reduce, h, w, sm_scale=sm_scale, num_iters=num_iters,
                             heads_per_pass=heads_per_pass, kv_block_order=True, one_kernel=one_kernel)
-    out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+    out = torch.empty(size, dtype=q.dtype, device=q.device)
     d = _desc(q, k_cache, v_cache, out, f_tied, h_reduce, w_reduce, h, w, sm_scale, 1, 0, num_iters, one_kernel)
     nbytes = monarch_workspace_bytes(d, heads_per_pass)
     ws = scratch(nbytes, q.device)
