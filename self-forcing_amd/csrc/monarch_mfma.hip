@@ -70,7 +70,10 @@ struct S1Lds {
 // CS: block-causal without the masked pairs: a wave all of whose columns are masked for a tile forms and stores nothing.  A
 //     training clip of three chunks (a = f = 3, b1 = 90, b2 = 52, 12 heads) has a third of its pairs masked: 99 -> 85 us,
 //     with R written 119 -> 98.
-template <class E, int D, int NT, bool WR = false, bool IT = false, bool KO = false, bool CS = false>
+// NW: a KV-cache call: the tiles of the new chunk come from the chunk and go to their cache rows too.  Its state costs every
+//     tile, so that the calls without a chunk have kernels without it: 40 heads x 64, 12 x 36 in half-height blocks, 21 frames
+//     275 us with it, 271 without; 19 x 128 of 9 x 95, 15 frames 238, 235.5.
+template <class E, int D, int NT, bool WR = false, bool IT = false, bool KO = false, bool CS = false, bool NW = false>
 __global__ __launch_bounds__(NT > 2 ? 512 : 768) __attribute__((amdgpu_waves_per_eu(NT > 2 ? 2 : 3, NT > 2 ? 2 : 3)))
 void monarch_step1_kernel(MonarchArgs p) {
     using L = S1Lds<D, NT, KO>;
@@ -132,7 +135,7 @@ void monarch_step1_kernel(MonarchArgs p) {
     };
 
     // tile x is of the new chunk, whose rows are not in the cache yet
-    auto is_new = [&](const Tile& x) { return !WR && !CS && p.new_kv && x.f >= p.new_f0 && x.f < p.new_f1; };
+    auto is_new = [&](const Tile& x) { return NW && x.f >= p.new_f0 && x.f < p.new_f1; };
 
     // Tile x into buffer `buf`: LDS position P (in 16-byte units) holds chunk (P % CPR) ^ swz(row) of row P / CPR.
     // Rows past the end of a short tile (l >= b2) load row b2 - 1 again; their logits are masked below.  Every wave
@@ -417,7 +420,7 @@ void monarch_step1_kernel(MonarchArgs p) {
                 }
             }
         }
-        if (!WR && !CS && fresh && cur.ac == 0 && is_new(cur)) write_new(cur, kt);
+        if (NW && fresh && cur.ac == 0 && is_new(cur)) write_new(cur, kt);
     }
 }
 
@@ -1400,8 +1403,12 @@ struct Step1Kernel {
 template <class E, int D, int NT>
 static Step1Kernel step1_kernel(const MonarchArgs& a, Step1 kind) {
     constexpr size_t whole = S1Lds<D, NT, false>::kGroup;
-    if (kind == Step1::kIterKbar) return {(const void*)monarch_step1_kernel<E, D, NT, false, true, true>, S1Lds<D, NT, true>::kGroup};
-    if (kind == Step1::kIter) return {(const void*)monarch_step1_kernel<E, D, NT, false, true>, whole};
+    if (kind == Step1::kIterKbar)
+        return {a.new_kv ? (const void*)monarch_step1_kernel<E, D, NT, false, true, true, false, true> : (const void*)monarch_step1_kernel<E, D, NT, false, true, true>,
+                S1Lds<D, NT, true>::kGroup};
+    if (kind == Step1::kIter)
+        return {a.new_kv ? (const void*)monarch_step1_kernel<E, D, NT, false, true, false, false, true> : (const void*)monarch_step1_kernel<E, D, NT, false, true>, whole};
+    if (a.new_kv) return {(const void*)monarch_step1_kernel<E, D, NT, false, false, false, false, true>, whole};
     const bool skip = a.causal && a.skip_masked;
     if constexpr (NT <= 2) {
         if (a.rb) return {skip ? (const void*)monarch_step1_kernel<E, D, NT, true, false, false, true> : (const void*)monarch_step1_kernel<E, D, NT, true>, whole};
