@@ -214,7 +214,7 @@ void monarch_step1_kernel(MonarchArgs p) {
     // wait for the loads can leave those stores in flight instead of draining them.
     u32x4 qb[DS];                                          // logits operand (B): this lane's query row
     u32x4 qn[DS];                                          // the next tile's, requested a tile ahead where it is another one
-    float wn = 1.f;                                        // IT: the weight of the next tile's representative
+    float wn = 1.f;                                        // IT: the weight of the next tile's representative (not AH: this tile's factor)
     uint32_t crow[4] = {0, 0, 0, 0};                       // byte offsets in the (f, k) slab of the four scratch rows this lane stores to
     uint32_t cloff = 0;                                    // same for cl
     int qkey = -1;
@@ -222,10 +222,14 @@ void monarch_step1_kernel(MonarchArgs p) {
 
     auto scratch_row = [&](const Tile& x) { return (uint32_t)x.ul * p.ws_unit + (uint32_t)x.k * p.ws_row + (uint32_t)x.f * fstep; };
     auto query_key = [&](const Tile& x) { return (x.ul * p.b1 + x.k) * p.n_achunks + x.ac; };     // one value per (unit, k, query chunk)
-    // Query rows of tile x.  They are asked for after the tile's own loads and before this round's stores, and so have landed
-    // with them: fetched where they are used, they are waited for behind all the stores of the tile before (3 refinement
-    // passes at three frames tied, which fetch them for every tile, 547 -> 534 us).  CS fetches them there all the same: a
-    // wave that skips a tile has no stores to count, and the whole clip's step 1 took 86.3 us this way, 83.6 that.
+    // Query rows of tile x.  AH: they are asked for a tile ahead, after the tile's own loads and before this round's stores, and so
+    // have landed with them: fetched where they are used, they are waited for behind all the stores of the tile before (3
+    // refinement passes at three frames tied, which fetch them for every tile, 547 -> 534 us).  The second copy of the fetch costs
+    // calls of few tiles and of short ones more than that: without a new chunk, 1 head x 128 of 22 x 50 in half-width blocks
+    // 38.7 us ahead, 37.4 where they are used, 4 heads of 30 x 52, 3 frames 29.0, 28.5; the refinement with one key tile, 6 x 64
+    // of 30 x 52 in half-width blocks 388, 373.  With a chunk, 38 x 64 of 30 x 52 in half-height blocks 554, 558.  CS: a wave that
+    // skips a tile has no stores to count, and the whole clip's step 1 took 86.3 us ahead, 83.6 where they are used.
+    constexpr bool AH = (IT && NT > 1) || NW;
     auto fetch_query = [&](const Tile& x, u32x4* to) {
         const int unit = p.unit0 + x.ul;
         const int b = unit / p.H, h = unit % p.H;
@@ -236,7 +240,7 @@ void monarch_step1_kernel(MonarchArgs p) {
         if (IT && p.iter_mode == 2) {
             const size_t rrow = (size_t)scratch_row(x) + (size_t)(x.a0 * b2 + cg) * p.ws_aj;
             qrow = (const uint16_t*)p.rep + rrow * D + 8 * hf;
-            wn = p.wgt[rrow];
+            wn = AH ? p.wgt[rrow] : fminf(1.0f / (p.wgt[rrow] + 1e-6f), 1e4f);
         }
 #pragma unroll
         for (int ds = 0; ds < DS; ++ds) to[ds] = *(const u32x4*)(qrow + 16 * ds);
@@ -244,10 +248,10 @@ void monarch_step1_kernel(MonarchArgs p) {
 
     Tile cur = decode(t0 + grp), nxt = cur;
     bool stored = true;                                    // CS: this wave stored rows in the round before
-    if (!CS) fetch_query(cur, qn);
+    if (AH) fetch_query(cur, qn);
     stage(cur, 0);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (!CS) {                                             // landed: a wait in the loop counts the loop's operations only
+    if (AH) {                                              // landed: a wait in the loop counts the loop's operations only
 #pragma unroll
         for (int ds = 0; ds < DS; ++ds) asm volatile("" : "+v"(qn[ds]));
         if (IT) asm volatile("" : "+v"(wn));
@@ -266,7 +270,7 @@ void monarch_step1_kernel(MonarchArgs p) {
         const uint32_t srow = scratch_row(cur);
         if ((IT && p.iter_mode == 2) || query_key(cur) != qkey) {
             qkey = query_key(cur);
-            if (CS) {
+            if (!AH) {
                 fetch_query(cur, qb);
 #pragma unroll
                 for (int ds = 0; ds < DS; ++ds) asm volatile("" : "+v"(qb[ds]));      // waited for here, before the tile loads below
@@ -274,7 +278,7 @@ void monarch_step1_kernel(MonarchArgs p) {
 #pragma unroll
                 for (int ds = 0; ds < DS; ++ds) qb[ds] = qn[ds];
             }
-            if (IT) wsc = p.iter_mode == 2 ? fminf(1.0f / (wn + 1e-6f), 1e4f) : 1.0f / (1.0f + 1e-6f);
+            if (IT) wsc = p.iter_mode != 2 ? 1.0f / (1.0f + 1e-6f) : AH ? fminf(1.0f / (wn + 1e-6f), 1e4f) : wn;
             const int cg = min(wave * 32 + m, cur.ncols - 1);
             cloff = (uint32_t)(cur.a0 * b2 + cg) * p.cl_aj * 4;
 #pragma unroll
@@ -288,7 +292,7 @@ void monarch_step1_kernel(MonarchArgs p) {
             const int tn = t0 + grp + (r + 1) * G;
             nxt = decode(tn < t1 ? tn : t0 + grp + (mine - 1) * G);
             stage(nxt, (r + 1) & 1);
-            if (!CS && ((IT && p.iter_mode == 2) || query_key(nxt) != qkey)) fetch_query(nxt, qn);
+            if (AH && ((IT && p.iter_mode == 2) || query_key(nxt) != qkey)) fetch_query(nxt, qn);
         }
 
         if (CS) {
