@@ -1440,7 +1440,7 @@ static int enqueue_step1(const MonarchArgs& a, int nunits, hipStream_t stream, S
                                     : step1_kernel<E, D, 1>(a, kind);
     MonarchArgs a1 = a;
     a1.s1_total = a.nf * a.b1 * nunits * a.n_achunks;
-    // One workgroup per CU, of as many wave groups as its LDS holds up to 8 waves, or two of 5 or 6 (8 waves in all where one has
+    // One workgroup per CU, of as many wave groups as its LDS holds up to 8 waves, or two of 5 (or 6, below; 8 waves in all where one has
     // 256 registers): a group's loads, logits, softmax and stores follow each other, and the other groups fill the gaps.  A
     // group has the waves that its columns need and no more.  With at least four, the others of which formed and stored the last
     // column again and again, and never more than two groups, three refinement passes at three frames tied (52 columns, 12
@@ -1449,7 +1449,9 @@ static int enqueue_step1(const MonarchArgs& a, int nunits, hipStream_t stream, S
     // at 7 heads of nine 23 x 31 frames, two 44.5.  Two or four waves for 32 columns, each with its part of the output, took
     // the refinement to 505 and 541 us: they fetch the query rows as often.
     const int cus = a.s1_wgs > 0 ? a.s1_wgs : cu_count();
-    const int by_waves = nt > 2 ? 8 / nwaves : std::min(12 / nwaves, std::max(2, 8 / nwaves));      // within the launch bounds
+    // Two groups of six waves are worth it at head_dim 64 only (176 columns of 44 x 44, 12 heads: 161 us, one group 172; head_dim 128
+    // 304, 297; 192 columns of 30 x 64 240, 232).
+    const int by_waves = nt > 2 ? 8 / nwaves : nwaves == 6 && D == 128 ? 1 : std::min(12 / nwaves, std::max(2, 8 / nwaves));      // within the launch bounds
     const int room = std::min(by_waves, (int)(160 * 1024 / k.group));
     a1.s1_groups = std::max(1, std::min(room, (a1.s1_total + cus - 1) / cus));
     const int wgs = std::min(cus, (a1.s1_total + a1.s1_groups - 1) / a1.s1_groups);

@@ -193,6 +193,10 @@ def test_step_1_writes_the_new_chunk_to_the_cache(dtype, B, H, D, tiling, q_fram
     (128, 52, 1, 5, 3),         # two waves; Kbar alone with four groups, the last pass with two
     (64, 9, 3, 6, 2),
     (128, 70, 1, 4, 2),         # three key tiles: one group, two of Kbar alone at most
+    (128, 60, 3, 2, 1),         # six waves: one group
+    (64, 60, 3, 2, 1),          # and two
+    (128, 60, 3, 2, 2),
+    (64, 30, 6, 2, 1),
 ])
 def test_step_1_wave_groups(D, w, q_frames, H, num_iters):
     """More tiles than two wave groups of every compute unit take, few columns: every number of waves and of groups."""
