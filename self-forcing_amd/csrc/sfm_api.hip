@@ -377,8 +377,15 @@ static int monarch_fwd_impl(const sfm_monarch_desc* desc, const void* q, const v
     a.stats_ld = (uint32_t)((pl.b1 + 31) / 32 * 32);
     if (nc && nc->end > nc->start) {
         const int64_t blk = (int64_t)pl.b1 * pl.b2;
-        if ((pl.mfma || pl.iter_mfma) && !pl.fused && nc->start % blk == 0) {
-            // step 1 loads the chunk's tiles from it and writes the cache itself: no launch in front, the chunk read once
+        // Step 1 can load the chunk's tiles from it and write the cache itself: no launch in front, the chunk read once, but every
+        // tile of a kernel that can do it costs more (its state is spilled), and every new one most.  Where that is more than the
+        // launch saves, the write goes in front: 12 heads x 64 of 45 x 80 in 15 x 20 blocks, three frames against themselves
+        // (76 new tiles to a compute unit) 532 us in step 1, 511 in front; 6 x 128 of 30 x 10, 18 frames (13) 156, 151; 4 x 64,
+        // 30 x 52 in quarter-width blocks, 3 frames against 6, two passes (6) 142, 132.  Against 12 heads x 128 of 30 x 52, 3
+        // frames against themselves (4) 64, 74; 45 x 80, 9 (57) 0.98 of the time.
+        const int64_t new_tiles = (int64_t)pl.units * pl.b1 * ((nc->end - nc->start) / blk) * a.n_achunks;
+        const int most = pl.iter ? (pl.b2 > 32 && desc->D == 128 ? 5 : 1) : (pl.b2 > 32 ? 60 : 10);
+        if ((pl.mfma || pl.iter_mfma) && !pl.fused && nc->start % blk == 0 && new_tiles <= (int64_t)most * cu_count()) {
             a.new_kv = 1;
             a.new_f0 = (int)(nc->start / blk);
             a.new_f1 = (int)(nc->end / blk);

@@ -157,6 +157,13 @@ def test_kv_cache_op_tilings(f_tied, h_reduce, w_reduce):
     (1, 2, 128, (1, 1, 1, 5, 20), 3, 3, 6, 6, 3),        # refinement: K in the first pass, V in the last
     (2, 2, 64, (3, 2, 1, 4, 10), 3, 0, 3, 6, 2),
     (1, 1, 128, (1, 1, 1, 4, 70), 3, 1, 4, 4, 2),
+    # new tiles of the chunk (heads x block rows x block-frames) at the most that step 1 takes on 256 compute units, and past it
+    (1, 8, 64, (1, 1, 1, 32, 3), 1, 1, 11, 12, 1),
+    (1, 8, 64, (1, 1, 1, 32, 3), 1, 1, 12, 12, 1),
+    (1, 8, 128, (1, 1, 1, 32, 33), 1, 0, 5, 6, 2),
+    (1, 8, 128, (1, 1, 1, 32, 33), 1, 0, 6, 6, 2),
+    (1, 8, 64, (1, 1, 1, 32, 33), 1, 0, 1, 3, 2),
+    (1, 8, 64, (1, 1, 1, 32, 33), 1, 0, 2, 3, 2),
 ])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_step_1_writes_the_new_chunk_to_the_cache(dtype, B, H, D, tiling, q_frames, first, last, frames, num_iters):
