@@ -1585,7 +1585,15 @@ template <class E, int D>
 static bool launch_weights(const MonarchArgs& a, int nunits, hipStream_t stream, int* rc) {
     switch ((a.b1 + 31) / 32) {
         case 1: return launch_weights_t<E, D, 1, 1, 4>(a, nunits, stream, rc) || launch_weights_t<E, D, 1, 4, 8>(a, nunits, stream, rc);
-        case 2: return launch_weights_t<E, D, 2, 8, 4>(a, nunits, stream, rc);
+        case 2: {
+            // Eight waves that get a chunk or none leave compute units, which hold one such workgroup, idle: with many columns the two
+            // kernels are faster.  18 heads x 64 of 40 x 44, 6 frames (8 chunks, 2376 columns) 82 us, 29 + 39; two passes of 12 x
+            // 64 of 40 x 40, 3 frames (4 chunks, 1440) 103, 91; 36 x 128 of these (4320) 399, 391, 18 x 128 0.97 of the time of two
+            // kernels, 2 x 64 of 40 x 16 0.82.
+            const int chunks = (a.nf * a.b1 + 31) / 32, cols = nunits * a.na * a.b2;
+            if (chunks <= (D == 64 ? 8 : 5) && cols > (D == 64 ? 1 : 10) * cu_count()) return false;
+            return launch_weights_t<E, D, 2, 8, 4>(a, nunits, stream, rc);
+        }
         case 3: return launch_weights_t<E, D, 3, 8, 3>(a, nunits, stream, rc);
         default: return false;
     }

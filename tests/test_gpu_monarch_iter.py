@@ -83,6 +83,20 @@ def test_representatives_from_logits_in_registers(dtype, D, h, w, frames):
             assert ((out.float().cpu() - ref).norm() / ref.norm()).item() < 30 / 2 ** (9 if dtype == torch.bfloat16 else 12)
 
 
+@pytest.mark.parametrize("D,H,frames", [
+    (64, 6, 6), (64, 6, 7),           # 300 columns: 8 chunks of 32 rows (two kernels), 9 (one)
+    (64, 5, 1),                       # 250 columns: one
+    (128, 52, 4), (128, 52, 5),       # 2600 columns: 5 chunks (two), 7 (one)
+])
+def test_two_query_tiles_with_many_columns(D, H, frames):
+    h, w, dtype = 40, 50, torch.bfloat16
+    q = randn((1, h * w, H, D), 70, dtype)
+    k, v = (randn((1, frames * h * w, H, D), 71 + i, dtype) for i in range(2))
+    ref = monarch.monarch_attn(q, k, v, 1, 1, 1, h, w, num_iters=2, dtype=torch.float32)
+    out = mattn.monarch_attn(q.to(DEV), k.to(DEV), v.to(DEV), 1, 1, 1, h, w, num_iters=2)
+    assert_close_16bit(out, ref, dtype)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_16bit_inputs_and_cache_entry_point(dtype):
     """Cache holds 2 of 3 frames, the third arrives with the call; rows are in block order (h_reduce = 2)."""
