@@ -60,9 +60,11 @@ def test_mfma_path_small_shapes(dtype, B, H, D, a, f, b1, b2):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("H,b1", [(2, 30), (520, 30), (2, 45), (2, 90), (2, 128)])      # shared columns, a wave each, teams of 2, 3 and 4
 @pytest.mark.parametrize("grow", [0.2, 1.5, -1.5])
-def test_step_2_rescales_where_a_maximum_moves(H, b1, grow, dtype):
-    """Logits that grow slowly from chunk to chunk, that grow fast, and that fall, so that the first chunk's maxima stay.  One column per block: the right factor is 1 and Kbar, Y are the rows themselves, so that the logits are exact."""
-    f, D = 8, 128
+@pytest.mark.parametrize("D", [64, 128])
+def test_step_2_rescales_where_a_maximum_moves(D, H, b1, grow, dtype):
+    """Logits that grow slowly from chunk to chunk, that grow fast, and that fall, so that the first chunk's maxima stay.  One column
+    per block: the right factor is 1 and Kbar, Y are the rows themselves, so that the logits are exact."""
+    f = 8
     q = randn((1, b1, H, D), 40, dtype)
     k, v = (randn((1, f * b1, H, D), 41 + i, dtype) for i in range(2))
     scale = torch.linspace(1.0, 1.0 + abs(grow) * f, f * b1)

@@ -5,6 +5,8 @@ monarch_attn.py:1880-1957) at sizes the oracle finishes in seconds.
 Tolerances: fp32 tensors <= 2e-4 of the gradient's max-abs (fp32 kernels, sums of ~10^3 terms); 16-bit tensors the
 reference harness's own raw bar, atol = rtol = 1e-2 (bf16) / 1e-3 (fp16) on the unscaled gradients
 (monarch_attn.py:1908-1920)."""
+import ctypes as C
+
 import pytest
 import torch
 
@@ -156,8 +158,8 @@ def test_480p_block_shape_bf16_one_head(bwd_path):
 @pytest.mark.parametrize("h,w,Fq,Fk,D,causal,dtype", [
     (4, 52, 3, 3, 128, True, torch.bfloat16),      # 156 (a, j) columns: every fused kernel, last column block partial
     (4, 52, 3, 5, 64, False, torch.float16),
-    (4, 52, 4, 4, 64, True, torch.bfloat16),       # 208 columns: two passes of the right-factor kernel over each tile
-    (4, 52, 7, 7, 128, False, torch.float16),      # 364 columns: three passes
+    (4, 52, 4, 4, 64, True, torch.bfloat16),       # 208 columns: four chunks of the right-factor kernel, the last of 16
+    (4, 52, 7, 7, 128, False, torch.float16),      # 364: six, the last of 44
     (5, 6, 2, 3, 64, False, torch.bfloat16),       # b2 = 6, not a multiple of 4
     (4, 20, 3, 9, 128, False, torch.bfloat16),     # 36 rows (f, k) per column: two chunks of the left factor, the second with 4 rows
     (8, 12, 2, 8, 64, False, torch.float16),       # 64 rows: two full chunks
@@ -182,7 +184,7 @@ def test_16bit_gradients_across_the_fused_kernels_limits(h, w, Fq, Fk, D, causal
 
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("b2", [1, 2, 3, 5, 26, 31, 33, 39, 63])
-def test_block_columns_that_are_no_multiple_of_four(b2, D):
+def test_block_columns_that_are_no_multiple_of_four(b2, D, switches):
     """The rows of dS1 hold whole pieces of four: gradients at block widths between them, block-causal and not, on a scratch
     full of NaN, and from the fused chain, whose workspace is smaller than the library chain's."""
     h, F, H, dtype = 5, 4, 2, torch.bfloat16
@@ -193,6 +195,15 @@ def test_block_columns_that_are_no_multiple_of_four(b2, D):
         monarch.monarch_attn(qr, kr, vr, 1, 1, 1, h, b2, **kw).backward(do.double())
         qd, kd, vd = _leaf(q0, DEV), _leaf(k0, DEV), _leaf(v0, DEV)
         out = mattn.monarch_attn(qd, kd, vd, 1, 1, 1, h, b2, **kw)
+        need = {}
+        for mask in (sfa.lib.SW_BWD_RIGHT_GEMM, 0):
+            switches(mask)
+            bd, n = sfa.lib.MonarchBwdDesc(), C.c_size_t(0)
+            bd.fwd = mattn._desc(qd, kd, vd, out, 1, 1, 1, h, b2, D ** -0.5, 0, 2 if kw else 0)
+            bd.dq_stride, bd.dkv_stride, bd.kv_grad_frame_end = sfa.lib.strides3(qd), sfa.lib.strides3(kd), F
+            sfa.lib.check(sfa.lib.load().sfm_monarch_bwd_workspace_bytes(C.byref(bd), 0, C.byref(n)))
+            need[mask] = n.value
+        assert need[0] < need[sfa.lib.SW_BWD_RIGHT_GEMM]
         mattn.scratch(256 << 20, torch.device(DEV)).fill_(0xff)
         out.backward(do.to(DEV))
         _close(qd.grad, qr.grad, dtype)
@@ -322,13 +333,14 @@ def test_each_fused_part_can_fall_back_to_the_library_chain(switch, switches):
     _close(vd.grad, vr.grad, dtype)
 
 
-def test_480p_block_shape_new_frame_gradients_only():
-    """b1 = 30, b2 = 52, D = 128: one query frame against a cache of three frames whose last one arrives with the call;
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("frames", [1, 3])      # 52 columns, and 156: the chunks of 64 of a skipped block-frame follow each other
+def test_480p_block_shape_new_frame_gradients_only(frames, dtype):
+    """b1 = 30, b2 = 52, D = 128: one or three query frames against a cache of three frames whose last one arrives with the call;
     grad_only_new_kv, so that the right-factor kernel skips the gradient products of two of the three block-frames."""
     h, w, H, D = 30, 52, 1, 128
-    dtype = torch.bfloat16
     n = h * w
-    q0, do = (randn((1, n, H, D), 190 + i, dtype) for i in range(2))
+    q0, do = (randn((1, frames * n, H, D), 190 + i, dtype) for i in range(2))
     k_old, v_old = (randn((1, 2 * n, H, D), 192 + i, dtype) for i in range(2))
     k_new, v_new = (randn((1, n, H, D), 194 + i, dtype) for i in range(2))
     qr, kor, vor, knr, vnr = (_leaf(t.double()) for t in (q0, k_old, v_old, k_new, v_new))

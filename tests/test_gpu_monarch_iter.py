@@ -97,6 +97,31 @@ def test_two_query_tiles_with_many_columns(D, H, frames):
     assert_close_16bit(out, ref, dtype)
 
 
+@pytest.mark.parametrize("what", ["q", "v"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), -float("inf")])
+@pytest.mark.parametrize("D,h,w,F,n", [
+    (128, 30, 26, 6, 2), (64, 10, 20, 3, 3),      # one query tile: four waves per column, one
+    (64, 45, 12, 3, 2), (128, 45, 12, 6, 2),      # two
+    (128, 90, 8, 2, 2),                           # three
+    (64, 100, 4, 9, 2),                           # four: two kernels
+    (128, 30, 52, 3, 1), (64, 64, 6, 9, 1), (128, 128, 4, 9, 1),      # one pass: step 2 alone, its teams
+])
+def test_what_is_not_finite_stays_in_its_column(D, h, w, F, n, value, what):
+    """A query that is not finite takes its head's column of its block-frame with it (that block row's Kbar is part of all
+    rows' logits), a value its head's channel; nothing else."""
+    q, k, v = (randn((1, F * h * w, 2, D), 80 + i, torch.bfloat16) for i in range(3))
+    row = 5 * w + 3
+    {"q": q, "v": v}[what][0, row, 1, 7] = value
+    out = mattn.monarch_attn(q.to(DEV), k.to(DEV), v.to(DEV), 1, 1, 1, h, w, num_iters=n)
+    bad = torch.zeros(F, h, w, 2, D, dtype=torch.bool, device=DEV)
+    if what == "q":
+        bad[0, :, 3, 1] = True
+    else:
+        bad[..., 1, 7] = True
+    bad = bad.view_as(out)
+    assert torch.isfinite(out[~bad]).all() and not torch.isfinite(out[bad]).any()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_16bit_inputs_and_cache_entry_point(dtype):
     """Cache holds 2 of 3 frames, the third arrives with the call; rows are in block order (h_reduce = 2)."""
