@@ -574,7 +574,7 @@ void plan_rounds(int64_t units, int Sq, int Skv, int nkv, int D, Rounds* rq, Rou
     const double f = D == 64 ? 0.55 : 1.0;
     *rq = split_last_round((Sq + 127) / 128 * units, (Skv + 63) / 64, 2 * cu_count(), 2640 * f, 1500 * f, 128 * D);
     // (times of the dkv kernel before its pipeline, which takes 0.87 of them for a whole column but not where a workgroup has a few
-    // tiles; with its own, 1 head x 64, 1000 queries x 5000 keys was not split: 66.0 us against 61.4; 1 x 128, 2904 x 13459, its own
+    // tiles; with its own, 1 head x 64, 1000 queries x 5000 keys was not split: 71.0 us against 66.0; 1 x 128, 2904 x 13459, its own
     // keys' gradients, in 5 ranges for 8: 139 against 134)
     *rkv = split_last_round((nkv + 127) / 128 * units, (Sq + 63) / 64, cu_count(), 2550 * f, 2100 * f, 256 * D);
 }
