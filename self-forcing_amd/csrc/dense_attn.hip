@@ -10,7 +10,7 @@
 // tile (K and V rows in LDS, row-major, 16-byte chunks XOR-swizzled):
 //     S^T[l, q] = K[l,:] . Q[q,:]          online softmax per query column (lane)
 //     O^T[d, q] += V^T[d, l] P^T[l, q]     V^T comes from transposing LDS reads (ds_read_tr16_b64), P^T from the
-//                                          accumulator layout (perm_row)
+//                                          accumulator layout
 // Tiles go from global memory straight into LDS (global_load_lds_dwordx4), two K and two V buffers, one
 // barrier per tile.  A wave's matrix and vector work are interleaved in its instruction stream: the logits of
 // tile n + 1 are contracted while the exponentials of tile n are taken, and the maximum of tile n + 1 is reduced

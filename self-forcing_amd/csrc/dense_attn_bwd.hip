@@ -101,33 +101,6 @@ struct Tile {
     static constexpr int DS = D / 16, DT = D / 32, CPR = D / 8, kPitch = 2 * D, kBytes = 64 * kPitch;
 };
 
-// logits of the tile's rows 32 tl + 0..31 against the wave's own rows: A = tile rows, B = own rows (registers)
-template <class E, int D>
-__device__ __forceinline__ void tile_products(const char* ta, const char* tb, uint32_t a_off, const u32x4 (&oa)[D / 16],
-                                              const u32x4 (&ob)[D / 16], f32x16 (&s)[2], f32x16 (&d)[2]) {
-    using T = Tile<D>;
-#pragma unroll
-    for (int tl = 0; tl < 2; ++tl)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) s[tl][v] = d[tl][v] = 0.f;
-#pragma unroll
-    for (int ds = 0; ds < T::DS; ++ds)
-#pragma unroll
-        for (int tl = 0; tl < 2; ++tl) {
-            const u32x4 xa = *(const u32x4*)(ta + tl * 32 * T::kPitch + (a_off ^ (uint32_t)(ds << 5)));
-            const u32x4 xb = *(const u32x4*)(tb + tl * 32 * T::kPitch + (a_off ^ (uint32_t)(ds << 5)));
-            s[tl] = E::mfma32(xa, oa[ds], s[tl]);
-            d[tl] = E::mfma32(xb, ob[ds], d[tl]);
-        }
-}
-
-// 16 accumulator values (streamed rows 8 g + 4 hf + e of a 32-row half) -> the B operands of the two 16-row steps
-template <class E>
-__device__ __forceinline__ void pack_steps(const f32x16& x, u32x4& lo, u32x4& hi) {
-    lo.x = pack2<E>(x[0], x[1]); lo.y = pack2<E>(x[2], x[3]); lo.z = pack2<E>(x[4], x[5]); lo.w = pack2<E>(x[6], x[7]);
-    hi.x = pack2<E>(x[8], x[9]); hi.y = pack2<E>(x[10], x[11]); hi.z = pack2<E>(x[12], x[13]); hi.w = pack2<E>(x[14], x[15]);
-}
-
 // A operand [m = head-dim 32 dt + lane % 32, k = the 16 rows of step st in accumulator order] of a tile, transposed
 template <int D>
 __device__ __forceinline__ u32x4 tile_tr(const char* tile, uint32_t tr_lo, uint32_t tr_hi, int st) {
@@ -543,9 +516,10 @@ __global__ __launch_bounds__(256) void dense_bwd_sum_kernel(DenseBwdArgs p) {
 // The rounds of a grid of `items` workgroups over `tiles` streamed tiles each, of which the chip holds `slots` at once.  The
 // last, partly filled round (1320 key blocks on 256 compute units: 40 blocks in a sixth round) is split into ranges where a
 // model of its time in ns says that saves a tenth: a tile takes `tile_ns` with the chip full, `half_ns` on half of the slots
-// or fewer; the sum's launch 5000, and the partials (`floats` each) are written and read at 3.5 TB/s.  Measured:
+// or fewer; the sum's launch 5000, and the partials (`floats` each) are written and read at 3.5 TB/s.  Measured,
+// with the dkv kernel before its pipeline:
 //     heads x queries x keys, us    before  now           heads x queries x keys, new keys' gradients only    before  now
-//     12 x 4680 x 14040 (dkv)         1132   925           9 x 1000 x 5000                                       154   94
+//     12 x 4680 x 14040 (dkv)         1132  1028           9 x 1000 x 5000                                       154   94
 //     1 x 500 x 16000                  365    64           21 x 202 x 2804                                        84   46
 //     1 x 4000 x 500                   153    46           3 x 4680 x 4680                                       267  177
 Rounds split_last_round(int64_t items, int tiles, int slots, double tile_ns, double half_ns, int floats) {

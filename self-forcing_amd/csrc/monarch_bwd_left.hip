@@ -224,7 +224,7 @@ void monarch_bwd_left_kernel(LeftArgs p) {
     };
     const uint32_t b_off = (uint32_t)m * kPitch + (uint32_t)((hf ^ bl_swz<CPR>(m)) << 4);     // row m of a tile as an operand
     // transposing reads of a tile: lane (m, hf) gets, for head-dim column 32 dt + m, rows 16 ks + 4 hf + {0..3} and + 8 +
-    // {0..3}, the order in which the packed accumulators hold them (two reads, see perm_row); for dt: tr[dt & 1] ^ (dt / 2) 128
+    // {0..3}, the order in which the packed accumulators hold them (two reads); for dt: tr[dt & 1] ^ (dt / 2) 128
     uint32_t tr[2][2], trx;
     {
         const int s16 = lane & 15, g16 = lane >> 4;

@@ -488,6 +488,8 @@ __global__ __launch_bounds__(1024) void monarch_bwd_dqk_kernel(DqkArgs p) {
 
 }  // namespace
 
+// The kernel takes the columns 64 at a time and has no need of a limit; 480 is as far as the fused right factor has been run and
+// compared, and the dQ kernel below, without which it would gain little, ends at 512.
 bool monarch_bwd_right_supported(int dtype, int D, int b2, int AJ) {
     return (dtype == SFM_BF16 || dtype == SFM_F16) && (D == 64 || D == 128) && b2 >= 1 && b2 <= 64 && AJ <= 480;
 }

@@ -10,7 +10,7 @@
 //          S^T[l,(a,j)] = K[f,k,l,:] . Q[a,k,j,:]           (MFMA, wave = 32 (a,j) columns)
 //          R = softmax_l(s S)       cl = sum_l R log2 R      (registers + one cross-half shuffle)
 //          Kbar^T = K^T R^T,  Y^T = V^T R^T                  (MFMA; R^T is fed straight from the
-//                                                             accumulator layout, see perm_row)
+//                                                             accumulator layout)
 //      rows Kbar[a,j,(f,k),:], Y[a,j,(f,k),:] go to the workspace straight from the accumulators: one
 //      v_permlane32_swap per dword pair leaves 8 consecutive head-dim elements per lane (16-byte stores).
 //
@@ -466,8 +466,9 @@ __device__ __forceinline__ void wait_vm() {
 //       this form 299 and 70.  Two query tiles in one wave need 290 registers and spill.)
 // A chunk is a chain, barrier to barrier: with the full exp2f and a row mask in every chunk a team's chunk took 1.2 us however
 // few columns there were, now 1.0 (2 heads x 30 columns of 1332 rows 50 -> 42 us).  Teams of three and four have three
-// waves per SIMD (168 registers), so that the 624 columns of 12 heads with three frames tied are one round: 69 -> 60 us,
-// head_dim 64 46 -> 31; a team of two gains nothing from a third wave.  A third chunk pair in LDS: 72.
+// waves per SIMD (168 registers, of which a team of three at head_dim 128 spills three), so that the 624 columns of 12 heads with
+// three frames tied are one round: 69 -> 60 us, head_dim 64 46 -> 31; a team of two gains nothing from a third wave (head_dim
+// 128).  A third chunk pair in LDS: 72.
 // SHARE (TEAM = 1): 2 or 4 (p.s2_split) waves of a workgroup share a column's rows, 32-row chunks dealt in turn, and merge
 // (maximum, sum, output) through LDS at the end: with few (a, j) columns the chip is otherwise idle and a wave's chain of
 // dependent chunks (about 2.5 us each) is the whole time.  A kernel of its own: with the number of waves an argument of one

@@ -93,9 +93,8 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // Orders a wave's own LDS writes before its later LDS reads (wave-private staging buffers).
 __device__ __forceinline__ void lds_wave_sync() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
-// Row of the 16x16-dword-permuted contraction index used when a D tile (rows = contraction
-// index) is fed back as a B operand: element e of lane-half hf in 16-wide step s.
-__device__ __forceinline__ int perm_row(int s, int hf, int e) { return 16 * s + 4 * hf + (e < 4 ? e : e + 4); }
+// A D tile (rows = contraction index) that is fed back as a B operand holds, as element e of lane-half hf in 16-wide step s, row
+// 16 s + 4 hf + {0, 1, 2, 3, 8, 9, 10, 11}[e]: the accumulator order, which the A operand beside it is read in.
 
 // ---------------------------------------------------------------------------------------------
 // Token index of a Monarch block coordinate (block-frame bf, block row i, block col 0).
