@@ -79,9 +79,10 @@ def write_traffic(fetch_csv, write_csv):
     mean = lambda v: sum(v) / len(v)
 
     def pick(table, key):
-        """(name, mean) of the instantiation of `key` with the most dispatches (the forward's own: the backward leg
-        launches a statistics-keeping instantiation a few times)."""
-        name = max((k for k in table if key + "<" in k), key=lambda k: len(table[k]))
+        """(name, mean) of the instantiation of `key` that the timed forward runs: without a new chunk, a refinement's pass or
+        the backward's matrices, each of which is a template flag; of several the one with the most dispatches."""
+        names = [k for k in table if key + "<" in k]
+        name = max([k for k in names if "true" not in k.split("(")[0]] or names, key=lambda k: len(table[k]))
         return name, mean(table[name])
 
     def copy_factor(table):
