@@ -354,8 +354,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     // Halves of 32 queries follow each other in a pipeline.  Step H of it, H = 2 t + tl, is the gradient products of half H - 1 and the
     // logits and dP of half H + 1, with the softmax backward of half H spread over all of their MFMAs: a wave alone on its SIMD
     // issues nothing else while it waits, and with the softmax beside every second run of MFMAs only, the other runs
-    // left the vector unit idle and these the matrix pipe: 12 heads x 4680 queries x 14040 keys took 1061 us where this takes 925
-    // (873 TFLOP/s; the clock is down to 1.95 GHz).  Two waves per SIMD, each with half of the head dim's sums, that hand
+    // left the vector unit idle and these the matrix pipe: 12 heads x 4680 queries x 14040 keys took 1061 us where this takes 915
+    // (882 TFLOP/s; the clock is down to 1.95 GHz).  Two waves per SIMD, each with half of the head dim's sums, that hand
     // their P and dS to each other through LDS: 1020.
     constexpr int NO = 4 * T::DT, NA = 2 * T::DS, NS = NO + NA;         // MFMAs of a half's gradients, of its logits, of a step
     constexpr int kAhead = 4, kRing = 8;                    // A operands are read this many MFMAs ahead, over the end of a step too
