@@ -161,6 +161,9 @@ def test_480p_block_shape_bf16_one_head(bwd_path):
     (4, 52, 4, 4, 64, True, torch.bfloat16),       # 208 columns: four chunks of the right-factor kernel, the last of 16
     (4, 52, 7, 7, 128, False, torch.float16),      # 364: six, the last of 44
     (5, 6, 2, 3, 64, False, torch.bfloat16),       # b2 = 6, not a multiple of 4
+    (2, 32, 15, 2, 128, False, torch.bfloat16),    # 480 columns, the most of the fused right factor
+    (2, 37, 13, 2, 64, False, torch.bfloat16),     # 481: the library chain
+    (2, 19, 27, 27, 128, True, torch.float16),     # 513, block-causal
     (4, 20, 3, 9, 128, False, torch.bfloat16),     # 36 rows (f, k) per column: two chunks of the left factor, the second with 4 rows
     (8, 12, 2, 8, 64, False, torch.float16),       # 64 rows: two full chunks
     (6, 10, 6, 6, 128, True, torch.bfloat16),      # block-causal with two chunks: the visible rows end inside a chunk
