@@ -92,6 +92,15 @@ int sfm_monarch_stats_bytes(const sfm_monarch_desc* desc, size_t* bytes);
 int sfm_monarch_fwd_stats(const sfm_monarch_desc* desc, const void* q, const void* k, const void* v, void* out, float* stats,
                           void* workspace, size_t workspace_bytes, void* stream);
 
+/* Forward that leaves its intermediates (Kbar, Y, the right factor and its entropy term) for the backward as well, which then does
+ * not run step 1 again.  They are in `kept`, sfm_monarch_kept_bytes of it (0: the backward of this descriptor would not take
+ * them, or they pass 2 GiB; then use sfm_monarch_fwd_stats), which is also the call's scratch; hand `kept`, untouched, to
+ * sfm_monarch_bwd_kept together with `stats` and `out`.  No counterpart in the reference, whose backward forms them again
+ * (monarch_attn.py:1326-1470). */
+int sfm_monarch_kept_bytes(const sfm_monarch_desc* desc, size_t* bytes);
+int sfm_monarch_fwd_kept(const sfm_monarch_desc* desc, const void* q, const void* k, const void* v, void* out, float* stats,
+                         void* kept, size_t kept_size, void* stream);
+
 /* Measurement variant of sfm_monarch_fwd: brackets the two kernels of every pass with hipEvents recorded on
  * `stream`, WAITS for them, and returns the summed kernel durations in milliseconds.  No counterpart in the
  * reference (its pipeline times whole chunks with torch.cuda.Event, pipeline/causal_inference.py:105-115). */
@@ -136,6 +145,15 @@ int sfm_monarch_bwd_saved(const sfm_monarch_bwd_desc* desc, const void* q, const
                           const float* stats, const void* dout, float* dq, void* dk, void* dv, void* workspace,
                           size_t workspace_bytes, void* stream);
 
+/* sfm_monarch_bwd_saved with what sfm_monarch_fwd_kept (or sfm_monarch_attn_with_kv_cache_kept) left, on the same forward
+ * descriptor; same results.  `kept` is only read.  SFM_ERR_UNSUPPORTED where sfm_monarch_kept_bytes is 0 or the gradients'
+ * rows are not 16-byte aligned.  Less workspace than sfm_monarch_bwd_kept_workspace_bytes, down to one (batch, head) unit's
+ * share, means more passes. */
+int sfm_monarch_bwd_kept_workspace_bytes(const sfm_monarch_bwd_desc* desc, size_t* bytes);
+int sfm_monarch_bwd_kept(const sfm_monarch_bwd_desc* desc, const void* q, const void* k, const void* v, const void* out,
+                         const float* stats, const void* kept, size_t kept_size, const void* dout, float* dq, void* dk, void* dv,
+                         void* workspace, size_t workspace_bytes, void* stream);
+
 /* Writes new_k/new_v [B, n_new, H, D] (token order) into k_cache/v_cache[:, start_idx:end_idx]
  * in Monarch block order.  Replaces monarch_attn.py:1784-1785 + 1230-1231.
  * strides: new_stride for new_k and new_v, cache_stride for both caches. */
@@ -158,6 +176,12 @@ int sfm_monarch_attn_with_kv_cache_stats(const sfm_monarch_desc* desc, const voi
                                          const void* new_k, const void* new_v, const int64_t new_stride[3],
                                          int64_t start_idx, int64_t end_idx, void* out, float* stats,
                                          void* workspace, size_t workspace_bytes, void* stream);
+
+/* The same, leaving the intermediates in `kept` (see sfm_monarch_fwd_kept), which is the scratch too. */
+int sfm_monarch_attn_with_kv_cache_kept(const sfm_monarch_desc* desc, const void* q, void* k_cache, void* v_cache,
+                                        const void* new_k, const void* new_v, const int64_t new_stride[3],
+                                        int64_t start_idx, int64_t end_idx, void* out, float* stats, void* kept,
+                                        size_t kept_size, void* stream);
 
 /* sfm_monarch_attn_with_kv_cache for callers that cannot allocate or hand over a workspace (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  The scratch is a

@@ -412,6 +412,8 @@ struct Parts {
     bool dqa;      // 8: the left factor's kernel forms its dQ too (with `dqk` in the caller's rows, to which the right factor's is added)
     bool right;    // 9, the right factor's softmax backward, 11-13 and the scatter of dk / dv in one kernel per tile t
     bool dqk;      // 10 in a kernel that reads K where the caller has it (with `right`: no gathered copy of K is needed)
+    bool fk() const { return dqa && right; }   // Kbar, Y and c are kept as the forward has them: a column's rows are consecutive
+    bool all() const { return left && fwd && dqa && right && dqk; }
 };
 
 Parts make_parts(const MonarchArgs& p, int dtype, const int64_t* dks) {
@@ -433,8 +435,9 @@ Parts make_parts(const MonarchArgs& p, int dtype, const int64_t* dks) {
     return f;
 }
 
-Layout make_layout(const MonarchArgs& p, int n, size_t e, const Parts& f) {
-    const size_t AJ = (size_t)p.na * p.b2, RR = (size_t)p.nf * p.b1, D = p.D;
+// With `kept` the forward's Kbar, Y, c and R are at hand.
+Layout make_layout(const MonarchArgs& p, int n, size_t e, const Parts& f, bool kept) {
+    const size_t AJ = (size_t)p.na * p.b2, RR = (size_t)p.nf * p.b1, D = p.D, RP = f.fk() ? p.r_pad : RR;
     const size_t MQ = (size_t)p.b1 * AJ, MK = (size_t)p.b1 * p.nf * p.b2, NL = (size_t)p.nf * p.b2;
     Layout l;
     size_t o = 0;
@@ -446,13 +449,13 @@ Layout make_layout(const MonarchArgs& p, int n, size_t e, const Parts& f) {
     l.Vk = take(!f.right, n * MK * D * e);
     l.S1f = take(!f.fwd, n * p.b1 * AJ * NL * 4);
     l.dRb = take(!f.right, n * p.b1 * AJ * NL * 4);
-    l.Rb = take(true, n * p.b1 * AJ * p.nf * (size_t)(p.b2 > 64 ? p.b2 : 64) * e);      // row pitch 64 when step 1 of the forward writes it
+    l.Rb = take(!kept, n * p.b1 * AJ * p.nf * (size_t)(p.b2 > 64 ? p.b2 : 64) * e);      // row pitch 64 when step 1 of the forward writes it
     l.dS1 = take(true, n * p.b1 * AJ * p.nf * (size_t)(f.right ? (p.b2 + 3) / 4 * 4 : p.b2) * e);
-    l.Kbar = take(true, n * AJ * RR * D * e);
-    l.Y = take(true, n * AJ * RR * D * e);
+    l.Kbar = take(!kept, n * AJ * RP * D * e);
+    l.Y = take(!kept, n * AJ * RP * D * e);
     l.dKbar = take(true, n * AJ * RR * D * e);
     l.dY = take(true, n * AJ * RR * D * e);
-    l.c = take(true, n * AJ * RR * 4);
+    l.c = take(!kept, n * AJ * RP * 4);
     l.dc = take(true, n * AJ * RR * 4);
     l.S2f = take(!f.left, n * AJ * p.b1 * RR * 4);
     l.dLmf = take(!f.left, n * AJ * p.b1 * RR * 4);
@@ -507,7 +510,7 @@ int run(const MonarchBwdArgs& g, int n, void* workspace, hipStream_t stream) {
     const MonarchArgs& p = g.p;
     const size_t e = sizeof(T);
     const Parts parts = make_parts(p, left_dtype<E>() >= 0 ? left_dtype<E>() : SFM_F32, g.dks);
-    const Layout lay = make_layout(p, n, e, parts);
+    const Layout lay = make_layout(p, n, e, parts, g.kept);
     char* ws = (char*)workspace;
     Ctx cx{nullptr, ws, 0, stream};                      // the rocBLAS handle is made by the first product that needs it
     const int b1 = p.b1, b2 = p.b2, nf = p.nf, na = p.na, D = p.D, H = p.H;
@@ -518,7 +521,7 @@ int run(const MonarchBwdArgs& g, int n, void* workspace, hipStream_t stream) {
 
     const int64_t nseg = (int64_t)n * b1 * AJ * nf;
     const bool fused_left = parts.left, fused_fwd = parts.fwd, fused_dqa = parts.dqa, fused_right = parts.right;
-    const bool skip = p.causal && parts.left && parts.fwd && parts.dqa && parts.right && parts.dqk;     // masked pairs are left out
+    const bool skip = p.causal && parts.all();           // masked pairs are left out
     const bool dq_direct = parts.dqa && parts.dqk;       // both parts of dq go to the caller's rows
     const int ds2_ld = fused_left ? (RR + 7) / 8 * 8 : RR;
     const int rb_ld = fused_fwd ? 64 : b2;
@@ -563,20 +566,30 @@ int run(const MonarchBwdArgs& g, int n, void* workspace, hipStream_t stream) {
     const Op dKbar_t{lay.dKbar, D, (int64_t)AJ * D}, dY_t{lay.dY, D, (int64_t)AJ * D};
 
     const Op Rb_t{lay.Rb, rb_ld, (int64_t)AJ * rb_ld};
-    if (fused_fwd) {
+    const bool fk = parts.fk();
+    const char* const kbar = g.kept ? (const char*)p.kbar : ws + lay.Kbar;
+    const char* const yy = g.kept ? (const char*)p.y : ws + lay.Y;
+    const float* const cc = g.kept ? p.cl : (const float*)(ws + lay.c);
+    const char* const rb = g.kept ? (const char*)p.rb : ws + lay.Rb;
+    if (g.kept) {
+        // step 1 ran in the forward
+    } else if (fused_fwd) {
         MonarchArgs f1 = p;
         f1.kbar = ws + lay.Kbar;
         f1.y = ws + lay.Y;
         f1.cl = (float*)(ws + lay.c);
         f1.rb = ws + lay.Rb;
         f1.skip_masked = skip;
-        f1.ws_unit = (uint32_t)((int64_t)RR * AJ);
-        f1.ws_aj = 1;
-        f1.ws_row = (uint32_t)(nf * AJ);
-        f1.ws_f = (uint32_t)AJ;
-        f1.cl_unit = f1.ws_unit;         // c sits where its scratch row does: [row][(a, j)]
-        f1.cl_aj = 1;
-        f1.cl_row = 1;
+        monarch_rb_tiles(&f1);
+        if (!fk) {                           // tile after tile, as the library products want them; else the forward's own arrangement
+            f1.ws_unit = (uint32_t)((int64_t)RR * AJ);
+            f1.ws_aj = 1;
+            f1.ws_row = (uint32_t)(nf * AJ);
+            f1.ws_f = (uint32_t)AJ;
+            f1.cl_unit = f1.ws_unit;         // c sits where its scratch row does: [row][(a, j)]
+            f1.cl_aj = 1;
+            f1.cl_row = 1;
+        }
         if (!cx.status) cx.status = launch_monarch_step1(f1, left_dtype<E>(), n, stream);
     } else {
         // 1. S1 = Qk Kk^T per (u, k)
@@ -591,8 +604,7 @@ int run(const MonarchBwdArgs& g, int n, void* workspace, hipStream_t stream) {
         // 4-7 in one kernel: statistics and gradients of the left factor without the [i x r] matrices in memory
         if (!cx.status)
             cx.status = launch_monarch_bwd_left(left_dtype<E>(), D, n, b1, b2, AJ, nf, p.causal, s, p.q, p.qs, g.dout, saved ? g.fout : nullptr,
-                                                g.dos, p.qmap, H, p.unit0, ws + lay.Kbar, ws + lay.Y, (const float*)(ws + lay.c),
-                                                fused_fwd ? 1 : 0, ws + lay.dKbar, ws + lay.dY, (float*)(ws + lay.dc),
+                                                g.dos, p.qmap, H, p.unit0, kbar, yy, cc, fk ? p.r_pad : 0, fused_fwd ? 1 : 0, ws + lay.dKbar, ws + lay.dY, (float*)(ws + lay.dc),
                                                 fused_dqa ? nullptr : ws + lay.dS2, ds2_ld,
                                                 !fused_dqa  ? nullptr
                                                 : dq_direct ? g.dq
@@ -636,8 +648,8 @@ int run(const MonarchBwdArgs& g, int n, void* workspace, hipStream_t stream) {
     }
     if (fused_right) {
         if (!cx.status)
-            cx.status = launch_monarch_bwd_right(left_dtype<E>(), D, nt, b1, b2, AJ, nf, s, p.k, p.ks, p.v, p.vs, ws + lay.Rb,
-                                                 ws + lay.dKbar, ws + lay.dY, (const float*)(ws + lay.dc), p.q, p.qs, p.qmap, ws + lay.dS1, parts.dqk, g.dk,
+            cx.status = launch_monarch_bwd_right(left_dtype<E>(), D, nt, b1, b2, AJ, nf, s, p.k, p.ks, p.v, p.vs, rb,
+                                                 ws + lay.dKbar, ws + lay.dY, (const float*)(ws + lay.dc), fk, p.q, p.qs, p.qmap, ws + lay.dS1, parts.dqk, g.dk,
                                                  g.dv, g.dks, g.dk_row0, p.kmap, H, p.unit0, g.kv_f0, g.kv_f1, skip ? p.causal : 0, stream);
     } else {
         // 9. dR block = dKbar block . K block^T + dY block . V block^T per t
@@ -695,12 +707,11 @@ int run(const MonarchBwdArgs& g, int n, void* workspace, hipStream_t stream) {
 bool monarch_bwd_gemm_available() { return blas_load(); }
 
 bool monarch_bwd_all_fused(const MonarchArgs& p, int dtype, const int64_t* dkv_stride) {
-    const Parts f = make_parts(p, dtype, dkv_stride);
-    return f.left && f.fwd && f.dqa && f.right && f.dqk;
+    return make_parts(p, dtype, dkv_stride).all();
 }
 
-size_t monarch_bwd_gemm_bytes(const MonarchArgs& p, int dtype, int nunits, const int64_t* dkv_stride) {
-    return make_layout(p, nunits, dtype == SFM_F32 ? 4 : 2, make_parts(p, dtype, dkv_stride)).total;
+size_t monarch_bwd_gemm_bytes(const MonarchArgs& p, int dtype, int nunits, const int64_t* dkv_stride, bool kept) {
+    return make_layout(p, nunits, dtype == SFM_F32 ? 4 : 2, make_parts(p, dtype, dkv_stride), kept).total;
 }
 
 int launch_monarch_bwd_gemm(const MonarchBwdArgs& g, int dtype, int nunits, void* workspace, hipStream_t stream) {

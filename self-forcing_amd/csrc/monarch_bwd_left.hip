@@ -22,6 +22,10 @@
 //       32 query rows and hands them to the others through LDS, and the sums over i are split by head-dim blocks, so that
 //       every Kbar / Y row is read once and every dKbar / dY row written once.
 //
+// Kbar, Y and the entropy terms are read as the forward arranges them (a column's rows one after the other, (f, k) order) where
+// every later part is fused too, so that the forward's own can be handed over; dKbar and dY are written tile after tile, as the
+// right factor reads them.
+//
 // Bound by HBM: Kbar, Y read and dKbar, dY written once.  At 12 heads, a = 3, f = 21, b1 = 30, b2 = 52, 1.3 GB in 283 us,
 // where the kernel without dQ took 306 and a second one that read Kbar again for dQ 117.  With three frames tied (a = 3,
 // f = 3, b1 = 90, b2 = 52) 217 us, block-causal over single block-frames, where a third of the rows is left out, 183; a
@@ -45,13 +49,16 @@ struct LeftArgs {
     int64_t qs[3], os[3];
     TokMap qmap;
     int H;
-    const uint16_t* kbar;    // row r of (u, aj) at ((u * RR + r) * AJ + aj) * D
+    // A column's rows x are taken in the order of kbar: with r_pad > 0, the forward's arrangement, x = f * b1 + k at ((u * AJ + aj) *
+    // r_pad + x) * D; else x = r = k * nf + f at ((u * RR + r) * AJ + aj) * D
+    const uint16_t* kbar;
     const uint16_t* y;
-    const float* c;          // c_rows == 0: [u][aj][RR], natural log units; c_rows == 1: [(u * RR + r) * AJ + aj], log2 units
-    int c_rows;
-    uint16_t* dkbar;         // like kbar
+    int r_pad;
+    const float* c;          // r_pad > 0: [u][r_pad][AJ], log2 units; else c_rows == 0: [u][aj][RR], natural log units; c_rows == 1:
+    int c_rows;              // [(u * RR + r) * AJ + aj], log2 units
+    uint16_t* dkbar;         // row r = k * nf + f of (u, aj) at ((u * RR + r) * AJ + aj) * D
     uint16_t* dy;
-    float* dc;               // [u][aj][RR]
+    float* dc;               // [u][aj][RR], in the order of kbar's rows
     uint16_t* ds2;           // optional: [u][aj][b1][ds2_ld], ds2_ld >= RR
     int ds2_ld;
     float* dq;               // optional: s sum_r dS2 Kbar, in the query's rows with strides dqs (dq_rows), else [u][aj][i][D]
@@ -173,23 +180,32 @@ void monarch_bwd_left_kernel(LeftArgs p) {
     const int a_blk = aj / p.b2;
     const int flim = p.causal ? min(p.nf, (a_blk / p.causal + 1) * p.causal) : p.nf;      // visible kv block-frames
     const int64_t rstride = (int64_t)p.AJ * D;                                           // elements between rows r, r + 1
-    const char* const kbb = (const char*)(p.kbar + ((int64_t)u * RR * p.AJ + aj) * D);
-    const char* const ybb = (const char*)(p.y + ((int64_t)u * RR * p.AJ + aj) * D);
-    const char* const cpb = (const char*)(p.c_rows ? p.c + (int64_t)u * RR * p.AJ + aj : p.c + uaj * RR);
+    const bool fk = p.r_pad > 0;                          // uniform: Kbar, Y and c are the forward's
+    const int64_t kbar0 = (fk ? uaj * p.r_pad : (int64_t)u * RR * p.AJ + aj) * D;
+    const char* const kbb = (const char*)(p.kbar + kbar0);
+    const char* const ybb = (const char*)(p.y + kbar0);
+    const char* const cpb = (const char*)(fk ? p.c + (int64_t)u * p.r_pad * p.AJ + aj : p.c_rows ? p.c + (int64_t)u * RR * p.AJ + aj : p.c + uaj * RR);
     const float cmul = p.c_rows ? 1.f : kLog2e;
     const float sc2 = p.scale * kLog2e;
-    // The rows of a column, in order: all of them, or (skip) those of its flim visible block-frames
+    // The rows of a column, in order: all of them, or (skip) those of its flim visible block-frames, which come first in the
+    // forward's arrangement
     const bool skip = p.skip && flim < p.nf;              // uniform
     const int RV = skip ? b1 * flim : RR;
     const int nch = (RV + 31) / 32;
-    auto row_of = [&](int x) { return skip ? x / flim * p.nf + x % flim : x; };
+    auto row_of = [&](int x) { return skip && !fk ? x / flim * p.nf + x % flim : x; };       // in Kbar, Y, c, dc
+    const float inv_b1 = 1.f / (float)b1;
+    auto grad_row = [&](int x) {                          // in dKbar, dY
+        if (!fk) return row_of(x);
+        const int f = (int)(((float)x + 0.5f) * inv_b1);  // x / b1, exact while x < 2^22
+        return (x - f * b1) * p.nf + f;
+    };
 
     // A chunk of 32 rows r goes from global memory into LDS (a row's 2 D bytes by consecutive lanes); there is one chunk
     // buffer.  A lone wave fills its operand registers from it and requests the next chunk at once; a team reads the operands
     // where they are used, and each wave requests its share of the next chunk when all of them are done with this one.
     char* const kt = base + L::kChunk;
     const uint32_t kt0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(size_t)(__attribute__((address_space(3))) char*)kt);
-    const uint32_t rsb = (uint32_t)(rstride * 2), csb = (uint32_t)((p.c_rows ? p.AJ : 1) * 4);
+    const uint32_t rsb = fk ? (uint32_t)kPitch : (uint32_t)(rstride * 2), csb = (uint32_t)((p.c_rows ? p.AJ : 1) * 4);
     auto piece_off = [&](int n, int g) {
         const int P = g * 64 + lane;
         const int r = P / CPR, c = (P % CPR) ^ bl_swz<CPR>(r);
@@ -298,7 +314,7 @@ void monarch_bwd_left_kernel(LeftArgs p) {
     };
     auto row_ok = [&](int n) {
         const int r = 32 * n + m;
-        return r < RV && (skip || (r % p.nf) < flim);
+        return r < RV && (skip || (fk ? r < b1 * flim : r % p.nf < flim));
     };
 
     float lse[16], delta[16];
@@ -447,7 +463,7 @@ void monarch_bwd_left_kernel(LeftArgs p) {
         for (int rb = 0; rb < 4; ++rb) {
             const int rr = 32 * n + (m & 7) + 8 * rb;
             row_in[rb] = rr < RV;
-            rowoff[rb] = (int64_t)row_of(min(rr, RV - 1)) * rstride + (4 * ((m >> 3) & 1) + 2 * ((m >> 4) & 1) + hf) * 8;
+            rowoff[rb] = (int64_t)grad_row(min(rr, RV - 1)) * rstride + (4 * ((m >> 3) & 1) + 2 * ((m >> 4) & 1) + hf) * 8;
         }
         auto half_rows = [&](int which, int dp) {
             const char* src = which == 0 ? dot_t : qt;
@@ -568,7 +584,7 @@ bool monarch_bwd_left_supported(int dtype, int D, int b1) {
 
 int launch_monarch_bwd_left(int dtype, int D, int n, int b1, int b2, int AJ, int nf, int causal, float scale, const void* q,
                             const int64_t* qs, const void* dout, const void* out, const int64_t* os, const TokMap& qmap, int H,
-                            int unit0, const void* kbar, const void* y, const float* c, int c_rows, void* dkbar, void* dy, float* dc,
+                            int unit0, const void* kbar, const void* y, const float* c, int r_pad, int c_rows, void* dkbar, void* dy, float* dc,
                             void* ds2, int ds2_ld, float* dq, const int64_t* dqs, const float* stats, int stats_ld, bool skip_masked,
                             hipStream_t stream) {
     LeftArgs a;
@@ -585,6 +601,7 @@ int launch_monarch_bwd_left(int dtype, int D, int n, int b1, int b2, int AJ, int
     a.H = H;
     a.stats = out ? stats : nullptr; a.stats_ld = stats_ld; a.unit0 = unit0;
     a.c_rows = c_rows;
+    a.r_pad = r_pad;
     a.kbar = (const uint16_t*)kbar; a.y = (const uint16_t*)y;
     a.c = c;
     a.dkbar = (uint16_t*)dkbar; a.dy = (uint16_t*)dy;

@@ -39,7 +39,8 @@ struct RightArgs {
     const char* rb;          // [t][AJ][64]
     const char* dkbar;       // [t][AJ][D]
     const char* dy;
-    const float* dc;         // [u][AJ][RR]
+    const float* dc;         // [u][AJ][RR], (k, f) of a column at k * dc_k + f * dc_f
+    int dc_k, dc_f;
     const char* q;           // caller's tensor: row (a, j) of (unit, k) is token qmap.row(a, k) + j, strides qs0, qs1, qs2
     int64_t qs0, qs1, qs2;
     TokMap qmap;
@@ -195,7 +196,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
         const uint32_t b_off = (uint32_t)col * kPitch + (uint32_t)((hf ^ br_swz<CPR>(m)) << 4);
         for (int c0 = cfirst; c0 < AJ; c0 += kCols) {
             const int nrows = min(kCols, AJ - c0);
-            const float dcv = col < nrows ? p.dc[(u * AJ + c0 + col) * ((int64_t)nf * p.b1) + (int64_t)k * nf + f] : 0.f;
+            const float dcv = col < nrows ? p.dc[(u * AJ + c0 + col) * ((int64_t)nf * p.b1) + (int64_t)k * p.dc_k + f * p.dc_f] : 0.f;
             loaded(nrows);
             // dR^T[l, aj] = K dKbar^T + V dY^T, then R (16 bit) of the l this lane holds: l = 32 tl + 8 g + 4 hf + 0..3
             f32x16 dr;
@@ -495,8 +496,8 @@ bool monarch_bwd_right_supported(int dtype, int D, int b2, int AJ) {
 }
 
 int launch_monarch_bwd_right(int dtype, int D, int64_t ntiles, int b1, int b2, int AJ, int nf, float scale, const void* kk,
-                             const int64_t* ks, const void* v, const int64_t* vs, const void* rb, const void* dkbar, const void* dy, const float* dc, const void* q,
-                             const int64_t* qs, const TokMap& qmap, void* ds1, bool ds1_tiles, void* dk, void* dv, const int64_t* dks, int64_t row0,
+                             const int64_t* ks, const void* v, const int64_t* vs, const void* rb, const void* dkbar, const void* dy, const float* dc,
+                             bool dc_fk, const void* q, const int64_t* qs, const TokMap& qmap, void* ds1, bool ds1_tiles, void* dk, void* dv, const int64_t* dks, int64_t row0,
                              const TokMap& kmap, int H, int unit0, int f0, int f1, int skip_causal, hipStream_t stream) {
     if ((dks[0] | dks[1] | dks[2] | vs[0] | vs[1] | vs[2] | ks[0] | ks[1] | ks[2]) % 8 ||
         ((uintptr_t)dk | (uintptr_t)dv | (uintptr_t)v | (uintptr_t)kk) % 16 || (int64_t)(b2 - 1) * vs[1] * 2 + 2 * D > 0xffffffffll ||
@@ -510,6 +511,8 @@ int launch_monarch_bwd_right(int dtype, int D, int64_t ntiles, int b1, int b2, i
     a.ks0 = ks[0]; a.ks1 = ks[1]; a.ks2 = ks[2];
     a.dkbar = (const char*)dkbar; a.dy = (const char*)dy;
     a.dc = dc;
+    a.dc_k = dc_fk ? 1 : nf;
+    a.dc_f = dc_fk ? b1 : 1;
     a.q = (const char*)q; a.qs0 = qs[0]; a.qs1 = qs[1]; a.qs2 = qs[2];
     a.qmap = qmap;
     a.ds1 = (uint16_t*)ds1;

@@ -61,7 +61,7 @@ struct S1Lds {
 // NT: 32-row tiles of the key axis l (b2 <= 32 NT).  Up to two tiles a wave has 170 registers and a workgroup is several
 //     wave groups: two of 5 waves at 156 columns.  Three and four tiles (b2 up to 128: the 720p and
 //     1080p grids) have 256 registers for up to 8 waves, and their tile buffers take 96 / 128 KB of LDS.
-// WR: also write the right factor R (16 bit, 64 values per scratch row) to p.rb; the backward uses it.
+// WR: also write the right factor R (16 bit, 64 values per row) to p.rb; the backward uses it.
 // IT: a pass of the iterated refinement (wan/modules/monarch_attn.py:1716-1722): the logits are scaled per (a, f, k, j)
 //     column and, after the first pass, the query operand of tile (f, k) is the column's representative p.rep[a, j, (f, k)]
 //     instead of Q[a, k, j]; the operand is then fetched for every tile.
@@ -353,7 +353,8 @@ void monarch_step1_kernel(MonarchArgs p) {
             if (WR) {
                 // R[l] for l = 16 st + 0..15: the lower half of the wave holds 0..3 and 8..11, the upper half 4..7 and
                 // 12..15; exchanging the lower half's second pair with the upper half's first leaves 8 consecutive values
-                char* rrow = (char*)p.rb + ((size_t)srow + cloff / 4) * 128 + 16 * hf;
+                const size_t r0 = (size_t)cur.ul * p.rb_unit + (uint32_t)cur.k * p.rb_k + (uint32_t)cur.f * p.rb_f;
+                char* rrow = (char*)p.rb + (r0 + cloff / 4) * 128 + 16 * hf;
 #pragma unroll
                 for (int st = 0; st < 2 * NT; ++st) {
                     auto rx = __builtin_amdgcn_permlane32_swap(pb[st].x, pb[st].z, false, false);
@@ -1413,6 +1414,9 @@ static Step1Kernel step1_kernel(const MonarchArgs& a, Step1 kind) {
                 S1Lds<D, NT, true>::kGroup};
     if (kind == Step1::kIter)
         return {a.new_kv ? (const void*)monarch_step1_kernel<E, D, NT, false, true, false, false, true> : (const void*)monarch_step1_kernel<E, D, NT, false, true>, whole};
+    if constexpr (NT <= 2) {
+        if (a.rb && a.new_kv) return {(const void*)monarch_step1_kernel<E, D, NT, true, false, false, false, true>, whole};
+    }
     if (a.new_kv) return {(const void*)monarch_step1_kernel<E, D, NT, false, false, false, false, true>, whole};
     const bool skip = a.causal && a.skip_masked;
     if constexpr (NT <= 2) {
@@ -1523,7 +1527,6 @@ template <class E, int D>
 static int launch_t(const MonarchArgs& a, int nunits, hipStream_t stream, const StepEvents* ev) {
     if (ev) (void)hipEventRecord(ev->ev[0], stream);
     MonarchArgs a0 = a;
-    a0.rb = nullptr;
     a0.skip_masked = 1;                                  // step 2 stops at a column's last visible row
     if (int rc = enqueue_step1<E, D>(a0, nunits, stream)) return rc;
     if (ev) (void)hipEventRecord(ev->ev[1], stream);

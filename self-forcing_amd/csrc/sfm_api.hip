@@ -341,6 +341,29 @@ static void init_args(const sfm_monarch_desc* desc, const MonarchPlan& pl, Monar
     a.s1_wgs = step1_wgs_override();            // tuning override: step-1 workgroups (default 0: one per CU)
 }
 
+// Bytes of what a forward can leave for its backward (monarch_kept_layout), or 0 where the backward would not take it: it does
+// where all of its parts are fused kernels.  Larger calls than 2 GiB run in passes on both sides and keep nothing.
+// `dkv_stride`: of the gradients, NULL for rows that are 16-byte aligned.
+static size_t kept_bytes(const sfm_monarch_desc* desc, const MonarchPlan& pl, const int64_t* dkv_stride) {
+    static const int64_t aligned[3] = {8, 8, 8};
+    if (!pl.mfma || pl.iter || pl.fused || (switches() & SFM_SW_BWD_SIMT)) return 0;
+    MonarchArgs a;
+    init_args(desc, pl, &a);
+    if (!monarch_bwd_all_fused(a, desc->dtype, dkv_stride ? dkv_stride : aligned)) return 0;
+    const size_t total = monarch_kept_layout(a, pl.units).total;
+    return total <= (size_t)2 << 30 ? total : 0;
+}
+
+// points the scratch at what is kept for `units` units
+static void bind_kept(MonarchArgs* a, void* kept, int units) {
+    const KeptLayout l = monarch_kept_layout(*a, units);
+    a->kbar = (char*)kept + l.kbar;
+    a->y = (char*)kept + l.y;
+    a->cl = (float*)((char*)kept + l.cl);
+    a->rb = (char*)kept + l.rb;
+    monarch_rb_tiles(a);
+}
+
 // The new chunk of a KV-cache call: token-order rows for cache rows [start, end) in block order.
 struct NewChunk {
     const void *k, *v;
@@ -350,7 +373,7 @@ struct NewChunk {
 
 static int monarch_fwd_impl(const sfm_monarch_desc* desc, const void* q, const void* k, const void* v, void* out,
                             void* workspace, size_t workspace_bytes, void* stream, float* step_ms, float* stats = nullptr,
-                            const NewChunk* nc = nullptr) {
+                            const NewChunk* nc = nullptr, bool keep = false) {
     MonarchPlan pl;
     int rc = plan_monarch(desc, &pl);
     if (rc) return rc;
@@ -366,7 +389,17 @@ static int monarch_fwd_impl(const sfm_monarch_desc* desc, const void* q, const v
         set_error("q, k, v and out must be 16-byte aligned");
         return SFM_ERR_ALIGN;
     }
-    if (!workspace || (((uintptr_t)workspace) & 255) || workspace_bytes < pl.per_unit) {
+    if (keep) {
+        const size_t need = kept_bytes(desc, pl, nullptr);
+        if (!need) {
+            set_error("nothing can be kept for this descriptor's backward (see sfm_monarch_kept_bytes)");
+            return SFM_ERR_UNSUPPORTED;
+        }
+        if (!workspace || (((uintptr_t)workspace) & 255) || workspace_bytes < need) {
+            set_error("kept must be non-NULL, 256-byte aligned and hold %zu bytes", need);
+            return SFM_ERR_WORKSPACE;
+        }
+    } else if (!workspace || (((uintptr_t)workspace) & 255) || workspace_bytes < pl.per_unit) {
         set_error("workspace must be non-NULL, 256-byte aligned and hold at least %zu bytes (one unit)", pl.per_unit);
         return SFM_ERR_WORKSPACE;
     }
@@ -429,6 +462,10 @@ static int monarch_fwd_impl(const sfm_monarch_desc* desc, const void* q, const v
             if (rc) return rc;
         }
         return SFM_OK;
+    }
+    if (keep) {
+        bind_kept(&a, workspace, pl.units);
+        return launch_monarch_mfma(a, desc->dtype, pl.units, (hipStream_t)stream, nullptr);
     }
     size_t upp_sz = workspace_bytes / pl.per_unit;
     if (upp_sz * pl.per_unit > ((size_t)3 << 30)) upp_sz = ((size_t)3 << 30) / pl.per_unit;   // 32-bit offsets
@@ -521,6 +558,27 @@ int sfm_monarch_fwd_stats(const sfm_monarch_desc* desc, const void* q, const voi
     return monarch_fwd_impl(desc, q, k, v, out, workspace, workspace_bytes, stream, nullptr, stats);
 }
 
+int sfm_monarch_kept_bytes(const sfm_monarch_desc* desc, size_t* bytes) {
+    if (!bytes) {
+        set_error("bytes is NULL");
+        return SFM_ERR_NULL;
+    }
+    MonarchPlan pl;
+    int rc = plan_monarch(desc, &pl);
+    if (rc) return rc;
+    *bytes = kept_bytes(desc, pl, nullptr);
+    return SFM_OK;
+}
+
+int sfm_monarch_fwd_kept(const sfm_monarch_desc* desc, const void* q, const void* k, const void* v, void* out, float* stats,
+                         void* kept, size_t kept_size, void* stream) {
+    if (!stats) {
+        set_error("stats is NULL");
+        return SFM_ERR_NULL;
+    }
+    return monarch_fwd_impl(desc, q, k, v, out, kept, kept_size, stream, nullptr, stats, nullptr, true);
+}
+
 int sfm_monarch_fwd_timed(const sfm_monarch_desc* desc, const void* q, const void* k, const void* v, void* out,
                           void* workspace, size_t workspace_bytes, void* stream, float* step1_ms, float* step2_ms) {
     if (!step1_ms || !step2_ms) {
@@ -611,7 +669,7 @@ int sfm_monarch_bwd_workspace_bytes(const sfm_monarch_bwd_desc* desc, int32_t he
 
 static int monarch_bwd_impl(const sfm_monarch_bwd_desc* desc, const void* q, const void* k, const void* v, const void* out,
                             const float* stats, const void* dout, float* dq, void* dk, void* dv, void* workspace,
-                            size_t workspace_bytes, void* stream);
+                            size_t workspace_bytes, void* stream, const void* kept = nullptr);
 
 int sfm_monarch_bwd(const sfm_monarch_bwd_desc* desc, const void* q, const void* k, const void* v, const void* dout,
                     float* dq, void* dk, void* dv, void* workspace, size_t workspace_bytes, void* stream) {
@@ -632,9 +690,59 @@ int sfm_monarch_bwd_saved(const sfm_monarch_bwd_desc* desc, const void* q, const
     return monarch_bwd_impl(desc, q, k, v, out, stats, dout, dq, dk, dv, workspace, workspace_bytes, stream);
 }
 
+// Checks a descriptor of the kept variant and what it keeps; returns the plan and the bytes kept.
+static int plan_bwd_kept(const sfm_monarch_bwd_desc* desc, MonarchPlan* pl, size_t* kept) {
+    size_t per_unit = 0;
+    int rc = plan_bwd(desc, pl, &per_unit);
+    if (rc) return rc;
+    *kept = kept_bytes(&desc->fwd, *pl, desc->dkv_stride);
+    if (!*kept) {
+        set_error("nothing can be kept for this descriptor's backward (see sfm_monarch_kept_bytes)");
+        return SFM_ERR_UNSUPPORTED;
+    }
+    return SFM_OK;
+}
+
+int sfm_monarch_bwd_kept_workspace_bytes(const sfm_monarch_bwd_desc* desc, size_t* bytes) {
+    if (!bytes) {
+        set_error("bytes is NULL");
+        return SFM_ERR_NULL;
+    }
+    MonarchPlan pl;
+    size_t kept = 0;
+    int rc = plan_bwd_kept(desc, &pl, &kept);
+    if (rc) return rc;
+    MonarchArgs a;
+    init_args(&desc->fwd, pl, &a);
+    *bytes = monarch_bwd_gemm_bytes(a, desc->fwd.dtype, pl.units, desc->dkv_stride, true);
+    return SFM_OK;
+}
+
+int sfm_monarch_bwd_kept(const sfm_monarch_bwd_desc* desc, const void* q, const void* k, const void* v, const void* out,
+                         const float* stats, const void* kept, size_t kept_size, const void* dout, float* dq, void* dk, void* dv,
+                         void* workspace, size_t workspace_bytes, void* stream) {
+    if (!out || !stats || !kept) {
+        set_error("out, stats and kept must be non-NULL");
+        return SFM_ERR_NULL;
+    }
+    if (!aligned16(out) || (((uintptr_t)stats) & 3) || (((uintptr_t)kept) & 255)) {
+        set_error("out must be 16-byte aligned, stats 4-byte aligned, kept 256-byte aligned");
+        return SFM_ERR_ALIGN;
+    }
+    MonarchPlan pl;
+    size_t need = 0;
+    int rc = plan_bwd_kept(desc, &pl, &need);
+    if (rc) return rc;
+    if (kept_size < need) {
+        set_error("kept holds %zu bytes, the forward of this descriptor leaves %zu", kept_size, need);
+        return SFM_ERR_WORKSPACE;
+    }
+    return monarch_bwd_impl(desc, q, k, v, out, stats, dout, dq, dk, dv, workspace, workspace_bytes, stream, kept);
+}
+
 static int monarch_bwd_impl(const sfm_monarch_bwd_desc* desc, const void* q, const void* k, const void* v, const void* out,
                             const float* stats, const void* dout, float* dq, void* dk, void* dv, void* workspace,
-                            size_t workspace_bytes, void* stream) {
+                            size_t workspace_bytes, void* stream, const void* kept) {
     MonarchPlan pl;
     size_t per_unit = 0;
     int rc = plan_bwd(desc, &pl, &per_unit);
@@ -651,15 +759,16 @@ static int monarch_bwd_impl(const sfm_monarch_bwd_desc* desc, const void* q, con
         set_error("workspace must be non-NULL and 256-byte aligned");
         return SFM_ERR_WORKSPACE;
     }
-    if (bwd_uses_chain(desc, pl)) {
+    if (kept || bwd_uses_chain(desc, pl)) {
         MonarchBwdArgs g;
         memset(&g, 0, sizeof(g));
         init_args(&desc->fwd, pl, &g.p);
+        g.kept = kept != nullptr;
         int n = pl.units;
-        while (n > 1 && monarch_bwd_gemm_bytes(g.p, desc->fwd.dtype, n, desc->dkv_stride) > workspace_bytes) --n;
-        if (monarch_bwd_gemm_bytes(g.p, desc->fwd.dtype, n, desc->dkv_stride) > workspace_bytes) {
+        while (n > 1 && monarch_bwd_gemm_bytes(g.p, desc->fwd.dtype, n, desc->dkv_stride, g.kept) > workspace_bytes) --n;
+        if (monarch_bwd_gemm_bytes(g.p, desc->fwd.dtype, n, desc->dkv_stride, g.kept) > workspace_bytes) {
             set_error("workspace holds %zu bytes, one (batch, head) unit needs %zu", workspace_bytes,
-                      monarch_bwd_gemm_bytes(g.p, desc->fwd.dtype, 1, desc->dkv_stride));
+                      monarch_bwd_gemm_bytes(g.p, desc->fwd.dtype, 1, desc->dkv_stride, g.kept));
             return SFM_ERR_WORKSPACE;
         }
         g.p.q = q; g.p.k = k; g.p.v = v;
@@ -675,6 +784,14 @@ static int monarch_bwd_impl(const sfm_monarch_bwd_desc* desc, const void* q, con
         g.dk_row0 = (int64_t)g.kv_f0 * pl.b1 * pl.b2;
         for (int u0 = 0; u0 < pl.units; u0 += n) {
             g.p.unit0 = u0;
+            if (kept) {                    // this pass's units
+                bind_kept(&g.p, const_cast<void*>(kept), pl.units);
+                const size_t rows = (size_t)g.p.ws_unit * u0;
+                g.p.kbar = (char*)g.p.kbar + rows * desc->fwd.D * 2;
+                g.p.y = (char*)g.p.y + rows * desc->fwd.D * 2;
+                g.p.cl += (size_t)g.p.cl_unit * u0;
+                g.p.rb = (char*)g.p.rb + (size_t)g.p.rb_unit * u0 * 128;
+            }
             rc = launch_monarch_bwd_gemm(g, desc->fwd.dtype, pl.units - u0 < n ? pl.units - u0 : n, workspace, (hipStream_t)stream);
             if (rc) return rc;
         }
@@ -781,7 +898,7 @@ int sfm_kv_cache_write(int32_t dtype, int32_t B, int32_t H, int32_t D, const sfm
 // sfm_kv_cache_write takes it
 static int with_kv_cache_impl(const sfm_monarch_desc* desc, const void* q, void* k_cache, void* v_cache, const void* new_k,
                               const void* new_v, const int64_t new_stride[3], int64_t start_idx, int64_t end_idx, void* out,
-                              float* stats, void* workspace, size_t workspace_bytes, void* stream) {
+                              float* stats, void* workspace, size_t workspace_bytes, void* stream, bool keep = false) {
     MonarchPlan pl;
     int rc = plan_monarch(desc, &pl);
     if (rc) return rc;
@@ -813,15 +930,21 @@ static int with_kv_cache_impl(const sfm_monarch_desc* desc, const void* q, void*
         set_error("q, caches and out must be 16-byte aligned");
         return SFM_ERR_ALIGN;
     }
-    if (!workspace || (((uintptr_t)workspace) & 255) || workspace_bytes < pl.per_unit) {
-        set_error("workspace must be non-NULL, 256-byte aligned and hold at least %zu bytes (one unit)", pl.per_unit);
+    const size_t kept = keep ? kept_bytes(desc, pl, nullptr) : 0;
+    if (keep && !kept) {
+        set_error("nothing can be kept for this descriptor's backward (see sfm_monarch_kept_bytes)");
+        return SFM_ERR_UNSUPPORTED;
+    }
+    if (!workspace || (((uintptr_t)workspace) & 255) || workspace_bytes < (keep ? kept : pl.per_unit)) {
+        set_error("%s must be non-NULL, 256-byte aligned and hold at least %zu bytes%s", keep ? "kept" : "workspace",
+                  keep ? kept : pl.per_unit, keep ? "" : " (one unit)");
         return SFM_ERR_WORKSPACE;
     }
     rc = check_cache_write(desc->dtype, desc->B, desc->H, desc->D, &desc->tiling, new_k, new_v, new_stride, k_cache, v_cache,
                            desc->k_stride, desc->kv_tokens, start_idx, end_idx);
     if (rc) return rc;
     const NewChunk nc = {new_k, new_v, new_stride, start_idx, end_idx};
-    return monarch_fwd_impl(desc, q, k_cache, v_cache, out, workspace, workspace_bytes, stream, nullptr, stats, &nc);
+    return monarch_fwd_impl(desc, q, k_cache, v_cache, out, workspace, workspace_bytes, stream, nullptr, stats, &nc, keep);
 }
 
 int sfm_monarch_attn_with_kv_cache(const sfm_monarch_desc* desc, const void* q, void* k_cache, void* v_cache,
@@ -842,6 +965,18 @@ int sfm_monarch_attn_with_kv_cache_stats(const sfm_monarch_desc* desc, const voi
     }
     return with_kv_cache_impl(desc, q, k_cache, v_cache, new_k, new_v, new_stride, start_idx, end_idx, out, stats, workspace,
                               workspace_bytes, stream);
+}
+
+int sfm_monarch_attn_with_kv_cache_kept(const sfm_monarch_desc* desc, const void* q, void* k_cache, void* v_cache,
+                                        const void* new_k, const void* new_v, const int64_t new_stride[3],
+                                        int64_t start_idx, int64_t end_idx, void* out, float* stats, void* kept,
+                                        size_t kept_size, void* stream) {
+    if (!stats) {
+        set_error("stats is NULL");
+        return SFM_ERR_NULL;
+    }
+    return with_kv_cache_impl(desc, q, k_cache, v_cache, new_k, new_v, new_stride, start_idx, end_idx, out, stats, kept, kept_size,
+                              stream, true);
 }
 
 }  // extern "C"

@@ -158,7 +158,7 @@ struct MonarchArgs {
     // writes as whole cache lines (one float per (a, j)-major row is a partial write of a 32-byte sector each, and 1.2 M of
     // those per call cost step 1 7 % of its time); step 2 gathers its column with that stride, out of the L2.
     uint32_t cl_unit, cl_aj, cl_row;
-    void* rb;        // MFMA step 1 only, optional: the right factor R, 16 bit, 64 values per scratch row (same row index)
+    void* rb;        // MFMA step 1 only, optional: the right factor R, 16 bit, 64 values per row (row index: rb_unit below)
     float* stats;    // MFMA step 2 only, optional: log2-sum-exp of each query row's left-factor logits,
     uint32_t stats_ld;   // at ((b*H + h) * na*b2 + a*b2 + j) * stats_ld + i
     int unit0;       // first (b*H + h) unit of this pass
@@ -180,6 +180,8 @@ struct MonarchArgs {
     const void* new_k;
     const void* new_v;
     int64_t ns[3];
+    // MFMA step 1 only, with rb: R of (ul, a, j, k, f) is row ul*rb_unit + k*rb_k + f*rb_f + a*b2 + j, a tile's columns in a run
+    uint32_t rb_unit, rb_k, rb_f;
 };
 
 // Backward: the forward arguments (scratch matrices in float) plus the gradient tensors.
@@ -199,7 +201,32 @@ struct MonarchBwdArgs {
     int kv_f0, kv_f1;        // kv block-frames whose dK / dV are wanted
     const void* fout;        // optional, with fstats: the forward's output (layout of dout) and its row statistics
     const float* fstats;     // (MonarchArgs::stats of that forward, row pitch round_up(b1, 32))
+    // p.kbar, p.y, p.cl and p.rb are what the forward left for this pass's units (monarch_kept_layout): step 1 is not run again
+    bool kept;
 };
+
+// What a forward can leave for the backward: Kbar, Y and cl in the forward's arrangement and R in the backward's (a tile
+// (unit, k, f) after the other), each for `units` units.  Byte offsets, all of them multiples of 256.
+struct KeptLayout {
+    size_t kbar, y, cl, rb, total;
+};
+inline KeptLayout monarch_kept_layout(const MonarchArgs& p, int units) {
+    const size_t aj = (size_t)p.na * p.b2, rows = aj * p.r_pad, mat = (rows * p.D * 2 * units + 255) / 256 * 256;
+    KeptLayout l;
+    l.kbar = 0;
+    l.y = mat;
+    l.cl = 2 * mat;
+    l.rb = l.cl + (rows * sizeof(float) * units + 255) / 256 * 256;
+    l.total = l.rb + aj * p.nf * p.b1 * 128 * units;
+    return l;
+}
+// R's rows in the backward's arrangement
+inline void monarch_rb_tiles(MonarchArgs* p) {
+    const uint32_t aj = (uint32_t)(p->na * p->b2);
+    p->rb_f = aj;
+    p->rb_k = aj * p->nf;
+    p->rb_unit = aj * p->nf * p->b1;
+}
 
 // Optional timing hooks: ev[0] is recorded before step 1, ev[1] between the steps, ev[2] after step 2.
 struct StepEvents {
@@ -226,26 +253,30 @@ bool rocblas_disabled();           // SFM_NO_ROCBLAS was set at load
 int step1_wgs_override();          // SFM_S1_WGS at load, 0 = none
 // every part of the chain runs as a fused kernel for this problem: no library GEMM is called
 bool monarch_bwd_all_fused(const MonarchArgs& p, int dtype, const int64_t* dkv_stride);
-size_t monarch_bwd_gemm_bytes(const MonarchArgs& p, int dtype, int nunits, const int64_t* dkv_stride);
+size_t monarch_bwd_gemm_bytes(const MonarchArgs& p, int dtype, int nunits, const int64_t* dkv_stride, bool kept = false);
 int launch_monarch_bwd_gemm(const MonarchBwdArgs& g, int dtype, int nunits, void* workspace, hipStream_t stream);
-// step 1 of the MFMA forward alone, with the scratch strides of `a` and, if a.rb is set, the right factor written out
+// step 1 of the MFMA forward alone, with the scratch strides of `a` and, if a.rb is set, the right factor written out (also by
+// launch_monarch_mfma)
 int launch_monarch_step1(const MonarchArgs& a, int dtype, int nunits, hipStream_t stream);
 // fused left-factor part of the backward (monarch_bwd_left.hip): q, dout (and out, with stats) are the callers' tensors,
-// 16-byte aligned rows; everything else in the GEMM path's scratch layouts.  dS2 (for a library product) and its dQ = s dS2
-// Kbar are each optional; dQ goes to the caller's rows (dqs) or, with dqs NULL, to a float matrix [u][aj][i][D]
+// 16-byte aligned rows; everything else in the GEMM path's scratch layouts, but with r_pad > 0, when kbar, y and c (log2 units) are
+// in the forward's: [u][aj][r_pad] rows in the order (f, k), c [u][r_pad][aj], and dc follows that row order.  dS2 (for a
+// library product; not with r_pad) and its dQ = s dS2 Kbar are each optional; dQ goes to the caller's rows (dqs) or, with dqs
+// NULL, to a float matrix [u][aj][i][D]
 bool monarch_bwd_left_supported(int dtype, int D, int b1);
 int launch_monarch_bwd_left(int dtype, int D, int n, int b1, int b2, int AJ, int nf, int causal, float scale, const void* q,
                             const int64_t* qs, const void* dout, const void* out, const int64_t* os, const TokMap& qmap, int H,
-                            int unit0, const void* kbar, const void* y, const float* c, int c_rows, void* dkbar, void* dy, float* dc,
+                            int unit0, const void* kbar, const void* y, const float* c, int r_pad, int c_rows, void* dkbar, void* dy, float* dc,
                             void* ds2, int ds2_ld, float* dq, const int64_t* dqs, const float* stats, int stats_ld, bool skip_masked,
                             hipStream_t stream);
 // fused right-factor part of the backward (monarch_bwd_right.hip): per tile t = (unit, k, f) the dS1 block (scratch, for
 // dQ = s dS1 K; rows [f][(a, j)] per (unit, k) with ds1_tiles, as launch_monarch_bwd_dqk reads them, else [(a, j)][f]) and the
-// finished dK / dV rows of kv block-frames [f0, f1) in the caller's tensors; q, k and v are the caller's tensors too
+// finished dK / dV rows of kv block-frames [f0, f1) in the caller's tensors; q, k and v are the caller's tensors too.  A column's
+// dc is in the order (f, k) with dc_fk, else (k, f)
 bool monarch_bwd_right_supported(int dtype, int D, int b2, int AJ);
 int launch_monarch_bwd_right(int dtype, int D, int64_t ntiles, int b1, int b2, int AJ, int nf, float scale, const void* kk,
-                             const int64_t* ks, const void* v, const int64_t* vs, const void* rb, const void* dkbar, const void* dy, const float* dc, const void* q,
-                             const int64_t* qs, const TokMap& qmap, void* ds1, bool ds1_tiles, void* dk, void* dv, const int64_t* dks, int64_t row0,
+                             const int64_t* ks, const void* v, const int64_t* vs, const void* rb, const void* dkbar, const void* dy, const float* dc,
+                             bool dc_fk, const void* q, const int64_t* qs, const TokMap& qmap, void* ds1, bool ds1_tiles, void* dk, void* dv, const int64_t* dks, int64_t row0,
                              const TokMap& kmap, int H, int unit0, int f0, int f1, int skip_causal, hipStream_t stream);
 
 // With `skip_masked` / `skip_causal` (the block-causal size) the three parts neither read nor write the scratch rows of masked

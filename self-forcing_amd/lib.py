@@ -27,7 +27,9 @@ SYMBOLS = [
     "sfm_dense_workspace_bytes", "sfm_dense_fwd_ws", "sfm_full_attention_with_kv_cache_ws",
     "sfm_dense_fwd", "sfm_full_attention_with_kv_cache", "sfm_qk_prologue", "sfm_ln_modulate", "sfm_gate_residual",
     "sfm_rms_norm", "sfm_gate_residual_ln", "sfm_linear", "sfm_monarch_bwd_workspace_bytes", "sfm_monarch_bwd", "sfm_monarch_bwd_uses_gemm",
-    "sfm_monarch_stats_bytes", "sfm_monarch_fwd_stats", "sfm_monarch_bwd_saved", "sfm_dense_bwd_workspace_bytes", "sfm_dense_bwd", "sfm_probe_mfma_bf16", "sfm_probe_tile_traffic", "sfm_probe_row_stream", "sfm_probe_l2_read", "sfm_conv3d_cl", "sfm_vae_norm_act", "sfm_set_switches", "sfm_get_switches", "sfm_last_error", "sfm_version",
+    "sfm_monarch_stats_bytes", "sfm_monarch_fwd_stats", "sfm_monarch_bwd_saved",
+    "sfm_monarch_kept_bytes", "sfm_monarch_fwd_kept", "sfm_monarch_bwd_kept_workspace_bytes", "sfm_monarch_bwd_kept",
+    "sfm_monarch_attn_with_kv_cache_kept", "sfm_dense_bwd_workspace_bytes", "sfm_dense_bwd", "sfm_probe_mfma_bf16", "sfm_probe_tile_traffic", "sfm_probe_row_stream", "sfm_probe_l2_read", "sfm_conv3d_cl", "sfm_vae_norm_act", "sfm_set_switches", "sfm_get_switches", "sfm_last_error", "sfm_version",
 ]
 
 
@@ -115,6 +117,11 @@ def load():
     lib.sfm_monarch_stats_bytes.argtypes = [C.POINTER(MonarchDesc), C.POINTER(C.c_size_t)]
     lib.sfm_monarch_fwd_stats.argtypes = [C.POINTER(MonarchDesc), P, P, P, P, P, P, C.c_size_t, P]
     lib.sfm_monarch_bwd_saved.argtypes = [C.POINTER(MonarchBwdDesc), P, P, P, P, P, P, P, P, P, P, C.c_size_t, P]
+    lib.sfm_monarch_kept_bytes.argtypes = [C.POINTER(MonarchDesc), C.POINTER(C.c_size_t)]
+    lib.sfm_monarch_fwd_kept.argtypes = [C.POINTER(MonarchDesc), P, P, P, P, P, P, C.c_size_t, P]
+    lib.sfm_monarch_bwd_kept_workspace_bytes.argtypes = [C.POINTER(MonarchBwdDesc), C.POINTER(C.c_size_t)]
+    lib.sfm_monarch_bwd_kept.argtypes = [C.POINTER(MonarchBwdDesc), P, P, P, P, P, P, C.c_size_t, P, P, P, P, P, C.c_size_t, P]
+    lib.sfm_monarch_attn_with_kv_cache_kept.argtypes = [C.POINTER(MonarchDesc), P, P, P, P, P, S3, I64, I64, P, P, P, C.c_size_t, P]
     lib.sfm_kv_cache_write.argtypes = [C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.POINTER(Tiling), P, P, S3, P, P,
                                        S3, I64, I64, I64, P]
     lib.sfm_monarch_attn_with_kv_cache.argtypes = [C.POINTER(MonarchDesc), P, P, P, P, P, S3, I64, I64, P, P,

@@ -13,6 +13,8 @@ differentiable torch and has no backward kernels either).
 """
 import contextlib
 import ctypes as C
+import threading
+import weakref
 
 import torch
 
@@ -71,6 +73,48 @@ def scratch(nbytes, device):
 
 def release_scratch():
     _SCRATCH.clear()
+
+
+class _KeptBudget:
+    """What the forwards of one device hold for backwards to come: at most a sixteenth of its memory (18 GB), which is a pass of
+    30 layers of 12 heads at 480p; beyond that a forward leaves nothing and its backward forms the intermediates again.  A
+    buffer is counted from its allocation until autograd lets go of it."""
+
+    def __init__(self, device):
+        self.left = torch.cuda.get_device_properties(device).total_memory // 16
+        self.lock = threading.RLock()            # a buffer's finalizer may run inside take(), from the garbage collector
+
+    def take(self, nbytes, device):
+        with self.lock:
+            if nbytes > self.left:
+                return None
+            self.left -= nbytes
+        try:
+            buf = torch.empty(nbytes, dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError:
+            self.give(nbytes)
+            return None
+        weakref.finalize(buf, self.give, nbytes).atexit = False
+        return buf
+
+    def give(self, nbytes):
+        with self.lock:
+            self.left += nbytes
+
+
+_KEPT = {}
+_top_hooks = getattr(torch._C._autograd, "_top_saved_tensors_default_hooks", None)
+
+
+def _kept_buffer(nbytes, device):
+    """A buffer for the intermediates of a forward under autograd, or None.  None too while hooks on saved tensors are set (they
+    would move or keep a buffer 50 times the inputs: activation checkpointing, save_on_cpu)."""
+    if not nbytes or _top_hooks is None or _top_hooks(False) is not None:
+        return None
+    budget = _KEPT.get(device.index)
+    if budget is None:
+        budget = _KEPT.setdefault(device.index, _KeptBudget(device))
+    return budget.take(nbytes, device)
 
 
 def monarch_workspace_bytes(desc, heads_per_pass=0):
@@ -137,13 +181,28 @@ def _monarch_fwd_stats(q, k, v, tiling, sm_scale, kv_block_order, cbf, heads_per
     """Forward for autograd, with new = (new_k, new_v, start_idx, end_idx) of the KV-cache operator: returns (out, stats)
     where stats is the opaque row-statistics tensor that sfm_monarch_bwd_saved takes, or None when the forward that runs for
     these tensors produces none (the reference's forward keeps z and z_lse the same way, monarch_attn.py:1309-1317)."""
+    return _monarch_fwd_kept(q, k, v, tiling, sm_scale, kv_block_order, cbf, heads_per_pass, new, keep=False)[:2]
+
+
+def _monarch_fwd_kept(q, k, v, tiling, sm_scale, kv_block_order, cbf, heads_per_pass=0, new=None, keep=True):
+    """_monarch_fwd_stats that returns (out, stats, kept): kept is the scratch of a forward whose intermediates
+    sfm_monarch_bwd_kept takes, or None (a bound on the heads of a pass bounds the scratch, which is then not held).  Forward and
+    backward of 12 heads at 480p, three frames against 21 (766 MB kept): 1159 us with step 1 run again by the backward, 976 so; a
+    block-causal clip of nine frames, three tied, 620 and 534."""
     out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     d = _desc(q, k, v, out, *tiling, sm_scale, kv_block_order, cbf, 1)
     n = C.c_size_t(0)
     _l.check(_l.load().sfm_monarch_stats_bytes(C.byref(d), C.byref(n)))
-    nbytes = monarch_workspace_bytes(d, heads_per_pass)
-    ws = scratch(nbytes, q.device)
     stats = torch.empty(n.value // 4, dtype=torch.float32, device=q.device) if n.value else None
+    kept = None
+    if keep and stats is not None and not heads_per_pass:
+        _l.check(_l.load().sfm_monarch_kept_bytes(C.byref(d), C.byref(n)))
+        kept = _kept_buffer(n.value, q.device)
+    if kept is not None:
+        nbytes, ws = n.value, kept
+    else:
+        nbytes = monarch_workspace_bytes(d, heads_per_pass)
+        ws = scratch(nbytes, q.device)
     if new is not None and (stats is None or not _like_q(q, new[0])):
         kv_cache_write(*new[:2], k, v, *new[2:], *tiling)
         new = None
@@ -154,22 +213,24 @@ def _monarch_fwd_stats(q, k, v, tiling, sm_scale, kv_block_order, cbf, heads_per
                 new_k, new_v = new_k.contiguous(), new_v.contiguous()
             if k.stride() != v.stride():
                 raise ValueError("k_cache and v_cache must share their strides")
-            _l.check(_l.load().sfm_monarch_attn_with_kv_cache_stats(
+            fn = _l.load().sfm_monarch_attn_with_kv_cache_stats if kept is None else _l.load().sfm_monarch_attn_with_kv_cache_kept
+            _l.check(fn(
                 C.byref(d), q.data_ptr(), k.data_ptr(), v.data_ptr(), new_k.data_ptr(), new_v.data_ptr(), _l.strides3(new_k),
                 start_idx, end_idx, out.data_ptr(), stats.data_ptr(), ws.data_ptr(), nbytes, _stream(q)))
         elif stats is None:
             _l.check(_l.load().sfm_monarch_fwd(C.byref(d), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
                                                ws.data_ptr(), nbytes, _stream(q)))
         else:
-            _l.check(_l.load().sfm_monarch_fwd_stats(C.byref(d), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-                                                     stats.data_ptr(), ws.data_ptr(), nbytes, _stream(q)))
-    return out, stats
+            fn = _l.load().sfm_monarch_fwd_stats if kept is None else _l.load().sfm_monarch_fwd_kept
+            _l.check(fn(C.byref(d), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), stats.data_ptr(), ws.data_ptr(), nbytes,
+                        _stream(q)))
+    return out, stats, kept
 
 
 def _monarch_bwd(q, k, v, dout, tiling, sm_scale, kv_block_order, cbf, kv_f0=0, kv_f1=None, heads_per_pass=0, out=None,
-                 stats=None):
-    """Raw call of sfm_monarch_bwd (or sfm_monarch_bwd_saved when the forward's `out` and `stats` are given): returns
-    (dq float32, dk, dv); dk, dv cover kv block-frames [kv_f0, kv_f1) in the row order of k."""
+                 stats=None, kept=None):
+    """Raw call of sfm_monarch_bwd (or sfm_monarch_bwd_saved when the forward's `out` and `stats` are given, sfm_monarch_bwd_kept
+    when its `kept` is too): returns (dq float32, dk, dv); dk, dv cover kv block-frames [kv_f0, kv_f1) in the row order of k."""
     f_tied, h_reduce, w_reduce, h, w = tiling
     per_frame = f_tied * (h // h_reduce) * (w // w_reduce)
     nf = k.shape[1] // per_frame
@@ -188,10 +249,21 @@ def _monarch_bwd(q, k, v, dout, tiling, sm_scale, kv_block_order, cbf, kv_f0=0, 
     bd.dkv_stride = _l.strides3(dk)
     bd.kv_grad_frame_start, bd.kv_grad_frame_end = kv_f0, kv_f1
     n = C.c_size_t(0)
-    _l.check(_l.load().sfm_monarch_bwd_workspace_bytes(C.byref(bd), heads_per_pass, C.byref(n)))
+    if kept is not None:
+        _l.check(_l.load().sfm_monarch_kept_bytes(C.byref(bd.fwd), C.byref(n)))
+        if n.value != kept.numel():              # the implementation switches were changed since the forward
+            kept = None
+    if kept is not None:
+        _l.check(_l.load().sfm_monarch_bwd_kept_workspace_bytes(C.byref(bd), C.byref(n)))
+    else:
+        _l.check(_l.load().sfm_monarch_bwd_workspace_bytes(C.byref(bd), heads_per_pass, C.byref(n)))
     ws = scratch(n.value, q.device)
     with _on_device(q.device):
-        if out is None or stats is None:
+        if kept is not None:
+            _l.check(_l.load().sfm_monarch_bwd_kept(C.byref(bd), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+                                                    stats.data_ptr(), kept.data_ptr(), kept.numel(), dout.data_ptr(), dq.data_ptr(),
+                                                    dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), n.value, _stream(q)))
+        elif out is None or stats is None:
             _l.check(_l.load().sfm_monarch_bwd(C.byref(bd), q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(),
                                                dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), n.value,
                                                _stream(q)))
@@ -200,6 +272,14 @@ def _monarch_bwd(q, k, v, dout, tiling, sm_scale, kv_block_order, cbf, kv_f0=0, 
                                                      stats.data_ptr(), dout.data_ptr(), dq.data_ptr(), dk.data_ptr(),
                                                      dv.data_ptr(), ws.data_ptr(), n.value, _stream(q)))
     return dq, dk, dv
+
+
+_KEPT_NAMES = ("out", "stats", "kept")
+
+
+def _save(ctx, inputs, out, stats, kept):
+    """The forward's tensors for the backward: the inputs, then as many of _KEPT_NAMES as it left."""
+    ctx.save_for_backward(*inputs, *(() if stats is None else (out, stats) if kept is None else (out, stats, kept)))
 
 
 class _MonarchFn(torch.autograd.Function):
@@ -213,21 +293,16 @@ class _MonarchFn(torch.autograd.Function):
         _check4("v", v, q.dtype, q.device)
         if k.stride() != v.stride():
             k, v = k.contiguous(), v.contiguous()
-        out, stats = _monarch_fwd_stats(q, k, v, tiling, sm_scale, 1 if kv_block_order else 0, cbf, heads_per_pass)
-        ctx.has_stats = stats is not None
-        if stats is not None:
-            ctx.save_for_backward(q, k, v, out, stats)
-        else:
-            ctx.save_for_backward(q, k, v)
+        out, *kept = _monarch_fwd_kept(q, k, v, tiling, sm_scale, 1 if kv_block_order else 0, cbf, heads_per_pass)
+        _save(ctx, (q, k, v), out, *kept)
         ctx.cfg = (tiling, sm_scale, cbf, kv_block_order)
         return out
 
     @staticmethod
     def backward(ctx, dout):
         q, k, v, *kept = ctx.saved_tensors
-        out, stats = kept if ctx.has_stats else (None, None)
         tiling, sm_scale, cbf, kv_block_order = ctx.cfg
-        dq, dk, dv = _monarch_bwd(q, k, v, dout, tiling, sm_scale, 1 if kv_block_order else 0, cbf, out=out, stats=stats)
+        dq, dk, dv = _monarch_bwd(q, k, v, dout, tiling, sm_scale, 1 if kv_block_order else 0, cbf, **dict(zip(_KEPT_NAMES, kept)))
         return dq.to(q.dtype), dk, dv, None, None, None, None, None
 
 
@@ -246,30 +321,26 @@ class _MonarchCacheFn(torch.autograd.Function):
             raise ValueError("k/v shapes differ")
         if new_k.shape[1] != end_idx - start_idx:
             raise ValueError(f"new_k holds {new_k.shape[1]} tokens but end_idx - start_idx = {end_idx - start_idx}")
-        out, stats = _monarch_fwd_stats(q, k_cache, v_cache, tiling, sm_scale, 1, 0, heads_per_pass,
-                                        new=(new_k, new_v, start_idx, end_idx))
-        ctx.has_stats = stats is not None
-        if stats is not None:
-            ctx.save_for_backward(q, k_cache, v_cache, out, stats)
-        else:
-            ctx.save_for_backward(q, k_cache, v_cache)
+        out, *kept = _monarch_fwd_kept(q, k_cache, v_cache, tiling, sm_scale, 1, 0, heads_per_pass,
+                                       new=(new_k, new_v, start_idx, end_idx))
+        _save(ctx, (q, k_cache, v_cache), out, *kept)
         ctx.cfg = (start_idx, end_idx, tiling, sm_scale, grad_only_new_kv)
         return out
 
     @staticmethod
     def backward(ctx, dout):
         q, k_cache, v_cache, *kept = ctx.saved_tensors
-        out, stats = kept if ctx.has_stats else (None, None)
+        kept = dict(zip(_KEPT_NAMES, kept))
         start_idx, end_idx, tiling, sm_scale, grad_only_new_kv = ctx.cfg
         f_tied, h_reduce, w_reduce, h, w = tiling
         per_frame = f_tied * (h // h_reduce) * (w // w_reduce)
         if grad_only_new_kv:
             dq, dk, dv = _monarch_bwd(q, k_cache, v_cache, dout, tiling, sm_scale, 1, 0, start_idx // per_frame,
-                                      end_idx // per_frame, out=out, stats=stats)
+                                      end_idx // per_frame, **kept)
             dk_cache = dv_cache = None
             dk_new, dv_new = dk, dv
         else:
-            dq, dk_cache, dv_cache = _monarch_bwd(q, k_cache, v_cache, dout, tiling, sm_scale, 1, 0, out=out, stats=stats)
+            dq, dk_cache, dv_cache = _monarch_bwd(q, k_cache, v_cache, dout, tiling, sm_scale, 1, 0, **kept)
             dk_new, dv_new = dk_cache[:, start_idx:end_idx], dv_cache[:, start_idx:end_idx]
         dk_new = _from_block_order(dk_new, *tiling)
         dv_new = _from_block_order(dv_new, *tiling)

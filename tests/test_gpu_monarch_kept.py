@@ -1,0 +1,113 @@
+"""The forward that leaves its intermediates for the backward (sfm_monarch_fwd_kept, sfm_monarch_attn_with_kv_cache_kept,
+sfm_monarch_bwd_kept) against the chain that forms them again: the same kernels on the same numbers, so the same bits.  The
+autograd tests of the operators hold this path to the oracle."""
+import ctypes as C
+
+import pytest
+import torch
+
+import self_forcing_amd as sfa
+from gpu_util import randn
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+mattn, L = sfa.monarch_attn, sfa.lib
+
+
+# rows per column just below, at and above whole chunks of 32, one and two key tiles, one to three query tiles, head_dim 64 / 128
+@pytest.mark.parametrize("tiling,Fq,Fk,H,D,causal", [
+    ((1, 1, 1, 1, 5), 1, 1, 1, 64, 0), ((1, 1, 1, 4, 8), 2, 8, 3, 128, 0), ((1, 1, 1, 31, 1), 1, 1, 2, 64, 0),
+    ((1, 1, 1, 11, 52), 3, 3, 2, 128, 0), ((1, 1, 1, 30, 52), 3, 6, 2, 128, 0), ((1, 2, 1, 8, 33), 1, 4, 2, 64, 0),
+    ((3, 1, 2, 7, 64), 3, 6, 1, 128, 0), ((3, 1, 1, 13, 20), 3, 3, 2, 64, 0), ((1, 1, 1, 90, 8), 1, 2, 2, 128, 0),
+    ((1, 1, 1, 5, 20), 6, 6, 2, 128, 2), ((3, 1, 1, 12, 16), 6, 6, 2, 64, 1),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_kept_intermediates_give_the_bits_of_the_recomputed_ones(tiling, Fq, Fk, H, D, causal, dtype):
+    f_tied, hr, wr, h, w = tiling
+    q, do = (randn((2, Fq * h * w, H, D), 500 + i, dtype).to(DEV) for i in range(2))
+    k, v = (randn((2, Fk * h * w, H, D), 502 + i, dtype).to(DEV) for i in range(2))
+    sc = D ** -0.5
+    out, stats = mattn._monarch_fwd_stats(q, k, v, tiling, sc, 0, causal)
+    d = mattn._desc(q, k, v, out, *tiling, sc, 0, causal)
+    n = C.c_size_t(0)
+    L.check(L.load().sfm_monarch_kept_bytes(C.byref(d), C.byref(n)))
+    assert n.value > 0
+    kept = torch.full((n.value + 4096,), 0xAB, dtype=torch.uint8, device=DEV)
+    out2, stats2 = torch.empty_like(out), torch.empty_like(stats)
+    args = (C.byref(d), q.data_ptr(), k.data_ptr(), v.data_ptr(), out2.data_ptr(), stats2.data_ptr(), kept.data_ptr())
+    assert L.load().sfm_monarch_fwd_kept(*args, n.value - 1, None) == -6
+    L.check(L.load().sfm_monarch_fwd_kept(*args, n.value, mattn._stream(q)))
+    assert torch.equal(out, out2) and bool((kept[n.value:] == 0xAB).all())
+    want = mattn._monarch_bwd(q, k, v, do, tiling, sc, 0, causal, out=out, stats=stats)
+    before = kept.clone()
+    for _ in range(2):                                        # only read: a second backward finds the same
+        got = mattn._monarch_bwd(q, k, v, do, tiling, sc, 0, causal, out=out2, stats=stats2, kept=kept[:n.value])
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+    assert torch.equal(kept, before)
+
+
+@pytest.mark.parametrize("start", [0, 3])
+def test_kept_with_a_new_chunk_and_in_several_passes(start):
+    """The cache call keeps what a call on the written cache does; a backward with room for one unit runs in passes."""
+    h, w, H, D, dtype = 9, 24, 3, 128, torch.bfloat16
+    per, tiling, sc = h * w, (1, 1, 1, 9, 24), 128 ** -0.5
+    q, do, nk, nv = (randn((1, 3 * per, H, D), 510 + i, dtype).to(DEV) for i in range(4))
+    kc, vc = (randn((1, 6 * per, H, D), 514 + i, dtype).to(DEV) for i in range(2))
+    out, stats, kept = mattn._monarch_fwd_kept(q, kc, vc, tiling, sc, 1, 0, new=(nk, nv, start * per, (start + 3) * per))
+    assert kept is not None and torch.equal(kc[:, start * per:(start + 3) * per], nk)
+    want = mattn._monarch_bwd(q, kc, vc, do, tiling, sc, 1, 0, start, start + 3)
+    got = mattn._monarch_bwd(q, kc, vc, do, tiling, sc, 1, 0, start, start + 3, out=out, stats=stats, kept=kept)
+    for a, b in zip(got, want):                                # `want` sums the left factor's statistics itself
+        torch.testing.assert_close(a.float(), b.float(), atol=2e-2, rtol=2e-2)
+    bd = L.MonarchBwdDesc()
+    dq, dk, dv = (torch.empty_like(t) for t in got)
+    bd.fwd = mattn._desc(q, kc, vc, do, *tiling, sc, 1, 0)
+    bd.dq_stride, bd.dkv_stride = L.strides3(dq), L.strides3(dk)
+    bd.kv_grad_frame_start, bd.kv_grad_frame_end = start, start + 3
+    n = C.c_size_t(0)
+    L.check(L.load().sfm_monarch_bwd_kept_workspace_bytes(C.byref(bd), C.byref(n)))
+    ws = torch.empty(n.value // 2, dtype=torch.uint8, device=DEV)       # one or two of the three units
+    L.check(L.load().sfm_monarch_bwd_kept(C.byref(bd), q.data_ptr(), kc.data_ptr(), vc.data_ptr(), out.data_ptr(), stats.data_ptr(),
+                                          kept.data_ptr(), kept.numel(), do.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+                                          ws.data_ptr(), ws.numel(), mattn._stream(q)))
+    assert all(torch.equal(a, b) for a, b in zip((dq, dk, dv), got))
+
+
+def test_what_is_kept_is_bounded_and_given_back(monkeypatch):
+    h, w, H, D, dtype = 6, 20, 2, 64, torch.bfloat16
+    q, k, v, do = (randn((1, 3 * h * w, H, D), 520 + i, dtype).to(DEV) for i in range(4))
+    leaves = [t.requires_grad_(True) for t in (q, k, v)]
+
+    def forward():
+        return mattn.monarch_attn(q, k, v, 1, 1, 1, h, w)
+
+    forward()
+    budget = mattn._KEPT[torch.cuda.current_device()]
+    full = budget.left
+    out = forward()
+    size = full - budget.left
+    assert size > 0
+    want = torch.autograd.grad(out, leaves, do)
+    assert budget.left == full
+    out = forward()
+    del out
+    assert budget.left == full
+    # no room: the backward forms the intermediates again
+    monkeypatch.setattr(budget, "left", size - 1)
+    got = torch.autograd.grad(forward(), leaves, do)
+    assert budget.left == size - 1 and all(torch.equal(a, b) for a, b in zip(got, want))
+    monkeypatch.setattr(budget, "left", full)
+    # hooks on saved tensors see the small ones only
+    seen = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: seen.append(t.numel()) or t, lambda t: t):
+        got = torch.autograd.grad(forward(), leaves, do)
+    assert budget.left == full and max(seen) <= q.numel() and all(torch.equal(a, b) for a, b in zip(got, want))
+    # another implementation than the forward ran with
+    out = forward()
+    old = L.load().sfm_set_switches(L.SW_BWD_SIMT)
+    try:
+        got = torch.autograd.grad(out, leaves, do)
+    finally:
+        L.load().sfm_set_switches(old)
+    for a, b in zip(got, want):
+        torch.testing.assert_close(a.float(), b.float(), atol=1e-2, rtol=1e-2)
