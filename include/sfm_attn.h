@@ -146,12 +146,13 @@ int sfm_monarch_bwd_saved(const sfm_monarch_bwd_desc* desc, const void* q, const
                           size_t workspace_bytes, void* stream);
 
 /* sfm_monarch_bwd_saved with what sfm_monarch_fwd_kept (or sfm_monarch_attn_with_kv_cache_kept) left, on the same forward
- * descriptor; same results.  `kept` is only read.  SFM_ERR_UNSUPPORTED where sfm_monarch_kept_bytes is 0 or the gradients'
+ * descriptor; same results, but dq comes in the tensor dtype (the float32 sum rounded once), dq_stride in its elements.  `kept`
+ * is only read.  SFM_ERR_UNSUPPORTED where sfm_monarch_kept_bytes is 0 or the gradients'
  * rows are not 16-byte aligned.  Less workspace than sfm_monarch_bwd_kept_workspace_bytes, down to one (batch, head) unit's
  * share, means more passes. */
 int sfm_monarch_bwd_kept_workspace_bytes(const sfm_monarch_bwd_desc* desc, size_t* bytes);
 int sfm_monarch_bwd_kept(const sfm_monarch_bwd_desc* desc, const void* q, const void* k, const void* v, const void* out,
-                         const float* stats, const void* kept, size_t kept_size, const void* dout, float* dq, void* dk, void* dv,
+                         const float* stats, const void* kept, size_t kept_size, const void* dout, void* dq, void* dk, void* dv,
                          void* workspace, size_t workspace_bytes, void* stream);
 
 /* Writes new_k/new_v [B, n_new, H, D] (token order) into k_cache/v_cache[:, start_idx:end_idx]

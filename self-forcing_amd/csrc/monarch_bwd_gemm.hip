@@ -427,9 +427,9 @@ Parts make_parts(const MonarchArgs& p, int dtype, const int64_t* dks) {
     f.dqa = f.left && !(sw & SFM_SW_BWD_DQA_GEMM);
     const bool direct_ok = (dks[0] | dks[1] | dks[2] | p.vs[0] | p.vs[1] | p.vs[2] | p.ks[0] | p.ks[1] | p.ks[2]) % 8 == 0 &&      // 16-byte rows of k, v, dk, dv
                            (int64_t)p.nf * p.b1 * p.b2 * p.ks[1] * 2 < ((int64_t)1 << 32);
-    f.dqk = monarch_bwd_dqk_supported(dtype, p.D, p.b2, p.na * p.b2) && !(sw & SFM_SW_BWD_DQK_GEMM);
+    f.dqk = monarch_bwd_dqk_supported(dtype, p.D) && !(sw & SFM_SW_BWD_DQK_GEMM);
     // the rows of dS1 are padded to whole 8-byte pieces, which the library product of part 10 does not know
-    f.right = f.fwd && direct_ok && monarch_bwd_right_supported(dtype, p.D, p.b2, p.na * p.b2) && (f.dqk || p.b2 % 4 == 0) &&
+    f.right = f.fwd && direct_ok && monarch_bwd_right_supported(dtype, p.D, p.b2) && p.na * p.b2 <= 480 && (f.dqk || p.b2 % 4 == 0) &&
               !(sw & SFM_SW_BWD_RIGHT_GEMM);
     f.dqk = f.dqk && f.right;
     return f;
@@ -461,7 +461,7 @@ Layout make_layout(const MonarchArgs& p, int n, size_t e, const Parts& f, bool k
     l.dLmf = take(!f.left, n * AJ * p.b1 * RR * 4);
     l.L = take(!f.left, n * AJ * p.b1 * RR * e);
     l.dS2 = take(!f.dqa, n * AJ * p.b1 * ((RR + 7) / 8 * 8) * e);                         // rows padded to 8 for the fused kernels
-    l.dQa = take(!f.dqa || !f.dqk, n * MQ * D * 4);
+    l.dQa = take(!f.dqa || !f.dqk || kept, n * MQ * D * 4);
     l.dQk = take(!f.dqa || !f.dqk, n * MQ * D * 4);
     l.dKk = take(!f.right, n * MK * D * 4);
     l.dVk = take(!f.right, n * MK * D * 4);
@@ -522,7 +522,7 @@ int run(const MonarchBwdArgs& g, int n, void* workspace, hipStream_t stream) {
     const int64_t nseg = (int64_t)n * b1 * AJ * nf;
     const bool fused_left = parts.left, fused_fwd = parts.fwd, fused_dqa = parts.dqa, fused_right = parts.right;
     const bool skip = p.causal && parts.all();           // masked pairs are left out
-    const bool dq_direct = parts.dqa && parts.dqk;       // both parts of dq go to the caller's rows
+    const bool dq_direct = parts.dqa && parts.dqk && !g.dq16;      // both parts of dq go to the caller's rows
     const int ds2_ld = fused_left ? (RR + 7) / 8 * 8 : RR;
     const int rb_ld = fused_fwd ? 64 : b2;
     if (fused_right && ((uintptr_t)g.dk | (uintptr_t)g.dv | (uintptr_t)p.v) % 16) {
@@ -668,8 +668,8 @@ int run(const MonarchBwdArgs& g, int n, void* workspace, hipStream_t stream) {
     if (parts.dqk) {
         if (!cx.status)
             cx.status = launch_monarch_bwd_dqk(left_dtype<E>(), D, nuk, b1, b2, AJ, nf, s, p.k, p.ks, p.kmap, ws + lay.dS1,
-                                               dq_direct ? g.dq : (float*)(ws + lay.dQk), dq_direct ? g.dqs : nullptr, p.qmap, H,
-                                               p.unit0, skip ? p.causal : 0, stream);
+                                               dq_direct ? g.dq : (float*)(ws + (g.dq16 ? lay.dQa : lay.dQk)), g.dq16,
+                                               dq_direct || g.dq16 ? g.dqs : nullptr, p.qmap, H, p.unit0, skip ? p.causal : 0, stream);
     } else {
         gemm(cx, false, false, AJ, D, NL, s, 0.f, dS1_uk, Kk_uk, dQk_uk, tE, tF, nuk);
     }
@@ -684,7 +684,7 @@ int run(const MonarchBwdArgs& g, int n, void* workspace, hipStream_t stream) {
     // scatter the gradients back to the callers' layouts
     {
         const int64_t tq = (int64_t)n * MQ * (D / 4);
-        if (!dq_direct)
+        if (!dq_direct && !g.dq16)
             hipLaunchKernelGGL(scatter_dq, dim3((unsigned)((tq + 255) / 256)), dim3(256), 0, stream, (const float*)(ws + lay.dQa),
                                (const float*)(ws + lay.dQk), g.dq, g.dqs[0], g.dqs[1], g.dqs[2], p.qmap, na, H, D, p.unit0, tq);
         const int64_t tk = (int64_t)n * b1 * (g.kv_f1 - g.kv_f0) * b2 * (D / 4);

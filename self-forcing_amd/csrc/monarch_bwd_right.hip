@@ -338,29 +338,37 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
 
 
 // ---------------------------------------------------------------------------------------------------------------
-// dQ of the right factor: dQk[(u, k)][aj, :] = s sum_{f, l} dS1[(u, k)][aj, (f, l)] K[(f, k, l), :], float, added to the
-// caller's dq rows, where the left factor's part is, or written to a scratch matrix.  One workgroup per (unit, k), one
-// wave per 32 columns (a, j); the K rows of the nf block-frames stream through LDS 64 at a time straight from the
-// caller's tensor (global_load_lds_dwordx4, double buffered, chunk swizzle) and come back transposed as the B operand
-// [n = d, k = (f, l)]; the A operand is dS1 straight from memory, two 8-byte pieces per step in the order in which the
-// transposing reads deliver the rows.
+// dQ of the right factor: dQk[(u, k)][aj, :] = s sum_{f, l} dS1[(u, k)][aj, (f, l)] K[(f, k, l), :], float, added to the left
+// factor's part, in the caller's float rows or on the way to 16-bit ones, or written to a scratch matrix.  A workgroup
+// takes up to kDqkWaves x 32 columns (a, j) of a (unit, k), a wave 32; the K rows of the nf block-frames stream through LDS 64
+// at a time straight from the caller's tensor (global_load_lds_dwordx4, double buffered, chunk swizzle) and come back
+// transposed as the A operand [m = d, k = (f, l)]; the B operand is dS1 straight from memory, two 8-byte pieces per step in the
+// order in which the transposing reads deliver the rows, so that a lane ends up with four consecutive d of its column.
 struct DqkArgs {
     const char* k;           // caller's tensor: row kmap.row(f, k) + l, strides ks0 (batch), ks1 (row), ks2 (head), in elements
     int64_t ks0, ks1, ks2;
     TokMap kmap;
     const uint16_t* ds1;     // [(u, k)][f][AJ][b2p] as the kernel above writes it
     uint32_t b2p_inv;        // 2^32 / b2p, rounded up: x / b2p is the upper half of the product for every x below 2^26
-    float* dqk;              // [(u, k)][AJ][D], or the caller's rows to add to: token qmap.row(a, k) + j, strides dqs
+    float* dqk;              // [(u, k)][AJ][D], or (add) the caller's rows to add to: token qmap.row(a, k) + j, strides dqs
+    const float* part;       // with dq16: the left factor's part, [u][AJ][b1][D]
+    uint16_t* dq16;          // optional: 16-bit rows for the sum, like dqk's with add
     int64_t dqs0, dqs1, dqs2;
     TokMap qmap;
     bool add;
     int causal;              // block-causal size: dS1 beyond a column's visible block-frames is not there; 0 = none
     int b1, b2, AJ, nf, H, unit0;
+    int nchunks, total;      // column chunks of a (unit, k), workgroups with work
     float scale;
 };
 
+// A (unit, k) of 156 columns as one workgroup of five waves is 360 of them for 256 compute units at 12 heads, b1 = 30: with three
+// and two waves 84 -> 73 us (f = 21), and at three frames tied, block-causal (three tiles to a workgroup) 69 -> 61; five waves as
+// the kernel is now 79 and 64, two 98 and 64.  Bound by its loads' latency: a tile's K rows and dS1 pieces are one tile ahead.
+constexpr int kDqkWaves = 4;
+
 template <class E, int D>
-__global__ __launch_bounds__(1024) void monarch_bwd_dqk_kernel(DqkArgs p) {
+__global__ __launch_bounds__(64 * kDqkWaves) __attribute__((amdgpu_waves_per_eu(4, 4))) void monarch_bwd_dqk_kernel(DqkArgs p) {
     constexpr int DT = D / 32, CPR = D / 8;
     constexpr int kPitch = 2 * D;
     constexpr int kTile = 64 * kPitch;
@@ -370,12 +378,15 @@ __global__ __launch_bounds__(1024) void monarch_bwd_dqk_kernel(DqkArgs p) {
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, hf = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nwaves = __builtin_amdgcn_readfirstlane((int)blockDim.x >> 6);
-    const int64_t uk = blockIdx.x;
+    const int item = xcd_item(p.total);                                  // the chunks of a (unit, k) read the same K rows
+    if (item >= p.total) return;
+    const int64_t uk = item / p.nchunks;
+    const int col0 = (item % p.nchunks) * nwaves * 32;                   // this workgroup's first column
     const int k = (int)(uk % p.b1);
     const int unit = p.unit0 + (int)(uk / p.b1);
     const int b2 = p.b2, b2p = (b2 + 3) & ~3, AJ = p.AJ, NL = p.nf * b2p;
-    const int nt = (NL + 63) / 64;
     auto visible = [&](int aj) { return p.causal ? min(p.nf, (aj / b2 / p.causal + 1) * p.causal) * b2p : NL; };      // elements of dS1 row aj
+    const int nt = (visible(min(col0 + nwaves * 32, AJ) - 1) + 63) / 64;                       // tiles that the last column sees
 
     const char* kbase = p.k + ((int64_t)(unit / p.H) * p.ks0 + (int64_t)(unit % p.H) * p.ks2) * 2;
     const uint32_t krb = (uint32_t)(p.ks1 * 2);
@@ -386,17 +397,20 @@ __global__ __launch_bounds__(1024) void monarch_bwd_dqk_kernel(DqkArgs p) {
             const int P = g * 64 + lane;
             const int r = P / CPR, c = (P % CPR) ^ br_swz<CPR>(r);
             const int x = min(64 * t + r, NL - 1);
-            const uint32_t tok = (uint32_t)(p.kmap.row(x / b2p, k) + min(x % b2p, b2 - 1));
+            const int f = (int)__umulhi((uint32_t)x, p.b2p_inv);
+            const uint32_t tok = (uint32_t)(p.kmap.row(f, k) + min(x - f * b2p, b2 - 1));
             br_load_lds16(kbase, tok * krb + (uint32_t)(c * 16), lds0 + (uint32_t)(t & 1) * kTile + (uint32_t)g * 1024);
         }
     };
-    // dS1 pieces of row aj = 32 wave + m: x = 64 t + 16 ks + 4 hf + {0..3} and + 8 + {0..3}
-    const int aj = min(32 * wave + m, AJ - 1);
+    // dS1 pieces of row aj: x = 64 t + 16 ks + 4 hf + {0..3} and + 8 + {0..3}
+    const int aj0 = col0 + 32 * wave;
+    const int aj = min(aj0 + m, AJ - 1);
     const uint16_t* arow = p.ds1 + uk * AJ * (int64_t)NL + aj * b2p;
     const uint32_t fstep = (uint32_t)((AJ - 1) * b2p);                  // from a row's end in one block-frame to its start in the next
     auto piece = [&](int x) { return *(const u32x2*)(arow + (uint32_t)x + __umulhi((uint32_t)x, p.b2p_inv) * fstep); };
     const int na = visible(aj);
-    const int nwave = __builtin_amdgcn_readfirstlane(visible(min(32 * wave + 31, AJ - 1)));      // of the wave's longest row
+    // of the wave's longest row; a wave past the last column only fetches tiles
+    const int nwave = __builtin_amdgcn_readfirstlane(aj0 < AJ ? visible(min(aj0 + 31, AJ - 1)) : 0);
     auto load_a = [&](int t, u32x4 (&a)[4]) {
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
@@ -444,55 +458,56 @@ __global__ __launch_bounds__(1024) void monarch_bwd_dqk_kernel(DqkArgs p) {
                 for (int dt = 0; dt < DT; ++dt) {
                     const u32x2 lo = br_read_tr(tile, tr[dt][0] + ks * 16 * kPitch);
                     const u32x2 hi = br_read_tr(tile, tr[dt][1] + ks * 16 * kPitch);
-                    const u32x4 bop = {lo.x, lo.y, hi.x, hi.y};
-                    acc[dt] = E::mfma32(acur[ks], bop, acc[dt]);
+                    const u32x4 kop = {lo.x, lo.y, hi.x, hi.y};
+                    acc[dt] = E::mfma32(kop, acur[ks], acc[dt]);
                 }
         }
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) acur[ks] = anext[ks];
     }
-    // lane (d = 32 dt + m) holds rows aj = 32 wave + 8 g + 4 hf + e
-    if (!p.add) {
-        float* const out = p.dqk + uk * AJ * D;
+    // lane (m, hf) holds d = 32 dt + 8 g + 4 hf + 0..3 of column aj0 + m
+    if (aj0 + m >= AJ) return;
+    const int64_t tok = p.qmap.row(aj / b2, k) + aj % b2;
+    if (p.dq16) {
+        const float* const from = p.part + ((uk / p.b1 * AJ + aj) * p.b1 + k) * D + 4 * hf;
+        uint16_t* const to = p.dq16 + (int64_t)(unit / p.H) * p.dqs0 + (int64_t)(unit % p.H) * p.dqs2 + tok * p.dqs1 + 8 * hf;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const int row = 32 * wave + 8 * (v >> 2) + 4 * hf + (v & 3);
-            if (row < AJ) {
+        for (int dt = 0; dt < DT; ++dt) {
+            f32x4 x[4];
 #pragma unroll
-                for (int dt = 0; dt < DT; ++dt) out[(int64_t)row * D + 32 * dt + m] = acc[dt][v] * p.scale;
+            for (int g = 0; g < 4; ++g) x[g] = *(const f32x4*)(from + 32 * dt + 8 * g);
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[g][e] += acc[dt][4 * g + e] * p.scale;
+            // the half swap leaves 8 consecutive elements per lane (both halves of a column are here)
+#pragma unroll
+            for (int gp = 0; gp < 2; ++gp) {
+                const f32x4 y = x[2 * gp], z = x[2 * gp + 1];
+                auto rx = __builtin_amdgcn_permlane32_swap(pack2<E>(y.x, y.y), pack2<E>(z.x, z.y), false, false);
+                auto ry = __builtin_amdgcn_permlane32_swap(pack2<E>(y.z, y.w), pack2<E>(z.z, z.w), false, false);
+                *(u32x4*)(to + 32 * dt + 16 * gp) = u32x4{(uint32_t)rx[0], (uint32_t)ry[0], (uint32_t)rx[1], (uint32_t)ry[1]};
             }
         }
         return;
     }
-    // four rows at a time: their loads are all in flight before the first sum is stored (one row after the other took
-    // 107 us where this takes 85, at 12 heads, a = 3, f = 21, b1 = 30, b2 = 52)
-    float* const out = p.dqk + (int64_t)(unit / p.H) * p.dqs0 + (int64_t)(unit % p.H) * p.dqs2 + m;
+    float* const to = (p.add ? p.dqk + (int64_t)(unit / p.H) * p.dqs0 + (int64_t)(unit % p.H) * p.dqs2 + tok * p.dqs1 : p.dqk + (uk * AJ + aj) * D) + 4 * hf;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        float* to[4];
-        float x[4][DT];
+    for (int dt = 0; dt < DT; ++dt) {
+        f32x4 x[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int row = min(32 * wave + 8 * g + 4 * hf + e, AJ - 1);
-            to[e] = out + (p.qmap.row(row / b2, k) + row % b2) * p.dqs1;
+        for (int g = 0; g < 4; ++g) x[g] = p.add ? *(const f32x4*)(to + 32 * dt + 8 * g) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt) x[e][dt] = to[e][32 * dt];
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (32 * wave + 8 * g + 4 * hf + e < AJ) {
-#pragma unroll
-                for (int dt = 0; dt < DT; ++dt) to[e][32 * dt] = x[e][dt] + acc[dt][4 * g + e] * p.scale;
-            }
+        for (int g = 0; g < 4; ++g)
+            *(f32x4*)(to + 32 * dt + 8 * g) = f32x4{x[g].x + acc[dt][4 * g] * p.scale, x[g].y + acc[dt][4 * g + 1] * p.scale,
+                                                    x[g].z + acc[dt][4 * g + 2] * p.scale, x[g].w + acc[dt][4 * g + 3] * p.scale};
     }
 }
 
 }  // namespace
 
-// The kernel takes the columns 64 at a time and has no need of a limit; 480 is as far as the fused right factor has been run and
-// compared, and the dQ kernel below, without which it would gain little, ends at 512.
-bool monarch_bwd_right_supported(int dtype, int D, int b2, int AJ) {
-    return (dtype == SFM_BF16 || dtype == SFM_F16) && (D == 64 || D == 128) && b2 >= 1 && b2 <= 64 && AJ <= 480;
+bool monarch_bwd_right_supported(int dtype, int D, int b2) {
+    return (dtype == SFM_BF16 || dtype == SFM_F16) && (D == 64 || D == 128) && b2 >= 1 && b2 <= 64;
 }
 
 int launch_monarch_bwd_right(int dtype, int D, int64_t ntiles, int b1, int b2, int AJ, int nf, float scale, const void* kk,
@@ -552,14 +567,13 @@ int launch_monarch_bwd_right(int dtype, int D, int64_t ntiles, int b1, int b2, i
     return SFM_OK;
 }
 
-// at most 16 waves of 32 columns each
-bool monarch_bwd_dqk_supported(int dtype, int D, int b2, int AJ) {
-    return (dtype == SFM_BF16 || dtype == SFM_F16) && (D == 64 || D == 128) && AJ <= 512;
+bool monarch_bwd_dqk_supported(int dtype, int D) {
+    return (dtype == SFM_BF16 || dtype == SFM_F16) && (D == 64 || D == 128);
 }
 
 int launch_monarch_bwd_dqk(int dtype, int D, int64_t nuk, int b1, int b2, int AJ, int nf, float scale, const void* k, const int64_t* ks,
-                           const TokMap& kmap, const void* ds1, float* dqk, const int64_t* dqs, const TokMap& qmap, int H, int unit0,
-                           int skip_causal, hipStream_t stream) {
+                           const TokMap& kmap, const void* ds1, float* dqk, void* dq16, const int64_t* dqs, const TokMap& qmap, int H,
+                           int unit0, int skip_causal, hipStream_t stream) {
     if ((ks[0] | ks[1] | ks[2]) % 8 || ((uintptr_t)k) % 16 || (int64_t)nf * b1 * b2 * ks[1] * 2 > 0xffffffffll) {
         set_error("monarch backward (dQ of the right factor): k rows must be 16-byte aligned and a (batch, head) slice under 4 GiB");
         return SFM_ERR_STRIDE;
@@ -569,16 +583,21 @@ int launch_monarch_bwd_dqk(int dtype, int D, int64_t nuk, int b1, int b2, int AJ
     a.kmap = kmap;
     a.ds1 = (const uint16_t*)ds1;
     a.b2p_inv = (uint32_t)((((uint64_t)1 << 32) + (b2 + 3) / 4 * 4 - 1) / (uint64_t)((b2 + 3) / 4 * 4));
-    a.dqk = dqk;
+    a.dqk = dq16 ? nullptr : dqk;
+    a.part = dq16 ? dqk : nullptr;
+    a.dq16 = (uint16_t*)dq16;
     a.add = dqs != nullptr;
     a.causal = skip_causal;
     a.dqs0 = dqs ? dqs[0] : 0; a.dqs1 = dqs ? dqs[1] : 0; a.dqs2 = dqs ? dqs[2] : 0;
     a.qmap = qmap;
     a.b1 = b1; a.b2 = b2; a.AJ = AJ; a.nf = nf; a.H = H; a.unit0 = unit0;
     a.scale = scale;
-    const int nwaves = (AJ + 31) / 32;
+    const int waves = (AJ + 31) / 32;
+    a.nchunks = (waves + kDqkWaves - 1) / kDqkWaves;
+    const int nwaves = (waves + a.nchunks - 1) / a.nchunks;
+    a.total = (int)nuk * a.nchunks;
     const size_t ldsb = (size_t)2 * 64 * 2 * D;
-    const dim3 grid((unsigned)nuk), block((unsigned)(64 * nwaves));
+    const dim3 grid((unsigned)xcd_grid(a.total)), block((unsigned)(64 * nwaves));
     if (dtype == SFM_BF16) {
         if (D == 128) hipLaunchKernelGGL((monarch_bwd_dqk_kernel<BF16, 128>), grid, block, ldsb, stream, a);
         else hipLaunchKernelGGL((monarch_bwd_dqk_kernel<BF16, 64>), grid, block, ldsb, stream, a);

@@ -667,6 +667,7 @@ int sfm_monarch_bwd_workspace_bytes(const sfm_monarch_bwd_desc* desc, int32_t he
     return SFM_OK;
 }
 
+// with `kept`, dq is in the tensor dtype
 static int monarch_bwd_impl(const sfm_monarch_bwd_desc* desc, const void* q, const void* k, const void* v, const void* out,
                             const float* stats, const void* dout, float* dq, void* dk, void* dv, void* workspace,
                             size_t workspace_bytes, void* stream, const void* kept = nullptr);
@@ -695,6 +696,7 @@ static int plan_bwd_kept(const sfm_monarch_bwd_desc* desc, MonarchPlan* pl, size
     size_t per_unit = 0;
     int rc = plan_bwd(desc, pl, &per_unit);
     if (rc) return rc;
+    if ((rc = check_strides("dq", desc->dq_stride, desc->fwd.q_tokens, desc->fwd.H, desc->fwd.D, desc->fwd.B, 2))) return rc;
     *kept = kept_bytes(&desc->fwd, *pl, desc->dkv_stride);
     if (!*kept) {
         set_error("nothing can be kept for this descriptor's backward (see sfm_monarch_kept_bytes)");
@@ -719,7 +721,7 @@ int sfm_monarch_bwd_kept_workspace_bytes(const sfm_monarch_bwd_desc* desc, size_
 }
 
 int sfm_monarch_bwd_kept(const sfm_monarch_bwd_desc* desc, const void* q, const void* k, const void* v, const void* out,
-                         const float* stats, const void* kept, size_t kept_size, const void* dout, float* dq, void* dk, void* dv,
+                         const float* stats, const void* kept, size_t kept_size, const void* dout, void* dq, void* dk, void* dv,
                          void* workspace, size_t workspace_bytes, void* stream) {
     if (!out || !stats || !kept) {
         set_error("out, stats and kept must be non-NULL");
@@ -737,7 +739,7 @@ int sfm_monarch_bwd_kept(const sfm_monarch_bwd_desc* desc, const void* q, const 
         set_error("kept holds %zu bytes, the forward of this descriptor leaves %zu", kept_size, need);
         return SFM_ERR_WORKSPACE;
     }
-    return monarch_bwd_impl(desc, q, k, v, out, stats, dout, dq, dk, dv, workspace, workspace_bytes, stream, kept);
+    return monarch_bwd_impl(desc, q, k, v, out, stats, dout, (float*)dq, dk, dv, workspace, workspace_bytes, stream, kept);
 }
 
 static int monarch_bwd_impl(const sfm_monarch_bwd_desc* desc, const void* q, const void* k, const void* v, const void* out,
@@ -764,6 +766,7 @@ static int monarch_bwd_impl(const sfm_monarch_bwd_desc* desc, const void* q, con
         memset(&g, 0, sizeof(g));
         init_args(&desc->fwd, pl, &g.p);
         g.kept = kept != nullptr;
+        g.dq16 = kept ? (void*)dq : nullptr;
         int n = pl.units;
         while (n > 1 && monarch_bwd_gemm_bytes(g.p, desc->fwd.dtype, n, desc->dkv_stride, g.kept) > workspace_bytes) --n;
         if (monarch_bwd_gemm_bytes(g.p, desc->fwd.dtype, n, desc->dkv_stride, g.kept) > workspace_bytes) {

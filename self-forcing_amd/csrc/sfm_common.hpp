@@ -190,6 +190,7 @@ struct MonarchBwdArgs {
     const void* dout;        // [B, Sq, H, D] tensor dtype, strides dos
     int64_t dos[3];
     float* dq;               // [B, Sq, H, D] float, strides dqs
+    void* dq16;              // in its place, where every part is fused: the tensor dtype
     int64_t dqs[3];
     void* dk;                // tensor dtype, rows kmap.row(f, k) + l - dk_row0, strides dks
     void* dv;
@@ -273,7 +274,7 @@ int launch_monarch_bwd_left(int dtype, int D, int n, int b1, int b2, int AJ, int
 // dQ = s dS1 K; rows [f][(a, j)] per (unit, k) with ds1_tiles, as launch_monarch_bwd_dqk reads them, else [(a, j)][f]) and the
 // finished dK / dV rows of kv block-frames [f0, f1) in the caller's tensors; q, k and v are the caller's tensors too.  A column's
 // dc is in the order (f, k) with dc_fk, else (k, f)
-bool monarch_bwd_right_supported(int dtype, int D, int b2, int AJ);
+bool monarch_bwd_right_supported(int dtype, int D, int b2);
 int launch_monarch_bwd_right(int dtype, int D, int64_t ntiles, int b1, int b2, int AJ, int nf, float scale, const void* kk,
                              const int64_t* ks, const void* v, const int64_t* vs, const void* rb, const void* dkbar, const void* dy, const float* dc,
                              bool dc_fk, const void* q, const int64_t* qs, const TokMap& qmap, void* ds1, bool ds1_tiles, void* dk, void* dv, const int64_t* dks, int64_t row0,
@@ -282,11 +283,12 @@ int launch_monarch_bwd_right(int dtype, int D, int64_t ntiles, int b1, int b2, i
 // With `skip_masked` / `skip_causal` (the block-causal size) the three parts neither read nor write the scratch rows of masked
 // (query, key) block-frame pairs; the caller passes it when all of them (and step 1) run.
 // dQ of the right factor (monarch_bwd_right.hip): dqk[(u, k)][aj][:] = s sum_{f, l} dS1 K, float, or, with dqs given, added
-// to the caller's rows; k is the caller's tensor
-bool monarch_bwd_dqk_supported(int dtype, int D, int b2, int AJ);
+// to the caller's rows, or, with dq16 too, added to dqk ([u][aj][i][:], the left factor's) and stored to 16-bit rows; k is the
+// caller's tensor
+bool monarch_bwd_dqk_supported(int dtype, int D);
 int launch_monarch_bwd_dqk(int dtype, int D, int64_t nuk, int b1, int b2, int AJ, int nf, float scale, const void* k, const int64_t* ks,
-                           const TokMap& kmap, const void* ds1, float* dqk, const int64_t* dqs, const TokMap& qmap, int H, int unit0,
-                           int skip_causal, hipStream_t stream);
+                           const TokMap& kmap, const void* ds1, float* dqk, void* dq16, const int64_t* dqs, const TokMap& qmap, int H,
+                           int unit0, int skip_causal, hipStream_t stream);
 
 // backward of the dense attention (dense_attn_bwd.hip); with less scratch than this (2*B*H*q_tokens floats at least) no
 // workgroup is split

@@ -75,6 +75,10 @@ def release_scratch():
     _SCRATCH.clear()
 
 
+class _KeptRef(weakref.ref):
+    __slots__ = ("nbytes",)
+
+
 class _KeptBudget:
     """What the forwards of one device hold for backwards to come: at most a sixteenth of its memory (18 GB), which is a pass of
     30 layers of 12 heads at 480p; beyond that a forward leaves nothing and its backward forms the intermediates again.  A
@@ -82,7 +86,8 @@ class _KeptBudget:
 
     def __init__(self, device):
         self.left = torch.cuda.get_device_properties(device).total_memory // 16
-        self.lock = threading.RLock()            # a buffer's finalizer may run inside take(), from the garbage collector
+        self.lock = threading.RLock()            # a buffer may die inside take(), in the garbage collector
+        self.refs = set()
 
     def take(self, nbytes, device):
         with self.lock:
@@ -92,14 +97,18 @@ class _KeptBudget:
         try:
             buf = torch.empty(nbytes, dtype=torch.uint8, device=device)
         except torch.OutOfMemoryError:
-            self.give(nbytes)
+            with self.lock:
+                self.left += nbytes
             return None
-        weakref.finalize(buf, self.give, nbytes).atexit = False
+        ref = _KeptRef(buf, self._died)
+        ref.nbytes = nbytes
+        self.refs.add(ref)
         return buf
 
-    def give(self, nbytes):
+    def _died(self, ref):
         with self.lock:
-            self.left += nbytes
+            self.refs.discard(ref)
+            self.left += ref.nbytes
 
 
 _KEPT = {}
@@ -191,12 +200,12 @@ def _monarch_fwd_kept(q, k, v, tiling, sm_scale, kv_block_order, cbf, heads_per_
     block-causal clip of nine frames, three tied, 620 and 534."""
     out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     d = _desc(q, k, v, out, *tiling, sm_scale, kv_block_order, cbf, 1)
-    n = C.c_size_t(0)
-    _l.check(_l.load().sfm_monarch_stats_bytes(C.byref(d), C.byref(n)))
+    lib, n = _l.load(), C.c_size_t(0)
+    _l.check(lib.sfm_monarch_stats_bytes(C.byref(d), C.byref(n)))
     stats = torch.empty(n.value // 4, dtype=torch.float32, device=q.device) if n.value else None
     kept = None
     if keep and stats is not None and not heads_per_pass:
-        _l.check(_l.load().sfm_monarch_kept_bytes(C.byref(d), C.byref(n)))
+        _l.check(lib.sfm_monarch_kept_bytes(C.byref(d), C.byref(n)))
         kept = _kept_buffer(n.value, q.device)
     if kept is not None:
         nbytes, ws = n.value, kept
@@ -213,15 +222,15 @@ def _monarch_fwd_kept(q, k, v, tiling, sm_scale, kv_block_order, cbf, heads_per_
                 new_k, new_v = new_k.contiguous(), new_v.contiguous()
             if k.stride() != v.stride():
                 raise ValueError("k_cache and v_cache must share their strides")
-            fn = _l.load().sfm_monarch_attn_with_kv_cache_stats if kept is None else _l.load().sfm_monarch_attn_with_kv_cache_kept
+            fn = lib.sfm_monarch_attn_with_kv_cache_stats if kept is None else lib.sfm_monarch_attn_with_kv_cache_kept
             _l.check(fn(
                 C.byref(d), q.data_ptr(), k.data_ptr(), v.data_ptr(), new_k.data_ptr(), new_v.data_ptr(), _l.strides3(new_k),
                 start_idx, end_idx, out.data_ptr(), stats.data_ptr(), ws.data_ptr(), nbytes, _stream(q)))
         elif stats is None:
-            _l.check(_l.load().sfm_monarch_fwd(C.byref(d), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-                                               ws.data_ptr(), nbytes, _stream(q)))
+            _l.check(lib.sfm_monarch_fwd(C.byref(d), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+                                         ws.data_ptr(), nbytes, _stream(q)))
         else:
-            fn = _l.load().sfm_monarch_fwd_stats if kept is None else _l.load().sfm_monarch_fwd_kept
+            fn = lib.sfm_monarch_fwd_stats if kept is None else lib.sfm_monarch_fwd_kept
             _l.check(fn(C.byref(d), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), stats.data_ptr(), ws.data_ptr(), nbytes,
                         _stream(q)))
     return out, stats, kept
@@ -230,7 +239,8 @@ def _monarch_fwd_kept(q, k, v, tiling, sm_scale, kv_block_order, cbf, heads_per_
 def _monarch_bwd(q, k, v, dout, tiling, sm_scale, kv_block_order, cbf, kv_f0=0, kv_f1=None, heads_per_pass=0, out=None,
                  stats=None, kept=None):
     """Raw call of sfm_monarch_bwd (or sfm_monarch_bwd_saved when the forward's `out` and `stats` are given, sfm_monarch_bwd_kept
-    when its `kept` is too): returns (dq float32, dk, dv); dk, dv cover kv block-frames [kv_f0, kv_f1) in the row order of k."""
+    when its `kept` is too): returns (dq float32, with `kept` in q's dtype, dk, dv); dk, dv cover kv
+    block-frames [kv_f0, kv_f1) in the row order of k."""
     f_tied, h_reduce, w_reduce, h, w = tiling
     per_frame = f_tied * (h // h_reduce) * (w // w_reduce)
     nf = k.shape[1] // per_frame
@@ -240,37 +250,38 @@ def _monarch_bwd(q, k, v, dout, tiling, sm_scale, kv_block_order, cbf, kv_f0=0, 
         dout = dout.contiguous()
     if out is not None and out.stride() != dout.stride():
         out = out.contiguous()
-    dq = torch.empty(q.shape, dtype=torch.float32, device=q.device)
     dk = torch.empty((k.shape[0], (kv_f1 - kv_f0) * per_frame, k.shape[2], k.shape[3]), dtype=k.dtype, device=k.device)
     dv = torch.empty_like(dk)
     bd = _l.MonarchBwdDesc()
     bd.fwd = _desc(q, k, v, dout, f_tied, h_reduce, w_reduce, h, w, sm_scale, kv_block_order, cbf)
-    bd.dq_stride = _l.strides3(dq)
     bd.dkv_stride = _l.strides3(dk)
     bd.kv_grad_frame_start, bd.kv_grad_frame_end = kv_f0, kv_f1
-    n = C.c_size_t(0)
+    lib, n = _l.load(), C.c_size_t(0)
     if kept is not None:
-        _l.check(_l.load().sfm_monarch_kept_bytes(C.byref(bd.fwd), C.byref(n)))
-        if n.value != kept.numel():              # the implementation switches were changed since the forward
+        dq = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+        bd.dq_stride = _l.strides3(dq)
+        rc = lib.sfm_monarch_bwd_kept_workspace_bytes(C.byref(bd), C.byref(n))
+        if rc == _l.SFM_ERR_UNSUPPORTED:         # the implementation switches were changed since the forward
             kept = None
-    if kept is not None:
-        _l.check(_l.load().sfm_monarch_bwd_kept_workspace_bytes(C.byref(bd), C.byref(n)))
-    else:
-        _l.check(_l.load().sfm_monarch_bwd_workspace_bytes(C.byref(bd), heads_per_pass, C.byref(n)))
+        else:
+            _l.check(rc)
+    if kept is None:
+        dq = torch.empty(q.shape, dtype=torch.float32, device=q.device)
+        bd.dq_stride = _l.strides3(dq)
+        _l.check(lib.sfm_monarch_bwd_workspace_bytes(C.byref(bd), heads_per_pass, C.byref(n)))
     ws = scratch(n.value, q.device)
     with _on_device(q.device):
         if kept is not None:
-            _l.check(_l.load().sfm_monarch_bwd_kept(C.byref(bd), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-                                                    stats.data_ptr(), kept.data_ptr(), kept.numel(), dout.data_ptr(), dq.data_ptr(),
-                                                    dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), n.value, _stream(q)))
+            _l.check(lib.sfm_monarch_bwd_kept(C.byref(bd), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+                                              stats.data_ptr(), kept.data_ptr(), kept.numel(), dout.data_ptr(), dq.data_ptr(),
+                                              dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), n.value, _stream(q)))
         elif out is None or stats is None:
-            _l.check(_l.load().sfm_monarch_bwd(C.byref(bd), q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(),
-                                               dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), n.value,
-                                               _stream(q)))
+            _l.check(lib.sfm_monarch_bwd(C.byref(bd), q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(), dq.data_ptr(),
+                                         dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), n.value, _stream(q)))
         else:
-            _l.check(_l.load().sfm_monarch_bwd_saved(C.byref(bd), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-                                                     stats.data_ptr(), dout.data_ptr(), dq.data_ptr(), dk.data_ptr(),
-                                                     dv.data_ptr(), ws.data_ptr(), n.value, _stream(q)))
+            _l.check(lib.sfm_monarch_bwd_saved(C.byref(bd), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+                                               stats.data_ptr(), dout.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+                                               ws.data_ptr(), n.value, _stream(q)))
     return dq, dk, dv
 
 
