@@ -429,7 +429,7 @@ Parts make_parts(const MonarchArgs& p, int dtype, const int64_t* dks) {
                            (int64_t)p.nf * p.b1 * p.b2 * p.ks[1] * 2 < ((int64_t)1 << 32);
     f.dqk = monarch_bwd_dqk_supported(dtype, p.D) && !(sw & SFM_SW_BWD_DQK_GEMM);
     // the rows of dS1 are padded to whole 8-byte pieces, which the library product of part 10 does not know
-    f.right = f.fwd && direct_ok && monarch_bwd_right_supported(dtype, p.D, p.b2) && p.na * p.b2 <= 480 && (f.dqk || p.b2 % 4 == 0) &&
+    f.right = f.fwd && direct_ok && monarch_bwd_right_supported(dtype, p.D, p.b2) && (f.dqk || p.b2 % 4 == 0) &&
               !(sw & SFM_SW_BWD_RIGHT_GEMM);
     f.dqk = f.dqk && f.right;
     return f;

@@ -1,5 +1,4 @@
-// Right-factor part of the Monarch backward on gfx950 MFMA (bf16 / fp16, head_dim 64 or 128, b2 <= 64, at most 480 (a, j)
-// columns).
+// Right-factor part of the Monarch backward on gfx950 MFMA (bf16 / fp16, head_dim 64 or 128, b2 <= 64).
 //
 // Replaces, per tile t = (unit, k, f), the small batched products and the row kernel of the GEMM chain
 //     dR[aj, l]  = dKbar[aj,:] . K[l,:] + dY[aj,:] . V[l,:]

@@ -19,6 +19,7 @@ mattn, L = sfa.monarch_attn, sfa.lib
     ((1, 1, 1, 1, 5), 1, 1, 1, 64, 0), ((1, 1, 1, 4, 8), 2, 8, 3, 128, 0), ((1, 1, 1, 31, 1), 1, 1, 2, 64, 0),
     ((1, 1, 1, 11, 52), 3, 3, 2, 128, 0), ((1, 1, 1, 30, 52), 3, 6, 2, 128, 0), ((1, 2, 1, 8, 33), 1, 4, 2, 64, 0),
     ((3, 1, 2, 7, 64), 3, 6, 1, 128, 0), ((3, 1, 1, 13, 20), 3, 3, 2, 64, 0), ((1, 1, 1, 90, 8), 1, 2, 2, 128, 0),
+    ((1, 2, 1, 4, 60), 9, 9, 1, 128, 6), ((1, 1, 1, 3, 43), 12, 2, 2, 64, 0),      # 1080 and 516 (a, j) columns
     ((1, 1, 1, 5, 20), 6, 6, 2, 128, 2), ((3, 1, 1, 12, 16), 6, 6, 2, 64, 1),
 ])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
