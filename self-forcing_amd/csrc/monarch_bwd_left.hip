@@ -18,19 +18,23 @@
 //
 //   TEAM = 1 (b1 <= 32): a wave per column, four to a workgroup that share nothing; the operands of a chunk are in
 //       registers (one wave per SIMD), so that the next chunk's loads run beside the whole computation.
-//   TEAM = 2..4 (b1 <= 128): a workgroup of TEAM waves per column shares its chunks; each wave forms L and dS2 of its own
-//       32 query rows and hands them to the others through LDS, and the sums over i are split by head-dim blocks, so that
-//       every Kbar / Y row is read once and every dKbar / dY row written once.
+//   TEAM = 2..4 (b1 <= 128): a workgroup of up to TEAM query tiles per column shares its chunks; a wave per tile forms L and
+//       dS2 of its 32 query rows and hands them to the others through LDS, and the sums over i are split by head-dim blocks,
+//       a pair of them of one matrix to each of four waves (head_dim 64: two), so that every Kbar / Y row is read once and
+//       every dKbar / dY row written once.
 //
 // Kbar, Y and the entropy terms are read as the forward arranges them (a column's rows one after the other, (f, k) order) where
 // every later part is fused too, so that the forward's own can be handed over; dKbar and dY are written tile after tile, as the
 // right factor reads them.
 //
-// Bound by HBM: Kbar, Y read and dKbar, dY written once.  At 12 heads, a = 3, f = 21, b1 = 30, b2 = 52, 1.3 GB in 283 us,
-// where the kernel without dQ took 306 and a second one that read Kbar again for dQ 117.  With three frames tied (a = 3,
-// f = 3, b1 = 90, b2 = 52) 217 us, block-causal over single block-frames, where a third of the rows is left out, 183; a
-// grid slice per 32 query rows, which read the rows three times and wrote partial sums, took 352, the kernel that added
-// them 179 and dQ 175.
+// TEAM = 1 is bound by HBM: Kbar, Y read and dKbar, dY written once.  At 12 heads, a = 3, f = 21, b1 = 30, b2 = 52, 1.3 GB
+// in 263 us (271 before its rows were fetched at once), where the kernel without dQ took 306 and a second one that read Kbar
+// again for dQ 117.  A team is bound by the latency of its own steps, 5200 cycles a chunk of 32 rows, of which 400 wait
+// for the rows.  Three frames tied (b1 = 90): against 21 frames 113 us, nine frames block-causal (a = f = 3, a third of the rows
+// left out, 565 MB) 143; that was 175 while the column's own rows came a row group after the other (20 000 cycles before the
+// first chunk), three waves shared four pairs of head-dim blocks (8400 cycles a chunk; 6600 so) and every request and store
+// worked out its row for either arrangement.  A grid slice per 32 query rows, which read the rows three times and wrote partial
+// sums, took 352, the kernel that added them 179 and dQ 175.
 
 #include <hip/hip_runtime.h>
 
@@ -108,16 +112,21 @@ struct LeftLds {
     static constexpr int kXWave = TEAM == 1 ? kX : 2 * kX;
     static constexpr int kDc = kXs + TEAM * kXWave;
     static constexpr int kBytes = (kDc + (TEAM == 1 ? 0 : TEAM * 128) + 255) / 256 * 256;
+    // a team has a wave per query tile and at least one per pair of head-dim blocks of the two matrices of gradient rows
+    static constexpr int kWaves = TEAM == 1 ? 4 : TEAM > D / 32 ? TEAM : D / 32;
     static __host__ __device__ constexpr size_t bytes() { return (size_t)(TEAM == 1 ? 4 : 1) * kBytes; }
 };
 
-template <class E, int D, int TEAM>
-__global__ __launch_bounds__(TEAM == 1 ? 256 : 64 * TEAM) __attribute__((amdgpu_waves_per_eu(TEAM == 1 ? 1 : 2, TEAM == 1 ? 1 : 2)))
+// FK: Kbar, Y and c are in the forward's arrangement (r_pad > 0), and no dS2 is wanted; the row arithmetic of the other
+// arrangement took a quarter of a team's instructions
+template <class E, int D, int TEAM, bool FK>
+__global__ __launch_bounds__((64 * LeftLds<D, TEAM>::kWaves)) __attribute__((amdgpu_waves_per_eu(TEAM == 1 ? 1 : 2, TEAM == 1 ? 1 : 2)))
 void monarch_bwd_left_kernel(LeftArgs p) {
     using L = LeftLds<D, TEAM>;
     constexpr int DS = D / 16, DT = D / 32, CPR = D / 8, NG = CPR / 2;      // NG: 1 KB pieces of a tile
     constexpr int kPitch = L::kPitch, kTile = L::kTile, kXPitch = L::kXPitch;
     constexpr bool SOLO = TEAM == 1;
+    constexpr int WAVES = L::kWaves;
     extern __shared__ __attribute__((aligned(256))) char lds[];
 
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, hf = lane >> 5;
@@ -130,72 +139,60 @@ void monarch_bwd_left_kernel(LeftArgs p) {
     if (aj >= p.AJ) return;                               // a lone wave: nothing is shared
     const int u = item / njg;
     const int w = SOLO ? 0 : wave;                        // this wave's query tile
+    const bool has_tile = SOLO || WAVES == TEAM || wave < TEAM;        // uniform: the others join for the gradient rows
     const int i0 = 32 * w;
     const int RR = p.RR, b1 = p.b1;
     const int64_t uaj = (int64_t)u * p.AJ + aj;
 
     char* const base = lds + (SOLO ? wave * L::kBytes : 0);
     char* const qt = base;                                // TEAM query tiles
-    char* const dot_t = base + TEAM * kTile;              // TEAM dO tiles
     char* const qs = qt + w * kTile;
-    char* const dos = dot_t + w * kTile;
+    char* const dos = qs + TEAM * kTile;                  // behind the query tiles TEAM dO tiles
     float* const dls = (float*)(base + L::kDot + w * 128);
     char* const xds = base + L::kXs + w * L::kXWave;      // this wave's dS2
     const bool saved = p.stats != nullptr;                // uniform: the forward's output and row statistics are at hand
+    // The column's query, dO (and output) rows: all of a wave's loads on their way at once, and behind them those of the first
+    // chunk (one row group after the other waited out the latency of each: 20 000 cycles before the first chunk)
+    u32x4 q_in[NG], do_in[NG], out_in[NG];
+    const int ch0 = lane % CPR, r0 = lane / CPR;          // piece g of a wave: 16 bytes of row r0 + g (64 / CPR)
     {
         const int unit = p.unit0 + u, bb = unit / p.H, hh = unit % p.H;
         const int a_q = aj / p.b2, j_q = aj % p.b2;
-        const char* qg = p.q + ((int64_t)bb * p.qs[0] + (int64_t)hh * p.qs[2]) * 2;
-        const char* dg = p.dout + ((int64_t)bb * p.os[0] + (int64_t)hh * p.os[2]) * 2;
-        const char* og = saved ? p.out + ((int64_t)bb * p.os[0] + (int64_t)hh * p.os[2]) * 2 : dg;
-        for (int cidx = lane; cidx < 32 * CPR; cidx += 64) {
-            const int r = cidx / CPR, ch = cidx % CPR;
-            u32x4 a = {0u, 0u, 0u, 0u}, b = a;
-            float dot = 0.f;
-            if (i0 + r < b1) {
-                const int64_t tok = p.qmap.row(a_q, i0 + r) + j_q;
-                a = *(const u32x4*)(qg + tok * p.qs[1] * 2 + ch * 16);
-                b = *(const u32x4*)(dg + tok * p.os[1] * 2 + ch * 16);
-                if (saved) {                              // sum_r L dLm of row i is dO_i . O_i
-                    const u32x4 o = *(const u32x4*)(og + tok * p.os[1] * 2 + ch * 16);
+        const char* qg = p.q + ((int64_t)bb * p.qs[0] + (int64_t)hh * p.qs[2]) * 2 + ch0 * 16;
+        const char* dg = p.dout + ((int64_t)bb * p.os[0] + (int64_t)hh * p.os[2]) * 2 + ch0 * 16;
+        const char* og = saved ? p.out + ((int64_t)bb * p.os[0] + (int64_t)hh * p.os[2]) * 2 + ch0 * 16 : dg;
+        const int64_t tok0 = p.qmap.row(a_q, 0) + j_q;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        dot += E::to_float((uint16_t)(b[e] & 0xffffu)) * E::to_float((uint16_t)(o[e] & 0xffffu)) +
-                               E::to_float((uint16_t)(b[e] >> 16)) * E::to_float((uint16_t)(o[e] >> 16));
-                }
-            }
-            const int at = r * kPitch + ((ch ^ bl_swz<CPR>(r)) << 4);
-            *(u32x4*)(qs + at) = a;
-            *(u32x4*)(dos + at) = b;
-            if (saved) {
-#pragma unroll
-                for (int o = 1; o < CPR; o <<= 1) dot += __shfl_xor(dot, o);
-                if (ch == 0) dls[r] = dot;
+        for (int g = 0; g < NG; ++g) {
+            const int i = i0 + r0 + g * (64 / CPR);
+            q_in[g] = do_in[g] = out_in[g] = u32x4{0u, 0u, 0u, 0u};
+            if (i < b1) {                                 // no row of a wave without a tile
+                const int64_t tok = tok0 + p.qmap.row_delta(i);
+                q_in[g] = *(const u32x4*)(qg + tok * p.qs[1] * 2);
+                do_in[g] = *(const u32x4*)(dg + tok * p.os[1] * 2);
+                if (saved) out_in[g] = *(const u32x4*)(og + tok * p.os[1] * 2);
             }
         }
     }
-    if (SOLO) lds_wave_sync();
-    else lds_barrier();
 
     const int a_blk = aj / p.b2;
     const int flim = p.causal ? min(p.nf, (a_blk / p.causal + 1) * p.causal) : p.nf;      // visible kv block-frames
     const int64_t rstride = (int64_t)p.AJ * D;                                           // elements between rows r, r + 1
-    const bool fk = p.r_pad > 0;                          // uniform: Kbar, Y and c are the forward's
-    const int64_t kbar0 = (fk ? uaj * p.r_pad : (int64_t)u * RR * p.AJ + aj) * D;
+    const int64_t kbar0 = (FK ? uaj * p.r_pad : (int64_t)u * RR * p.AJ + aj) * D;
     const char* const kbb = (const char*)(p.kbar + kbar0);
     const char* const ybb = (const char*)(p.y + kbar0);
-    const char* const cpb = (const char*)(fk ? p.c + (int64_t)u * p.r_pad * p.AJ + aj : p.c_rows ? p.c + (int64_t)u * RR * p.AJ + aj : p.c + uaj * RR);
-    const float cmul = p.c_rows ? 1.f : kLog2e;
+    const char* const cpb = (const char*)(FK ? p.c + (int64_t)u * p.r_pad * p.AJ + aj : p.c_rows ? p.c + (int64_t)u * RR * p.AJ + aj : p.c + uaj * RR);
+    const float cmul = FK || p.c_rows ? 1.f : kLog2e;
     const float sc2 = p.scale * kLog2e;
     // The rows of a column, in order: all of them, or (skip) those of its flim visible block-frames, which come first in the
     // forward's arrangement
     const bool skip = p.skip && flim < p.nf;              // uniform
     const int RV = skip ? b1 * flim : RR;
     const int nch = (RV + 31) / 32;
-    auto row_of = [&](int x) { return skip && !fk ? x / flim * p.nf + x % flim : x; };       // in Kbar, Y, c, dc
+    auto row_of = [&](int x) { return !FK && skip ? x / flim * p.nf + x % flim : x; };       // in Kbar, Y, c, dc
     const float inv_b1 = 1.f / (float)b1;
     auto grad_row = [&](int x) {                          // in dKbar, dY
-        if (!fk) return row_of(x);
+        if (!FK) return row_of(x);
         const int f = (int)(((float)x + 0.5f) * inv_b1);  // x / b1, exact while x < 2^22
         return (x - f * b1) * p.nf + f;
     };
@@ -205,7 +202,7 @@ void monarch_bwd_left_kernel(LeftArgs p) {
     // where they are used, and each wave requests its share of the next chunk when all of them are done with this one.
     char* const kt = base + L::kChunk;
     const uint32_t kt0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(size_t)(__attribute__((address_space(3))) char*)kt);
-    const uint32_t rsb = fk ? (uint32_t)kPitch : (uint32_t)(rstride * 2), csb = (uint32_t)((p.c_rows ? p.AJ : 1) * 4);
+    const uint32_t rsb = FK ? (uint32_t)kPitch : (uint32_t)(rstride * 2), csb = (uint32_t)((FK || p.c_rows ? p.AJ : 1) * 4);
     auto piece_off = [&](int n, int g) {
         const int P = g * 64 + lane;
         const int r = P / CPR, c = (P % CPR) ^ bl_swz<CPR>(r);
@@ -231,12 +228,12 @@ void monarch_bwd_left_kernel(LeftArgs p) {
             }
         } else {
 #pragma unroll
-            for (int q0 = 0; q0 < 2 * NG; q0 += TEAM) {
+            for (int q0 = 0; q0 < 2 * NG; q0 += WAVES) {
                 const int q = q0 + wave;
-                if (q < 2 * NG) bl_load_lds16(q < NG ? kbb : ybb, piece_off(n, q % NG), kt0 + (uint32_t)q * 1024);
+                if (2 * NG % WAVES == 0 || q < 2 * NG) bl_load_lds16(q < NG ? kbb : ybb, piece_off(n, q % NG), kt0 + (uint32_t)q * 1024);
             }
         }
-        if (wave == (SOLO ? wave : TEAM - 1)) bl_load_lds4_at<2 * kTile>(cpb, (uint32_t)row_of(min(32 * n + m, RV - 1)) * csb, kt0);
+        if (SOLO || wave == WAVES - 1) bl_load_lds4_at<2 * kTile>(cpb, (uint32_t)row_of(min(32 * n + m, RV - 1)) * csb, kt0);
     };
     const uint32_t b_off = (uint32_t)m * kPitch + (uint32_t)((hf ^ bl_swz<CPR>(m)) << 4);     // row m of a tile as an operand
     // transposing reads of a tile: lane (m, hf) gets, for head-dim column 32 dt + m, rows 16 ks + 4 hf + {0..3} and + 8 +
@@ -263,9 +260,15 @@ void monarch_bwd_left_kernel(LeftArgs p) {
 
     u32x4 kcur[SOLO ? DS : 1], ycur[SOLO ? DS : 1], ktr[SOLO ? DT : 1][2];
     float ccur = 0.f;
-    // waits for the chunk requested last; a lone wave fills its registers from it and requests chunk `next`
-    auto open_chunk = [&](int next, bool want_t) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // The gradient rows' store instructions that a wave issues behind a request: they may stay in flight when the requested
+    // chunk is waited for (vector memory operations complete in order)
+    constexpr int kStores = SOLO ? 4 * DT : 4;
+    const bool stores = SOLO || wave < DT;                // uniform
+    // waits for the chunk requested last (`stored`: gradient rows were stored since); a lone wave fills its registers from it
+    // and requests chunk `next`
+    auto open_chunk = [&](int next, bool want_t, bool stored) {
+        if (stored && stores) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kStores) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if constexpr (SOLO) {
 #pragma unroll
             for (int ds = 0; ds < DS; ++ds) {
@@ -314,11 +317,33 @@ void monarch_bwd_left_kernel(LeftArgs p) {
     };
     auto row_ok = [&](int n) {
         const int r = 32 * n + m;
-        return r < RV && (skip || (fk ? r < b1 * flim : r % p.nf < flim));
+        return FK ? r < b1 * flim : r < RV && (skip || r % p.nf < flim);
     };
 
-    float lse[16], delta[16];
     request(0);
+    if (has_tile) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            const int r = r0 + g * (64 / CPR);
+            const int at = r * kPitch + ((ch0 ^ bl_swz<CPR>(r)) << 4);
+            *(u32x4*)(qs + at) = q_in[g];
+            *(u32x4*)(dos + at) = do_in[g];
+            if (saved) {                                      // sum_r L dLm of row i is dO_i . O_i
+                float dot = 0.f;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    dot += E::to_float((uint16_t)(do_in[g][e] & 0xffffu)) * E::to_float((uint16_t)(out_in[g][e] & 0xffffu)) +
+                           E::to_float((uint16_t)(do_in[g][e] >> 16)) * E::to_float((uint16_t)(out_in[g][e] >> 16));
+#pragma unroll
+                for (int o = 1; o < CPR; o <<= 1) dot += __shfl_xor(dot, o);
+                if (ch0 == 0) dls[r] = dot;
+            }
+        }
+    }
+    if (SOLO) lds_wave_sync();
+    else lds_barrier();
+
+    float lse[16], delta[16];
     if (saved) {
         const float* st = p.stats + ((int64_t)(p.unit0 + u) * p.AJ + aj) * p.stats_ld;
 #pragma unroll
@@ -337,11 +362,12 @@ void monarch_bwd_left_kernel(LeftArgs p) {
         }
         for (int n = 0; n < nch; ++n) {
             const int next = n + 1 < nch ? n + 1 : 0;      // after the last chunk the first one, for pass 2
-            open_chunk(next, false);
+            open_chunk(next, false, false);
             f32x16 s, d;
-            products(s, d);
+            if (has_tile) products(s, d);
             const float cl2 = ccur;
             close_chunk(next);
+            if (!has_tile) continue;
             const bool ok = row_ok(n);
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
@@ -385,67 +411,69 @@ void monarch_bwd_left_kernel(LeftArgs p) {
 
     for (int n = 0; n < nch; ++n) {
         const int next = n + 1 < nch ? n + 1 : -1;
-        open_chunk(next, true);
-        f32x16 s, d;
-        products(s, d);
-        const float cl2 = ccur;
-        const bool ok = row_ok(n);
+        open_chunk(next, true, n > 0);
         const bool r_in = 32 * n + m < RV;
         const int r = row_of(32 * n + m);
-        float dsum = 0.f;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const float pv = ok ? fast_exp2(s[v] * sc2 - cl2 - lse[v]) : 0.f;
-            const float gv = pv * (d[v] - delta[v]);
-            s[v] = pv;                                   // L[i, r]
-            d[v] = gv;                                   // dS2[i, r]
-            dsum += gv;
-        }
-        dsum = xhalf_sum(dsum);
-        if (SOLO) {
-            if (r_in && hf == 0) dcp[r] = -dsum;
-        } else if (hf == 0) {
-            *(float*)(base + L::kDc + w * 128 + m * 4) = dsum;
-        }
-        if (p.ds2 && r_in) {
-            uint16_t* const ds2p = p.ds2 + uaj * b1 * p.ds2_ld;
+        u32x4 pl[2], pg[2];                              // B operands [n = r, k = i] for the two steps of 16 rows i
+        if (has_tile) {
+            f32x16 s, d;
+            products(s, d);
+            const float cl2 = ccur;
+            const bool ok = row_ok(n);
+            float dsum = 0.f;
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
-                const int i = i0 + 8 * (v >> 2) + 4 * hf + (v & 3);
-                if (i < b1) ds2p[(int64_t)i * p.ds2_ld + r] = E::from_float(d[v]);
+                const float pv = ok ? fast_exp2(s[v] * sc2 - cl2 - lse[v]) : 0.f;
+                const float gv = pv * (d[v] - delta[v]);
+                s[v] = pv;                                   // L[i, r]
+                d[v] = gv;                                   // dS2[i, r]
+                dsum += gv;
             }
-        }
-        u32x4 pl[2], pg[2];                              // B operands [n = r, k = i] for the two steps of 16 rows i
+            dsum = xhalf_sum(dsum);
+            if (SOLO) {
+                if (r_in && hf == 0) dcp[r] = -dsum;
+            } else if (hf == 0) {
+                *(float*)(base + L::kDc + w * 128 + m * 4) = dsum;
+            }
+            if (!FK && p.ds2 && r_in) {
+                uint16_t* const ds2p = p.ds2 + uaj * b1 * p.ds2_ld;
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            pl[ks].x = pack2<E>(s[8 * ks + 0], s[8 * ks + 1]); pl[ks].y = pack2<E>(s[8 * ks + 2], s[8 * ks + 3]);
-            pl[ks].z = pack2<E>(s[8 * ks + 4], s[8 * ks + 5]); pl[ks].w = pack2<E>(s[8 * ks + 6], s[8 * ks + 7]);
-            pg[ks].x = pack2<E>(d[8 * ks + 0], d[8 * ks + 1]); pg[ks].y = pack2<E>(d[8 * ks + 2], d[8 * ks + 3]);
-            pg[ks].z = pack2<E>(d[8 * ks + 4], d[8 * ks + 5]); pg[ks].w = pack2<E>(d[8 * ks + 6], d[8 * ks + 7]);
-            char* const x = xds + m * kXPitch + (16 * ks + 4 * hf) * 2;
-            *(u32x2*)x = u32x2{pg[ks].x, pg[ks].y};
-            *(u32x2*)(x + 16) = u32x2{pg[ks].z, pg[ks].w};
-            if (!SOLO) {
-                *(u32x2*)(x + L::kX) = u32x2{pl[ks].x, pl[ks].y};
-                *(u32x2*)(x + L::kX + 16) = u32x2{pl[ks].z, pl[ks].w};
+                for (int v = 0; v < 16; ++v) {
+                    const int i = i0 + 8 * (v >> 2) + 4 * hf + (v & 3);
+                    if (i < b1) ds2p[(int64_t)i * p.ds2_ld + r] = E::from_float(d[v]);
+                }
             }
-        }
-        lds_wave_sync();
-        if (p.dq) {
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks) {
-                const u32x2 lo = bl_read_tr(xds, trx + ks * 16 * kXPitch);
-                const u32x2 hi = bl_read_tr(xds, trx + (8 + ks * 16) * kXPitch);
-                const u32x4 bop = {lo.x, lo.y, hi.x, hi.y};
+                pl[ks].x = pack2<E>(s[8 * ks + 0], s[8 * ks + 1]); pl[ks].y = pack2<E>(s[8 * ks + 2], s[8 * ks + 3]);
+                pl[ks].z = pack2<E>(s[8 * ks + 4], s[8 * ks + 5]); pl[ks].w = pack2<E>(s[8 * ks + 6], s[8 * ks + 7]);
+                pg[ks].x = pack2<E>(d[8 * ks + 0], d[8 * ks + 1]); pg[ks].y = pack2<E>(d[8 * ks + 2], d[8 * ks + 3]);
+                pg[ks].z = pack2<E>(d[8 * ks + 4], d[8 * ks + 5]); pg[ks].w = pack2<E>(d[8 * ks + 6], d[8 * ks + 7]);
+                char* const x = xds + m * kXPitch + (16 * ks + 4 * hf) * 2;
+                *(u32x2*)x = u32x2{pg[ks].x, pg[ks].y};
+                *(u32x2*)(x + 16) = u32x2{pg[ks].z, pg[ks].w};
+                if (!SOLO) {
+                    *(u32x2*)(x + L::kX) = u32x2{pl[ks].x, pl[ks].y};
+                    *(u32x2*)(x + L::kX + 16) = u32x2{pl[ks].z, pl[ks].w};
+                }
+            }
+            lds_wave_sync();
+            if (p.dq) {
 #pragma unroll
-                for (int dt = 0; dt < DT; ++dt) {
-                    if constexpr (SOLO) dqa[dt] = E::mfma32(ktr[dt][ks], bop, dqa[dt]);
-                    else dqa[dt] = E::mfma32(read_t(kt, dt & 1, dt >> 1, ks), bop, dqa[dt]);
+                for (int ks = 0; ks < 2; ++ks) {
+                    const u32x2 lo = bl_read_tr(xds, trx + ks * 16 * kXPitch);
+                    const u32x2 hi = bl_read_tr(xds, trx + (8 + ks * 16) * kXPitch);
+                    const u32x4 bop = {lo.x, lo.y, hi.x, hi.y};
+#pragma unroll
+                    for (int dt = 0; dt < DT; ++dt) {
+                        if constexpr (SOLO) dqa[dt] = E::mfma32(ktr[dt][ks], bop, dqa[dt]);
+                        else dqa[dt] = E::mfma32(read_t(kt, dt & 1, dt >> 1, ks), bop, dqa[dt]);
+                    }
                 }
             }
         }
         close_chunk(next);
-        if (!SOLO && wave == TEAM - 1 && r_in && hf == 0) {
+        if (!SOLO && wave == WAVES - 1 && r_in && hf == 0) {
             float t = 0.f;
 #pragma unroll
             for (int x = 0; x < TEAM; ++x) t += *(const float*)(base + L::kDc + x * 128 + m * 4);
@@ -457,17 +485,19 @@ void monarch_bwd_left_kernel(LeftArgs p) {
         // (v_permlane16_swap) and lane bit 3 for the block within the pair (a rotation by 8 within rows of 16 lanes),
         // after which a lane holds the 16-byte piece 4 (bit 3) + 2 (bit 4) + hf of the rows (r & 7) + 8 rb, rb = 0..3:
         // one store instruction writes 128 contiguous bytes of each of 8 rows.
-        int64_t rowoff[4];
+        uint64_t rowoff[4];                              // bytes
         bool row_in[4];
 #pragma unroll
         for (int rb = 0; rb < 4; ++rb) {
             const int rr = 32 * n + (m & 7) + 8 * rb;
             row_in[rb] = rr < RV;
-            rowoff[rb] = (int64_t)grad_row(min(rr, RV - 1)) * rstride + (4 * ((m >> 3) & 1) + 2 * ((m >> 4) & 1) + hf) * 8;
+            rowoff[rb] = (uint64_t)(uint32_t)grad_row(min(rr, RV - 1)) * (uint32_t)(rstride * 2) + (4 * ((m >> 3) & 1) + 2 * ((m >> 4) & 1) + hf) * 16;
         }
-        auto half_rows = [&](int which, int dp) {
-            const char* src = which == 0 ? dot_t : qt;
-            uint16_t* const obase = which == 0 ? dyb : dkb;
+        // N pairs of head-dim blocks from dp0 on: 2 N independent chains of matrix instructions that share their B operands
+        auto half_rows = [&](int which, int dp0, auto n_c) {
+            constexpr int N = decltype(n_c)::value;
+            const char* const src = qt + (which == 0 ? TEAM * kTile : 0);
+            char* const obase = (char*)(which == 0 ? dyb : dkb);
             const float osc = which == 0 ? 1.f : p.scale;
             u32x4 bop[TEAM][2];
 #pragma unroll
@@ -482,53 +512,67 @@ void monarch_bwd_left_kernel(LeftArgs p) {
                         bop[t][ks] = u32x4{lo.x, lo.y, hi.x, hi.y};
                     }
                 }
-            uint32_t wd[2][2][4];                        // [block in pair][gp][dword]
+            f32x16 o[2 * N];
 #pragma unroll
-            for (int dl = 0; dl < 2; ++dl) {
-                f32x16 o;
+            for (int x = 0; x < 2 * N; ++x)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) o[v] = 0.f;
+                for (int v = 0; v < 16; ++v) o[x][v] = 0.f;
 #pragma unroll
-                for (int t = 0; t < TEAM; ++t)
+            for (int t = 0; t < TEAM; ++t)
 #pragma unroll
-                    for (int ks = 0; ks < 2; ++ks) o = E::mfma32(read_t(src + t * kTile, dl, dp, ks), bop[t][ks], o);
+                for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-                for (int gp = 0; gp < 2; ++gp) {
-                    const int g0 = 2 * gp, g1 = 2 * gp + 1;
-                    auto rx = __builtin_amdgcn_permlane32_swap(pack2<E>(o[4 * g0 + 0] * osc, o[4 * g0 + 1] * osc),
-                                                               pack2<E>(o[4 * g1 + 0] * osc, o[4 * g1 + 1] * osc), false, false);
-                    auto ry = __builtin_amdgcn_permlane32_swap(pack2<E>(o[4 * g0 + 2] * osc, o[4 * g0 + 3] * osc),
-                                                               pack2<E>(o[4 * g1 + 2] * osc, o[4 * g1 + 3] * osc), false, false);
-                    wd[dl][gp][0] = rx[0]; wd[dl][gp][1] = ry[0]; wd[dl][gp][2] = rx[1]; wd[dl][gp][3] = ry[1];
+                    for (int x = 0; x < 2 * N; ++x) o[x] = E::mfma32(read_t(src + t * kTile, x & 1, dp0 + (x >> 1), ks), bop[t][ks], o[x]);
+#pragma unroll
+            for (int dp = 0; dp < N; ++dp) {
+                uint32_t wd[2][2][4];                    // [block in pair][gp][dword]
+#pragma unroll
+                for (int dl = 0; dl < 2; ++dl) {
+                    const f32x16& a = o[2 * dp + dl];
+#pragma unroll
+                    for (int gp = 0; gp < 2; ++gp) {
+                        const int g0 = 2 * gp, g1 = 2 * gp + 1;
+                        auto rx = __builtin_amdgcn_permlane32_swap(pack2<E>(a[4 * g0 + 0] * osc, a[4 * g0 + 1] * osc),
+                                                                   pack2<E>(a[4 * g1 + 0] * osc, a[4 * g1 + 1] * osc), false, false);
+                        auto ry = __builtin_amdgcn_permlane32_swap(pack2<E>(a[4 * g0 + 2] * osc, a[4 * g0 + 3] * osc),
+                                                                   pack2<E>(a[4 * g1 + 2] * osc, a[4 * g1 + 3] * osc), false, false);
+                        wd[dl][gp][0] = rx[0]; wd[dl][gp][1] = ry[0]; wd[dl][gp][2] = rx[1]; wd[dl][gp][3] = ry[1];
+                    }
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        auto x = __builtin_amdgcn_permlane16_swap(wd[dl][0][q], wd[dl][1][q], false, false);
+                        wd[dl][0][q] = x[0]; wd[dl][1][q] = x[1];
+                    }
                 }
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    auto x = __builtin_amdgcn_permlane16_swap(wd[dl][0][q], wd[dl][1][q], false, false);
-                    wd[dl][0][q] = x[0]; wd[dl][1][q] = x[1];
-                }
-            }
+                for (int r4 = 0; r4 < 2; ++r4) {
+                    u32x4 lo, hi;
 #pragma unroll
-            for (int r4 = 0; r4 < 2; ++r4) {
-                u32x4 lo, hi;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const uint32_t x0 = wd[0][r4][q], x1 = wd[1][r4][q];
-                    // row_ror:8 within 16 lanes; bank mask 0xc writes lanes 8..15 of a row, 0x3 lanes 0..7
-                    lo[q] = (uint32_t)__builtin_amdgcn_update_dpp((int)x0, (int)x1, 0x128, 0xf, 0xc, false);
-                    hi[q] = (uint32_t)__builtin_amdgcn_update_dpp((int)x1, (int)x0, 0x128, 0xf, 0x3, false);
+                    for (int q = 0; q < 4; ++q) {
+                        const uint32_t x0 = wd[0][r4][q], x1 = wd[1][r4][q];
+                        // row_ror:8 within 16 lanes; bank mask 0xc writes lanes 8..15 of a row, 0x3 lanes 0..7
+                        lo[q] = (uint32_t)__builtin_amdgcn_update_dpp((int)x0, (int)x1, 0x128, 0xf, 0xc, false);
+                        hi[q] = (uint32_t)__builtin_amdgcn_update_dpp((int)x1, (int)x0, 0x128, 0xf, 0x3, false);
+                    }
+                    // non-temporal: the rows are read once, by the right factor's kernel, after this grid has finished.  Before
+                    // the last chunk every row exists, and the stores are counted by open_chunk.
+                    char* const at_lo = obase + (rowoff[2 * r4 + 0] + 128 * (dp0 + dp));
+                    char* const at_hi = obase + (rowoff[2 * r4 + 1] + 128 * (dp0 + dp));
+                    if (next >= 0) {
+                        __builtin_nontemporal_store(lo, (u32x4*)at_lo);
+                        __builtin_nontemporal_store(hi, (u32x4*)at_hi);
+                    } else {
+                        if (row_in[2 * r4 + 0]) __builtin_nontemporal_store(lo, (u32x4*)at_lo);
+                        if (row_in[2 * r4 + 1]) __builtin_nontemporal_store(hi, (u32x4*)at_hi);
+                    }
                 }
-                // non-temporal: the rows are read once, by the right factor's kernel, after this grid has finished
-                if (row_in[2 * r4 + 0]) __builtin_nontemporal_store(lo, (u32x4*)(obase + rowoff[2 * r4 + 0] + 64 * dp));
-                if (row_in[2 * r4 + 1]) __builtin_nontemporal_store(hi, (u32x4*)(obase + rowoff[2 * r4 + 1] + 64 * dp));
             }
         };
         if constexpr (SOLO) {
-#pragma unroll
-            for (int which = 0; which < 2; ++which)
-#pragma unroll
-                for (int dp = 0; dp < DT / 2; ++dp) half_rows(which, dp);
-        } else {
-            for (int x = wave; x < DT; x += TEAM) half_rows(x / (DT / 2), x % (DT / 2));
+            half_rows(0, 0, std::integral_constant<int, DT / 2>{});
+            half_rows(1, 0, std::integral_constant<int, DT / 2>{});
+        } else if (stores) {
+            half_rows(wave / (DT / 2), wave % (DT / 2), std::integral_constant<int, 1>{});
         }
     }
     if (p.dq && i0 + m < b1) {
@@ -548,10 +592,10 @@ void monarch_bwd_left_kernel(LeftArgs p) {
     }
 }
 
-template <class E, int D, int TEAM>
+template <class E, int D, int TEAM, bool FK>
 int launch_left(const LeftArgs& a, hipStream_t stream) {
     const size_t ldsb = LeftLds<D, TEAM>::bytes();
-    const void* fn = (const void*)monarch_bwd_left_kernel<E, D, TEAM>;
+    const void* fn = (const void*)monarch_bwd_left_kernel<E, D, TEAM, FK>;
     hipError_t e = hipSuccess;
     if (ldsb > 64 * 1024) e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsb);
     if (e != hipSuccess) {
@@ -559,7 +603,7 @@ int launch_left(const LeftArgs& a, hipStream_t stream) {
         return SFM_ERR_HIP;
     }
     const int per_wg = TEAM == 1 ? 4 : 1;
-    const dim3 grid((unsigned)xcd_grid((a.AJ + per_wg - 1) / per_wg * a.nunits)), block(TEAM == 1 ? 256 : 64 * TEAM);
+    const dim3 grid((unsigned)xcd_grid((a.AJ + per_wg - 1) / per_wg * a.nunits)), block(64 * LeftLds<D, TEAM>::kWaves);
     LeftArgs arg = a;
     void* kargs[] = {&arg};
     e = hipLaunchKernel(fn, grid, block, kargs, ldsb, stream);
@@ -568,6 +612,11 @@ int launch_left(const LeftArgs& a, hipStream_t stream) {
         return SFM_ERR_HIP;
     }
     return SFM_OK;
+}
+
+template <class E, int D, int TEAM>
+int launch_left(const LeftArgs& a, hipStream_t stream) {
+    return a.r_pad > 0 ? launch_left<E, D, TEAM, true>(a, stream) : launch_left<E, D, TEAM, false>(a, stream);
 }
 
 template <class E, int D>
