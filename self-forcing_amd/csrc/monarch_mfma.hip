@@ -217,6 +217,7 @@ void monarch_step1_kernel(MonarchArgs p) {
     float wn = 1.f;                                        // IT: the weight of the next tile's representative (not AH: this tile's factor)
     uint32_t crow[4] = {0, 0, 0, 0};                       // byte offsets in the (f, k) slab of the four scratch rows this lane stores to
     uint32_t cloff = 0;                                    // same for cl
+    uint32_t roff[4] = {0, 0, 0, 0};                       // WR: of the four rows of R
     int qkey = -1;
     float wsc = 1.f;                                       // IT: the column's logits factor
 
@@ -285,6 +286,7 @@ void monarch_step1_kernel(MonarchArgs p) {
             for (int rb = 0; rb < 4; ++rb) {
                 const int sg = min(wave * 32 + (m & 7) + 8 * rb, cur.ncols - 1);
                 crow[rb] = (uint32_t)(cur.a0 * b2 + sg) * p.ws_aj * (D * 2) + piece;
+                if (WR) roff[rb] = (uint32_t)(cur.a0 * b2 + sg) * 128 + piece;
             }
         }
         if (r + 1 < rounds) {
@@ -354,13 +356,42 @@ void monarch_step1_kernel(MonarchArgs p) {
                 // R[l] for l = 16 st + 0..15: the lower half of the wave holds 0..3 and 8..11, the upper half 4..7 and
                 // 12..15; exchanging the lower half's second pair with the upper half's first leaves 8 consecutive values
                 const size_t r0 = (size_t)cur.ul * p.rb_unit + (uint32_t)cur.k * p.rb_k + (uint32_t)cur.f * p.rb_f;
-                char* rrow = (char*)p.rb + (r0 + cloff / 4) * 128 + 16 * hf;
+                u32x4 w[2 * NT];
 #pragma unroll
                 for (int st = 0; st < 2 * NT; ++st) {
                     auto rx = __builtin_amdgcn_permlane32_swap(pb[st].x, pb[st].z, false, false);
                     auto ry = __builtin_amdgcn_permlane32_swap(pb[st].y, pb[st].w, false, false);
-                    const u32x4 w = {(uint32_t)rx[0], (uint32_t)ry[0], (uint32_t)rx[1], (uint32_t)ry[1]};
-                    *(u32x4*)(rrow + 32 * st) = w;
+                    w[st] = u32x4{(uint32_t)rx[0], (uint32_t)ry[0], (uint32_t)rx[1], (uint32_t)ry[1]};
+                }
+                if constexpr (NT == 2) {
+                    // Eight whole rows of 128 bytes per store and past the caches, like the rows of Kbar and Y below and by the
+                    // same exchanges: 32-byte pieces of 32 rows, written back under step 2, cost that kernel 18 us (12 heads,
+                    // 4680 x 32760: 139 -> 121).
+                    char* rbase = (char*)p.rb + r0 * 128;
+                    u32x4 row[2][2];
+#pragma unroll
+                    for (int dl = 0; dl < 2; ++dl)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            auto x = __builtin_amdgcn_permlane16_swap(w[2 * dl][q], w[2 * dl + 1][q], false, false);
+                            row[dl][0][q] = x[0];
+                            row[dl][1][q] = x[1];
+                        }
+#pragma unroll
+                    for (int r4 = 0; r4 < 2; ++r4) {
+                        u32x4 lo, hi;
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            lo[q] = (uint32_t)__builtin_amdgcn_update_dpp((int)row[0][r4][q], (int)row[1][r4][q], 0x128, 0xf, 0xc, false);
+                            hi[q] = (uint32_t)__builtin_amdgcn_update_dpp((int)row[1][r4][q], (int)row[0][r4][q], 0x128, 0xf, 0x3, false);
+                        }
+                        __builtin_nontemporal_store(lo, (u32x4*)(rbase + roff[2 * r4 + 0]));
+                        __builtin_nontemporal_store(hi, (u32x4*)(rbase + roff[2 * r4 + 1]));
+                    }
+                } else {
+                    char* rrow = (char*)p.rb + (r0 + cloff / 4) * 128 + 16 * hf;
+#pragma unroll
+                    for (int st = 0; st < 2 * NT; ++st) *(u32x4*)(rrow + 32 * st) = w[st];
                 }
             }
         }
