@@ -1145,6 +1145,11 @@ __global__ __launch_bounds__(64 * (RepLds<D, NQ>::kWaves)) void monarch_rep_kern
 // heads x 128: 604 MB) 148 us where the two kernels took 69 + 150, bound by that traffic; at three (three frames tied: 201
 // MB) 75 for 46 + 62, where one workgroup fills a compute unit and its loads, logits, reductions and stores follow each
 // other.  (98 with every value's maximum and sum reduced in all lanes, and with exp2f.)
+// RUN: a workgroup walks a run of columns, the next one's first chunk requested as soon as this one's has been read; the products
+// of all chunks share their query rows, and the representatives leave in whole lines, past the caches: 75 -> 70 us at three
+// frames tied.  A column's 44 000 cycles there: logits 8500, maxima, exponentials and sums 6500, waiting for the other waves
+// 2800, scales and weights 3300, representatives and their stores 10 000, the next column's query rows behind the stores of all
+// compute units 12 000.  Held in registers until those rows are requested, the representatives spill (81 us and more).
 // ------------------------------------------------------------------------------------------------
 template <int D, int NQ, int W>
 struct WtLds {
@@ -1188,8 +1193,8 @@ __device__ __forceinline__ float half_reduce(float* x, int m) {
     return op(x[0], dpp_move<0xb1>(x[0]));                                               // quad_perm:[1,0,3,2]
 }
 
-template <class E, int D, int NQ, int W, int C>
-__global__ __launch_bounds__(64 * (WtLds<D, NQ, W>::kWaves)) __attribute__((amdgpu_waves_per_eu(2, 2))) void monarch_weights_kernel(MonarchArgs p) {
+template <class E, int D, int NQ, int W, int C, bool RUN>
+__global__ __launch_bounds__(64 * (WtLds<D, NQ, W>::kWaves)) __attribute__((amdgpu_waves_per_eu(2, 2))) void monarch_weights_kernel(MonarchArgs p, int items) {
     using L = WtLds<D, NQ, W>;
     constexpr int DS = D / 16, DT = D / 32, CPR = D / 8;
     constexpr int NG = CPR / 2;                            // 1 KB pieces of a chunk
@@ -1197,216 +1202,346 @@ __global__ __launch_bounds__(64 * (WtLds<D, NQ, W>::kWaves)) __attribute__((amdg
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lane = tid & 63;
-    const int m = lane & 31;
-    const int hf = lane >> 5;
 
     const int b2 = p.b2;
     const int njg = (b2 + L::kCols - 1) / L::kCols;
-    const int a = blockIdx.x / njg;
     const int col = W == 1 ? wave : 0;                     // this wave's column of the workgroup's
-    const int j = min((int)(blockIdx.x % njg) * L::kCols + col, b2 - 1);      // past the last column: that one again, with the same results
     const int w = W == 1 ? 0 : wave;                       // its chunks: w, w + W, ...
-    const int ul = blockIdx.y;
-    const int unit = p.unit0 + ul;
-    const int b = unit / p.H, h = unit % p.H;
+    // an item is a workgroup's columns (unit, a, kCols of j); RUN: every workgroup takes an equal run of them, else a unit's in x
+    int item = RUN ? (int)((int64_t)items * blockIdx.x / gridDim.x) : (int)blockIdx.x;
+    const int end = RUN ? (int)((int64_t)items * (blockIdx.x + 1) / gridDim.x) : 0;
 
     const int r_lim = p.nf * p.b1;
     const int nch = (r_lim + 31) / 32;
-    const int64_t blk = (int64_t)ul * p.ws_unit + (int64_t)(a * b2 + j) * p.ws_aj;
-    const char* kb = (const char*)p.kbar + blk * (2 * D);
-    const char* clp = (const char*)(p.cl + (int64_t)ul * p.cl_unit + (int64_t)(a * b2 + j) * p.cl_aj);
     const uint32_t cl_ld = p.cl_row * 4;
-    char* repb = (char*)p.rep + blk * (2 * D);
-    float* wgt = p.wgt + blk;
+    struct Column {
+        int ul, a, j;
+        int64_t blk;       // its first scratch row
+    };
+    auto column = [&](int x) {
+        Column c;
+        const int g = x / njg;
+        c.j = min((x - g * njg) * L::kCols + col, b2 - 1);      // past the last column: that one again, with the same results
+        c.ul = RUN ? g / p.na : (int)blockIdx.y;
+        c.a = RUN ? g - c.ul * p.na : g;
+        c.blk = (int64_t)c.ul * p.ws_unit + (int64_t)(c.a * b2 + c.j) * p.ws_aj;
+        return c;
+    };
 
     char* const wl = lds_s2 + wave * L::kWave;
     const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)wl;
     char* const qt = lds_s2 + L::kWaves * L::kWave + col * NQ * L::kTile;     // the column's query rows, laid out like chunks of scratch rows
     const uint32_t qt0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)qt;
 
-    // query rows into LDS (rows past b1 repeat the last one; their scale is zero)
-    const uint16_t* qg = (const uint16_t*)p.q + (int64_t)b * p.qs[0] + (int64_t)h * p.qs[2];
-    for (int g = w; g < NQ * NG; g += W) {
-        const int P = g * 64 + lane;
-        const int r = P / CPR, c = (P % CPR) ^ s1_swz<CPR>(r);
-        const uint32_t off = (uint32_t)((p.qmap.row(a, min(r, p.b1 - 1)) + j) * p.qs[1] * 2) + (uint32_t)c * 16;
-        s1_load_lds16((const char*)qg, off, qt0 + (uint32_t)g * 1024);
-    }
-    auto issue = [&](int n, int buf) {
-        const uint32_t dst = lds0 + (uint32_t)buf * L::kBuf;
-#pragma unroll
-        for (int g = 0; g < NG; ++g) {
-            const int P = g * 64 + lane;
-            const int r = P / CPR, c = (P % CPR) ^ s1_swz<CPR>(r);
-            const uint32_t off = (uint32_t)min(32 * n + r, r_lim - 1) * (2 * D) + (uint32_t)c * 16;
-            s1_load_lds16(kb, off, dst + (uint32_t)g * 1024);
-        }
-        s2_load_lds4(clp, (uint32_t)(32 * n + m) * cl_ld, dst + L::kTile);
-    };
-    if (w < nch) issue(w, 0);
-    if (w + W < nch) issue(w + W, 1);
-    const uint32_t b_off = (uint32_t)m * L::kPitch + (uint32_t)((hf ^ s1_swz<CPR>(m)) << 4);   // row m of a 32-row tile as an MFMA operand
-    uint32_t tr[DT][2];            // Q^T as the representatives' A operand: transposing reads
-    {
-        const int s16 = lane & 15, g16 = lane >> 4;
-        const int rl = 4 * hf + (s16 >> 2);
-        const int cl = 2 * (g16 & 1) + ((s16 & 3) >> 1);
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-            for (int half = 0; half < 2; ++half) {
-                const int r = rl + 8 * half;
-                tr[dt][half] = (uint32_t)(r * L::kPitch + (((4 * dt + cl) ^ s1_swz<CPR>(r)) << 4) + (s16 & 1) * 8);
+    Column cur = column(item);
+    for (bool first = true;; ++item, first = false) {
+        // what follows from the lane is formed again for every item: kept, it does not fit beside the logits
+        int lane = tid & 63;
+        if (RUN) asm volatile("" : "+v"(lane));
+        const int m = lane & 31;
+        const int hf = lane >> 5;
+        // query rows into LDS (rows past b1 repeat the last one; their scale is zero)
+        auto queries = [&](const Column& x) {
+            const int unit = p.unit0 + x.ul;
+            const uint16_t* qg = (const uint16_t*)p.q + (int64_t)(unit / p.H) * p.qs[0] + (int64_t)(unit % p.H) * p.qs[2];
+            for (int g = w; g < NQ * NG; g += W) {
+                const int P = g * 64 + lane;
+                const int r = P / CPR, c = (P % CPR) ^ s1_swz<CPR>(r);
+                const uint32_t off = (uint32_t)((p.qmap.row(x.a, min(r, p.b1 - 1)) + x.j) * p.qs[1] * 2) + (uint32_t)c * 16;
+                s1_load_lds16((const char*)qg, off, qt0 + (uint32_t)g * 1024);
             }
-    }
-    const float sc2 = p.scale * kLog2e;
-    const f32x16 kZero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-
-    // this wave's share of the query rows has landed when only its first two chunks are outstanding
-    if (w + W < nch) wait_vm<2 * (NG + 1)>();
-    else if (w < nch) wait_vm<NG + 1>();
-    else wait_vm<0>();
-    lds_barrier();
-
-    f32x16 z[C][NQ];               // S[i = 32 qi + 8 g + 4 hf + e, r = 32 n + m], then its exponentials
+        };
+        auto issue = [&](const Column& x, int n, int buf) {
+            const char* const kb = (const char*)p.kbar + x.blk * (2 * D);
+            const char* const clp = (const char*)(p.cl + (int64_t)x.ul * p.cl_unit + (int64_t)(x.a * b2 + x.j) * p.cl_aj);
+            const uint32_t dst = lds0 + (uint32_t)buf * L::kBuf;
 #pragma unroll
-    for (int c = 0; c < C; ++c) {
-        const int n = w + c * W;
-        if (n >= nch) {
+            for (int g = 0; g < NG; ++g) {
+                const int P = g * 64 + lane;
+                const int r = P / CPR, c = (P % CPR) ^ s1_swz<CPR>(r);
+                const uint32_t off = (uint32_t)min(32 * n + r, r_lim - 1) * (2 * D) + (uint32_t)c * 16;
+                s1_load_lds16(kb, off, dst + (uint32_t)g * 1024);
+            }
+            s2_load_lds4(clp, (uint32_t)(32 * n + m) * cl_ld, dst + L::kTile);
+        };
+        const uint32_t b_off = (uint32_t)m * L::kPitch + (uint32_t)((hf ^ s1_swz<CPR>(m)) << 4);   // row m of a 32-row tile as an MFMA operand
+        uint32_t tr[DT][2];            // Q^T as the representatives' A operand: transposing reads
+        {
+            const int s16 = lane & 15, g16 = lane >> 4;
+            const int rl = 4 * hf + (s16 >> 2);
+            const int cl = 2 * (g16 & 1) + ((s16 & 3) >> 1);
 #pragma unroll
-            for (int qi = 0; qi < NQ; ++qi)
+            for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) z[c][qi][v] = -INFINITY;
-            continue;
+                for (int half = 0; half < 2; ++half) {
+                    const int r = rl + 8 * half;
+                    tr[dt][half] = (uint32_t)(r * L::kPitch + (((4 * dt + cl) ^ s1_swz<CPR>(r)) << 4) + (s16 & 1) * 8);
+                }
         }
-        // chunk n has landed when only the one requested after it is outstanding
-        if (n + W < nch) wait_vm<NG + 1>();
-        else wait_vm<0>();
-        const char* kt = wl + (c & 1) * L::kBuf;
-        const float cc = *(const float*)(kt + L::kTile + m * 4);
-        const bool rok = 32 * n + m < r_lim;
+        const float sc2 = p.scale * kLog2e;
+        const f32x16 kZero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (first) {
+            queries(cur);
+            if (w < nch) issue(cur, w, 0);
+            if (w + W < nch) issue(cur, w + W, 1);
+            // this wave's share of the query rows has landed when only its first two chunks are outstanding
+            if (w + W < nch) wait_vm<2 * (NG + 1)>();
+            else if (w < nch) wait_vm<NG + 1>();
+            else wait_vm<0>();
+            lds_barrier();
+        }
+        const bool more = RUN && item + 1 < end;           // uniform over the workgroup
+        const Column next = RUN ? column(more ? item + 1 : item) : cur;
+        f32x16 z[C][NQ];               // S[i = 32 qi + 8 g + 4 hf + e, r = 32 n + m], then its exponentials
 #pragma unroll
-        for (int qi = 0; qi < NQ; ++qi) {
-            f32x16 t;
+        for (int c = 0; c < C; ++c) {
+            const int n = w + c * W;
+            if (n >= nch) {
+#pragma unroll
+                for (int qi = 0; qi < NQ; ++qi)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) z[c][qi][v] = -INFINITY;
+                continue;
+            }
+            // chunk n has landed when only the one requested after it is outstanding
+            if (n + W < nch) wait_vm<NG + 1>();
+            else wait_vm<0>();
+            const char* kt = wl + (c & 1) * L::kBuf;
+            const float cc = *(const float*)(kt + L::kTile + m * 4);
+            const bool rok = 32 * n + m < r_lim;
+            // a row of Kbar is read once for the query tiles, whose products are independent chains
 #pragma unroll
             for (int ds = 0; ds < DS; ++ds) {
                 const u32x4 bk = *(const u32x4*)(kt + (b_off ^ (uint32_t)(ds << 5)));
-                const u32x4 aq = *(const u32x4*)(qt + qi * L::kTile + (b_off ^ (uint32_t)(ds << 5)));
-                t = E::mfma32(aq, bk, ds ? t : kZero);
-            }
 #pragma unroll
-            for (int v = 0; v < 16; ++v) z[c][qi][v] = rok ? t[v] * sc2 - cc : -INFINITY;
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // the chunk has been read: the next but one may land on it
-        if (n + 2 * W < nch) issue(n + 2 * W, c & 1);
-    }
-
-    // Rows' maxima and sums over this wave's chunks, to the (dead) front of its chunk buffers: [NQ * 32] maxima, sums
-    float* const own = (float*)wl;
-    const int at = half_reduce_at(m), myrow = 8 * (at >> 2) + 4 * hf + (at & 3);
-#pragma unroll
-    for (int qi = 0; qi < NQ; ++qi) {
-        float t[16];
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            t[v] = z[0][qi][v];
-#pragma unroll
-            for (int c = 1; c < C; ++c) t[v] = fmaxf(t[v], z[c][qi][v]);
-        }
-        own[32 * qi + myrow] = half_reduce<true>(t, m);
-    }
-    lds_wave_sync();
-#pragma unroll
-    for (int qi = 0; qi < NQ; ++qi) {
-        float t[16];
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const f32x4 mx = *(const f32x4*)(own + 32 * qi + 8 * g + 4 * hf);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float base = mx[e] == -INFINITY ? 0.f : mx[e];       // a wave without chunks
-                t[4 * g + e] = 0.f;
-#pragma unroll
-                for (int c = 0; c < C; ++c) {
-                    z[c][qi][4 * g + e] = fast_exp2(z[c][qi][4 * g + e] - base);
-                    t[4 * g + e] += z[c][qi][4 * g + e];
+                for (int qi = 0; qi < NQ; ++qi) {
+                    const u32x4 aq = *(const u32x4*)(qt + qi * L::kTile + (b_off ^ (uint32_t)(ds << 5)));
+                    z[c][qi] = E::mfma32(aq, bk, ds ? z[c][qi] : kZero);
                 }
             }
-        }
-        own[NQ * 32 + 32 * qi + myrow] = half_reduce<false>(t, m);
-    }
-    if (W > 1) lds_barrier();
-    else lds_wave_sync();
-    // scale of row i for this wave: exp2(max_wave - max) / sum, behind the maxima and sums that other waves still read
-    for (int i = lane; i < NQ * 32; i += 64) {
-        float M = -INFINITY, sum = 0.f;
-#pragma unroll
-        for (int x = 0; x < W; ++x) M = fmaxf(M, *(const float*)((W == 1 ? wl : lds_s2 + x * L::kWave) + i * 4));
-#pragma unroll
-        for (int x = 0; x < W; ++x) {
-            const float* o = (const float*)(W == 1 ? wl : lds_s2 + x * L::kWave);
-            sum += o[NQ * 32 + i] * exp2f(o[i] - M);             // a wave without chunks: 0 * exp2(-inf)
-        }
-        own[2 * NQ * 32 + i] = i < p.b1 ? exp2f(own[i] - M) / sum : 0.f;
-    }
-    lds_wave_sync();
-
-#pragma unroll
-    for (int qi = 0; qi < NQ; ++qi)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const f32x4 fac = *(const f32x4*)(own + 2 * NQ * 32 + 32 * qi + 8 * g + 4 * hf);
-#pragma unroll
-            for (int c = 0; c < C; ++c)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) z[c][qi][4 * g + e] *= fac[e];
-        }
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-        const int n = w + c * W;
-        if (n >= nch) break;
-        float wsum = 0.f;
-        u32x4 pb[NQ][2];
-#pragma unroll
-        for (int qi = 0; qi < NQ; ++qi) {
-#pragma unroll
-            for (int v = 0; v < 16; ++v) wsum += z[c][qi][v];
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                pb[qi][q].x = pack2<E>(z[c][qi][8 * q + 0], z[c][qi][8 * q + 1]);
-                pb[qi][q].y = pack2<E>(z[c][qi][8 * q + 2], z[c][qi][8 * q + 3]);
-                pb[qi][q].z = pack2<E>(z[c][qi][8 * q + 4], z[c][qi][8 * q + 5]);
-                pb[qi][q].w = pack2<E>(z[c][qi][8 * q + 6], z[c][qi][8 * q + 7]);
-            }
-        }
-        wsum = xhalf_sum(wsum);
-        if (hf == 0) wgt[32 * n + m] = wsum;
-        char* rrow = repb + (size_t)(32 * n + m) * (2 * D);
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-            f32x16 acc;
 #pragma unroll
             for (int qi = 0; qi < NQ; ++qi)
 #pragma unroll
-                for (int q = 0; q < 2; ++q) {
-                    const u32x2 lo = s1_read_tr(qt + qi * L::kTile, tr[dt][0] + q * 16 * L::kPitch);
-                    const u32x2 hi = s1_read_tr(qt + qi * L::kTile, tr[dt][1] + q * 16 * L::kPitch);
-                    const u32x4 aq = {lo.x, lo.y, hi.x, hi.y};
-                    acc = E::mfma32(aq, pb[qi][q], (qi | q) ? acc : kZero);
-                }
-            // rep^T[d = 32 dt + 8 g + 4 hf + e, r]: the half-swap leaves 8 consecutive d per lane
+                for (int v = 0; v < 16; ++v) z[c][qi][v] = z[c][qi][v] * sc2 - cc;
+            if (32 * n + 32 > r_lim) {                       // uniform: the last chunk, where it is not a whole one
 #pragma unroll
-            for (int gp = 0; gp < 2; ++gp) {
-                const int g0 = 2 * gp, g1 = 2 * gp + 1;
-                auto rx = __builtin_amdgcn_permlane32_swap(pack2<E>(acc[4 * g0 + 0], acc[4 * g0 + 1]),
-                                                           pack2<E>(acc[4 * g1 + 0], acc[4 * g1 + 1]), false, false);
-                auto ry = __builtin_amdgcn_permlane32_swap(pack2<E>(acc[4 * g0 + 2], acc[4 * g0 + 3]),
-                                                           pack2<E>(acc[4 * g1 + 2], acc[4 * g1 + 3]), false, false);
-                const u32x4 o = {(uint32_t)rx[0], (uint32_t)ry[0], (uint32_t)rx[1], (uint32_t)ry[1]};
-                *(u32x4*)(rrow + (32 * dt + 16 * gp + 8 * hf) * 2) = o;
+                for (int qi = 0; qi < NQ; ++qi)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) z[c][qi][v] = rok ? z[c][qi][v] : -INFINITY;
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // the chunk has been read: the next but one may land on it
+            if (n + 2 * W < nch) issue(cur, n + 2 * W, c & 1);
+        }
+        if (more && w < nch) issue(next, w, 0);                      // both chunk buffers have been read
+
+        // Rows' maxima and sums over this wave's chunks, to the front of its second chunk buffer: [NQ * 32] maxima, sums
+        float* const own = (float*)(wl + L::kBuf);
+        const int at = half_reduce_at(m), myrow = 8 * (at >> 2) + 4 * hf + (at & 3);
+#pragma unroll
+        for (int qi = 0; qi < NQ; ++qi) {
+            float t[16];
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                t[v] = z[0][qi][v];
+#pragma unroll
+                for (int c = 1; c < C; ++c) t[v] = fmaxf(t[v], z[c][qi][v]);
+            }
+            own[32 * qi + myrow] = half_reduce<true>(t, m);
+        }
+        lds_wave_sync();
+#pragma unroll
+        for (int qi = 0; qi < NQ; ++qi) {
+            float t[16];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const f32x4 mx = *(const f32x4*)(own + 32 * qi + 8 * g + 4 * hf);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float base = mx[e] == -INFINITY ? 0.f : mx[e];       // a wave without chunks
+                    t[4 * g + e] = 0.f;
+#pragma unroll
+                    for (int c = 0; c < C; ++c) {
+                        z[c][qi][4 * g + e] = fast_exp2(z[c][qi][4 * g + e] - base);
+                        t[4 * g + e] += z[c][qi][4 * g + e];
+                    }
+                }
+            }
+            own[NQ * 32 + 32 * qi + myrow] = half_reduce<false>(t, m);
+        }
+        if (W > 1) lds_barrier();
+        else lds_wave_sync();
+        // scale of row i for this wave: exp2(max_wave - max) / sum, behind the maxima and sums that other waves still read
+        for (int i = lane; i < NQ * 32; i += 64) {
+            float mx[W], sm[W], M = -INFINITY, sum = 0.f;
+#pragma unroll
+            for (int x = 0; x < W; ++x) {
+                const float* o = (const float*)((W == 1 ? wl : lds_s2 + x * L::kWave) + L::kBuf);
+                mx[x] = o[i];
+                sm[x] = o[NQ * 32 + i];
+            }
+#pragma unroll
+            for (int x = 0; x < W; ++x) M = fmaxf(M, mx[x]);
+#pragma unroll
+            for (int x = 0; x < W; ++x) sum += sm[x] * fast_exp2(mx[x] - M);          // a wave without chunks: 0 * exp2(-inf)
+            own[2 * NQ * 32 + i] = i < p.b1 ? fast_exp2(own[i] - M) / sum : 0.f;
+        }
+        lds_wave_sync();
+
+#pragma unroll
+        for (int qi = 0; qi < NQ; ++qi)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const f32x4 fac = *(const f32x4*)(own + 2 * NQ * 32 + 32 * qi + 8 * g + 4 * hf);
+#pragma unroll
+                for (int c = 0; c < C; ++c)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) z[c][qi][4 * g + e] *= fac[e];
+            }
+        if constexpr (RUN) {
+            // weights; the scaled values become the B operands of the representatives
+            u32x4 pb[C][NQ][2];
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                const int n = w + c * W;
+                float wsum = 0.f;
+#pragma unroll
+                for (int qi = 0; qi < NQ; ++qi) {
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) wsum += z[c][qi][v];
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        pb[c][qi][q].x = pack2<E>(z[c][qi][8 * q + 0], z[c][qi][8 * q + 1]);
+                        pb[c][qi][q].y = pack2<E>(z[c][qi][8 * q + 2], z[c][qi][8 * q + 3]);
+                        pb[c][qi][q].z = pack2<E>(z[c][qi][8 * q + 4], z[c][qi][8 * q + 5]);
+                        pb[c][qi][q].w = pack2<E>(z[c][qi][8 * q + 6], z[c][qi][8 * q + 7]);
+                    }
+                }
+                wsum = xhalf_sum(wsum);
+                if (n < nch && hf == 0) p.wgt[cur.blk + 32 * n + m] = wsum;
+            }
+            // rep^T[d = 32 dt + 8 g + 4 hf + e, r], a pair of head-dim blocks at a time: their query rows are read once for all
+            // chunks, whose products are independent chains, and the exchanges of step 1 leave whole lines to store, 128 bytes of
+            // each of 8 rows an instruction.
+            const uint32_t piece = (uint32_t)(4 * ((m >> 3) & 1) + 2 * ((m >> 4) & 1) + hf) * 16;
+#pragma unroll
+            for (int dp = 0; dp < DT / 2; ++dp) {
+                u32x4 aq[2][NQ][2];
+#pragma unroll
+                for (int dl = 0; dl < 2; ++dl)
+#pragma unroll
+                    for (int qi = 0; qi < NQ; ++qi)
+#pragma unroll
+                        for (int q = 0; q < 2; ++q) {
+                            const u32x2 lo = s1_read_tr(qt + qi * L::kTile, tr[2 * dp + dl][0] + q * 16 * L::kPitch);
+                            const u32x2 hi = s1_read_tr(qt + qi * L::kTile, tr[2 * dp + dl][1] + q * 16 * L::kPitch);
+                            aq[dl][qi][q] = u32x4{lo.x, lo.y, hi.x, hi.y};
+                        }
+#pragma unroll
+                for (int c = 0; c < C; ++c) {
+                    const int n = w + c * W;
+                    if (n >= nch) break;
+                    f32x16 acc[2];
+#pragma unroll
+                    for (int qi = 0; qi < NQ; ++qi)
+#pragma unroll
+                        for (int q = 0; q < 2; ++q)
+#pragma unroll
+                            for (int dl = 0; dl < 2; ++dl) acc[dl] = E::mfma32(aq[dl][qi][q], pb[c][qi][q], (qi | q) ? acc[dl] : kZero);
+                    uint32_t x[2][2][4];             // [block in pair][gp][dword]
+#pragma unroll
+                    for (int dl = 0; dl < 2; ++dl) {
+#pragma unroll
+                        for (int gp = 0; gp < 2; ++gp) {
+                            const int g0 = 2 * gp, g1 = 2 * gp + 1;
+                            auto rx = __builtin_amdgcn_permlane32_swap(pack2<E>(acc[dl][4 * g0 + 0], acc[dl][4 * g0 + 1]),
+                                                                       pack2<E>(acc[dl][4 * g1 + 0], acc[dl][4 * g1 + 1]), false, false);
+                            auto ry = __builtin_amdgcn_permlane32_swap(pack2<E>(acc[dl][4 * g0 + 2], acc[dl][4 * g0 + 3]),
+                                                                       pack2<E>(acc[dl][4 * g1 + 2], acc[dl][4 * g1 + 3]), false, false);
+                            x[dl][gp][0] = rx[0]; x[dl][gp][1] = ry[0]; x[dl][gp][2] = rx[1]; x[dl][gp][3] = ry[1];
+                        }
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            auto y = __builtin_amdgcn_permlane16_swap(x[dl][0][q], x[dl][1][q], false, false);
+                            x[dl][0][q] = y[0]; x[dl][1][q] = y[1];
+                        }
+                    }
+                    char* const rows = (char*)p.rep + (cur.blk + 32 * n + (m & 7)) * (2 * D) + 128 * dp + piece;
+#pragma unroll
+                    for (int r4 = 0; r4 < 2; ++r4) {
+                        u32x4 lo, hi;
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            lo[q] = (uint32_t)__builtin_amdgcn_update_dpp((int)x[0][r4][q], (int)x[1][r4][q], 0x128, 0xf, 0xc, false);
+                            hi[q] = (uint32_t)__builtin_amdgcn_update_dpp((int)x[1][r4][q], (int)x[0][r4][q], 0x128, 0xf, 0x3, false);
+                        }
+                        u32x4* const at = (u32x4*)(rows + 2 * r4 * 8 * (2 * D));
+                        u32x4* const at_hi = (u32x4*)(rows + (2 * r4 + 1) * 8 * (2 * D));
+                        __builtin_nontemporal_store(lo, at);
+                        __builtin_nontemporal_store(hi, at_hi);
+                    }
+                }
+            }
+        } else {
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                const int n = w + c * W;
+                if (n >= nch) break;
+                float wsum = 0.f;
+                u32x4 pb[NQ][2];
+#pragma unroll
+                for (int qi = 0; qi < NQ; ++qi) {
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) wsum += z[c][qi][v];
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        pb[qi][q].x = pack2<E>(z[c][qi][8 * q + 0], z[c][qi][8 * q + 1]);
+                        pb[qi][q].y = pack2<E>(z[c][qi][8 * q + 2], z[c][qi][8 * q + 3]);
+                        pb[qi][q].z = pack2<E>(z[c][qi][8 * q + 4], z[c][qi][8 * q + 5]);
+                        pb[qi][q].w = pack2<E>(z[c][qi][8 * q + 6], z[c][qi][8 * q + 7]);
+                    }
+                }
+                wsum = xhalf_sum(wsum);
+                if (hf == 0) p.wgt[cur.blk + 32 * n + m] = wsum;
+                char* rrow = (char*)p.rep + (cur.blk + 32 * n + m) * (2 * D);
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) {
+                    f32x16 acc;
+#pragma unroll
+                    for (int qi = 0; qi < NQ; ++qi)
+#pragma unroll
+                        for (int q = 0; q < 2; ++q) {
+                            const u32x2 lo = s1_read_tr(qt + qi * L::kTile, tr[dt][0] + q * 16 * L::kPitch);
+                            const u32x2 hi = s1_read_tr(qt + qi * L::kTile, tr[dt][1] + q * 16 * L::kPitch);
+                            const u32x4 aq = {lo.x, lo.y, hi.x, hi.y};
+                            acc = E::mfma32(aq, pb[qi][q], (qi | q) ? acc : kZero);
+                        }
+                    // rep^T[d = 32 dt + 8 g + 4 hf + e, r]: the half-swap leaves 8 consecutive d per lane
+#pragma unroll
+                    for (int gp = 0; gp < 2; ++gp) {
+                        const int g0 = 2 * gp, g1 = 2 * gp + 1;
+                        auto rx = __builtin_amdgcn_permlane32_swap(pack2<E>(acc[4 * g0 + 0], acc[4 * g0 + 1]),
+                                                                   pack2<E>(acc[4 * g1 + 0], acc[4 * g1 + 1]), false, false);
+                        auto ry = __builtin_amdgcn_permlane32_swap(pack2<E>(acc[4 * g0 + 2], acc[4 * g0 + 3]),
+                                                                   pack2<E>(acc[4 * g1 + 2], acc[4 * g1 + 3]), false, false);
+                        const u32x4 o = {(uint32_t)rx[0], (uint32_t)ry[0], (uint32_t)rx[1], (uint32_t)ry[1]};
+                        *(u32x4*)(rrow + (32 * dt + 16 * gp + 8 * hf) * 2) = o;
+                    }
+                }
             }
         }
+        if (!more) return;
+        // The next column's first chunk is on its way since its buffer was read; the queries take the place of this one's, and
+        // the second chunk that of the maxima and sums, when every wave is done with them.
+        lds_barrier();
+        cur = next;
+        queries(cur);
+        if (w + W < nch) {
+            issue(cur, w + W, 1);
+            wait_vm<NG + 1>();
+        } else {
+            wait_vm<0>();
+        }
+        lds_barrier();
     }
 }
 
@@ -1606,11 +1741,18 @@ template <class E, int D, int NQ, int W, int C>
 static bool launch_weights_t(const MonarchArgs& a, int nunits, hipStream_t stream, int* rc) {
     using L = WtLds<D, NQ, W>;
     if ((a.nf * a.b1 + 31) / 32 > W * C) return false;
-    const void* fn = (const void*)monarch_weights_kernel<E, D, NQ, W, C>;
+    int items = nunits * a.na * ((a.b2 + L::kCols - 1) / L::kCols);
+    const int room = std::min((int)(160 * 1024 / L::bytes()), 8 / L::kWaves) * cu_count();      // workgroups at a time
+    // More columns than the chip holds at a time are taken in runs, unless the representatives are so small that the next pass finds
+    // them in the caches, which these kernels store past: three passes at three frames tied (100 MB) 444 us against 471, 5 heads x 64
+    // of 23 x 41, 15 frames (9 MB) 137 against 127.  One query tile gains 1 % at most and loses 8 % where columns are few.
+    constexpr bool kRun = NQ > 1 && !(D == 64 && NQ == 3);    // (registers)
+    const bool run = kRun && items > room && (int64_t)nunits * a.na * a.b2 * a.r_pad * (2 * D) > (int64_t)64 << 20;
+    const void* fn = run ? (const void*)monarch_weights_kernel<E, D, NQ, W, C, kRun> : (const void*)monarch_weights_kernel<E, D, NQ, W, C, false>;
     hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)L::bytes());
     MonarchArgs a1 = a;
-    void* args[] = {&a1};
-    if (e == hipSuccess) e = hipLaunchKernel(fn, dim3(a.na * ((a.b2 + L::kCols - 1) / L::kCols), nunits), dim3(64 * L::kWaves), args, L::bytes(), stream);
+    void* args[] = {&a1, &items};
+    if (e == hipSuccess) e = hipLaunchKernel(fn, run ? dim3(room) : dim3(items / nunits, nunits), dim3(64 * L::kWaves), args, L::bytes(), stream);
     if (e != hipSuccess) set_error("hip launch failed: %s", hipGetErrorString(e));
     *rc = e == hipSuccess ? SFM_OK : SFM_ERR_HIP;
     return true;

@@ -212,6 +212,23 @@ def test_refinement_around_query_tiles_and_row_chunks(b1, fk, D):
     assert_close_16bit(out, ref, torch.bfloat16)
 
 
+# two and three query tiles; row chunks below, at and past the number of waves, whole and ragged; runs of equal and unequal length
+@pytest.mark.parametrize("b1,fk,cols,H,D", [(36, 6, 50, 24, 128), (64, 8, 19, 28, 128), (45, 21, 36, 8, 128), (40, 24, 50, 11, 64), (90, 7, 52, 8, 128),
+                                            (65, 11, 24, 16, 128)])
+def test_refinement_in_runs_of_columns(b1, fk, cols, H, D):
+    """More columns than the chip holds at a time, with representatives beyond 64 MiB, are taken several to a workgroup: the bits of
+    passes that give every column its own, and one head against the oracle."""
+    q = randn((1, b1 * cols, H, D), 430 + b1, torch.bfloat16)
+    k, v = (randn((1, fk * b1 * cols, H, D), 431 + b1 + i, torch.bfloat16) for i in range(2))
+    qd, kd, vd = (t.to(DEV) for t in (q, k, v))
+    out = mattn.monarch_attn(qd, kd, vd, 1, 1, 1, b1, cols, num_iters=3)
+    part = mattn.monarch_attn(qd, kd, vd, 1, 1, 1, b1, cols, num_iters=3, heads_per_pass=3)
+    assert torch.equal(out, part)
+    h = H - 1
+    ref = monarch.monarch_attn(q[:, :, h:], k[:, :, h:], v[:, :, h:], 1, 1, 1, b1, cols, num_iters=3, dtype=torch.float32)
+    assert_close_16bit(out[:, :, h:], ref, torch.bfloat16)
+
+
 def test_mfma_refinement_golden_vectors_in_bf16():
     """The reference's own refinement outputs (float64 golden vectors), inputs rounded to bf16: D = 64 case of the
     fixture, num_iters 2, 3 and 8, on the MFMA kernels."""
