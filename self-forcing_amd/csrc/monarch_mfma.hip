@@ -403,59 +403,66 @@ void monarch_step1_kernel(MonarchArgs p) {
         // bit 3 for the block within the pair (a rotation by 8 within rows of 16 lanes).  Afterwards a lane
         // holds, for each of the four row groups rb, the piece 4 (dt0 + bit 3) + 2 bit 4 + hf of column
         // (c & 7) + 8 rb, so that one store instruction writes 128 contiguous bytes of each of 8 rows.
+        // Past the caches or through them: see enqueue_step1
+        auto contract = [&](auto cached) {
 #pragma unroll
-        for (int which = 0; which < (KO ? 1 : 2); ++which) {
-            const char* tbase = which == 0 ? kt : vt;
-            char* og = (char*)(which == 0 ? p.kbar : p.y) + (size_t)srow * (D * 2);
+            for (int which = 0; which < (KO ? 1 : 2); ++which) {
+                const char* tbase = which == 0 ? kt : vt;
+                char* og = (char*)(which == 0 ? p.kbar : p.y) + (size_t)srow * (D * 2);
 #pragma unroll
-            for (int dp = 0; dp < D / 64; ++dp) {
-                uint32_t w[2][2][4];             // [block in pair][gp][dword]
+                for (int dp = 0; dp < D / 64; ++dp) {
+                    uint32_t w[2][2][4];             // [block in pair][gp][dword]
 #pragma unroll
-                for (int dl = 0; dl < 2; ++dl) {
-                    const int dt = 2 * dp + dl;
-                    f32x16 acc;
+                    for (int dl = 0; dl < 2; ++dl) {
+                        const int dt = 2 * dp + dl;
+                        f32x16 acc;
 #pragma unroll
-                    for (int st = 0; st < 2 * NT; ++st) {
-                        const u32x2 lo = s1_read_tr(tbase, tr[dt][0] + st * 16 * L::kPitch);
-                        const u32x2 hi = s1_read_tr(tbase, tr[dt][1] + st * 16 * L::kPitch);
-                        const u32x4 a = {lo.x, lo.y, hi.x, hi.y};
-                        acc = E::mfma32(a, pb[st], st ? acc : kZero);
+                        for (int st = 0; st < 2 * NT; ++st) {
+                            const u32x2 lo = s1_read_tr(tbase, tr[dt][0] + st * 16 * L::kPitch);
+                            const u32x2 hi = s1_read_tr(tbase, tr[dt][1] + st * 16 * L::kPitch);
+                            const u32x4 a = {lo.x, lo.y, hi.x, hi.y};
+                            acc = E::mfma32(a, pb[st], st ? acc : kZero);
+                        }
+#pragma unroll
+                        for (int gp = 0; gp < 2; ++gp) {
+                            const int g0 = 2 * gp, g1 = 2 * gp + 1;
+                            auto rx = __builtin_amdgcn_permlane32_swap(pack2<E>(acc[4 * g0 + 0], acc[4 * g0 + 1]),
+                                                                       pack2<E>(acc[4 * g1 + 0], acc[4 * g1 + 1]), false, false);
+                            auto ry = __builtin_amdgcn_permlane32_swap(pack2<E>(acc[4 * g0 + 2], acc[4 * g0 + 3]),
+                                                                       pack2<E>(acc[4 * g1 + 2], acc[4 * g1 + 3]), false, false);
+                            w[dl][gp][0] = rx[0]; w[dl][gp][1] = ry[0]; w[dl][gp][2] = rx[1]; w[dl][gp][3] = ry[1];
+                        }
+                        // lane bit 4 <-> gp: slot 0 then holds rows (c & 15), slot 1 rows (c & 15) + 16
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            auto x = __builtin_amdgcn_permlane16_swap(w[dl][0][q], w[dl][1][q], false, false);
+                            w[dl][0][q] = x[0]; w[dl][1][q] = x[1];
+                        }
                     }
+                    // lane bit 3 <-> block within the pair
 #pragma unroll
-                    for (int gp = 0; gp < 2; ++gp) {
-                        const int g0 = 2 * gp, g1 = 2 * gp + 1;
-                        auto rx = __builtin_amdgcn_permlane32_swap(pack2<E>(acc[4 * g0 + 0], acc[4 * g0 + 1]),
-                                                                   pack2<E>(acc[4 * g1 + 0], acc[4 * g1 + 1]), false, false);
-                        auto ry = __builtin_amdgcn_permlane32_swap(pack2<E>(acc[4 * g0 + 2], acc[4 * g0 + 3]),
-                                                                   pack2<E>(acc[4 * g1 + 2], acc[4 * g1 + 3]), false, false);
-                        w[dl][gp][0] = rx[0]; w[dl][gp][1] = ry[0]; w[dl][gp][2] = rx[1]; w[dl][gp][3] = ry[1];
+                    for (int r4 = 0; r4 < 2; ++r4) {
+                        u32x4 lo, hi;
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            const uint32_t a = w[0][r4][q], b = w[1][r4][q];
+                            // row_ror:8 within 16 lanes; bank mask 0xc writes lanes 8..15 of a row, 0x3 lanes 0..7
+                            lo[q] = (uint32_t)__builtin_amdgcn_update_dpp((int)a, (int)b, 0x128, 0xf, 0xc, false);
+                            hi[q] = (uint32_t)__builtin_amdgcn_update_dpp((int)b, (int)a, 0x128, 0xf, 0x3, false);
+                        }
+                        if constexpr (decltype(cached)::value) {
+                            *(u32x4*)(og + crow[2 * r4 + 0] + 128 * dp) = lo;
+                            *(u32x4*)(og + crow[2 * r4 + 1] + 128 * dp) = hi;
+                        } else {
+                            __builtin_nontemporal_store(lo, (u32x4*)(og + crow[2 * r4 + 0] + 128 * dp));
+                            __builtin_nontemporal_store(hi, (u32x4*)(og + crow[2 * r4 + 1] + 128 * dp));
+                        }
                     }
-                    // lane bit 4 <-> gp: slot 0 then holds rows (c & 15), slot 1 rows (c & 15) + 16
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        auto x = __builtin_amdgcn_permlane16_swap(w[dl][0][q], w[dl][1][q], false, false);
-                        w[dl][0][q] = x[0]; w[dl][1][q] = x[1];
-                    }
-                }
-                // lane bit 3 <-> block within the pair
-#pragma unroll
-                for (int r4 = 0; r4 < 2; ++r4) {
-                    u32x4 lo, hi;
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const uint32_t a = w[0][r4][q], b = w[1][r4][q];
-                        // row_ror:8 within 16 lanes; bank mask 0xc writes lanes 8..15 of a row, 0x3 lanes 0..7
-                        lo[q] = (uint32_t)__builtin_amdgcn_update_dpp((int)a, (int)b, 0x128, 0xf, 0xc, false);
-                        hi[q] = (uint32_t)__builtin_amdgcn_update_dpp((int)b, (int)a, 0x128, 0xf, 0x3, false);
-                    }
-                    // Non-temporal: the rows are read exactly once, by step 2, after the whole grid has finished.
-                    // Ordinary stores leave them dirty in the caches and their write-back then competes with
-                    // step 2's reads (measured at 4680 x 32760, 12 heads: step 1 +15 us, step 2 -45 us).
-                    __builtin_nontemporal_store(lo, (u32x4*)(og + crow[2 * r4 + 0] + 128 * dp));
-                    __builtin_nontemporal_store(hi, (u32x4*)(og + crow[2 * r4 + 1] + 128 * dp));
                 }
             }
-        }
+        };
+        if (p.s1_cached) contract(std::true_type{});
+        else contract(std::false_type{});
         if (NW && fresh && cur.ac == 0 && is_new(cur)) write_new(cur, kt);
     }
 }
@@ -1619,6 +1626,16 @@ static int enqueue_step1(const MonarchArgs& a, int nunits, hipStream_t stream, S
     // tied frames against themselves 50 -> 46; 24 columns of nine 30 x 24 frames 52 -> 39.  Four groups of three waves: 50 us
     // at 7 heads of nine 23 x 31 frames, two 44.5.  Two or four waves for 32 columns, each with its part of the output, took
     // the refinement to 505 and 541 us: they fetch the query rows as often.
+    // What a pass writes goes through the caches where the memory-side one (256 MB) can still hold most of it for the kernel that reads
+    // it next, and past them where it cannot (written back under that kernel's reads) or where it is little (the L2s give their dirty
+    // lines up at the kernel's end).  us past the caches and through them, 12 heads x 128 of 30 x 52 unless named: three frames
+    // against 3 (86 MB) 67, 63.5, 6 (173) 112, 104, 9 (259) 154, 143, 12 (345) 201, 193, 21 (604) 322, 331; 45 x 80, 6 frames (398)
+    // 245, 242; 12 frames in half-height blocks (690) 341, 376; three passes at three frames tied (100 and 201) 450, 424; 2 heads, 6
+    // frames (29) 29.4, 29.3; 1 head, 3 frames (7) 21.8, 22.9; three frames tied against themselves (29) 44.6, 47.4.  Kbar alone is
+    // followed by as many bytes of representatives: two passes, 21 frames (302) 624, 637.
+    const size_t scratch_rows = (size_t)nunits * a.na * a.b2 * a.nf * a.b1;
+    const size_t written = scratch_rows * ((kind == Step1::kIterKbar ? 2 : 4) * D + (a.rb ? 128 : 0));
+    a1.s1_cached = written >= (size_t)40 << 20 && written <= (size_t)(kind == Step1::kIterKbar ? 256 : 384) << 20;
     const int cus = a.s1_wgs > 0 ? a.s1_wgs : cu_count();
     // Two groups of six waves are worth it at head_dim 64 only (176 columns of 44 x 44, 12 heads: 161 us, one group 172; head_dim 128
     // 304, 297; 192 columns of 30 x 64 240, 232).

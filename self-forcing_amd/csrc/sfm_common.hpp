@@ -182,6 +182,7 @@ struct MonarchArgs {
     int64_t ns[3];
     // MFMA step 1 only, with rb: R of (ul, a, j, k, f) is row ul*rb_unit + k*rb_k + f*rb_f + a*b2 + j, a tile's columns in a run
     uint32_t rb_unit, rb_k, rb_f;
+    int s1_cached;   // MFMA step 1 only: Kbar and Y are stored through the caches, not past them
 };
 
 // Backward: the forward arguments (scratch matrices in float) plus the gradient tensors.

@@ -430,3 +430,17 @@ def test_wrappers_reuse_one_scratch_buffer_per_stream():
     assert (0, side.cuda_stream) in mattn._SCRATCH and torch.equal(other, small_first)
     mattn.release_scratch()
     assert not mattn._SCRATCH
+
+
+# passes whose scratch lies below, within and beyond the sizes that step 1 stores through the caches; with the right factor too
+@pytest.mark.parametrize("heads,heads_per_pass,q_frames,frames,D,dtype", [(6, 2, 3, 3, 128, torch.bfloat16), (12, 4, 3, 21, 128, torch.float16),
+                                                                         (14, 5, 3, 9, 64, torch.bfloat16)])
+def test_scratch_through_and_past_the_caches_gives_the_same_bits(heads, heads_per_pass, q_frames, frames, D, dtype):
+    h, w = 30, 52
+    q = randn((1, q_frames * h * w, heads, D), 440, dtype).to(DEV)
+    k, v = (randn((1, frames * h * w, heads, D), 441 + i, dtype).to(DEV) for i in range(2))
+    for n in (1, 2):
+        whole = mattn.monarch_attn(q, k, v, 1, 1, 1, h, w, num_iters=n)
+        assert torch.equal(whole, mattn.monarch_attn(q, k, v, 1, 1, 1, h, w, num_iters=n, heads_per_pass=heads_per_pass))
+    out = mattn.monarch_attn(q.clone().requires_grad_(True), k, v, 1, 1, 1, h, w)
+    assert torch.equal(out, mattn.monarch_attn(q, k, v, 1, 1, 1, h, w, heads_per_pass=1))
