@@ -444,3 +444,17 @@ def test_scratch_through_and_past_the_caches_gives_the_same_bits(heads, heads_pe
         assert torch.equal(whole, mattn.monarch_attn(q, k, v, 1, 1, 1, h, w, num_iters=n, heads_per_pass=heads_per_pass))
     out = mattn.monarch_attn(q.clone().requires_grad_(True), k, v, 1, 1, 1, h, w)
     assert torch.equal(out, mattn.monarch_attn(q, k, v, 1, 1, 1, h, w, heads_per_pass=1))
+
+
+@pytest.mark.parametrize("heads", [5, 8])
+def test_default_passes_give_the_bits_of_other_passes(heads):
+    """Scratch of 352 to 600 MiB at head_dim 128 is gone through in two passes by default, of equal and of unequal length."""
+    q_frames, frames, h, w = (3, 21, 45, 80) if heads == 5 else (3, 21, 31, 52)
+    q, nk, nv = (randn((1, q_frames * h * w, heads, 128), 450 + i, torch.bfloat16).to(DEV) for i in range(3))
+    k, v = (randn((1, frames * h * w, heads, 128), 453 + i, torch.bfloat16).to(DEV) for i in range(2))
+    d = mattn._desc(q, k, v, q, 1, 1, 1, h, w, 128 ** -0.5, 1, 0)
+    assert mattn.monarch_workspace_bytes(d) == mattn.monarch_workspace_bytes(d, (heads + 1) // 2)
+    end = frames * h * w
+    out = [mattn.monarch_attn_with_kv_cache(q, k.clone(), v.clone(), nk, nv, end - q_frames * h * w, end, 1, 1, 1, h, w, heads_per_pass=n)
+           for n in (0, 1, heads)]
+    assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
