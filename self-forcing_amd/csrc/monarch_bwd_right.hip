@@ -64,6 +64,11 @@ __device__ __forceinline__ void br_load_lds16(const char* base, uint32_t off, ui
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(off), "s"(base) : "memory", "m0");
 }
 
+// the same past the caches, for rows that are read once: dS1, which the dQ kernel reads next, and the K, V and query rows keep
+// their place (forward and backward, three frames against themselves 208 -> 202 us, 21 frames 938 -> 930)
+__device__ __forceinline__ void br_load_lds16_nt(const char* base, uint32_t off, uint32_t lds_addr) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds_addr), "v"(off), "s"(base) : "memory", "m0");
+}
 // chunk c (16 bytes) of row r sits at chunk position c ^ swz(r); rows of CPR chunks (16: 256-byte rows, 8: 128-byte rows)
 template <int CPR>
 __device__ __forceinline__ int br_swz(int r) {
@@ -105,21 +110,23 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
     // LDS position P (16-byte units) of a tile holds chunk (P % C) ^ swz(row) of row P / C; 64 rows, those past the end repeat
     // the last one.  Key rows past the end land in rows of dK and dV that are not stored; columns are cleared below; a query
     // row that is not finite has made its column's dS1, and with it all of dK, NaN already
-    auto stage = [&](const char* src, uint32_t row_bytes, int nrows, uint32_t dst, auto cpr_c) {
+    auto stage = [&](const char* src, uint32_t row_bytes, int nrows, uint32_t dst, auto cpr_c, auto once_c) {
         constexpr int C = decltype(cpr_c)::value;
 #pragma unroll
         for (int g = 0; g < C / kWaves; ++g) {
             const int P = (wave + g * kWaves) * 64 + lane;
             const int r = P / C, c = (P % C) ^ br_swz<C>(r);
-            br_load_lds16(src, (uint32_t)min(r, nrows - 1) * row_bytes + (uint32_t)(c * 16), lds0 + dst + (uint32_t)(wave + g * kWaves) * 1024);
+            const uint32_t off = (uint32_t)min(r, nrows - 1) * row_bytes + (uint32_t)(c * 16), to = lds0 + dst + (uint32_t)(wave + g * kWaves) * 1024;
+            if constexpr (decltype(once_c)::value) br_load_lds16_nt(src, off, to);
+            else br_load_lds16(src, off, to);
         }
     };
     using c_d = std::integral_constant<int, CPR>;
     using c_r = std::integral_constant<int, 8>;
     stage(p.kk + ((int64_t)(unit / p.H) * p.ks0 + (int64_t)(unit % p.H) * p.ks2 + p.kmap.row(f, k) * p.ks1) * 2, (uint32_t)(p.ks1 * 2), b2,
-          L::oK, c_d{});
+          L::oK, c_d{}, std::false_type{});
     stage(p.v + ((int64_t)(unit / p.H) * p.vs0 + (int64_t)(unit % p.H) * p.vs2 + p.kmap.row(f, k) * p.vs1) * 2, (uint32_t)(p.vs1 * 2), b2,
-          L::oV, c_d{});
+          L::oV, c_d{}, std::false_type{});
     const bool want = f >= p.f0 && f < p.f1;                             // uniform: dK / dV of this kv block-frame are asked for
 
     const char* qbase = p.q + ((int64_t)(unit / p.H) * p.qs0 + (int64_t)(unit % p.H) * p.qs2) * 2;
@@ -128,9 +135,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
     const int cfirst = p.causal ? f / p.causal * p.causal * b2 : 0;      // the first column (a, j) that sees key block-frame f
 
     // What every wave does in a chunk; the two kinds of waves meet in the same four barriers.
-    auto load_g = [&](int c0) { stage(p.dkbar + (t * AJ + c0) * kPitch, kPitch, min(kCols, AJ - c0), L::oG, c_d{}); };
-    auto load_h = [&](int c0) { stage(p.dy + (t * AJ + c0) * kPitch, kPitch, min(kCols, AJ - c0), L::oH, c_d{}); };
-    auto load_r = [&](int c0) { stage(p.rb + (t * AJ + c0) * 128, 128, min(kCols, AJ - c0), L::oR, c_r{}); };
+    auto load_g = [&](int c0) { stage(p.dkbar + (t * AJ + c0) * kPitch, kPitch, min(kCols, AJ - c0), L::oG, c_d{}, std::true_type{}); };
+    auto load_h = [&](int c0) { stage(p.dy + (t * AJ + c0) * kPitch, kPitch, min(kCols, AJ - c0), L::oH, c_d{}, std::true_type{}); };
+    auto load_r = [&](int c0) { stage(p.rb + (t * AJ + c0) * 128, 128, min(kCols, AJ - c0), L::oR, c_r{}, std::true_type{}); };
     // the next chunk's rows are requested as soon as their tiles are free: dKbar (and dY, where no query rows take its place)
     // behind the products, the others at the chunk's end
     auto next_early = [&](int c1) {
