@@ -47,6 +47,10 @@ __device__ __forceinline__ u32x2 s1_read_tr(const char* lds, uint32_t off) {
 __device__ __forceinline__ void s1_load_lds16(const char* base, uint32_t off, uint32_t lds_addr) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(off), "s"(base) : "memory", "m0");
 }
+// past the caches
+__device__ __forceinline__ void s1_load_lds16_nt(const char* base, uint32_t off, uint32_t lds_addr) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds_addr), "v"(off), "s"(base) : "memory", "m0");
+}
 template <int CPR>
 __device__ __forceinline__ int s1_swz(int r) {
     return CPR >= 16 ? (((r & 3) << 2) | ((r >> 2) & 3)) : ((((r >> 1) & 1) << 2) | ((r >> 2) & 3));
@@ -513,7 +517,7 @@ __device__ __forceinline__ void wait_vm() {
 // dependent chunks (about 2.5 us each) is the whole time.  A kernel of its own: with the number of waves an argument of one
 // kernel for both, a call of three 480p frames against themselves (12 heads), whose columns are not shared, took 76.2 us
 // instead of 75.4 (two runs differ by 0.1).
-template <class E, int D, int TEAM, bool SHARE = false>
+template <class E, int D, int TEAM, bool SHARE = false, bool PAST = false>
 __global__ __launch_bounds__(TEAM == 1 ? 256 : 64 * TEAM) __attribute__((amdgpu_waves_per_eu(TEAM >= 3 ? 3 : 2, TEAM >= 3 ? 3 : 2)))
 void monarch_step2_kernel(MonarchArgs p) {
     using L = S2Lds<D>;
@@ -603,7 +607,8 @@ void monarch_step2_kernel(MonarchArgs p) {
             const int P = g * 64 + lane;
             const int r = P / CPR, c = (P % CPR) ^ s1_swz<CPR>(r);
             const uint32_t off = (uint32_t)min(32 * n + r, r_lim - 1) * (2 * D) + (uint32_t)c * 16;
-            s1_load_lds16(mat, off, dst + (uint32_t)g * 1024);
+            if constexpr (PAST) s1_load_lds16_nt(mat, off, dst + (uint32_t)g * 1024);          // see enqueue_step2
+            else s1_load_lds16(mat, off, dst + (uint32_t)g * 1024);
         }
     };
     // buffers of the chunk at position `it` of this wave's sequence: a team alternates between two pairs
@@ -1329,8 +1334,8 @@ __global__ __launch_bounds__(64 * (WtLds<D, NQ, W>::kWaves)) __attribute__((amdg
 #pragma unroll
             for (int qi = 0; qi < NQ; ++qi)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) z[c][qi][v] = z[c][qi][v] * sc2 - cc;
-            if (32 * n + 32 > r_lim) {                       // uniform: the last chunk, where it is not a whole one
+                for (int v = 0; v < 16; ++v) z[c][qi][v] = RUN || rok ? z[c][qi][v] * sc2 - cc : -INFINITY;
+            if (RUN && 32 * n + 32 > r_lim) {                // uniform: the last chunk, where it is not a whole one
 #pragma unroll
                 for (int qi = 0; qi < NQ; ++qi)
 #pragma unroll
@@ -1630,12 +1635,12 @@ static int enqueue_step1(const MonarchArgs& a, int nunits, hipStream_t stream, S
     // it next, and past them where it cannot (written back under that kernel's reads) or where it is little (the L2s give their dirty
     // lines up at the kernel's end).  us past the caches and through them, 12 heads x 128 of 30 x 52 unless named: three frames
     // against 3 (86 MB) 67, 63.5, 6 (173) 112, 104, 9 (259) 154, 143, 12 (345) 201, 193, 21 (604) 322, 331; 45 x 80, 6 frames (398)
-    // 245, 242; 12 frames in half-height blocks (690) 341, 376; three passes at three frames tied (100 and 201) 450, 424; 2 heads, 6
+    // 245, 242 (the other way round since step 2 reads past them); 12 frames in half-height blocks (690) 341, 376; three passes at three frames tied (100 and 201) 450, 424; 2 heads, 6
     // frames (29) 29.4, 29.3; 1 head, 3 frames (7) 21.8, 22.9; three frames tied against themselves (29) 44.6, 47.4.  Kbar alone is
     // followed by as many bytes of representatives: two passes, 21 frames (302) 624, 637.
     const size_t scratch_rows = (size_t)nunits * a.na * a.b2 * a.nf * a.b1;
     const size_t written = scratch_rows * ((kind == Step1::kIterKbar ? 2 : 4) * D + (a.rb ? 128 : 0));
-    a1.s1_cached = written >= (size_t)40 << 20 && written <= (size_t)(kind == Step1::kIterKbar ? 256 : 384) << 20;
+    a1.s1_cached = written >= (size_t)40 << 20 && written <= (size_t)(kind == Step1::kIterKbar ? 256 : 364) << 20;
     const int cus = a.s1_wgs > 0 ? a.s1_wgs : cu_count();
     // Two groups of six waves are worth it at head_dim 64 only (176 columns of 44 x 44, 12 heads: 161 us, one group 172; head_dim 128
     // 304, 297; 192 columns of 30 x 64 240, 232).
@@ -1660,17 +1665,27 @@ static int enqueue_step1(const MonarchArgs& a, int nunits, hipStream_t stream, S
     return SFM_OK;
 }
 
+template <class E, int D, int TEAM>
+static const void* step2_kernel(bool past) {
+    return past ? (const void*)monarch_step2_kernel<E, D, TEAM, false, true> : (const void*)monarch_step2_kernel<E, D, TEAM>;
+}
+
 // Enqueues step 2: a wave per column (a, j) of up to 32 query rows, a team of waves for more.  `stats_only` (b1 <= 128):
 // the row statistics without the output.
 template <class E, int D>
 static int enqueue_step2(const MonarchArgs& a, int nunits, hipStream_t stream, bool stats_only = false) {
     const int team = a.b1 > 96 ? 4 : (a.b1 + 31) / 32;
+    // From the size on where the memory-side cache holds part of Kbar and Y only, their rows, read once, are read past it: us
+    // through the caches and past them, 12 heads x 128 of 30 x 52, three frames against 9 (259 MB) 143, 140, 12 (345) 193, 179, in
+    // half-height blocks (690) 342, 336; 6 heads, 21 frames (302) 155, 146; 40 heads, 21 (2013) 1038, 1002.  Below, they would leave it: 6 heads,
+    // 12 frames (173 MB) 96.3, 98.6; three frames tied against 21 (201) 146, 149.
+    const bool past = (size_t)nunits * a.na * a.b2 * a.nf * a.b1 * 4 * D >= (size_t)240 << 20;
     const void* fn = stats_only ? (team == 4   ? (const void*)monarch_left_stats_kernel<E, D, 4>
                                    : team == 3 ? (const void*)monarch_left_stats_kernel<E, D, 3>
                                    : team == 2 ? (const void*)monarch_left_stats_kernel<E, D, 2>
                                                : (const void*)monarch_left_stats_kernel<E, D, 1>)
-                   : team == 4 ? (const void*)monarch_step2_kernel<E, D, 4> : team == 3 ? (const void*)monarch_step2_kernel<E, D, 3>
-                   : team == 2 ? (const void*)monarch_step2_kernel<E, D, 2> : (const void*)monarch_step2_kernel<E, D, 1>;
+                   : team == 4 ? step2_kernel<E, D, 4>(past) : team == 3 ? step2_kernel<E, D, 3>(past)
+                   : team == 2 ? step2_kernel<E, D, 2>(past) : step2_kernel<E, D, 1>(past);
     const size_t lds = stats_only ? (team == 4   ? StLds<D, 4>::bytes()
                                      : team == 3 ? StLds<D, 3>::bytes()
                                      : team == 2 ? StLds<D, 2>::bytes()
