@@ -1635,8 +1635,8 @@ static int enqueue_step1(const MonarchArgs& a, int nunits, hipStream_t stream, S
     // it next, and past them where it cannot (written back under that kernel's reads) or where it is little (the L2s give their dirty
     // lines up at the kernel's end).  us past the caches and through them, 12 heads x 128 of 30 x 52 unless named: three frames
     // against 3 (86 MB) 67, 63.5, 6 (173) 112, 104, 9 (259) 154, 143, 12 (345) 201, 193, 21 (604) 322, 331; 45 x 80, 6 frames (398)
-    // 245, 242 (the other way round since step 2 reads past them); 12 frames in half-height blocks (690) 341, 376; three passes at three frames tied (100 and 201) 450, 424; 2 heads, 6
-    // frames (29) 29.4, 29.3; 1 head, 3 frames (7) 21.8, 22.9; three frames tied against themselves (29) 44.6, 47.4.  Kbar alone is
+    // 245, 242, but level since step 2 reads past them; 12 frames in half-height blocks (690) 341, 376; three passes at three frames
+    // tied (100 and 201) 450, 424; 2 heads, 6 frames (29) 29.4, 29.3; 1 head, 3 frames (7) 21.8, 22.9; three frames tied against themselves (29) 44.6, 47.4.  Kbar alone is
     // followed by as many bytes of representatives: two passes, 21 frames (302) 624, 637.
     const size_t scratch_rows = (size_t)nunits * a.na * a.b2 * a.nf * a.b1;
     const size_t written = scratch_rows * ((kind == Step1::kIterKbar ? 2 : 4) * D + (a.rb ? 128 : 0));

@@ -257,7 +257,7 @@ static int plan_monarch(const sfm_monarch_desc* d, MonarchPlan* pl) {
 }
 
 // Default number of units per pass: all of them while the scratch stays under 4 GiB (one launch pair
-// fills the chip best), or half of them where step 2 then finds the scratch in the memory-side cache (step 1 stores 40 to 384 MB of it
+// fills the chip best), or half of them where step 2 then finds the scratch in the memory-side cache (step 1 stores 40 to 364 MiB of it
 // through the caches) and both halves still fill the chip.  us as one pass and as two, 12 heads x 128 of 30 x 52, three frames
 // against 15 (431 MB) 243, 231, against 18 (517) 282, 268, 21 (604) 322, 316; 8 heads, 21 (403) 230, 204; 30 of 22 x 40, 12 frames (486)
 // 268, 251; 11 of 56 x 40, 15 (567) 312, 289; 4 of 45 x 80, 21 (464) 247, 245.  Not outside these limits: 12 heads, 12 frames
