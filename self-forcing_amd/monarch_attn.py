@@ -67,6 +67,7 @@ def scratch(nbytes, device):
     key = (index, _raw_stream(index))
     buf = _SCRATCH.get(key)
     if buf is None or buf.numel() < nbytes:
+        _drop_kept(index)
         buf = _SCRATCH[key] = torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
     return buf
 
@@ -79,17 +80,30 @@ class _KeptRef(weakref.ref):
     __slots__ = ("nbytes",)
 
 
-class _KeptBudget:
-    """What the forwards of one device hold for backwards to come: at most a sixteenth of its memory (18 GB), which is a pass of
-    30 layers of 12 heads at 480p; beyond that a forward leaves nothing and its backward forms the intermediates again.  A
-    buffer is counted from its allocation until autograd lets go of it."""
+class _Kept:
+    """What one forward left for its backward, while nobody else has had it dropped."""
+    __slots__ = ("buf", "__weakref__")
 
-    def __init__(self, device):
-        self.left = torch.cuda.get_device_properties(device).total_memory // 16
+    def __init__(self, buf):
+        self.buf = buf
+
+
+class _KeptBudget:
+    """What the forwards of one device hold for backwards to come: the newest one's intermediates, 2 GiB at most.  The workspace of a
+    backward that finds them is smaller by as much, so a program that calls forward and backward in turn has no more memory
+    in use than if every backward formed them again (12 heads at 480p, three frames against 21: 769 + 760 MB, else 1500 and 29
+    of dq in float32).  They are dropped, and their backward forms them again, for the next forward's, for a backward that has
+    none and needs the larger workspace, and where a workspace grows.  A buffer is counted from its allocation until
+    nothing refers to it."""
+
+    def __init__(self):
+        self.left = 2 << 30                      # sfm_monarch_kept_bytes never asks for more
         self.lock = threading.RLock()            # a buffer may die inside take(), in the garbage collector
         self.refs = set()
+        self.pending = None                      # the newest _Kept, weakly: it dies with its graph
 
     def take(self, nbytes, device):
+        self.drop()
         with self.lock:
             if nbytes > self.left:
                 return None
@@ -110,20 +124,45 @@ class _KeptBudget:
             self.refs.discard(ref)
             self.left += ref.nbytes
 
+    def hold(self, buf):
+        kept = _Kept(buf)
+        with self.lock:
+            self.pending = weakref.ref(kept)
+        return kept
+
+    def claim(self, kept):
+        """The buffer, for one backward: from here on nobody drops it, and it dies with its last use."""
+        with self.lock:
+            buf, kept.buf = kept.buf, None
+            if self.pending is not None and self.pending() is kept:
+                self.pending = None
+        return buf
+
+    def drop(self):
+        with self.lock:
+            kept, self.pending = self.pending and self.pending(), None
+            if kept is not None:
+                kept.buf = None
+
 
 _KEPT = {}
 _top_hooks = getattr(torch._C._autograd, "_top_saved_tensors_default_hooks", None)
 
 
 def _kept_buffer(nbytes, device):
-    """A buffer for the intermediates of a forward under autograd, or None.  None too while hooks on saved tensors are set (they
-    would move or keep a buffer 50 times the inputs: activation checkpointing, save_on_cpu)."""
+    """A buffer for the intermediates of a forward under autograd, or None.  None too while hooks on saved tensors are set: their
+    program wants little memory between forward and backward (activation checkpointing, save_on_cpu)."""
     if not nbytes or _top_hooks is None or _top_hooks(False) is not None:
         return None
     budget = _KEPT.get(device.index)
     if budget is None:
-        budget = _KEPT.setdefault(device.index, _KeptBudget(device))
+        budget = _KEPT.setdefault(device.index, _KeptBudget())
     return budget.take(nbytes, device)
+
+
+def _drop_kept(index):
+    if index in _KEPT:
+        _KEPT[index].drop()
 
 
 def monarch_workspace_bytes(desc, heads_per_pass=0):
@@ -285,12 +324,22 @@ def _monarch_bwd(q, k, v, dout, tiling, sm_scale, kv_block_order, cbf, kv_f0=0, 
     return dq, dk, dv
 
 
-_KEPT_NAMES = ("out", "stats", "kept")
-
-
 def _save(ctx, inputs, out, stats, kept):
-    """The forward's tensors for the backward: the inputs, then as many of _KEPT_NAMES as it left."""
-    ctx.save_for_backward(*inputs, *(() if stats is None else (out, stats) if kept is None else (out, stats, kept)))
+    """The forward's tensors for the backward: the inputs, then the output and its row statistics if it left any.  `kept` is no saved
+    tensor: it may be dropped before."""
+    ctx.save_for_backward(*inputs, *(() if stats is None else (out, stats)))
+    ctx.kept = None if kept is None else _KEPT[kept.device.index].hold(kept)
+
+
+def _saved(ctx):
+    """(inputs, what _monarch_bwd takes of the forward's)."""
+    q, k, v, *left = ctx.saved_tensors
+    left = dict(zip(("out", "stats"), left))
+    if ctx.kept is not None:
+        left["kept"] = _KEPT[q.device.index].claim(ctx.kept)
+    if left.get("kept") is None:
+        _drop_kept(q.device.index)
+    return (q, k, v), left
 
 
 class _MonarchFn(torch.autograd.Function):
@@ -311,9 +360,9 @@ class _MonarchFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dout):
-        q, k, v, *kept = ctx.saved_tensors
+        (q, k, v), left = _saved(ctx)
         tiling, sm_scale, cbf, kv_block_order = ctx.cfg
-        dq, dk, dv = _monarch_bwd(q, k, v, dout, tiling, sm_scale, 1 if kv_block_order else 0, cbf, **dict(zip(_KEPT_NAMES, kept)))
+        dq, dk, dv = _monarch_bwd(q, k, v, dout, tiling, sm_scale, 1 if kv_block_order else 0, cbf, **left)
         return dq.to(q.dtype), dk, dv, None, None, None, None, None
 
 
@@ -340,18 +389,17 @@ class _MonarchCacheFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dout):
-        q, k_cache, v_cache, *kept = ctx.saved_tensors
-        kept = dict(zip(_KEPT_NAMES, kept))
+        (q, k_cache, v_cache), left = _saved(ctx)
         start_idx, end_idx, tiling, sm_scale, grad_only_new_kv = ctx.cfg
         f_tied, h_reduce, w_reduce, h, w = tiling
         per_frame = f_tied * (h // h_reduce) * (w // w_reduce)
         if grad_only_new_kv:
             dq, dk, dv = _monarch_bwd(q, k_cache, v_cache, dout, tiling, sm_scale, 1, 0, start_idx // per_frame,
-                                      end_idx // per_frame, **kept)
+                                      end_idx // per_frame, **left)
             dk_cache = dv_cache = None
             dk_new, dv_new = dk, dv
         else:
-            dq, dk_cache, dv_cache = _monarch_bwd(q, k_cache, v_cache, dout, tiling, sm_scale, 1, 0, **kept)
+            dq, dk_cache, dv_cache = _monarch_bwd(q, k_cache, v_cache, dout, tiling, sm_scale, 1, 0, **left)
             dk_new, dv_new = dk_cache[:, start_idx:end_idx], dv_cache[:, start_idx:end_idx]
         dk_new = _from_block_order(dk_new, *tiling)
         dv_new = _from_block_order(dv_new, *tiling)
@@ -466,7 +514,8 @@ def monarch_attn_with_kv_cache(q, k_cache, v_cache, new_k, new_v, start_idx, end
                                sm_scale=None, num_iters=1, grad_only_new_kv=False, heads_per_pass=0, one_kernel=False):
     """Writes new_k/new_v into k_cache/v_cache[:, start_idx:end_idx] (block order, in place) and
     returns one-iteration Monarch attention of q against the whole cache view.  `heads_per_pass` and `one_kernel`
-    (no counterparts in the reference) bound the scratch and select the forward that keeps its intermediates in LDS."""
+    (no counterparts in the reference) bound the scratch and select the forward that keeps its intermediates in LDS.  Under
+    autograd, `heads_per_pass` also keeps the forward from holding its intermediates, up to 2 GiB, for its backward."""
     if _needs_grad(q, k_cache, v_cache, new_k, new_v):
         if sm_scale is None:
             sm_scale = q.shape[-1] ** -0.5
@@ -539,7 +588,7 @@ def monarch_attn(q, k, v, f_tied, h_reduce, w_reduce, h, w, sm_scale=None, block
     """One-iteration Monarch attention without a cache write; `block_causal_size` (tokens) masks
     block-frames of later causal blocks.  `kv_block_order=True` (no counterpart in the reference) says
     that k, v are a KV-cache view whose rows are already in Monarch block order, e.g. after
-    prologue.qk_prologue wrote them."""
+    prologue.qk_prologue wrote them.  `heads_per_pass` and `one_kernel` as in monarch_attn_with_kv_cache."""
     if _needs_grad(q, k, v):
         if sm_scale is None:
             sm_scale = q.shape[-1] ** -0.5

@@ -113,3 +113,65 @@ def test_what_is_kept_is_bounded_and_given_back(monkeypatch):
         L.load().sfm_set_switches(old)
     for a, b in zip(got, want):
         torch.testing.assert_close(a.float(), b.float(), atol=1e-2, rtol=1e-2)
+
+
+def test_the_newest_forward_alone_holds_its_intermediates():
+    """Layers whose backwards come later hold one buffer between them, not one each: the others' backwards, a second one of a
+    retained graph and one whose buffer made room for a larger workspace form the intermediates again, with the same bits."""
+    h, w, H, D, dtype = 6, 20, 2, 64, torch.bfloat16
+    q, k, v, do = (randn((1, 3 * h * w, H, D), 530 + i, dtype).to(DEV) for i in range(4))
+    leaves = [t.requires_grad_(True) for t in (q, k, v)]
+
+    def forward(**kw):
+        return mattn.monarch_attn(q, k, v, 1, 1, 1, h, w, **kw)
+
+    want = torch.autograd.grad(forward(heads_per_pass=H), leaves, do)
+    first = forward()
+    budget = mattn._KEPT[torch.cuda.current_device()]
+    left = budget.left
+    assert len(budget.refs) == 1
+    second = forward()
+    assert budget.left == left and len(budget.refs) == 1
+    forward(heads_per_pass=H)                                       # holds none, and leaves the newest that does its own
+    assert budget.left == left
+    for _ in range(2):
+        got = torch.autograd.grad(second, leaves, do, retain_graph=True)
+        assert not budget.refs and all(torch.equal(a, b) for a, b in zip(got, want))
+    held = forward()
+    assert len(budget.refs) == 1
+    got = torch.autograd.grad(first, leaves, do)                    # its workspace is the larger one
+    assert not budget.refs and all(torch.equal(a, b) for a, b in zip(got, want))
+    got = torch.autograd.grad(held, leaves, do)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    held = forward()
+    key = (torch.cuda.current_device(), torch.cuda.current_stream().cuda_stream)
+    mattn.scratch(mattn._SCRATCH[key].numel() + 1, q.device)
+    assert not budget.refs
+    got = torch.autograd.grad(held, leaves, do)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    layers = [forward() for _ in range(6)]
+    assert len(budget.refs) <= 1
+    for o in reversed(layers):
+        got = torch.autograd.grad(o, leaves, do)
+        assert len(budget.refs) <= 1 and all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_forward_and_backward_in_turn_take_no_more_memory_than_without_what_is_kept(monkeypatch):
+    h, w, H, D, dtype = 30, 52, 4, 128, torch.bfloat16
+    q, k, v, do = (randn((1, 3 * h * w, H, D), 540 + i, dtype).to(DEV) for i in range(4))
+    leaves = [t.requires_grad_(True) for t in (q, k, v)]
+
+    def peak():
+        mattn.release_scratch()
+        torch.cuda.empty_cache()
+        for i in range(3):
+            if i == 1:                                              # the first pass allocates the workspace
+                torch.cuda.reset_peak_memory_stats()
+            out = mattn.monarch_attn(q, k, v, 1, 1, 1, h, w)
+            torch.autograd.grad(out, leaves, do)
+            del out
+        return torch.cuda.max_memory_allocated()
+
+    kept = peak()
+    monkeypatch.setattr(mattn, "_kept_buffer", lambda *a: None)
+    assert kept <= peak() + (2 << 20)                               # allocations are rounded up to 512 bytes and more
