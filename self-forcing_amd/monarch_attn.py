@@ -161,6 +161,8 @@ def _kept_buffer(nbytes, device):
 
 
 def _drop_kept(index):
+    """Every call that writes cache rows makes this one too: a backward takes K and V from the caches as it finds them, and with rows
+    written since its forward it has to form the right factor from those too, not from the ones that the forward saw."""
     if index in _KEPT:
         _KEPT[index].drop()
 
@@ -211,6 +213,7 @@ def kv_cache_write(new_k, new_v, k_cache, v_cache, start_idx, end_idx, f_tied, h
     B, _, H, D = new_k.shape
     if B > k_cache.shape[0] or H > k_cache.shape[2] or D > k_cache.shape[3]:
         raise ValueError(f"new_k {tuple(new_k.shape)} holds more batches, heads or channels than the cache {tuple(k_cache.shape)}")
+    _drop_kept(k_cache.device.index)
     with _on_device(new_k.device):
         _l.check(_l.load().sfm_kv_cache_write(_DT[new_k.dtype], B, H, D, C.byref(_l.Tiling(f_tied, h_reduce, w_reduce, h, w)),
                                               new_k.data_ptr(), new_v.data_ptr(), _l.strides3(new_k), k_cache.data_ptr(),
@@ -243,6 +246,8 @@ def _monarch_fwd_kept(q, k, v, tiling, sm_scale, kv_block_order, cbf, heads_per_
     _l.check(lib.sfm_monarch_stats_bytes(C.byref(d), C.byref(n)))
     stats = torch.empty(n.value // 4, dtype=torch.float32, device=q.device) if n.value else None
     kept = None
+    if new is not None:
+        _drop_kept(q.device.index)
     if keep and stats is not None and not heads_per_pass:
         _l.check(lib.sfm_monarch_kept_bytes(C.byref(d), C.byref(n)))
         kept = _kept_buffer(n.value, q.device)
@@ -369,7 +374,8 @@ class _MonarchFn(torch.autograd.Function):
 class _MonarchCacheFn(torch.autograd.Function):
     """monarch_attn_with_kv_cache under autograd (_attention_with_cache, monarch_attn.py:1225-1470): the caches
     are written in place in the forward and saved by reference, as the reference does; with grad_only_new_kv
-    only the block-frames written by this call get K/V gradients (:1364-1374)."""
+    only the block-frames written by this call get K/V gradients (:1364-1374).  Rows that another call writes before the
+    backward are what it computes with, right factor included (_drop_kept); the output and its statistics are the forward's."""
 
     @staticmethod
     def forward(ctx, q, k_cache, v_cache, new_k, new_v, start_idx, end_idx, tiling, sm_scale, grad_only_new_kv,
@@ -546,6 +552,7 @@ def monarch_attn_with_kv_cache(q, k_cache, v_cache, new_k, new_v, start_idx, end
     d = _desc(q, k_cache, v_cache, out, f_tied, h_reduce, w_reduce, h, w, sm_scale, 1, 0, num_iters, one_kernel)
     nbytes = monarch_workspace_bytes(d, heads_per_pass)
     ws = scratch(nbytes, q.device)
+    _drop_kept(q.device.index)
     with _on_device(q.device):
         _l.check(_l.load().sfm_monarch_attn_with_kv_cache(
             C.byref(d), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), new_k.data_ptr(), new_v.data_ptr(),
@@ -576,6 +583,7 @@ def monarch_attn_with_kv_cache_static(q, k_cache, v_cache, new_k, new_v, start_i
         if out.shape != q.shape:
             raise ValueError("out must have q's shape")
     d = _desc(q, k_cache, v_cache, out, f_tied, h_reduce, w_reduce, h, w, sm_scale, 1, 0, num_iters)
+    _drop_kept(q.device.index)
     with _on_device(q.device):
         _l.check(_l.load().sfm_monarch_attn_with_kv_cache_static(
             C.byref(d), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), new_k.data_ptr(), new_v.data_ptr(),

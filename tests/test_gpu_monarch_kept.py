@@ -175,3 +175,45 @@ def test_forward_and_backward_in_turn_take_no_more_memory_than_without_what_is_k
     kept = peak()
     monkeypatch.setattr(mattn, "_kept_buffer", lambda *a: None)
     assert kept <= peak() + (2 << 20)                               # allocations are rounded up to 512 bytes and more
+
+
+@pytest.mark.parametrize("writer", ["kv_cache_write", "operator", "operator_static", "operator_under_autograd", "dense", "prologue"])
+def test_cache_rows_written_before_the_backward_are_what_it_computes_with(writer):
+    """The caches are saved by reference: a call that writes rows between forward and backward makes the backward form all of its
+    intermediates from the new ones, as one does whose forward held none."""
+    h, w, H, D, dtype = 6, 20, 2, 64, torch.bfloat16
+    per, tiling = h * w, (1, 1, 1, 6, 20)
+    q, do, nk, nv, other_k, other_v = (randn((1, 3 * per, H, D), 550 + i, dtype).to(DEV) for i in range(6))
+    caches = [randn((1, 6 * per, H, D), 556 + i, dtype).to(DEV) for i in range(2)]
+    leaves = [t.requires_grad_(True) for t in (q, nk, nv)]
+    ones, rope = torch.ones(H * D, dtype=dtype, device=DEV), sfa.prologue.rope_table(D, device=DEV)
+    flat = [t.detach().reshape(1, 3 * per, H * D) for t in (q, other_k, other_v)]
+
+    def write(kc, vc):
+        rows = (other_k, other_v, 3 * per, 6 * per)
+        if writer == "operator_under_autograd":
+            return mattn.monarch_attn_with_kv_cache(q, kc, vc, *rows, *tiling, heads_per_pass=H)
+        with torch.no_grad():
+            if writer == "kv_cache_write":
+                mattn.kv_cache_write(*rows[:2], kc, vc, *rows[2:], *tiling)
+            elif writer == "operator":
+                mattn.monarch_attn_with_kv_cache(q, kc, vc, *rows, *tiling)
+            elif writer == "operator_static":
+                mattn.monarch_attn_with_kv_cache_static(q, kc, vc, *rows, *tiling)
+            elif writer == "dense":
+                sfa.attention.full_attention_with_kv_cache(q, kc, vc, *rows)
+            else:
+                sfa.prologue.qk_prologue(*flat, ones, ones, H, (3, h, w), 3, rope, kc, vc, 3 * per)
+
+    def grads(overwrite, **kw):
+        kc, vc = (t.clone() for t in caches)
+        out = mattn.monarch_attn_with_kv_cache(q, kc, vc, nk, nv, 3 * per, 6 * per, *tiling, grad_only_new_kv=True, **kw)
+        if overwrite:
+            write(kc, vc)
+        return torch.autograd.grad(out, leaves, do)
+
+    plain, want = grads(False), grads(True, heads_per_pass=H)
+    assert not torch.equal(plain[0], want[0])
+    for got in (grads(True), grads(True)):
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+    assert all(torch.equal(a, b) for a, b in zip(grads(False), plain))
