@@ -3,6 +3,8 @@ declares, and rejects bad arguments with error codes before touching any device.
 import ctypes as C
 import os
 import re
+import shutil
+import subprocess
 
 import pytest
 
@@ -399,3 +401,29 @@ def test_linear_descriptor_errors():
     assert call(out=0x10000 + 256) == -4 and b"overlaps" in lib.sfm_last_error()  # out inside x
     assert call(out=0x200000 - 64) == -4                                          # out runs into w
     assert call(x=0x10008) == -7
+
+
+def test_stores_past_the_caches_keep_their_hint(tmp_path):
+    """Step 1 has its stores of Kbar and Y twice, through the caches and past them; a compiler that merges the ends of the two drops
+    the hint of the second.  Every kernel of the library has to have as many 16-byte stores past the caches as a tile
+    has: D / 16 of Kbar and as many of Y."""
+    objdump = "/opt/rocm/llvm/bin/llvm-objdump"
+    if not os.path.exists(objdump):
+        pytest.skip("no llvm-objdump")
+    shutil.copy(L.LIB_PATH, tmp_path / "lib.so")
+    subprocess.run([objdump, "--offloading", "lib.so"], cwd=tmp_path, check=True, capture_output=True)
+    stores = {}
+    for obj in sorted(tmp_path.glob("lib.so.*gfx950")):
+        if b"monarch_step1_kernel" not in obj.read_bytes():
+            continue
+        name = None
+        text = subprocess.run([objdump, "-d", "--no-show-raw-insn", "--no-leading-addr", str(obj)], check=True, capture_output=True, text=True).stdout
+        for line in text.splitlines():
+            if line.startswith("<"):
+                name = line
+            elif "global_store_dwordx4" in line and "monarch_step1_kernel" in name:
+                stores[name] = stores.get(name, 0) + (line.split("//")[0].split()[-1] == "nt")
+    assert stores
+    for name, past in stores.items():
+        D, kbar_alone = re.search(r"INS_\w+?ELi(\d+)ELi\dELb\dELb\dELb(\d)", name).groups()
+        assert past >= int(D) // 16 * (1 if kbar_alone == "1" else 2), name
