@@ -94,16 +94,21 @@ class _KeptBudget:
     in use than if every backward formed them again (12 heads at 480p, three frames against 21: 769 + 760 MB, else 1500 and 29
     of dq in float32).  They are dropped, and their backward forms them again, for the next forward's, for a backward that has
     none and needs the larger workspace, and where a workspace grows.  A buffer is counted from its allocation until
-    nothing refers to it."""
+    nothing refers to it.
+
+    To leave them costs a forward up to 9 % (12 heads at 480p, 21 frames: 323 us without, 347), lost where no backward takes them: an
+    evaluation with gradients on, several layers in front of their backwards.  After two in a row that nothing took, forwards
+    leave nothing until a backward comes that would have found its own."""
 
     def __init__(self):
         self.left = 2 << 30                      # sfm_monarch_kept_bytes never asks for more
         self.lock = threading.RLock()            # a buffer may die inside take(), in the garbage collector
         self.refs = set()
         self.pending = None                      # the newest _Kept, weakly: it dies with its graph
+        self.unused = 0                          # that no backward took, since one did
+        self.turn = 0                            # what a forward leaves, or would have left, is there until the next turn
 
     def take(self, nbytes, device):
-        self.drop()
         with self.lock:
             if nbytes > self.left:
                 return None
@@ -127,8 +132,14 @@ class _KeptBudget:
     def hold(self, buf):
         kept = _Kept(buf)
         with self.lock:
-            self.pending = weakref.ref(kept)
+            self.pending = weakref.ref(kept, self._graph_died)
         return kept
+
+    def _graph_died(self, ref):
+        with self.lock:
+            if self.pending is ref:
+                self.pending = None
+                self.unused += 1
 
     def claim(self, kept):
         """The buffer, for one backward: from here on nobody drops it, and it dies with its last use."""
@@ -136,28 +147,42 @@ class _KeptBudget:
             buf, kept.buf = kept.buf, None
             if self.pending is not None and self.pending() is kept:
                 self.pending = None
+                self.unused = 0
         return buf
 
+    def missed(self, turn):
+        """A backward whose forward left nothing: would it be there?"""
+        with self.lock:
+            if turn == self.turn:
+                self.unused = 0
+
     def drop(self):
+        self.turn += 1                           # one lost to another thread costs a forward that leaves something for nobody
+        if self.pending is None:
+            return
         with self.lock:
             kept, self.pending = self.pending and self.pending(), None
             if kept is not None:
                 kept.buf = None
+                self.unused += 1
 
 
 _KEPT = {}
 _top_hooks = getattr(torch._C._autograd, "_top_saved_tensors_default_hooks", None)
 
 
-def _kept_buffer(nbytes, device):
+def _kept_buffer(desc, device):
     """A buffer for the intermediates of a forward under autograd, or None.  None too while hooks on saved tensors are set: their
     program wants little memory between forward and backward (activation checkpointing, save_on_cpu)."""
-    if not nbytes or _top_hooks is None or _top_hooks(False) is not None:
-        return None
     budget = _KEPT.get(device.index)
     if budget is None:
         budget = _KEPT.setdefault(device.index, _KeptBudget())
-    return budget.take(nbytes, device)
+    budget.drop()
+    if budget.unused > 1 or _top_hooks is None or _top_hooks(False) is not None:
+        return None
+    n = C.c_size_t(0)
+    _l.check(_l.load().sfm_monarch_kept_bytes(C.byref(desc), C.byref(n)))
+    return budget.take(n.value, device) if n.value else None
 
 
 def _drop_kept(index):
@@ -246,13 +271,12 @@ def _monarch_fwd_kept(q, k, v, tiling, sm_scale, kv_block_order, cbf, heads_per_
     _l.check(lib.sfm_monarch_stats_bytes(C.byref(d), C.byref(n)))
     stats = torch.empty(n.value // 4, dtype=torch.float32, device=q.device) if n.value else None
     kept = None
-    if new is not None:
-        _drop_kept(q.device.index)
     if keep and stats is not None and not heads_per_pass:
-        _l.check(lib.sfm_monarch_kept_bytes(C.byref(d), C.byref(n)))
-        kept = _kept_buffer(n.value, q.device)
+        kept = _kept_buffer(d, q.device)
+    elif new is not None:
+        _drop_kept(q.device.index)
     if kept is not None:
-        nbytes, ws = n.value, kept
+        nbytes, ws = kept.numel(), kept
     else:
         nbytes = monarch_workspace_bytes(d, heads_per_pass)
         ws = scratch(nbytes, q.device)
@@ -333,7 +357,9 @@ def _save(ctx, inputs, out, stats, kept):
     """The forward's tensors for the backward: the inputs, then the output and its row statistics if it left any.  `kept` is no saved
     tensor: it may be dropped before."""
     ctx.save_for_backward(*inputs, *(() if stats is None else (out, stats)))
-    ctx.kept = None if kept is None else _KEPT[kept.device.index].hold(kept)
+    budget = _KEPT.get(out.device.index)
+    ctx.kept = None if kept is None else budget.hold(kept)
+    ctx.turn = budget.turn if budget is not None else -1
 
 
 def _saved(ctx):
@@ -342,6 +368,8 @@ def _saved(ctx):
     left = dict(zip(("out", "stats"), left))
     if ctx.kept is not None:
         left["kept"] = _KEPT[q.device.index].claim(ctx.kept)
+    elif q.device.index in _KEPT:
+        _KEPT[q.device.index].missed(ctx.turn)
     if left.get("kept") is None:
         _drop_kept(q.device.index)
     return (q, k, v), left

@@ -217,3 +217,33 @@ def test_cache_rows_written_before_the_backward_are_what_it_computes_with(writer
     for got in (grads(True), grads(True)):
         assert all(torch.equal(a, b) for a, b in zip(got, want))
     assert all(torch.equal(a, b) for a, b in zip(grads(False), plain))
+
+
+def test_forwards_that_get_no_backward_stop_leaving_anything():
+    h, w, H, D, dtype = 6, 20, 2, 64, torch.bfloat16
+    q, k, v, do = (randn((1, 3 * h * w, H, D), 570 + i, dtype).to(DEV) for i in range(4))
+    leaves = [t.requires_grad_(True) for t in (q, k, v)]
+
+    def forward():
+        return mattn.monarch_attn(q, k, v, 1, 1, 1, h, w)
+
+    def backward(out):
+        return torch.autograd.grad(out, leaves, do)
+
+    def leaves_something(out):
+        return len(budget.refs) == 1
+
+    want = backward(forward())
+    budget = mattn._KEPT[torch.cuda.current_device()]
+    backward(forward())
+    assert all(leaves_something(forward()) for _ in range(2))       # their graphs die here
+    assert not any(leaves_something(forward()) for _ in range(3))
+    out = forward()
+    assert not leaves_something(out)
+    assert all(torch.equal(a, b) for a, b in zip(backward(out), want))      # it would have found its own
+    out = forward()
+    assert leaves_something(out) and all(torch.equal(a, b) for a, b in zip(backward(out), want))
+    layers = [forward() for _ in range(5)]                          # each makes room for the next
+    assert not leaves_something(layers)
+    backward(layers[0])                                             # would not
+    assert not leaves_something(forward())
