@@ -273,7 +273,7 @@ static int default_units_per_pass(const MonarchPlan& pl, int D) {
     if (n > (size_t)pl.units) n = pl.units;
     const size_t cols = (size_t)pl.na * pl.b2, all = cols * pl.nf * pl.b1 * 4 * D * pl.units, half = ((size_t)pl.units + 1) / 2;
     if (pl.mfma && !pl.iter && D == 128 && pl.b1 >= 20 && pl.b2 > 32 && cols >= 96 && pl.na <= 256 / pl.b2 &&
-        all > (size_t)352 << 20 && all <= (size_t)600 << 20 && 2 * cols * (pl.units / 2) >= 3 * (size_t)cu_count())
+        all > (size_t)352 << 20 && all <= (size_t)600 << 20 && 2 * cols * (pl.units / 2) >= 3 * (size_t)kChipCus)
         n = half;
     return (int)n;
 }

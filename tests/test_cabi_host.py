@@ -427,3 +427,28 @@ def test_stores_past_the_caches_keep_their_hint(tmp_path):
     for name, past in stores.items():
         D, kbar_alone = re.search(r"INS_\w+?ELi(\d+)ELi\dELb\dELb\dELb(\d)", name).groups()
         assert past >= int(D) // 16 * (1 if kbar_alone == "1" else 2), name
+
+
+def test_workspace_query_asks_no_device(tmp_path):
+    """sfm_monarch_workspace_bytes is arithmetic on its descriptor: the answer depends on no device, and none is asked for."""
+    import sys
+    (tmp_path / "count.cpp").write_text('static int n; extern "C" int hipGetDevice(int*) { ++n; return 100; } extern "C" int asked() { return n; }')
+    subprocess.run(["g++", "-shared", "-fPIC", "-o", str(tmp_path / "count.so"), str(tmp_path / "count.cpp")], check=True)
+    code = f"""
+import ctypes as C, sys
+sys.path[:0] = [{ROOT!r}, {os.path.join(ROOT, "tests")!r}]
+from self_forcing_amd import lib as L
+from test_cabi_host import _desc, _ws
+n, counter = C.c_size_t(0), C.CDLL({str(tmp_path / "count.so")!r})
+lib = L.load()
+before = counter.asked()
+for heads in (2, 8, 12, 40):
+    for kw in (dict(), dict(num_iters=3), dict(dtype=L.SFM_F32), dict(D=64)):
+        d = _desc(H=heads, **kw)
+        assert lib.sfm_monarch_workspace_bytes(C.byref(d), 0, C.byref(n)) == 0
+    assert lib.sfm_monarch_kept_bytes(C.byref(_desc(H=heads)), C.byref(n)) == 0
+assert counter.asked() == before, counter.asked() - before
+"""
+    preload = [str(tmp_path / "count.so")] + [p for p in [os.environ.get("LD_PRELOAD")] if p]
+    r = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, LD_PRELOAD=":".join(preload)), capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr
