@@ -71,7 +71,7 @@ typedef struct sfm_monarch_desc {
 } sfm_monarch_desc;
 
 /* Bytes of device scratch sfm_monarch_fwd needs when it processes `heads_per_pass`
- * (batch x head) units at a time (0 = library default: all of them, or half where that is faster).  Replaces the per-call torch.empty
+ * (batch x head) units at a time (0 = library default).  Replaces the per-call torch.empty
  * scratch of monarch_attn.py:1246-1259.  The size is not proportional to heads_per_pass. */
 int sfm_monarch_workspace_bytes(const sfm_monarch_desc* desc, int32_t heads_per_pass, size_t* bytes);
 

@@ -257,24 +257,18 @@ static int plan_monarch(const sfm_monarch_desc* d, MonarchPlan* pl) {
 }
 
 // Default number of units per pass: all of them while the scratch stays under 4 GiB (one launch pair
-// fills the chip best), or half of them where step 2 then finds the scratch in the memory-side cache (step 1 stores 40 to 364 MiB of it
-// through the caches) and both halves still fill the chip.  us as one pass and as two, 12 heads x 128 of 30 x 52, three frames
-// against 15 (431 MB) 243, 231, against 18 (517) 282, 268, 21 (604) 322, 316; 8 heads, 21 (403) 230, 204; 30 of 22 x 40, 12 frames (486)
-// 268, 251; 11 of 56 x 40, 15 (567) 312, 289; 4 of 45 x 80, 21 (464) 247, 245.  Not outside these limits: 12 heads, 12 frames
-// (345) 195, 198; 10 of 45 x 80 in half-width blocks, 6 frames (664) 345, 351; 16 block rows (15 heads of 16 x 66, 18) 223, 236, blocks
-// of 26 columns (18 heads of 30 x 52 in halves, 6) 266, 283, 31 columns in all (33 heads of 54 x 31, 21) 382, 400, two chunks
-// of them (6 heads of 30 x 52 in half-height blocks, 21) 278, 312, one unit to a pass (2 heads of 45 x 80 in halves, 21) 228, 252;
-// head_dim 64 (16 heads of 45 x 80, 12) 305, 314; a refinement of two passes, 21 frames, 624, 648.
-static int default_units_per_pass(const MonarchPlan& pl, int D) {
+// fills the chip best; smaller passes only pay when the scratch would not fit).  Halves of which the memory-side cache holds the scratch
+// between the steps are no rule: of 7000 random calls (250 to 1400 MiB, 2 to 40 heads, inputs in turn) two passes took 1.07 times as
+// long in the mean, and more than one in the mean whatever the bytes, rounds of step 1 or waves of step 2 in a pass.  Limits drawn
+// around the calls that gain (head_dim 128, 20 block rows, 96 columns of blocks wider than 32, 352 to 600 MiB) picked 521 of which 393
+// were slower, 1.05 times in the mean: 12 heads x 128 of 30 x 52, three frames against 21, 307 us as one pass and 300 as two, 8 heads 218, 205;
+// but 10 heads 255, 272, 13 heads, 12 frames 188, 214, and four of 46 x 100 in half-height blocks, 21, 210, 273.
+static int default_units_per_pass(const MonarchPlan& pl) {
     if (pl.fused) return pl.units;                // a few MB per unit
     const size_t budget = (size_t)3 << 30;        // keeps 32-bit element offsets into each scratch matrix
     size_t n = budget / pl.per_unit;
     if (n < 1) n = 1;
     if (n > (size_t)pl.units) n = pl.units;
-    const size_t cols = (size_t)pl.na * pl.b2, all = cols * pl.nf * pl.b1 * 4 * D * pl.units, half = ((size_t)pl.units + 1) / 2;
-    if (pl.mfma && !pl.iter && D == 128 && pl.b1 >= 20 && pl.b2 > 32 && cols >= 96 && pl.na <= 256 / pl.b2 &&
-        all > (size_t)352 << 20 && all <= (size_t)600 << 20 && 2 * cols * (pl.units / 2) >= 3 * (size_t)kChipCus)
-        n = half;
     return (int)n;
 }
 
@@ -310,7 +304,7 @@ int sfm_monarch_workspace_bytes(const sfm_monarch_desc* desc, int32_t heads_per_
         set_error("heads_per_pass must be >= 0");
         return SFM_ERR_SHAPE;
     }
-    int upp = heads_per_pass == 0 ? default_units_per_pass(pl, desc->D) : (heads_per_pass > pl.units ? pl.units : heads_per_pass);
+    int upp = heads_per_pass == 0 ? default_units_per_pass(pl) : (heads_per_pass > pl.units ? pl.units : heads_per_pass);
     *bytes = pass_bytes(pl, upp);
     return SFM_OK;
 }

@@ -301,6 +301,5 @@ int launch_dense_bwd(const sfm_dense_desc& d, const int64_t* dq_stride, const in
 
 void set_error(const char* fmt, ...);
 int cu_count();                                  // compute units of the current device (cached per thread)
-constexpr int kChipCus = 256;                    // of the chip, for sizes that are worked out on the host alone
 
 }  // namespace sfm

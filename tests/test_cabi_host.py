@@ -89,6 +89,16 @@ def _ws(d, hpp=0):
     return rc, n.value
 
 
+def test_default_passes_hold_all_heads_below_the_scratch_limit():
+    """Whatever the memory-side cache could hold of a part of them: 12, 8 and 30 heads of 384 to 640 MiB, and a block-causal call."""
+    for kw in (dict(H=12), dict(H=8), dict(H=10), dict(H=13, kv_tokens=12 * 30 * 52), dict(H=7, q_tokens=9 * 30 * 52, kv_tokens=9 * 30 * 52, causal_block_frames=3),
+               dict(H=30, q_tokens=3 * 22 * 40, kv_tokens=12 * 22 * 40, tiling=L.Tiling(1, 1, 1, 22, 40))):
+        d = _desc(**kw)
+        assert _ws(d) == _ws(d, d.H) and _ws(d)[0] == 0
+    d = _desc(H=80)                                          # 3.75 GiB: as many as fit 3 GiB
+    assert _ws(d)[1] <= 3 << 30 < _ws(d, 80)[1]
+
+
 def _fused_bytes(na, nf, b1, b2, units, cus=256):
     """Scratch of the one-kernel forward for a pass over `units` units: one output block [b1, 128] (16 bit) and 32
     floats per (unit, stream slot, column); streams = compute units // column groups of (up to) 12."""
