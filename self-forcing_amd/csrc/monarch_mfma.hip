@@ -26,6 +26,7 @@
 // The running output stays in fp32 for the whole KV range (the reference rounds it to 16 bit
 // between KV chunks, monarch_attn.py:795,838).
 
+#include "monarch_rules.hpp"
 #include "sfm_common.hpp"
 
 #include <algorithm>
@@ -407,7 +408,7 @@ void monarch_step1_kernel(MonarchArgs p) {
         // bit 3 for the block within the pair (a rotation by 8 within rows of 16 lanes).  Afterwards a lane
         // holds, for each of the four row groups rb, the piece 4 (dt0 + bit 3) + 2 bit 4 + hf of column
         // (c & 7) + 8 rb, so that one store instruction writes 128 contiguous bytes of each of 8 rows.
-        // Past the caches or through them: see enqueue_step1
+        // Past the caches or through them: see step1_through_caches
         auto contract = [&](auto cached) {
 #pragma unroll
             for (int which = 0; which < (KO ? 1 : 2); ++which) {
@@ -613,7 +614,7 @@ void monarch_step2_kernel(MonarchArgs p) {
             const int P = g * 64 + lane;
             const int r = P / CPR, c = (P % CPR) ^ s1_swz<CPR>(r);
             const uint32_t off = (uint32_t)min(32 * n + r, r_lim - 1) * (2 * D) + (uint32_t)c * 16;
-            if constexpr (PAST) s1_load_lds16_nt(mat, off, dst + (uint32_t)g * 1024);          // see enqueue_step2
+            if constexpr (PAST) s1_load_lds16_nt(mat, off, dst + (uint32_t)g * 1024);          // see step2_past_caches
             else s1_load_lds16(mat, off, dst + (uint32_t)g * 1024);
         }
     };
@@ -1637,16 +1638,7 @@ static int enqueue_step1(const MonarchArgs& a, int nunits, hipStream_t stream, S
     // tied frames against themselves 50 -> 46; 24 columns of nine 30 x 24 frames 52 -> 39.  Four groups of three waves: 50 us
     // at 7 heads of nine 23 x 31 frames, two 44.5.  Two or four waves for 32 columns, each with its part of the output, took
     // the refinement to 505 and 541 us: they fetch the query rows as often.
-    // What a pass writes goes through the caches where the memory-side one (256 MB) can still hold most of it for the kernel that reads
-    // it next, and past them where it cannot (written back under that kernel's reads) or where it is little (the L2s give their dirty
-    // lines up at the kernel's end).  us past the caches and through them, 12 heads x 128 of 30 x 52 unless named: three frames
-    // against 3 (86 MB) 67, 63.5, 6 (173) 112, 104, 9 (259) 154, 143, 12 (345) 201, 193, 21 (604) 322, 331; 45 x 80, 6 frames (398)
-    // 245, 242, but level since step 2 reads past them; 12 frames in half-height blocks (690) 341, 376; three passes at three frames
-    // tied (100 and 201) 450, 424; 2 heads, 6 frames (29) 29.4, 29.3; 1 head, 3 frames (7) 21.8, 22.9; three frames tied against themselves (29) 44.6, 47.4.  Kbar alone is
-    // followed by as many bytes of representatives: two passes, 21 frames (302) 624, 637.
-    const size_t scratch_rows = (size_t)nunits * a.na * a.b2 * a.nf * a.b1;
-    const size_t written = scratch_rows * ((kind == Step1::kIterKbar ? 2 : 4) * D + (a.rb ? 128 : 0));
-    a1.s1_cached = written >= (size_t)40 << 20 && written <= (size_t)(kind == Step1::kIterKbar ? 256 : 364) << 20;
+    a1.s1_cached = step1_through_caches(a, nunits, kind == Step1::kIterKbar);
     const int cus = a.s1_wgs > 0 ? a.s1_wgs : cu_count();
     // Two groups of six waves are worth it at head_dim 64 only (176 columns of 44 x 44, 12 heads: 161 us, one group 172; head_dim 128
     // 304, 297; 192 columns of 30 x 64 240, 232).
@@ -1681,11 +1673,7 @@ static const void* step2_kernel(bool past) {
 template <class E, int D>
 static int enqueue_step2(const MonarchArgs& a, int nunits, hipStream_t stream, bool stats_only = false) {
     const int team = a.b1 > 96 ? 4 : (a.b1 + 31) / 32;
-    // From the size on where the memory-side cache holds part of Kbar and Y only, their rows, read once, are read past it: us
-    // through the caches and past them, 12 heads x 128 of 30 x 52, three frames against 9 (259 MB) 143, 140, 12 (345) 193, 179, in
-    // half-height blocks (690) 342, 336; 6 heads, 21 frames (302) 155, 146; 40 heads, 21 (2013) 1038, 1002.  Below, they would leave it: 6 heads,
-    // 12 frames (173 MB) 96.3, 98.6; three frames tied against 21 (201) 146, 149.
-    const bool past = (size_t)nunits * a.na * a.b2 * a.nf * a.b1 * 4 * D >= (size_t)240 << 20;
+    const bool past = step2_past_caches(a, nunits);
     const void* fn = stats_only ? (team == 4   ? (const void*)monarch_left_stats_kernel<E, D, 4>
                                    : team == 3 ? (const void*)monarch_left_stats_kernel<E, D, 3>
                                    : team == 2 ? (const void*)monarch_left_stats_kernel<E, D, 2>
