@@ -23,12 +23,15 @@ inline bool step1_skips_masked(const MonarchArgs& a) { return a.causal && a.skip
 // 245, 242, but level since step 2 reads past them; 12 frames in half-height blocks (690) 341, 376; three passes at three frames
 // tied (100 and 201) 450, 424; 2 heads, 6 frames (29) 29.4, 29.3; 1 head, 3 frames (7) 21.8, 22.9; three frames tied against themselves (29) 44.6, 47.4.  Kbar alone is
 // followed by as many bytes of representatives: two passes, 21 frames (302) 624, 637.
+// Teams of waves (more than 32 query rows in step 2) need 64 MiB: 80 random calls of 36 to 70 are 0.988 times as long with that limit as with 40,
+// block-causal ones 0.982 (through the caches, with more than 64 rows, 1.02 times; half-height blocks of 30 x 52, three tied, 4 heads x 64, 55 MiB: 51.5 us, 53.0).  Up to 32 rows 51 calls of 40 to 64 take 0.98 times as long through them.
 // What is too little is what the pass does write, masked pairs left out: counted with them, block-causal calls of 25 to 40 MiB took up
 // to 4 % longer.  The upper limit counts them: of 240 to 300 MiB without, such calls took 3 % longer through the caches (12 frames
 // of 30 x 52, 4 heads, 274 MiB of 439: 173, 182).
 inline bool step1_through_caches(const MonarchArgs& a, int nunits, bool kbar_alone) {
     const size_t row = (kbar_alone ? 2 : 4) * a.D + (a.rb ? 128 : 0);
-    return scratch_rows(a, nunits, step1_skips_masked(a)) * row >= (size_t)40 << 20 &&
+    const size_t least = a.b1 > 32 && !kbar_alone ? 64 : 40;
+    return scratch_rows(a, nunits, step1_skips_masked(a)) * row >= least << 20 &&
            scratch_rows(a, nunits, false) * row <= (size_t)(kbar_alone ? 256 : 364) << 20;
 }
 

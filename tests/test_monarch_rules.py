@@ -46,9 +46,15 @@ def test_masked_rows_are_not_counted(rules, na, causal):
 
 
 def test_block_causal_calls_are_too_small_by_the_rows_they_write(rules):
-    assert rules(5, 5, 66, 40, 2)[1] and not rules(5, 5, 66, 40, 2, causal=1)[1]       # 39 MiB of 64
-    assert rules(5, 5, 66, 40, 3, causal=1)[1]
-    assert rules(5, 5, 66, 40, 2, causal=1, new_kv=1)[1]                               # with a new chunk step 1 forms all rows
+    assert rules(5, 5, 32, 40, 4)[1] and not rules(5, 5, 32, 40, 4, causal=1)[1]       # 37 MiB of 62
+    assert rules(5, 5, 32, 40, 5, causal=1)[1]
+    assert rules(5, 5, 32, 40, 4, causal=1, new_kv=1)[1]                               # with a new chunk step 1 forms all rows
     # the upper limits go by all rows: nine frames of 30 x 52, three tied, 12 heads, 165 MiB of 247; 14 frame pairs, 329 of 494
     assert rules(3, 3, 90, 52, 12, causal=1)[1:] == (True, True)
     assert rules(6, 6, 45, 52, 12, causal=2)[1:] == (False, True)
+
+
+def test_teams_need_more(rules):
+    assert rules(2, 8, 32, 26, 7)[1] and not rules(2, 8, 33, 26, 7)[1]                 # 46 and 47 MiB
+    assert rules(2, 8, 33, 26, 10)[1] and not rules(2, 8, 32, 26, 6)[1]                # 67 and 39
+    assert rules(2, 8, 33, 26, 14, kbar_alone=1)[1]                                    # 47 of Kbar alone, which step 2 does not read
