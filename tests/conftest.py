@@ -32,3 +32,13 @@ def pytest_collection_modifyitems(config, items):
     for item in items:
         if "gpu" in item.keywords:
             item.add_marker(skip)
+
+
+@pytest.fixture(autouse=True)
+def _nothing_kept_for_backwards(request):
+    """Whether a Monarch forward under autograd leaves its intermediates follows what became of earlier ones: every GPU test starts
+    as a program does, whatever ran before it."""
+    if "gpu" in request.keywords:
+        import self_forcing_amd as sfa
+        sfa.monarch_attn._KEPT.clear()
+    yield
