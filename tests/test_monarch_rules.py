@@ -49,9 +49,21 @@ def test_block_causal_calls_are_too_small_by_the_rows_they_write(rules):
     assert rules(5, 5, 32, 40, 4)[1] and not rules(5, 5, 32, 40, 4, causal=1)[1]       # 37 MiB of 62
     assert rules(5, 5, 32, 40, 5, causal=1)[1]
     assert rules(5, 5, 32, 40, 4, causal=1, new_kv=1)[1]                               # with a new chunk step 1 forms all rows
-    # the upper limits go by all rows: nine frames of 30 x 52, three tied, 12 heads, 165 MiB of 247; 14 frame pairs, 329 of 494
-    assert rules(3, 3, 90, 52, 12, causal=1)[1:] == (True, True)
-    assert rules(6, 6, 45, 52, 12, causal=2)[1:] == (False, True)
+
+
+def test_the_most_depends_on_the_query_block_frames(rules):
+    for na, most in ((1, 1100), (3, 1100), (5, 1100), (6, 240), (12, 240)):
+        per_head = na * 12 * 32 * 40 * 512 / 2**20
+        fits = int(most / per_head)
+        assert rules(na, 12, 32, 40, fits)[1] and not rules(na, 12, 32, 40, fits + 1)[1], na
+        assert rules(na, 12, 32, 40, int(512 / per_head), kbar_alone=1)[1] and not rules(na, 12, 32, 40, int(512 / per_head) + 1, kbar_alone=1)[1]
+    # masked pairs count from six block-frames on, where step 2 reads past the caches, and not below: 1069 MiB of 1604
+    assert rules(3, 3, 90, 52, 78, causal=1)[1] and rules(6, 6, 45, 52, 5, causal=2)[1] and not rules(6, 6, 45, 52, 6, causal=2)[1]
+
+
+def test_step_2_reads_past_the_caches_from_240_mib_on(rules):
+    assert not rules(3, 21, 30, 52, 5)[2] and rules(3, 21, 30, 52, 6)[2]               # 239.9 and 288 MiB
+    assert rules(3, 3, 90, 52, 12, causal=1)[2]                                        # masked pairs count
 
 
 def test_teams_need_more(rules):
