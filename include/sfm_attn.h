@@ -147,8 +147,8 @@ int sfm_monarch_bwd_saved(const sfm_monarch_bwd_desc* desc, const void* q, const
 
 /* sfm_monarch_bwd_saved with what sfm_monarch_fwd_kept (or sfm_monarch_attn_with_kv_cache_kept) left, on the same forward
  * descriptor; same results, but dq comes in the tensor dtype (the float32 sum rounded once), dq_stride in its elements.  `kept`
- * is only read.  SFM_ERR_UNSUPPORTED where sfm_monarch_kept_bytes is 0 or the gradients'
- * rows are not 16-byte aligned.  Less workspace than sfm_monarch_bwd_kept_workspace_bytes, down to one (batch, head) unit's
+ * is only read.  SFM_ERR_UNSUPPORTED where sfm_monarch_kept_bytes is 0, for sfm_monarch_bwd_saved to take the call; gradients
+ * whose rows are not 16-byte aligned are SFM_ERR_STRIDE or SFM_ERR_ALIGN here as there.  Less workspace than sfm_monarch_bwd_kept_workspace_bytes, down to one (batch, head) unit's
  * share, means more passes. */
 int sfm_monarch_bwd_kept_workspace_bytes(const sfm_monarch_bwd_desc* desc, size_t* bytes);
 int sfm_monarch_bwd_kept(const sfm_monarch_bwd_desc* desc, const void* q, const void* k, const void* v, const void* out,

@@ -413,6 +413,29 @@ def test_linear_descriptor_errors():
     assert call(x=0x10008) == -7
 
 
+def test_kept_backward_errors():
+    """Nothing to keep is SFM_ERR_UNSUPPORTED, misaligned gradients are what they are to the other backwards."""
+    lib, n, fake = L.load(), C.c_size_t(0), 0x10000
+
+    def bwd(dq=fake, dk=fake, kept_size=1 << 40, dq_stride=None, dkv_stride=None, **kw):
+        bd = L.MonarchBwdDesc()
+        bd.fwd = _desc(kv_tokens=3 * 30 * 52, **kw)
+        bd.dq_stride = (C.c_int64 * 3)(*(dq_stride or bd.fwd.q_stride))
+        bd.dkv_stride = (C.c_int64 * 3)(*(dkv_stride or bd.fwd.k_stride))
+        bd.kv_grad_frame_start, bd.kv_grad_frame_end = 0, 1
+        return (lib.sfm_monarch_bwd_kept_workspace_bytes(C.byref(bd), C.byref(n)),
+                lib.sfm_monarch_bwd_kept(C.byref(bd), *[fake] * 6, kept_size, fake, dq, dk, fake, None, 0, None))
+
+    rows = 3 * 30 * 52 * 256
+    assert bwd() == (0, -6) and n.value > 0                                # all but the workspace is in order
+    assert bwd(kept_size=1 << 20) == (0, -6)
+    assert bwd(D=32) == (-9, -9) and b"kept" in lib.sfm_last_error()       # head_dim 32 has no MFMA kernels
+    assert bwd(num_iters=2) == (-9, -9)
+    assert bwd(dq_stride=(rows, 260, 128)) == (-5, -5)                     # 520 bytes: whole 16-byte pieces in float32 only
+    assert bwd(dkv_stride=(rows, 260, 128)) == (-5, -5)
+    assert bwd(dq=fake + 8) == (0, -7) and bwd(dk=fake + 2) == (0, -7)
+
+
 def test_stores_past_the_caches_keep_their_hint(tmp_path):
     """Step 1 has its stores of Kbar and Y twice, through the caches and past them; a compiler that merges the ends of the two drops
     the hint of the second.  Every kernel of the library has to have as many 16-byte stores past the caches as a tile
