@@ -434,7 +434,9 @@ def test_wrappers_reuse_one_scratch_buffer_per_stream():
 
 # passes whose scratch lies below, within and beyond the sizes that step 1 stores through the caches; with the right factor too
 @pytest.mark.parametrize("heads,heads_per_pass,q_frames,frames,D,dtype", [(6, 2, 3, 3, 128, torch.bfloat16), (12, 4, 3, 21, 128, torch.float16),
-                                                                         (14, 5, 3, 9, 64, torch.bfloat16)])
+                                                                         (14, 5, 3, 9, 64, torch.bfloat16),
+                                                                         # six query block-frames: 329 MiB past them, 219 through
+                                                                         (6, 4, 6, 12, 128, torch.bfloat16)])
 def test_scratch_through_and_past_the_caches_gives_the_same_bits(heads, heads_per_pass, q_frames, frames, D, dtype):
     h, w = 30, 52
     q = randn((1, q_frames * h * w, heads, D), 440, dtype).to(DEV)

@@ -161,9 +161,9 @@ def test_480p_block_shape_bf16_one_head(bwd_path):
     (4, 52, 4, 4, 64, True, torch.bfloat16),       # 208 columns: four chunks of the right-factor kernel, the last of 16
     (4, 52, 7, 7, 128, False, torch.float16),      # 364: six, the last of 44
     (5, 6, 2, 3, 64, False, torch.bfloat16),       # b2 = 6, not a multiple of 4
-    (2, 32, 15, 2, 128, False, torch.bfloat16),    # 480 columns, the most of the fused right factor
-    (2, 37, 13, 2, 64, False, torch.bfloat16),     # 481: the library chain
-    (2, 19, 27, 27, 128, True, torch.float16),     # 513, block-causal
+    (2, 32, 15, 2, 128, False, torch.bfloat16),    # 480 columns: eight chunks of the right factor, the last of 32
+    (2, 37, 13, 2, 64, False, torch.bfloat16),     # 481: the last of 33
+    (2, 19, 27, 27, 128, True, torch.float16),     # 513, block-causal: nine, the last of one
     (4, 20, 3, 9, 128, False, torch.bfloat16),     # 36 rows (f, k) per column: two chunks of the left factor, the second with 4 rows
     (8, 12, 2, 8, 64, False, torch.float16),       # 64 rows: two full chunks
     (6, 10, 6, 6, 128, True, torch.bfloat16),      # block-causal with two chunks: the visible rows end inside a chunk
@@ -179,6 +179,10 @@ def test_16bit_gradients_across_the_fused_kernels_limits(h, w, Fq, Fk, D, causal
     qr, kr, vr = _leaf(q0.double()), _leaf(k0.double()), _leaf(v0.double())
     monarch.monarch_attn(qr, kr, vr, 1, 1, 1, h, w, **kw).backward(do.double())
     qd, kd, vd = _leaf(q0, DEV), _leaf(k0, DEV), _leaf(v0, DEV)
+    # every part is a fused kernel, whatever the columns: only then is there something to keep
+    desc, n = mattn._desc(qd, kd, vd, qd, 1, 1, 1, h, w, D ** -0.5, 0, int(causal), 1), C.c_size_t(0)
+    sfa.lib.check(sfa.lib.load().sfm_monarch_kept_bytes(C.byref(desc), C.byref(n)))
+    assert n.value > 0
     mattn.monarch_attn(qd, kd, vd, 1, 1, 1, h, w, **kw).backward(do.to(DEV))
     _close(qd.grad, qr.grad, dtype)
     _close(kd.grad, kr.grad, dtype)

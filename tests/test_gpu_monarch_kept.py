@@ -247,3 +247,28 @@ def test_forwards_that_get_no_backward_stop_leaving_anything():
     assert not leaves_something(layers)
     backward(layers[0])                                             # would not
     assert not leaves_something(forward())
+
+
+@pytest.mark.parametrize("tiling,D", [((1, 1, 1, 9, 24), 128), ((3, 1, 1, 12, 16), 64), ((1, 2, 1, 8, 33), 128)])
+def test_kept_intermediates_of_strided_tensors(tiling, D):
+    """q out of a fused projection, the new chunk too, caches that are some rows and heads of larger ones, a gradient with another
+    order: the bits of the path that keeps nothing, and of contiguous tensors."""
+    f_tied, hr, wr, h, w = tiling
+    per, H, B, dtype = h * w, 3, 2, torch.bfloat16
+    qkv = randn((B, 3 * per, 3, H, D), 580, dtype).to(DEV)
+    q, nk, nv = qkv.unbind(2)
+    big_k, big_v = (randn((B, 11 * per, H + 2, D), 581 + i, dtype).to(DEV) for i in range(2))
+    do = randn((B, H, 3 * per, D), 583, dtype).to(DEV).transpose(1, 2)
+    grads = []
+    for kw in ({}, dict(heads_per_pass=B * H)):
+        for dense in (False, True):
+            ql, nkl, nvl = (t.detach().clone(memory_format=torch.contiguous_format) if dense else t.detach() for t in (q, nk, nv))
+            assert dense or not ql.is_contiguous()
+            kc, vc = (t.clone()[:, 2 * per:8 * per, 1:H + 1] for t in (big_k, big_v))
+            kc, vc = (t.contiguous() if dense else t for t in (kc, vc))
+            leaves = [t.requires_grad_(True) for t in (ql, nkl, nvl)]
+            out = mattn.monarch_attn_with_kv_cache(ql, kc, vc, nkl, nvl, 3 * per, 6 * per, *tiling, grad_only_new_kv=True, **kw)
+            assert bool(kw) == (len(mattn._KEPT[torch.cuda.current_device()].refs) == 0)
+            grads.append((out, *torch.autograd.grad(out, leaves, do)))
+    for g in grads[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(grads[0], g))
