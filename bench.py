@@ -251,6 +251,20 @@ def op_level(torch, sfa, args):
         torch.cuda.synchronize()
         bwd[name] = (time.perf_counter() - t0) * 1e3 / 3
     bwd_ms = bwd["saved"]
+    # forward and backward as a program under autograd runs them: the backward takes the forward's intermediates
+    leaves = [t.detach().requires_grad_(True) for t in (q, kc, vc)]
+
+    def forward_backward():
+        return torch.autograd.grad(sfa.monarch_attn.monarch_attn(*leaves, 1, 1, 1, B1, B2, kv_block_order=True), leaves, do)
+
+    forward_backward()
+    torch.cuda.synchronize()
+    t0 = time.perf_counter()
+    for _ in range(3):
+        forward_backward()
+    torch.cuda.synchronize()
+    fwd_bwd_ms = (time.perf_counter() - t0) * 1e3 / 3
+    del leaves
 
     # backward of the dense fallback at the same shape (all keys, and the new chunk's keys only)
     from self_forcing_amd.attention import _dense_bwd, _dense_fwd
@@ -321,7 +335,8 @@ def op_level(torch, sfa, args):
                          "ms_per_call": iter_ms, "ms_per_call_fp32_simt_kernels": iter_simt_ms,
                          "tflops": 8 * MONARCH_FLOPS / (iter_ms * 1e-3) / 1e12},
         "monarch_bwd": {"workload": "gradients of q and of all 21 cached K/V frames at the same shape",
-                        "ms_per_call": bwd_ms, "ms_per_call_recomputing_statistics": bwd["recompute"]},
+                        "ms_per_call": bwd_ms, "ms_per_call_recomputing_statistics": bwd["recompute"],
+                        "ms_per_forward_and_backward_under_autograd": fwd_bwd_ms},
         "l2_read_probe_tbs": l2_tbs,
         "dense_fallback": {"ms_per_call": dense_ms, "tflops": dense_tfl, "mfma_frac": dense_tfl / MFMA_BF16_PEAK_TFLOPS,
                            "mfma_probe_tflops": probe.value, "frac_of_probe": dense_tfl / probe.value,
