@@ -86,13 +86,12 @@ template <int CPR>
 __device__ __forceinline__ int bl_swz(int r) {
     return CPR >= 16 ? (((r & 3) << 2) | ((r >> 2) & 3)) : ((((r >> 1) & 1) << 2) | ((r >> 2) & 3));
 }
-// 64 lanes' 16 bytes into LDS past the caches: Kbar and Y are read once here, and what they would displace is read again (training
-// step, 12 heads, three frames against 21: 931 -> 899 us; 6 against themselves 335 -> 325; teams: 80 random calls of 100 to 900 MiB 0.99 times
-// as long, block-causal ones too)
 __device__ __forceinline__ void bl_load_lds16(const char* base, uint32_t off, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds_addr), "v"(off), "s"(base) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(off), "s"(base) : "memory", "m0");
 }
-// the same with the LDS address as a scalar base plus a compile-time offset (one scalar register for all of a chunk's loads)
+// the same with the LDS address as a scalar base plus a compile-time offset (one scalar register for all of a chunk's loads), past
+// the caches: Kbar and Y are read once here, and what they would displace is read again (training step, 12 heads, three frames
+// against 21: 931 -> 899 us; 6 against themselves 335 -> 325)
 template <int OFF>
 __device__ __forceinline__ void bl_load_lds16_at(const char* base, uint32_t off, uint32_t lds_base) {
     asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds_base), "v"(off), "s"(base), "n"(OFF) : "memory", "m0", "scc");
