@@ -86,6 +86,8 @@ template <int CPR>
 __device__ __forceinline__ int bl_swz(int r) {
     return CPR >= 16 ? (((r & 3) << 2) | ((r >> 2) & 3)) : ((((r >> 1) & 1) << 2) | ((r >> 2) & 3));
 }
+// (through the caches: teams that read past them gain 1 % where only a new chunk's keys get gradients, and with all keys take up to 2 %
+// longer, 12 heads x 128 of 30 x 52 in half-height blocks, three tied, 15 frames: 600, 610 us)
 __device__ __forceinline__ void bl_load_lds16(const char* base, uint32_t off, uint32_t lds_addr) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(off), "s"(base) : "memory", "m0");
 }
