@@ -187,7 +187,8 @@ def _kept_buffer(desc, device):
 
 def _drop_kept(index):
     """Every call that writes cache rows makes this one too: a backward takes K and V from the caches as it finds them, and with rows
-    written since its forward it has to form the right factor from those too, not from the ones that the forward saw."""
+    written since its forward it has to form the right factor from those too, not from the ones that the forward saw.  (A replayed
+    graph makes no call: rows that it writes reach K and V alone.)"""
     if index in _KEPT:
         _KEPT[index].drop()
 
