@@ -9,7 +9,7 @@ import warnings
 import torch
 
 from . import lib as _l
-from .monarch_attn import _DT, _check4, _drop_kept, _on_device, _stream, scratch as _scratch
+from .monarch_attn import _DT, _KEPT, _check4, _drop_kept, _on_device, _stream, scratch as _scratch
 
 
 def _dense_desc(q, k, v, out, sm_scale):
@@ -163,7 +163,8 @@ def _dense_cache_fwd(q, k_cache, v_cache, new_k, new_v, start_idx, end_idx, sm_s
     out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     lse = torch.empty((q.shape[0], q.shape[2], q.shape[1]), dtype=torch.float32, device=q.device) if want_lse else None
     d = _dense_desc(q, k_cache, v_cache, out, sm_scale)
-    _drop_kept(q.device.index)
+    if _KEPT:
+        _drop_kept(q.device.index)
     with _on_device(q.device):
         ws, nbytes = _dense_workspace(d, q.device)
         _l.check(_l.load().sfm_full_attention_with_kv_cache_ws(

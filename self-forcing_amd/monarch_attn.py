@@ -76,16 +76,16 @@ def release_scratch():
     _SCRATCH.clear()
 
 
-class _KeptRef(weakref.ref):
-    __slots__ = ("nbytes",)
-
-
 class _Kept:
-    """What one forward left for its backward, while nobody else has had it dropped."""
-    __slots__ = ("buf", "__weakref__")
+    """What one forward left for its backward, until that takes it, another call has it dropped or its graph dies."""
+    __slots__ = ("buf", "budget", "__weakref__")
 
-    def __init__(self, buf):
-        self.buf = buf
+    def __init__(self, buf, budget):
+        self.buf, self.budget = buf, budget
+
+    def __del__(self):
+        if self.buf is not None:
+            self.budget.graph_died(self)
 
 
 class _KeptBudget:
@@ -93,8 +93,7 @@ class _KeptBudget:
     backward that finds them is smaller by as much, so a program that calls forward and backward in turn has no more memory
     in use than if every backward formed them again (12 heads at 480p, three frames against 21: 769 + 760 MB, else 1500 and 29
     of dq in float32).  They are dropped, and their backward forms them again, for the next forward's, for a backward that has
-    none and needs the larger workspace, and where a workspace grows.  A buffer is counted from its allocation until
-    nothing refers to it.
+    none and needs the larger workspace, and where a workspace grows.
 
     To leave them costs a forward 10 % (12 heads at 480p, 21 frames: 291 us without, 320), lost where no backward takes them: an
     evaluation with gradients on, several layers in front of their backwards.  After two in a row that nothing took, forwards
@@ -102,68 +101,61 @@ class _KeptBudget:
 
     def __init__(self):
         self.left = 2 << 30                      # sfm_monarch_kept_bytes never asks for more
-        self.lock = threading.RLock()            # a buffer may die inside take(), in the garbage collector
-        self.refs = set()
-        self.pending = None                      # the newest _Kept, weakly: it dies with its graph
+        self.lock = threading.RLock()            # a _Kept may die inside any of these, in the garbage collector
+        self.pending = None                      # the one _Kept with a buffer, weakly: it dies with its graph
         self.unused = 0                          # that no backward took, since one did
         self.turn = 0                            # what a forward leaves, or would have left, is there until the next turn
 
     def take(self, nbytes, device):
-        with self.lock:
-            if nbytes > self.left:
-                return None
-            self.left -= nbytes
-        try:
-            buf = torch.empty(nbytes, dtype=torch.uint8, device=device)
-        except torch.OutOfMemoryError:
-            with self.lock:
-                self.left += nbytes
+        if nbytes > self.left:
             return None
-        ref = _KeptRef(buf, self._died)
-        ref.nbytes = nbytes
-        self.refs.add(ref)
-        return buf
-
-    def _died(self, ref):
-        with self.lock:
-            self.refs.discard(ref)
-            self.left += ref.nbytes
+        try:
+            return torch.empty(nbytes, dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError:
+            return None
 
     def hold(self, buf):
-        kept = _Kept(buf)
+        kept = _Kept(buf, self)
         with self.lock:
-            self.pending = weakref.ref(kept, self._graph_died)
+            if self.pending is not None:         # of another thread, since this one's forward began
+                self.drop()
+            self.left -= buf.numel()
+            self.pending = weakref.ref(kept)
         return kept
 
-    def _graph_died(self, ref):
-        with self.lock:
-            if self.pending is ref:
-                self.pending = None
-                self.unused += 1
+    def _release(self, kept):
+        """The buffer that `kept` no longer holds (with the lock)."""
+        buf, kept.buf = kept.buf, None
+        if buf is not None:
+            self.left += buf.numel()
+            self.pending = None
+        return buf
 
     def claim(self, kept):
         """The buffer, for one backward: from here on nobody drops it, and it dies with its last use."""
         with self.lock:
-            buf, kept.buf = kept.buf, None
-            if self.pending is not None and self.pending() is kept:
-                self.pending = None
+            buf = self._release(kept)
+            if buf is not None:
                 self.unused = 0
         return buf
 
+    def graph_died(self, kept):
+        with self.lock:
+            if self._release(kept) is not None:
+                self.unused += 1
+
     def missed(self, turn):
         """A backward whose forward left nothing: would it be there?"""
-        with self.lock:
-            if turn == self.turn:
-                self.unused = 0
+        if turn == self.turn:
+            self.unused = 0
 
     def drop(self):
         self.turn += 1                           # one lost to another thread costs a forward that leaves something for nobody
         if self.pending is None:
             return
         with self.lock:
-            kept, self.pending = self.pending and self.pending(), None
-            if kept is not None:
-                kept.buf = None
+            kept = self.pending and self.pending()
+            if kept is not None and self._release(kept) is not None:
                 self.unused += 1
 
 
@@ -186,7 +178,7 @@ def _kept_buffer(desc, device):
 
 
 def _drop_kept(index):
-    """Every call that writes cache rows makes this one too: a backward takes K and V from the caches as it finds them, and with rows
+    """Every call that writes cache rows makes this one too (where anything was ever kept: its cost is 0.3 of the smallest call's 18 us): a backward takes K and V from the caches as it finds them, and with rows
     written since its forward it has to form the right factor from those too, not from the ones that the forward saw.  (A replayed
     graph makes no call: rows that it writes reach K and V alone.)"""
     if index in _KEPT:
@@ -239,7 +231,8 @@ def kv_cache_write(new_k, new_v, k_cache, v_cache, start_idx, end_idx, f_tied, h
     B, _, H, D = new_k.shape
     if B > k_cache.shape[0] or H > k_cache.shape[2] or D > k_cache.shape[3]:
         raise ValueError(f"new_k {tuple(new_k.shape)} holds more batches, heads or channels than the cache {tuple(k_cache.shape)}")
-    _drop_kept(k_cache.device.index)
+    if _KEPT:
+        _drop_kept(k_cache.device.index)
     with _on_device(new_k.device):
         _l.check(_l.load().sfm_kv_cache_write(_DT[new_k.dtype], B, H, D, C.byref(_l.Tiling(f_tied, h_reduce, w_reduce, h, w)),
                                               new_k.data_ptr(), new_v.data_ptr(), _l.strides3(new_k), k_cache.data_ptr(),
@@ -274,7 +267,7 @@ def _monarch_fwd_kept(q, k, v, tiling, sm_scale, kv_block_order, cbf, heads_per_
     kept = None
     if keep and stats is not None and not heads_per_pass:
         kept = _kept_buffer(d, q.device)
-    elif new is not None:
+    elif new is not None and _KEPT:
         _drop_kept(q.device.index)
     if kept is not None:
         nbytes, ws = kept.numel(), kept
@@ -357,23 +350,27 @@ def _monarch_bwd(q, k, v, dout, tiling, sm_scale, kv_block_order, cbf, kv_f0=0, 
 def _save(ctx, inputs, out, stats, kept):
     """The forward's tensors for the backward: the inputs, then the output and its row statistics if it left any.  `kept` is no saved
     tensor: it may be dropped before."""
-    ctx.save_for_backward(*inputs, *(() if stats is None else (out, stats)))
+    if stats is None:
+        ctx.save_for_backward(*inputs)
+    else:
+        ctx.save_for_backward(*inputs, out, stats)
     budget = _KEPT.get(out.device.index)
     ctx.kept = None if kept is None else budget.hold(kept)
-    ctx.turn = budget.turn if budget is not None else -1
+    ctx.turn = -1 if budget is None else budget.turn
 
 
 def _saved(ctx):
     """(inputs, what _monarch_bwd takes of the forward's)."""
     q, k, v, *left = ctx.saved_tensors
-    left = dict(zip(("out", "stats"), left))
+    out, stats = left or (None, None)
+    budget, kept = _KEPT.get(q.device.index), None
     if ctx.kept is not None:
-        left["kept"] = _KEPT[q.device.index].claim(ctx.kept)
-    elif q.device.index in _KEPT:
-        _KEPT[q.device.index].missed(ctx.turn)
-    if left.get("kept") is None:
-        _drop_kept(q.device.index)
-    return (q, k, v), left
+        kept = ctx.kept.budget.claim(ctx.kept)
+    elif budget is not None:
+        budget.missed(ctx.turn)
+    if kept is None and budget is not None:
+        budget.drop()
+    return (q, k, v), {"out": out, "stats": stats, "kept": kept}
 
 
 class _MonarchFn(torch.autograd.Function):
@@ -581,7 +578,8 @@ def monarch_attn_with_kv_cache(q, k_cache, v_cache, new_k, new_v, start_idx, end
     d = _desc(q, k_cache, v_cache, out, f_tied, h_reduce, w_reduce, h, w, sm_scale, 1, 0, num_iters, one_kernel)
     nbytes = monarch_workspace_bytes(d, heads_per_pass)
     ws = scratch(nbytes, q.device)
-    _drop_kept(q.device.index)
+    if _KEPT:
+        _drop_kept(q.device.index)
     with _on_device(q.device):
         _l.check(_l.load().sfm_monarch_attn_with_kv_cache(
             C.byref(d), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), new_k.data_ptr(), new_v.data_ptr(),
@@ -612,7 +610,8 @@ def monarch_attn_with_kv_cache_static(q, k_cache, v_cache, new_k, new_v, start_i
         if out.shape != q.shape:
             raise ValueError("out must have q's shape")
     d = _desc(q, k_cache, v_cache, out, f_tied, h_reduce, w_reduce, h, w, sm_scale, 1, 0, num_iters)
-    _drop_kept(q.device.index)
+    if _KEPT:
+        _drop_kept(q.device.index)
     with _on_device(q.device):
         _l.check(_l.load().sfm_monarch_attn_with_kv_cache_static(
             C.byref(d), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), new_k.data_ptr(), new_v.data_ptr(),

@@ -10,7 +10,7 @@ import math
 import torch
 
 from . import lib as _l
-from .monarch_attn import _DT, _drop_kept, _stream
+from .monarch_attn import _DT, _KEPT, _drop_kept, _stream
 
 
 def rope_table(head_dim, max_pos=1024, theta=10000.0, device=None):
@@ -63,7 +63,8 @@ def qk_prologue(xq, xk, xv, wq, wk, num_heads, grid, start_frame, rope, k_cache,
     d.cache_stride = _l.strides3(k_cache)
     d.cache_tokens = k_cache.shape[1]
     d.start_idx = start_idx
-    _drop_kept(xq.device.index)
+    if _KEPT:
+        _drop_kept(xq.device.index)
     with torch.cuda.device(xq.device):
         _l.check(_l.load().sfm_qk_prologue(
             C.byref(d), xq.data_ptr(), xk.data_ptr(), xv.data_ptr(), wq.contiguous().data_ptr(),
